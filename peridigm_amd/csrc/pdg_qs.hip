@@ -27,6 +27,7 @@
 
 #include "pdg_ctx.hpp"
 #include "pdg_device.hpp"
+#include "pdg_qs_tiles.hpp"
 
 namespace pdg {
 
@@ -45,6 +46,9 @@ struct QsState {
          *beta = nullptr, *theta = nullptr, *dtheta = nullptr, *g = nullptr, *out = nullptr,
          *dinv = nullptr;
   signed char* fixed = nullptr;  // 3n, 1 = prescribed DOF
+  // tiled passes: node records
+  f64x2* rec = nullptr;  // the arrays of QsRecords, 6n
+  double vol1 = 0.0;     // > 0: every node's volume
   // solver vectors (internal order, 3n)
   double *xs = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *b = nullptr,
          *part = nullptr, *scal = nullptr;
@@ -927,6 +931,9 @@ static int ensure(Ctx* c) {
     if (!rc) rc = A((void**)&S->qh[k], 24 * (size_t)N);
   }
   if (!rc) rc = A((void**)&S->fixed, 3 * (size_t)N);
+  if (!rc && c->ntiles > 0) rc = A((void**)&S->rec, 6 * sizeof(f64x2) * (size_t)N);
+  if (N > 0 && std::all_of(c->vol.begin(), c->vol.end(), [&](double v) { return v == c->vol[0]; }))
+    S->vol1 = std::max(c->vol[0], 0.0);
   if (rc) return rc;
   // constants in internal order
   std::vector<double> hx(3 * (size_t)N), hv(N), hm(N), ha(N), hb(N);
@@ -967,24 +974,56 @@ static int to_dev(Ctx* c, const double* h, double* d) {
 
 static int to_host(Ctx* c, const double* d, double* h) { return c->download_vec3(d, h); }
 
-// device u -> residual in S->out (internal order)
-static int residual(Ctx* c) {
-  QsArgs a = args(c);
-  hipStream_t s = c->stream;
-  qs_theta<false, false>(a, s);
-  qs_force<0>(a, s);
+static QsTileArgs tile_args(Ctx* c) {
+  QsState* S = c->qs;
+  QsTileArgs a{};
+  a.t = c->tile_args();
+  a.n = c->N; a.row = c->d_row; a.mw = c->d_mw; a.mask = c->d_mask; a.vol1 = S->vol1;
+  a.m = S->m; a.beta = S->beta; a.alpha = S->alpha; a.vol = S->vol; a.x = S->x; a.u = S->u;
+  a.L = c->L; a.hhat = c->horizon / c->L; a.influence = c->infl;
+  a.linear = c->material == PDG_MATERIAL_LINEAR_LPS;
+  a.dT = c->thermal() ? S->dT : nullptr;
+  a.alphaT = c->alpha_t;
+  a.fixed = S->fixed; a.theta = S->theta;
+  f64x2** const at[] = {&a.rec.xu[0], &a.rec.xu[1], &a.rec.xu[2], &a.rec.aq, &a.rec.wd[0], &a.rec.wd[1]};
+  for (int k = 0; k < 6; k++) *at[k] = S->rec + (size_t)k * c->N;
+  return a;
+}
+
+// theta at the device state S->u, with what the tangent's passes read there.
+static int state(Ctx* c) {
+  if (c->tiled())
+    return c->hip(launch_qs_state(tile_args(c), c->tile_lanes(), c->stream), "qs state");
+  qs_theta<false, false>(args(c), c->stream);
+  return c->hip(hipGetLastError(), "qs state");
+}
+
+// f V at the device state S->u into S->out (internal order); `all`: on the
+// prescribed DOFs too, which are 0 otherwise. Leaves theta in S->theta.
+static int residual(Ctx* c, bool all = false) {
+  int rc = state(c);
+  if (rc) return rc;
+  if (c->tiled())
+    return c->hip(launch_qs_residual(tile_args(c), all, c->qs->out, c->tile_lanes(), c->stream),
+                  "qs residual");
+  if (all) qs_force<2>(args(c), c->stream);
+  else qs_force<0>(args(c), c->stream);
   return c->hip(hipGetLastError(), "qs residual");
 }
 
-// K w for device w (S->w), output in `out`; needs theta at the current u
-static int tangent(Ctx* c, const double* w, double* out, bool theta_ready) {
-  QsArgs a = args(c);
-  a.w = w;
-  a.out = out;
+// K w for device w, output in `out`; needs state() at the current u
+static int tangent(Ctx* c, const double* w, double* out) {
   hipStream_t s = c->stream;
-  (void)theta_ready;  // the dual pass recomputes theta with its derivative
-  qs_theta<true, false>(a, s);
-  qs_force<1>(a, s);
+  if (c->tiled()) {
+    int rc = c->hip(launch_qs_tangent(tile_args(c), w, out, c->tile_lanes(), s), "qs tangent");
+    if (rc) return rc;
+  } else {
+    QsArgs a = args(c);
+    a.w = w;
+    a.out = out;
+    qs_theta<true, false>(a, s);
+    qs_force<1>(a, s);
+  }
   if (c->qs->damped) {
     const int n3 = 3 * c->N;
     hipLaunchKernelGGL(k_damp_add, dim3((n3 + RB - 1) / RB), dim3(RB), 0, s, n3, c->qs->dampv, w, out);
@@ -1085,6 +1124,7 @@ static int coarse_build(Ctx* c) {
   const int reach = std::max(1, (int)std::ceil((2.0 * G.H + 2.0 * bc) / G.H - 1e-12) - 1);
   const int stride = 2 * reach + 1;
   const int sc[3] = {std::min(stride, G.d[0]), std::min(stride, G.d[1]), std::min(stride, G.d[2])};
+  if ((rc = state(c))) return rc;
   std::vector<int> pcol;  // probe -> colour code (cx, cy, cz, k0)
   for (int cz = 0; cz < sc[2]; cz++)
     for (int cy = 0; cy < sc[1]; cy++)
@@ -1094,7 +1134,7 @@ static int coarse_build(Ctx* c) {
           pcol.push_back(((cz * sc[1] + cy) * sc[0] + cx) * 3 + k0);
           hipLaunchKernelGGL(k_coarse_probe, dim3(nb), dim3(RB), 0, s, N, G, stride, cx, cy, cz, k0,
                              S->x, S->fixed, S->z);
-          if ((rc = tangent(c, S->z, S->q, true))) return rc;
+          if ((rc = tangent(c, S->z, S->q))) return rc;
           hipLaunchKernelGGL(k_coarse_partial, dim3(np * kCoarseSplit), dim3(RB), 0, s, S->cstart,
                              S->clist, S->wlist, S->fixed, S->q, S->cpart);
           hipLaunchKernelGGL(k_coarse_finish<false>, dim3(1), dim3(RB), 0, s, nc, S->cpart, nullptr,
@@ -1213,12 +1253,8 @@ static int residual_norm(Ctx* c, double* norm) {
 // the Newton tolerance (src/core/Peridigm.cpp:2716-2732). Leaves S->out
 // holding f V on every DOF.
 static int reaction_norm(Ctx* c, double* norm) {
-  QsArgs a = args(c);
-  hipStream_t s = c->stream;
-  qs_theta<false, false>(a, s);
-  qs_force<2>(a, s);
   double ninf = 0.0;
-  int rc = c->hip(hipGetLastError(), "qs reactions");
+  int rc = residual(c, true);
   if (!rc) rc = norms(c, c->qs->out, c->qs->fixed, norm, &ninf);
   return rc;
 }
@@ -1239,7 +1275,7 @@ static void drop_graphs(Ctx* c) {
 
 }  // namespace qs
 
-int qs_tangent_apply(Ctx* c, const double* w, double* out) { return qs::tangent(c, w, out, true); }
+int qs_tangent_apply(Ctx* c, const double* w, double* out) { return qs::tangent(c, w, out); }
 int qs_dot(Ctx* c, const double* x, const double* y, double* out) { return qs::dot(c, x, y, out); }
 
 double* Ctx::qs_dinv() { return qs ? qs->dinv : nullptr; }
@@ -1249,6 +1285,7 @@ int pdg_qs_prepare(Ctx* c, const double* u) {
   int rc = qs::ensure(c);
   if (!rc) rc = qs::to_dev(c, u, c->qs->u);
   if (!rc) rc = qs::block_jacobi(c);
+  if (!rc) rc = qs::state(c);
   return rc;
 }
 
@@ -1273,6 +1310,7 @@ void Ctx::free_extra() {
     }
     qs::drop_graphs(this);
     if (S->fixed) (void)hipFree(S->fixed);
+    if (S->rec) (void)hipFree(S->rec);
     if (S->hscal) (void)hipHostFree(S->hscal);
     delete S;
     qs = nullptr;
@@ -1339,7 +1377,8 @@ int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int ma
   // r = b - K x; z = M r; p = z
   int cur = 0;  // flexible CG: history slot of the current direction
   double* p = flexible ? S->ph[0] : S->p;
-  if ((rc = qs::tangent(c, x, S->q, false))) return rc;
+  if ((rc = qs::state(c))) return rc;
+  if ((rc = qs::tangent(c, x, S->q))) return rc;
   hipLaunchKernelGGL(k_sub, dim3(vb), blk, 0, s, n3, b, S->q, S->r);
   rc = c->hip(hipMemsetAsync(S->scal, 0, 8 * kScal, s), "zero scalars");
   if (!rc) rc = precond_apply(S->r, S->z);
@@ -1373,7 +1412,7 @@ int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int ma
   auto seq_a = [&](int cs, bool rr) -> int {
     double* pp = flexible ? S->ph[cs] : S->p;
     double* qq = flexible ? S->qh[cs] : S->q;
-    int r2 = qs::tangent(c, pp, qq, true);
+    int r2 = qs::tangent(c, pp, qq);
     if (r2) return r2;
     double* rrp = S->part;  // r.r partials
     if (flexible) {
@@ -1559,7 +1598,8 @@ int pdg_qs_tangent_apply(pdg_ctx* h, const double* u, const double* w, double* K
   int rc = qs::ensure(c);
   if (!rc) rc = qs::to_dev(c, u, c->qs->u);
   if (!rc) rc = qs::to_dev(c, w, c->qs->w);
-  if (!rc) rc = qs::tangent(c, c->qs->w, c->qs->out, false);
+  if (!rc) rc = qs::state(c);
+  if (!rc) rc = qs::tangent(c, c->qs->w, c->qs->out);
   if (!rc) rc = qs::to_host(c, c->qs->out, Kw);
   return rc;
 }
@@ -1678,11 +1718,8 @@ int pdg_qs_force_dilatation(pdg_ctx* h, const double* u, double* force, double* 
   QsState* S = c->qs;
   if (!rc) rc = qs::to_dev(c, u, S->u);
   if (rc) return rc;
-  QsArgs a = qs::args(c);
   hipStream_t s = c->stream;
-  qs_theta<false, false>(a, s);
-  qs_force<2>(a, s);
-  rc = c->hip(hipGetLastError(), "qs force");
+  rc = qs::residual(c, true);
   if (!rc) rc = qs::to_host(c, S->out, force);
   if (rc) return rc;
   for (int p = 0; p < c->N; p++)

@@ -1,0 +1,446 @@
+// LDS-tiled FP64 bond passes of the quasi-static path: dilatation, residual
+// force, and the tangent's two passes (derivative of the dilatation, then of
+// the force) over the Hilbert tiles of the explicit path.
+//
+// One workgroup owns a tile: it stages its halo's records in LDS as arrays of
+// 16-byte slots, and groups of G lanes own the tile's nodes. Lanes reading
+// distinct residues of 16 halo slots, which the tiles' bond order provides,
+// meet distinct LDS banks, as in the explicit passes.
+//
+// The untiled kernels gather 80 to 112 bytes a bond through L1 and L2 and are
+// bound by those gathers' latency; here HBM and L2 see each halo record once
+// per tile and a 2-byte index a bond. Bound by FP64 issue (about 70
+// instructions a bond in the tangent's force pass) and, on small meshes, by
+// the launch and the two rounds of loads before the bond loop. One tangent
+// product, dilatation + force pass, against the untiled kernels:
+//   3,000-node bar:     6.0 + 6.6 us   (9.5 + 10.5)
+//   24,000-node bar:   11.0 + 14.0 us  (32 + 41)
+//   200,000-node bar:  55 + 77 us      (223 + 313)
+// Records as one 80- to 112-byte structure a node instead of arrays measured
+// 61 + 125 us on the last (each lane's load then touches a line of its own,
+// and 112 bytes leave one workgroup to a CU in the force pass).
+//
+// Bond arithmetic, in units of L: X = x_j - x_i, D = u_j - u_i, Y = X + D.
+// One reciprocal square root t = 1/sqrt(|X|^2 |Y|^2) gives both quantities
+// that the formulas need,
+//   g = zeta/|Y| = |X|^2 t   and   1/|Y|^2 = g t,
+// where the untiled kernels take two square roots and a division. With
+// q = beta theta (less the thermal term), a = alpha_i + alpha_j and
+// S = T/|Y| = w [(q_i + q_j) g + a e/|Y|]:
+//   d theta_i = 3/m_i sum w V_j g Y.dY,
+//   df_i = sum V_j ([w g (dq_i + dq_j) + (w a - S) (Y.dY)/|Y|^2] Y + S dY).
+// e/|Y| is 1 - g in the tangent, where it is a geometric term of the order of
+// the strain, and (|Y|^2 - |X|^2)/|Y|^2 / (1 + g) in the residual, with
+// |Y|^2 - |X|^2 = D.(2X + D), which has no cancellation.
+
+#include <algorithm>
+
+#include "pdg_device.hpp"
+#include "pdg_qs_tiles.hpp"
+
+namespace pdg {
+namespace {
+
+using namespace dev;
+
+constexpr int WG = kTileThreads;
+
+__device__ __forceinline__ int tile_of_block(int bid, int ntiles) {
+  const int per = (ntiles + 7) >> 3;  // a contiguous run of tiles per XCD
+  return (bid & 7) * per + (bid >> 3);
+}
+inline unsigned tile_blocks(int ntiles) { return 8u * (unsigned)((ntiles + 7) >> 3); }
+
+// 1/sqrt(a) and 1/a from the hardware estimates (relative error below 2^-20)
+// and one third-order step, which cubes that error.
+__device__ __forceinline__ double rsqrt64(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  const double e = fma(-(a * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double rcp64(double a) {
+  const double r = __builtin_amdgcn_rcp(a);
+  const double e = fma(-a, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+
+// Influence function of a bond with squared length z2 (lengths in units of
+// L). The reciprocals depend on the horizon alone, so they leave the loops.
+template <int INFL>
+__device__ __forceinline__ double omega64(double z2, double hhat) {
+  if (INFL == PDG_INFLUENCE_ONE) return 1.0;
+  if (INFL == PDG_INFLUENCE_PARABOLIC_DECAY) {
+    const double zeta = sqrt(z2);
+    if (zeta > hhat) return 0.0;
+    const double s = zeta * (1.0 / hhat);
+    return s < 0.5 ? 1.0 : -4.0 * s * s + 4.0 * s;
+  }
+  return exp(z2 * (-1.0 / (hhat * hhat * 0.4 * 0.4)));
+}
+
+template <int G, int HV>
+__device__ __forceinline__ double lanes_sum(double v) {
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if (HV == 2) v += __shfl_xor(v, 16);
+  return v;
+}
+
+// What a pass does with a bond.
+enum { QP_THETA, QP_DTHETA, QP_FORCE, QP_DFORCE };
+
+// LDS arrays of a pass, 16-byte slots of one halo node each, at compile-time
+// distances (one byte offset addresses all of them): xu[0..2], then
+//   QP_THETA   (V, -)
+//   QP_DTHETA  (w0, w1), (w2, V)
+//   QP_FORCE   (alpha, q), (V, -)
+//   QP_DFORCE  (alpha, q), (w0, w1), (w2, dq), and an array of V unless every
+//              node has the same.
+constexpr int HS = kTileHaloMax;
+template <int PASS>
+constexpr int units() { return PASS == QP_THETA ? 4 : PASS == QP_DFORCE ? 6 : 5; }
+template <int PASS, bool UNIV>
+constexpr int lds_bytes() { return 16 * HS * units<PASS>() + (PASS == QP_DFORCE && !UNIV ? 8 * HS : 0); }
+
+// Workgroups of 512 threads, two to a CU (at most 80 KB of LDS each). The
+// tangent's force pass with a volume array takes 83 KB: one workgroup to a CU
+// then, of 1,024 threads, each node's bonds shared by two lane groups.
+template <int PASS, bool UNIV>
+constexpr int halves() { return lds_bytes<PASS, UNIV>() > 81920 ? 2 : 1; }
+
+// A halo node's record in registers.
+template <int PASS>
+struct Rec {
+  f64x2 v[units<PASS>()];
+  double vj;  // QP_DFORCE: V
+  __device__ double x(int c) const { return c == 0 ? v[0].x : c == 1 ? v[0].y : v[1].x; }
+  __device__ double u(int c) const { return c == 0 ? v[1].y : c == 1 ? v[2].x : v[2].y; }
+  __device__ double vol() const {
+    return PASS == QP_THETA ? v[3].x : PASS == QP_DTHETA ? v[units<PASS>() - 1].y
+           : PASS == QP_FORCE ? v[units<PASS>() - 1].x : vj;
+  }
+  __device__ double alpha() const { return v[3].x; }  // force passes
+  __device__ double q() const { return v[3].y; }      // force passes
+  __device__ double w(int c) const {                  // tangent passes
+    constexpr int k = units<PASS>() - 2;
+    return c == 0 ? v[k].x : c == 1 ? v[k].y : v[k + 1].x;
+  }
+  __device__ double dq() const { return v[units<PASS>() - 1].y; }
+};
+
+template <int PASS, bool UNIV>
+__device__ __forceinline__ void rec_read(Rec<PASS>& r, const char* lds, int jb, double vol1) {
+#pragma unroll
+  for (int k = 0; k < units<PASS>(); k++)
+    r.v[k] = *reinterpret_cast<const f64x2*>(lds + 16 * HS * k + jb);
+  if (PASS == QP_DFORCE)
+    r.vj = UNIV ? vol1 : *reinterpret_cast<const double*>(lds + 16 * HS * units<PASS>() + (jb >> 1));
+}
+
+// One bond of a pass: the sums of the lane (one for the dilatation passes,
+// three for the force passes).
+template <int PASS, int INFL, bool LIN>
+__device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, double hhat,
+                                     double thermal, double (&b)[3]) {
+  const double X0 = nb.x(0) - me.x(0), X1 = nb.x(1) - me.x(1), X2 = nb.x(2) - me.x(2);
+  const double z2 = fma(X2, X2, fma(X1, X1, X0 * X0));
+  const double om = omega64<INFL>(z2, hhat);
+  double d0 = 0.0, d1 = 0.0, d2 = 0.0;
+  if (PASS == QP_DTHETA || PASS == QP_DFORCE) {
+    d0 = nb.w(0) - me.w(0); d1 = nb.w(1) - me.w(1); d2 = nb.w(2) - me.w(2);
+  }
+  const double D0 = nb.u(0) - me.u(0), D1 = nb.u(1) - me.u(1), D2 = nb.u(2) - me.u(2);
+  if (LIN) {
+    // theta and force linear in u, the force along the reference bond
+    const bool dual = PASS == QP_DTHETA || PASS == QP_DFORCE;
+    const double pr = fma(X2, dual ? d2 : D2, fma(X1, dual ? d1 : D1, X0 * (dual ? d0 : D0)));
+    if (PASS == QP_THETA || PASS == QP_DTHETA) {
+      b[0] = om * nb.vol() * pr;
+    } else {
+      const double qs = PASS == QP_FORCE ? me.q() + nb.q() : me.dq() + nb.dq();
+      const double t = om * nb.vol() * fma(me.alpha() + nb.alpha(), pr * rcp64(z2), qs);
+      b[0] = t * X0; b[1] = t * X1; b[2] = t * X2;
+    }
+    return;
+  }
+  const double Y0 = X0 + D0, Y1 = X1 + D1, Y2 = X2 + D2;
+  const double yy = fma(Y2, Y2, fma(Y1, Y1, Y0 * Y0));
+  const double t = rsqrt64(z2 * yy);
+  double g = z2 * t, ryy = g * t;
+  if (z2 == 0.0) {  // points that coincide in the reference configuration
+    g = 0.0;
+    ryy = rcp64(yy);
+  }
+  if (PASS == QP_THETA) {
+    const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
+    b[0] = om * nb.vol() * (dd * g * rcp64(1.0 + g) - thermal * z2);
+  } else if (PASS == QP_DTHETA) {
+    b[0] = om * nb.vol() * g * fma(Y2, d2, fma(Y1, d1, Y0 * d0));
+  } else if (PASS == QP_FORCE) {
+    const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
+    const double ey = dd * ryy * rcp64(1.0 + g);
+    const double s = om * nb.vol() * fma(me.alpha() + nb.alpha(), ey, (me.q() + nb.q()) * g);
+    b[0] = s * Y0; b[1] = s * Y1; b[2] = s * Y2;
+  } else {
+    const double a = me.alpha() + nb.alpha();
+    const double S = om * fma(a, 1.0 - g, (me.q() + nb.q()) * g);
+    const double yd = fma(Y2, d2, fma(Y1, d1, Y0 * d0));
+    const double c = fma(om * g, me.dq() + nb.dq(), (om * a - S) * (yd * ryy)) * nb.vol();
+    const double sv = S * nb.vol();
+    b[0] = fma(sv, d0, c * Y0);
+    b[1] = fma(sv, d1, c * Y1);
+    b[2] = fma(sv, d2, c * Y2);
+  }
+}
+
+// What the pass writes, besides what QsTileArgs holds.
+struct QsOut {
+  const double* w;  // QP_DTHETA: the direction, 3n
+  double* out;      // force passes: 3n
+  int all;          // QP_FORCE: prescribed DOFs too
+};
+
+// A node group's row: CSR range, then the lane's intact bits (two words,
+// shifted down by the lane; bits past the row's end clear) and the local
+// indices of its first round.
+template <int U>
+struct Row {
+  int rs, deg, mw;
+  unsigned long long in[2];
+  int lj[U];
+};
+
+template <int U>
+__device__ __forceinline__ void row_range(const QsTileArgs& a, int node, int n0, int n1, Row<U>& r) {
+  const unsigned nd = (unsigned)(node < n1 ? node : n0);
+  r.rs = a.row[nd];
+  const int re = a.row[nd + 1u];
+  r.mw = a.mw[nd];
+  r.deg = node < n1 ? re - r.rs : 0;
+}
+
+template <int GB, int U>
+__device__ __forceinline__ void row_data(const QsTileArgs& a, int l, Row<U>& r) {
+  const unsigned long long* mp = a.mask + (unsigned)r.mw;
+  const unsigned short* lp = a.t.lcol + (unsigned)(r.rs + l);
+#pragma unroll
+  for (int k = 0; k < U; k++) r.lj[k] = lp[k * GB];
+#pragma unroll
+  for (int w = 0; w < 2; w++) {
+    const int left = r.deg - 64 * w;
+    const unsigned long long vb = left >= 64 ? ~0ull : (left <= 0 ? 0ull : (1ull << left) - 1ull);
+    r.in[w] = (~mp[w] & vb) >> l;
+  }
+}
+
+// What a pass stages of halo node i.
+template <int PASS, bool UNIV>
+__device__ __forceinline__ void slot_load(const QsTileArgs& a, const QsOut& o, unsigned i,
+                                          Rec<PASS>& r) {
+#pragma unroll
+  for (int k = 0; k < 3; k++) r.v[k] = a.rec.xu[k][i];
+  if (PASS == QP_FORCE || PASS == QP_DFORCE) r.v[3] = a.rec.aq[i];
+  if (PASS == QP_DTHETA) {
+    const double* w = o.w + 3u * i;
+    r.v[units<PASS>() - 2] = f64x2{w[0], w[1]};
+    r.v[units<PASS>() - 1] = f64x2{w[2], a.vol[i]};
+  } else if (PASS == QP_DFORCE) {
+    r.v[units<PASS>() - 2] = a.rec.wd[0][i];
+    r.v[units<PASS>() - 1] = a.rec.wd[1][i];
+    if (!UNIV) r.vj = a.vol[i];
+  } else {
+    r.v[units<PASS>() - 1] = f64x2{a.vol[i], 0.0};
+  }
+}
+
+template <int PASS, bool UNIV>
+__device__ __forceinline__ void slot_store(char* lds, int h, const Rec<PASS>& r) {
+#pragma unroll
+  for (int k = 0; k < units<PASS>(); k++)
+    *reinterpret_cast<f64x2*>(lds + 16 * (HS * k + h)) = r.v[k];
+  if (PASS == QP_DFORCE && !UNIV)
+    *reinterpret_cast<double*>(lds + 16 * HS * units<PASS>() + 8 * h) = r.vj;
+}
+
+// One pass over one tile. A node has HV groups of G lanes; group h's lane l
+// takes bonds h G + l, + HV G, ... in the tile's bond order, U of them per
+// round so that their LDS reads and the next round's local indices are in
+// flight together (two groups of a node sit in neighbouring 16-lane rows, so
+// each row still reads what the bond order made conflict-free). Bonds past
+// the row's end and broken bonds are computed like the others and selected
+// away: a local index past the row's end belongs to a later row or the zero
+// padding, so it addresses a slot of the arrays.
+// U = 4 in the force pass of the tangent took 77.3 us against 78.9 with 2 and
+// 82.4 with 1 on the 200,000-node bar; in the others 4 spills registers and 2
+// is as fast.
+template <int G, int PASS, bool UNIV, int INFL, bool LIN>
+__global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTileArgs a, QsOut o) {
+  constexpr int HV = halves<PASS, UNIV>();
+  constexpr int U = PASS == QP_DFORCE && HV == 1 && INFL == PDG_INFLUENCE_ONE ? 4 : 2;
+  __shared__ __align__(16) char lds[lds_bytes<PASS, UNIV>()];
+  constexpr int NG = WG / G;
+  constexpr int T = WG * HV;
+  constexpr int GB = G * HV;  // bonds of a node per step
+  constexpr int kHaloRounds = (kTileHaloMax + T - 1) / T;
+  const int tile = tile_of_block(blockIdx.x, a.t.ntiles);
+  if (tile >= a.t.ntiles) return;
+  const int n0 = a.t.tile_start[tile], n1 = a.t.tile_start[tile + 1];
+  const int h0 = a.t.halo_off[tile], hn = min(a.t.halo_off[tile + 1] - h0, HS);
+  const int own = a.t.own_off[tile];
+  const int l = (threadIdx.x & (G - 1)) + (HV == 2 ? ((threadIdx.x >> 4) & 1) * G : 0);
+  const int grp = HV == 2 ? (threadIdx.x >> 5) * (16 / G) + (threadIdx.x & 15) / G : threadIdx.x / G;
+  // Two phases of loads, each in flight together: the halo's node ids and the
+  // first round's CSR ranges, then the records, mask words and local indices
+  // they address. All unconditional (a thread without a slot or a node reads
+  // the tile's first).
+  int idx[kHaloRounds];
+#pragma unroll
+  for (int r = 0; r < kHaloRounds; r++) {
+    const int h = threadIdx.x + r * T;
+    idx[r] = a.t.halo[(unsigned)(h0 + (h < hn ? h : 0))];
+  }
+  Row<U> rw;
+  row_range(a, n0 + grp, n0, n1, rw);
+  row_data<GB, U>(a, l, rw);
+#pragma unroll
+  for (int r = 0; r < kHaloRounds; r++) {
+    if (r > 0 && r * T >= hn) break;
+    Rec<PASS> v;
+    slot_load<PASS, UNIV>(a, o, (unsigned)idx[r], v);
+    const int h = threadIdx.x + r * T;
+    if (h < hn) slot_store<PASS, UNIV>(lds, h, v);
+  }
+  __syncthreads();
+  for (int base = n0; base < n1; base += NG) {
+    const int node = base + grp;
+    const bool valid = node < n1;
+    const int nd = valid ? node : n0;
+    if (base != n0) {
+      row_range(a, node, n0, n1, rw);
+      row_data<GB, U>(a, l, rw);
+    }
+    const int deg = rw.deg;
+    const unsigned short* lp = a.t.lcol + (unsigned)(rw.rs + l);
+    Rec<PASS> me;
+    rec_read<PASS, UNIV>(me, lds, kLdsSlot * (own + (nd - n0)), a.vol1);
+    double thermal = 0.0;
+    if (PASS == QP_THETA && a.dT) thermal = a.alphaT * a.dT[(unsigned)nd];
+    // nodes of a tile are ordered by descending degree: the wave's first
+    // group has the largest
+    const int rounds = (__builtin_amdgcn_readfirstlane(deg) + GB * U - 1) / (GB * U);
+    double s[3] = {0.0, 0.0, 0.0};
+    int (&lj)[U] = rw.lj;
+    for (int c = 0; c < rounds; c++) {
+      int ln[U];
+      const unsigned short* np = lp + min(c + 1, rounds - 1) * (GB * U);
+#pragma unroll
+      for (int k = 0; k < U; k++) ln[k] = np[k * GB];
+      const int b0 = c * (GB * U);
+      const unsigned long long bits = (b0 < 64 ? rw.in[0] : rw.in[1]) >> (b0 & 63);
+#pragma unroll
+      for (int k = 0; k < U; k++) {
+        Rec<PASS> nb;
+        rec_read<PASS, UNIV>(nb, lds, lj[k], a.vol1);
+        double b[3] = {0.0, 0.0, 0.0};
+        bond<PASS, INFL, LIN>(me, nb, a.hhat, thermal, b);
+        const bool ok = (bits >> (k * GB)) & 1ull;
+#pragma unroll
+        for (int d = 0; d < (PASS == QP_FORCE || PASS == QP_DFORCE ? 3 : 1); d++)
+          s[d] = ok ? s[d] + b[d] : s[d];
+      }
+#pragma unroll
+      for (int k = 0; k < U; k++) lj[k] = ln[k];
+    }
+    if (PASS == QP_THETA || PASS == QP_DTHETA) {
+      const double sum = lanes_sum<G, HV>(s[0]);
+      if (!valid || l != 0) continue;
+      const double m = a.m[(unsigned)node];
+      const double c = m > 0.0 ? 3.0 / m : 0.0;
+      if (PASS == QP_THETA) {
+        const double th = c * (a.L * a.L) * sum;
+        a.theta[(unsigned)node] = th;
+        double q = a.beta[(unsigned)node] * th;
+        if (a.dT) q -= thermal * a.alpha[(unsigned)node];
+        a.rec.aq[(unsigned)node].y = q;
+      } else {
+        const double dq = a.L * (a.beta[(unsigned)node] * (c * a.L * sum));
+        a.rec.wd[0][(unsigned)node] = f64x2{me.w(0), me.w(1)};
+        a.rec.wd[1][(unsigned)node] = f64x2{me.w(2), dq};
+      }
+    } else {
+      const double f0 = lanes_sum<G, HV>(s[0]), f1 = lanes_sum<G, HV>(s[1]), f2 = lanes_sum<G, HV>(s[2]);
+      if (!valid || l >= 3) continue;
+      const double f = (l == 0 ? f0 : (l == 1 ? f1 : f2)) * me.vol();
+      const unsigned q = 3u * (unsigned)node + (unsigned)l;
+      const bool fx = a.fixed[q] != 0;
+      if (PASS == QP_FORCE) o.out[q] = fx && !o.all ? 0.0 : a.L * f;
+      else o.out[q] = fx ? (l == 0 ? me.w(0) : (l == 1 ? me.w(1) : me.w(2))) : -f;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_qs_pack(QsTileArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.n) return;
+  const double iL = 1.0 / a.L;  // exact
+  const double* x = a.x + 3 * (size_t)i;
+  const double* u = a.u + 3 * (size_t)i;
+  a.rec.xu[0][i] = f64x2{x[0] * iL, x[1] * iL};
+  a.rec.xu[1][i] = f64x2{x[2] * iL, u[0] * iL};
+  a.rec.xu[2][i] = f64x2{u[1] * iL, u[2] * iL};
+  a.rec.aq[i] = f64x2{a.alpha[i], 0.0};
+}
+
+// G lanes per node: at least enough that one round covers a tile, and at most
+// 16, the width of the LDS service groups that the bond order is made for
+// (wider settings run as 16 and loop over the tile's nodes).
+template <int PASS, bool UNIV, int INFL, bool LIN>
+hipError_t launch_g(const QsTileArgs& a, const QsOut& o, int lanes, hipStream_t s) {
+  const dim3 grid(tile_blocks(a.t.ntiles)), blk(WG * halves<PASS, UNIV>());
+  if (lanes <= 4) hipLaunchKernelGGL((k_qs_tile<4, PASS, UNIV, INFL, LIN>), grid, blk, 0, s, a, o);
+  else if (lanes == 8) hipLaunchKernelGGL((k_qs_tile<8, PASS, UNIV, INFL, LIN>), grid, blk, 0, s, a, o);
+  else hipLaunchKernelGGL((k_qs_tile<16, PASS, UNIV, INFL, LIN>), grid, blk, 0, s, a, o);
+  return hipGetLastError();
+}
+
+template <int PASS, int INFL, bool LIN>
+hipError_t launch_v(const QsTileArgs& a, const QsOut& o, int lanes, hipStream_t s) {
+  if (PASS == QP_DFORCE && a.vol1 > 0.0) return launch_g<PASS, PASS == QP_DFORCE, INFL, LIN>(a, o, lanes, s);
+  return launch_g<PASS, false, INFL, LIN>(a, o, lanes, s);
+}
+
+template <int PASS>
+hipError_t launch(const QsTileArgs& a, const QsOut& o, int lanes, hipStream_t s) {
+  if (a.t.ntiles <= 0) return hipErrorInvalidValue;
+  if (a.influence == PDG_INFLUENCE_ONE)
+    return a.linear ? launch_v<PASS, 0, true>(a, o, lanes, s) : launch_v<PASS, 0, false>(a, o, lanes, s);
+  if (a.influence == PDG_INFLUENCE_PARABOLIC_DECAY)
+    return a.linear ? launch_v<PASS, 1, true>(a, o, lanes, s) : launch_v<PASS, 1, false>(a, o, lanes, s);
+  return a.linear ? launch_v<PASS, 2, true>(a, o, lanes, s) : launch_v<PASS, 2, false>(a, o, lanes, s);
+}
+
+}  // namespace
+
+hipError_t launch_qs_state(const QsTileArgs& a, int lanes, hipStream_t s) {
+  hipLaunchKernelGGL(k_qs_pack, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a);
+  return launch<QP_THETA>(a, QsOut{}, lanes, s);
+}
+
+hipError_t launch_qs_residual(const QsTileArgs& a, bool all, double* out, int lanes,
+                              hipStream_t s) {
+  QsOut o{};
+  o.out = out;
+  o.all = all ? 1 : 0;
+  return launch<QP_FORCE>(a, o, lanes, s);
+}
+
+hipError_t launch_qs_tangent(const QsTileArgs& a, const double* w, double* out, int lanes,
+                             hipStream_t s) {
+  QsOut o{};
+  o.w = w;
+  o.out = out;
+  hipError_t e = launch<QP_DTHETA>(a, o, lanes, s);
+  return e == hipSuccess ? launch<QP_DFORCE>(a, o, lanes, s) : e;
+}
+
+}  // namespace pdg
