@@ -47,7 +47,7 @@ struct QsState {
          *dinv = nullptr;
   signed char* fixed = nullptr;  // 3n, 1 = prescribed DOF
   // tiled passes: node records
-  f64x2* rec = nullptr;  // the arrays of QsRecords, 6n
+  f64x2* rec = nullptr;  // the arrays of QsRecords, 8n
   double vol1 = 0.0;     // > 0: every node's volume
   // solver vectors (internal order, 3n)
   double *xs = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *b = nullptr,
@@ -57,13 +57,24 @@ struct QsState {
   double* qh[4] = {};
   int nblk = 0;
   double* hscal = nullptr;  // pinned host copy of the solver scalars
+  // conjugate gradients: scalars on the device, their pinned set-up copy and
+  // status, partial sums of r.z and r.r (kCgParts each) and p.Kp, and an event
+  // per chunk of iterations in flight
+  QsCg* cg = nullptr;
+  QsCg* hcg = nullptr;
+  QsCgStatus* hstat = nullptr;
+  double *rz_part = nullptr, *rr_part = nullptr, *pq_part = nullptr;
+  hipEvent_t cev[2] = {nullptr, nullptr};
   bool graphs = false;      // replay the CG iteration sequences as HIP graphs
-  // captured iteration sequences, per preconditioner, sequence (A, B) and
-  // flexible-CG history slot; valid for the x and b vectors and the network
-  // buffers they were captured with
-  hipGraphExec_t gexec[3][2][4] = {};
+  // captured launch sequences: a chunk of CG iterations per preconditioner,
+  // and the flexible iteration's two sequences (A, B) per history slot; valid
+  // for the x and b vectors, the kernel variant and the network buffers they
+  // were captured with
+  hipGraphExec_t gchunk[2] = {};
+  hipGraphExec_t gexec[2][4] = {};
   const double* gx = nullptr;
   const double* gb = nullptr;
+  bool gtiled = false;
   unsigned gepoch = 0;
   int fallbacks = 0;  // learned-preconditioner solves handed over to block-Jacobi CG
   std::vector<signed char> hfixed;
@@ -109,6 +120,7 @@ constexpr int kQsWideNodes = 100000;
 constexpr int kScal = 32;   // solver scalar slots on the device
 constexpr int kFcgSlots = 4;  // flexible CG keeps kFcgSlots - 1 previous directions
 constexpr int RB = 256; // reduction block
+constexpr int kCgParts = 512;  // most workgroups of the CG update (partial sums a value)
 
 __device__ __forceinline__ double infl64(int kind, double zeta, double horizon) {
   if (kind == PDG_INFLUENCE_ONE) return 1.0;
@@ -424,78 +436,85 @@ __global__ __launch_bounds__(RB) void k_final(int nb, const double* part, int st
   }
 }
 
-// z = Dinv r (block) on 3-vectors of nodes
-__global__ __launch_bounds__(RB) void k_block_apply(int n, const double* dinv, const double* r, double* z) {
-  const int i = blockIdx.x * RB + threadIdx.x;
-  if (i >= n) return;
-  const double* D = dinv + 9 * i;
-  const double r0 = r[3 * i], r1 = r[3 * i + 1], r2 = r[3 * i + 2];
-  z[3 * i] = D[0] * r0 + D[1] * r1 + D[2] * r2;
-  z[3 * i + 1] = D[3] * r0 + D[4] * r1 + D[5] * r2;
-  z[3 * i + 2] = D[6] * r0 + D[7] * r1 + D[8] * r2;
-}
-
-// z = Dinv r and partial sums of r.z in one pass (grid-stride over nodes, one
-// partial per block, like k_dot)
-__global__ __launch_bounds__(RB) void k_block_apply_dot(int n, const double* dinv, const double* r,
-                                                        double* z, double* part) {
-  __shared__ double sh[RB / 64];
-  double s = 0.0;
-  for (int i = blockIdx.x * RB + threadIdx.x; i < n; i += gridDim.x * RB) {
-    const double* D = dinv + 9 * i;
-    const double r0 = r[3 * i], r1 = r[3 * i + 1], r2 = r[3 * i + 2];
-    const double z0 = D[0] * r0 + D[1] * r1 + D[2] * r2;
-    const double z1 = D[3] * r0 + D[4] * r1 + D[5] * r2;
-    const double z2 = D[6] * r0 + D[7] * r1 + D[8] * r2;
-    z[3 * i] = z0;
-    z[3 * i + 1] = z1;
-    z[3 * i + 2] = z2;
-    s += r0 * z0 + r1 * z1 + r2 * z2;
+// Conjugate-gradient update of one iteration: al = r.z / p.Kp (p.Kp from its
+// npq partial sums, al = 0 after a breakdown), x += al p, r -= al q, then
+// z = Dinv r (PREC 1; z is r itself without a preconditioner, and formed later
+// by the two-level one) and the partial sums of r.z and r.r, a node per thread
+// (grid-stride). With INIT: r = b - q and the same sums. One pass over the
+// vectors in place of five kernels (dot, step, reduction, preconditioner with
+// its dot, direction); 24,000-node bar: 5.4 us, where those took 17.
+struct CgVecs {
+  const f64x2 *p0, *p1;  // tiled: the direction's records
+  const double* p;       // untiled: the direction
+  const double *q, *b, *dinv;
+  double *x, *r, *z;
+};
+template <int T, int PREC, bool INIT>
+__global__ __launch_bounds__(T) void k_cg_update(int n, QsCg* cg, int npq, const double* pq_part,
+                                                 CgVecs v, double* rz_part, double* rr_part) {
+  __shared__ double sh[2 * T / 64];
+  double al = 0.0;
+  if (!INIT) {
+    if (cg->done) return;
+    double pq = 0.0, none = 0.0;
+    for (int i = threadIdx.x; i < npq; i += T) pq += pq_part[i];
+    block_sum2<T>(pq, none, sh);
+    al = pq > 0.0 ? cg->rz / pq : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      if (!(pq > 0.0)) cg->brk = 1;
+      cg->it = cg->it + 1;
+    }
   }
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-// x += al p; r -= al q; partial sums of r.r
-// Solver scalars kept on the device (slots of `sc`), so a CG iteration needs
-// no host round trip: RZ = r.z, PQ = p.Kp, RR = r.r, RZN = new r.z, ZQ = z.Kp,
-// BETA, BRK = 1 after a breakdown (p.Kp <= 0).
-enum { SC_RZ = 0, SC_PQ = 1, SC_RR = 2, SC_RZN = 3, SC_ZQ = 4, SC_BETA = 5, SC_BRK = 6 };
-// flexible CG: PR = p.r, then per history slot k: PQH + k = p_k.Kp_k, ZQH + k = z.Kp_k
-enum { SC_PR = 7, SC_PQH = 8, SC_ZQH = 12 };
-
-// x += al p, r -= al q, partial sums of r.r (into rr_part); al = RZ / PQ (0
-// after a breakdown), PQ summed from the partials of k_dot (pq_part)
-__global__ __launch_bounds__(RB) void k_cg_step(int n, int nb, double* sc, const double* pq_part,
-                                                const double* p, const double* q, double* x,
-                                                double* r, double* rr_part) {
-  // p.Kp from k_dot's partials, summed by every block in k_final's order (so
-  // the same value); block 0 stores it for the breakdown test
-  __shared__ double sh[RB / 64];
-  __shared__ double pq_s;
-  double t = 0.0;
-  for (int i = threadIdx.x; i < nb; i += RB) t += pq_part[i];
-  t = block_sum(t, sh);
+  double rz = 0.0, rr = 0.0;
+  for (int i = blockIdx.x * T + threadIdx.x; i < n; i += gridDim.x * T) {
+    double r[3], z[3];
+    if (INIT) {
+      for (int c = 0; c < 3; c++) r[c] = v.b[3 * i + c] - v.q[3 * i + c];
+    } else {
+      double p[3];
+      if (v.p) {
+        for (int c = 0; c < 3; c++) p[c] = v.p[3 * i + c];
+      } else {
+        const f64x2 a = v.p0[i];
+        p[0] = a.x; p[1] = a.y; p[2] = v.p1[i].x;
+      }
+      for (int c = 0; c < 3; c++) {
+        v.x[3 * i + c] += al * p[c];
+        r[c] = v.r[3 * i + c] - al * v.q[3 * i + c];
+      }
+    }
+    for (int c = 0; c < 3; c++) v.r[3 * i + c] = r[c];
+    if (PREC == 1) {
+      const double* D = v.dinv + 9 * (size_t)i;
+      for (int c = 0; c < 3; c++) z[c] = D[3 * c] * r[0] + D[3 * c + 1] * r[1] + D[3 * c + 2] * r[2];
+      for (int c = 0; c < 3; c++) v.z[3 * i + c] = z[c];
+      rz += r[0] * z[0] + r[1] * z[1] + r[2] * z[2];
+    }
+    rr += r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+  }
+  if (PREC == 0) rz = rr;
+  block_sum2<T>(rz, rr, sh);
   if (threadIdx.x == 0) {
-    pq_s = t;
-    if (blockIdx.x == 0) sc[SC_PQ] = t;
+    if (PREC != 3) rz_part[blockIdx.x] = rz;
+    rr_part[blockIdx.x] = rr;
   }
-  __syncthreads();
-  const double pq = pq_s;
-  // r.z of this iteration is in RZN (from k_cg_dir or the set-up); block 0
-  // moves it to RZ for the next direction's beta (no block reads RZ here)
-  const double al = pq > 0.0 ? sc[SC_RZN] / pq : 0.0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) sc[SC_RZ] = sc[SC_RZN];
-  double s = 0.0;
-  for (int i = blockIdx.x * RB + threadIdx.x; i < n; i += gridDim.x * RB) {
-    x[i] += al * p[i];
-    const double ri = r[i] - al * q[i];
-    r[i] = ri;
-    s += ri * ri;
-  }
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) rr_part[blockIdx.x] = s;
 }
+
+// Direction of an iteration on an untiled mesh: p = z + beta p.
+__global__ __launch_bounds__(RB) void k_cg_dir(int n, QsCgStart s, const double* z, double* p) {
+  __shared__ double sh[2 * RB / 64];
+  if (s.cg->done) return;
+  double beta;
+  if (cg_start<RB>(s, sh, beta)) return;
+  for (int i = blockIdx.x * RB + threadIdx.x; i < n; i += gridDim.x * RB)
+    p[i] = beta != 0.0 ? z[i] + beta * p[i] : z[i];
+}
+
+// Solver scalars of flexible CG kept on the device (slots of `sc`), so an
+// iteration needs no host round trip: RR = r.r, BRK = 1 after a breakdown
+// (p.Kp <= 0), PR = p.r, then per history slot k: PQH + k = p_k.Kp_k,
+// ZQH + k = z.Kp_k
+enum { SC_RR = 2, SC_BRK = 6, SC_PR = 7, SC_PQH = 8, SC_ZQH = 12 };
 
 __global__ __launch_bounds__(RB) void k_fcg_step(int n, double* sc, int slot, const double* p,
                                                  const double* q, double* x, double* r,
@@ -533,33 +552,6 @@ __global__ __launch_bounds__(RB) void k_fcg_dir(int n, const double* sc, const d
     v -= c * h.p[k][i];
   }
   pnew[i] = v;
-}
-
-// p = z + beta p
-// p = z + beta p with beta = RZN / RZ (grid-stride, launched with as many
-// blocks as there are partials): every block sums the r.z partials
-// (rz_part) in the order of a single-block reduction; block 0 stores the sum
-// in RZN (read by the next step; no block reads RZN here), BETA, and the
-// breakdown flag
-__global__ __launch_bounds__(RB) void k_cg_dir(int n, int nb, double* sc, const double* rz_part,
-                                               const double* z, double* p) {
-  __shared__ double sh[RB / 64];
-  __shared__ double beta_s;
-  double t = 0.0;
-  for (int i = threadIdx.x; i < nb; i += RB) t += rz_part[i];
-  t = block_sum(t, sh);
-  if (threadIdx.x == 0) {
-    const double beta = t / sc[SC_RZ];
-    beta_s = beta;
-    if (blockIdx.x == 0) {
-      sc[SC_RZN] = t;
-      sc[SC_BETA] = beta;
-      if (!(sc[SC_PQ] > 0.0)) sc[SC_BRK] = 1.0;
-    }
-  }
-  __syncthreads();
-  const double beta = beta_s;
-  for (int i = blockIdx.x * RB + threadIdx.x; i < n; i += gridDim.x * RB) p[i] = z[i] + beta * p[i];
 }
 
 __global__ __launch_bounds__(RB) void k_axpby(int n, double a, const double* x, double b, double* y) {
@@ -781,8 +773,7 @@ __global__ __launch_bounds__(RB) void k_coarse_cells(int n, CoarseGrid G, const 
 }
 
 // z = Dinv r + P y (the two-level preconditioner), with the partial sums of
-// r.z when DOT (grid-stride over nodes, one partial per block, like k_dot)
-template <bool DOT>
+// r.z (grid-stride over nodes, one partial per block, like k_dot)
 __global__ __launch_bounds__(RB) void k_two_level_apply(int n, const double* __restrict__ dinv,
                                                         CoarseGrid G, const double* __restrict__ x,
                                                         const signed char* __restrict__ fixed,
@@ -810,12 +801,10 @@ __global__ __launch_bounds__(RB) void k_two_level_apply(int n, const double* __r
     z[3 * i] = z0;
     z[3 * i + 1] = z1;
     z[3 * i + 2] = z2;
-    if (DOT) s += r0 * z0 + r1 * z1 + r2 * z2;
+    s += r0 * z0 + r1 * z1 + r2 * z2;
   }
-  if (DOT) {
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
-  }
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 __global__ __launch_bounds__(RB) void k_zero_fixed(int n, const signed char* fixed, double* v) {
@@ -926,12 +915,20 @@ static int ensure(Ctx* c) {
   if (!rc) rc = A((void**)&S->part, 8 * (size_t)S->nblk * 2);
   if (!rc) rc = A((void**)&S->scal, 8 * kScal);
   if (!rc) rc = c->hip(hipHostMalloc((void**)&S->hscal, 8 * kScal, hipHostMallocDefault), "pinned alloc");
+  if (!rc) rc = A((void**)&S->cg, sizeof(QsCg));
+  if (!rc) rc = A((void**)&S->rz_part, 8 * (size_t)std::max(kCgParts, S->nblk));
+  if (!rc) rc = A((void**)&S->rr_part, 8 * (size_t)kCgParts);
+  if (!rc) rc = A((void**)&S->pq_part, 8 * (size_t)std::max(c->ntiles, S->nblk));
+  if (!rc) rc = c->hip(hipHostMalloc((void**)&S->hcg, sizeof(QsCg), hipHostMallocDefault), "pinned alloc");
+  if (!rc) rc = c->hip(hipHostMalloc((void**)&S->hstat, sizeof(QsCgStatus), hipHostMallocCoherent), "pinned alloc");
+  for (hipEvent_t& e : S->cev)
+    if (!rc) rc = c->hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
   for (int k = 0; k < 4 && !rc; k++) {
     rc = A((void**)&S->ph[k], 24 * (size_t)N);
     if (!rc) rc = A((void**)&S->qh[k], 24 * (size_t)N);
   }
   if (!rc) rc = A((void**)&S->fixed, 3 * (size_t)N);
-  if (!rc && c->ntiles > 0) rc = A((void**)&S->rec, 6 * sizeof(f64x2) * (size_t)N);
+  if (!rc && c->ntiles > 0) rc = A((void**)&S->rec, 8 * sizeof(f64x2) * (size_t)N);
   if (N > 0 && std::all_of(c->vol.begin(), c->vol.end(), [&](double v) { return v == c->vol[0]; }))
     S->vol1 = std::max(c->vol[0], 0.0);
   if (rc) return rc;
@@ -985,8 +982,10 @@ static QsTileArgs tile_args(Ctx* c) {
   a.dT = c->thermal() ? S->dT : nullptr;
   a.alphaT = c->alpha_t;
   a.fixed = S->fixed; a.theta = S->theta;
-  f64x2** const at[] = {&a.rec.xu[0], &a.rec.xu[1], &a.rec.xu[2], &a.rec.aq, &a.rec.wd[0], &a.rec.wd[1]};
-  for (int k = 0; k < 6; k++) *at[k] = S->rec + (size_t)k * c->N;
+  a.damp = S->damped ? S->dampv : nullptr;
+  f64x2** const at[] = {&a.rec.xu[0], &a.rec.xu[1], &a.rec.xu[2], &a.rec.aq,
+                        &a.rec.wd[0], &a.rec.wd[1], &a.rec.wp[0], &a.rec.wp[1]};
+  for (int k = 0; k < 8; k++) *at[k] = S->rec + (size_t)k * c->N;
   return a;
 }
 
@@ -1014,16 +1013,13 @@ static int residual(Ctx* c, bool all = false) {
 // K w for device w, output in `out`; needs state() at the current u
 static int tangent(Ctx* c, const double* w, double* out) {
   hipStream_t s = c->stream;
-  if (c->tiled()) {
-    int rc = c->hip(launch_qs_tangent(tile_args(c), w, out, c->tile_lanes(), s), "qs tangent");
-    if (rc) return rc;
-  } else {
-    QsArgs a = args(c);
-    a.w = w;
-    a.out = out;
-    qs_theta<true, false>(a, s);
-    qs_force<1>(a, s);
-  }
+  if (c->tiled())
+    return c->hip(launch_qs_tangent(tile_args(c), w, out, c->tile_lanes(), s), "qs tangent");
+  QsArgs a = args(c);
+  a.w = w;
+  a.out = out;
+  qs_theta<true, false>(a, s);
+  qs_force<1>(a, s);
   if (c->qs->damped) {
     const int n3 = 3 * c->N;
     hipLaunchKernelGGL(k_damp_add, dim3((n3 + RB - 1) / RB), dim3(RB), 0, s, n3, c->qs->dampv, w, out);
@@ -1264,13 +1260,17 @@ static void drop_graphs(Ctx* c) {
   QsState* S = c->qs;
   if (!S) return;
   bool any = false;
-  for (auto& a : S->gexec) for (auto& b : a) for (hipGraphExec_t g : b) any = any || g;
+  auto each = [&](auto&& f) {
+    for (hipGraphExec_t& g : S->gchunk) f(g);
+    for (auto& a : S->gexec) for (hipGraphExec_t& g : a) f(g);
+  };
+  each([&](hipGraphExec_t& g) { any = any || g; });
   if (!any) return;
   (void)hipStreamSynchronize(c->stream);
-  for (auto& a : S->gexec)
-    for (auto& b : a)
-      for (hipGraphExec_t& g : b)
-        if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
+  each([&](hipGraphExec_t& g) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  });
 }
 
 }  // namespace qs
@@ -1311,6 +1311,11 @@ void Ctx::free_extra() {
     qs::drop_graphs(this);
     if (S->fixed) (void)hipFree(S->fixed);
     if (S->rec) (void)hipFree(S->rec);
+    void* gptrs[] = {S->cg, S->rz_part, S->rr_part, S->pq_part};
+    for (void* p : gptrs) if (p) (void)hipFree(p);
+    if (S->hcg) (void)hipHostFree(S->hcg);
+    if (S->hstat) (void)hipHostFree(S->hstat);
+    for (hipEvent_t e : S->cev) if (e) (void)hipEventDestroy(e);
     if (S->hscal) (void)hipHostFree(S->hscal);
     delete S;
     qs = nullptr;
@@ -1319,24 +1324,157 @@ void Ctx::free_extra() {
   free_contact();  // sized by the topology and horizon
 }
 
+namespace qs {
+
+// Captures what `body` launches on the context's stream as a graph.
+template <class F>
+static int capture(Ctx* c, hipGraphExec_t* out, F&& body) {
+  hipGraph_t g = nullptr;
+  int r2 = c->hip(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "begin capture");
+  if (r2) return r2;
+  const int rb = body();
+  const hipError_t e = hipStreamEndCapture(c->stream, &g);
+  if (rb) { if (g) (void)hipGraphDestroy(g); return rb; }
+  r2 = c->hip(e, "end capture");
+  if (!r2) r2 = c->hip(hipGraphInstantiate(out, g, nullptr, nullptr, 0), "instantiate");
+  if (g) (void)hipGraphDestroy(g);
+  return r2;
+}
+
+// Preconditioned CG from the initial guess x (precond 0, 1 or 3). An iteration
+// is three kernels on a tiled mesh: direction with the dilatation pass, force
+// pass with p.Kp, update with the preconditioner (which the two-level one
+// follows with its coarse part). The decision to stop is made on the device,
+// so the host runs ahead: it launches chunks of kCgChunk iterations, each
+// followed by a wait for that chunk's first product only, and launches left
+// over after the end return at once. (Waiting for a copy of the residual at
+// every look left the GPU idle for about 15 us each time.)
+constexpr int kCgChunk = 4;  // even: the directions alternate between two buffers
+
+static int cg_solve(Ctx* c, double* x, const double* b, double bnorm, int precond, double tol,
+                    int maxit, int* iters, double* rel) {
+  QsState* S = c->qs;
+  const int N = c->N, n3 = 3 * N;
+  hipStream_t s = c->stream;
+  const bool tiled = c->tiled(), wide = N > 65536;
+  const int T = wide ? 256 : 128;
+  const int nup = std::max(1, std::min(kCgParts, (N + T - 1) / T));
+  const int npq = tiled ? c->ntiles : S->nblk;
+  const int nrz = precond == 3 ? S->nblk : nup;
+  double* const z = precond == 0 ? S->r : S->z;
+  // the tile arguments of even and odd iterations
+  QsTileArgs ta[2];
+  if (tiled) {
+    ta[0] = ta[1] = tile_args(c);
+    std::swap(ta[1].rec.wd, ta[1].rec.wp);
+  }
+  auto update = [&](int k, bool init) -> int {
+    CgVecs v{};
+    if (tiled) { v.p0 = ta[k & 1].rec.wd[0]; v.p1 = ta[k & 1].rec.wd[1]; }
+    else v.p = S->p;
+    v.q = S->q; v.b = b; v.dinv = S->dinv; v.x = x; v.r = S->r; v.z = S->z;
+    auto go = [&](auto fn) {
+      hipLaunchKernelGGL(fn, dim3(nup), dim3(T), 0, s, N, S->cg, npq, S->pq_part, v, S->rz_part, S->rr_part);
+    };
+    if (precond == 1) {
+      if (init) wide ? go(k_cg_update<256, 1, true>) : go(k_cg_update<128, 1, true>);
+      else wide ? go(k_cg_update<256, 1, false>) : go(k_cg_update<128, 1, false>);
+    } else if (precond == 3) {
+      if (init) wide ? go(k_cg_update<256, 3, true>) : go(k_cg_update<128, 3, true>);
+      else wide ? go(k_cg_update<256, 3, false>) : go(k_cg_update<128, 3, false>);
+      hipLaunchKernelGGL(k_coarse_partial, dim3(S->cgr.points() * kCoarseSplit), dim3(RB), 0, s,
+                         S->cstart, S->clist, S->wlist, S->fixed, S->r, S->cpart);
+      hipLaunchKernelGGL(k_coarse_finish<true>, dim3((S->nc + RB / 64 - 1) / (RB / 64)), dim3(RB),
+                         0, s, S->nc, S->cpart, S->cinv, S->cy);
+      hipLaunchKernelGGL(k_two_level_apply, dim3(S->nblk), dim3(RB), 0, s, N, S->dinv, S->cgr,
+                         S->x, S->fixed, S->cy, S->r, S->z, S->rz_part);
+    } else {
+      if (init) wide ? go(k_cg_update<256, 0, true>) : go(k_cg_update<128, 0, true>);
+      else wide ? go(k_cg_update<256, 0, false>) : go(k_cg_update<128, 0, false>);
+    }
+    return c->hip(hipGetLastError(), "cg update");
+  };
+  const QsCgStart start{S->cg, S->rz_part, S->rr_part, nrz, nup, S->hstat};
+  // iteration k's direction and product
+  auto product = [&](int k) -> int {
+    if (tiled)
+      return c->hip(launch_qs_tangent_cg(ta[k & 1], start, z, S->q, S->pq_part, c->tile_lanes(), s),
+                    "cg product");
+    hipLaunchKernelGGL(k_cg_dir, dim3(S->nblk), dim3(RB), 0, s, n3, start, z, S->p);
+    int r2 = tangent(c, S->p, S->q);
+    if (r2) return r2;
+    hipLaunchKernelGGL(k_dot, dim3(S->nblk), dim3(RB), 0, s, n3, S->p, S->q, S->pq_part);
+    return c->hip(hipGetLastError(), "cg product");
+  };
+  int rc = tangent(c, x, S->q);
+  *S->hcg = QsCg{};
+  S->hcg->maxit = maxit;
+  S->hcg->bnorm = bnorm;
+  S->hcg->tol = tol;
+  *S->hstat = QsCgStatus{};
+  if (!rc) rc = c->hip(hipMemcpyAsync(S->cg, S->hcg, sizeof(QsCg), hipMemcpyHostToDevice, s), "h2d");
+  if (!rc) rc = update(0, true);
+  if (rc) return rc;
+  // the damped tangent and the two-level preconditioner run without graphs
+  const bool graphs = S->graphs && !S->damped && precond < 3;
+  if (graphs && (S->gx != x || S->gb != b || S->gtiled != tiled)) {
+    drop_graphs(c);
+    S->gx = x; S->gb = b; S->gtiled = tiled;
+  }
+  volatile const QsCgStatus* st = S->hstat;
+  for (int chunk = 0; !st->done; chunk++) {
+    if (chunk > std::max(maxit, 0) / kCgChunk + 2) return c->fail(PDG_E_HIP, "CG did not report its end");
+    hipEvent_t ev = S->cev[chunk & 1];
+    if (graphs) {
+      hipGraphExec_t* g = &S->gchunk[precond];
+      auto body = [&]() -> int {
+        int r2 = 0;
+        for (int k = 0; k < kCgChunk && !r2; k++) {
+          r2 = product(k);
+          if (!r2) r2 = update(k, false);
+        }
+        return r2;
+      };
+      if (!*g) rc = capture(c, g, body);
+      if (!rc) rc = c->hip(hipGraphLaunch(*g, s), "graph launch");
+      if (!rc) rc = c->hip(hipEventRecord(ev, s), "event");
+      if (!rc && chunk > 0) rc = c->hip(hipEventSynchronize(S->cev[(chunk - 1) & 1]), "sync");
+    } else {
+      for (int k = 0; k < kCgChunk && !rc; k++) {
+        rc = product(k);
+        if (!rc && k == 0) rc = c->hip(hipEventRecord(ev, s), "event");
+        if (!rc) rc = update(k, false);
+      }
+      if (!rc) rc = c->hip(hipEventSynchronize(ev), "sync");
+    }
+    if (rc) return rc;
+  }
+  if (st->brk) return c->fail(PDG_E_NOCONV, "CG breakdown: p.Kp <= 0");
+  const double relres = std::sqrt(st->rr) / bnorm;
+  *iters = st->it;
+  *rel = relres;
+  if (relres > tol) return c->fail(PDG_E_NOCONV, "linear solve did not converge");
+  return PDG_OK;
+}
+
+}  // namespace qs
+
 // K x = b on device vectors in internal order; x holds the initial guess.
 // Returns iterations in *iters, the final relative residual in *rel.
 // Preconditioned CG (precond 0: none, 1: block Jacobi, 3: block Jacobi plus
-// the coarse correction, built by coarse_build) or, for the learned
-// preconditioner (precond 2), Notay's flexible CG truncated to the last
-// kFcgSlots - 1 directions: the new direction is z minus its K-projections on
-// them, alpha = p.r / p.Kp. Scalars stay on the device; the host reads the
-// residual norm at checks only: every iteration for the first 8, then every 4
-// (a solve may run up to 3 iterations past the tolerance).
+// the coarse correction, built by coarse_build; qs::cg_solve) or, for the
+// learned preconditioner (precond 2), Notay's flexible CG truncated to the
+// last kFcgSlots - 1 directions: the new direction is z minus its
+// K-projections on them, alpha = p.r / p.Kp. Scalars stay on the device. The
+// residual is looked at every iteration for the first 8, then every 4 (a
+// solve may run up to 3 iterations past the tolerance).
 int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int maxit, int* iters,
              double* rel) {
   QsState* S = c->qs;
   const int n3 = 3 * c->N;
   hipStream_t s = c->stream;
   const unsigned vb = (unsigned)((n3 + RB - 1) / RB);
-  const unsigned nb = (unsigned)((c->N + RB - 1) / RB);
   const dim3 red(S->nblk), blk(RB);
-  const bool flexible = precond == 2;
   int rc = 0;
   double bb = 0.0;
   if ((rc = qs::dot(c, b, b, &bb))) return rc;
@@ -1347,44 +1485,21 @@ int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int ma
     *rel = 0.0;
     return rc;
   }
+  if ((rc = qs::state(c))) return rc;
+  if (precond != 2) return qs::cg_solve(c, x, b, bnorm, precond, tol, maxit, iters, rel);
   // device dot product into scalar slot k
   auto ddot = [&](const double* u, const double* v, int k) {
     hipLaunchKernelGGL(k_dot, red, blk, 0, s, n3, u, v, S->part);
     hipLaunchKernelGGL(k_final, dim3(1), blk, 0, s, S->nblk, S->part, 1, S->scal + k);
   };
-  // coarse part of the two-level preconditioner: y = A_c^-1 P^T r
-  auto coarse = [&](const double* r) -> int {
-    hipLaunchKernelGGL(k_coarse_partial, dim3(S->cgr.points() * kCoarseSplit), blk, 0, s,
-                       S->cstart, S->clist, S->wlist, S->fixed, r, S->cpart);
-    hipLaunchKernelGGL(k_coarse_finish<true>, dim3((S->nc + RB / 64 - 1) / (RB / 64)), blk, 0, s,
-                       S->nc, S->cpart, S->cinv, S->cy);
-    return c->hip(hipGetLastError(), "coarse solve");
-  };
-  auto precond_apply = [&](const double* r, double* z) -> int {
-    if (precond == 2) return gnn_apply(c, r, z);
-    if (precond == 3) {
-      int r2 = coarse(r);
-      if (!r2) hipLaunchKernelGGL((k_two_level_apply<false>), dim3(nb), blk, 0, s, c->N, S->dinv,
-                                  S->cgr, S->x, S->fixed, S->cy, r, z, nullptr);
-      return r2 ? r2 : c->hip(hipGetLastError(), "two-level apply");
-    }
-    if (precond == 1) {
-      hipLaunchKernelGGL(k_block_apply, dim3(nb), blk, 0, s, c->N, S->dinv, r, z);
-      return c->hip(hipGetLastError(), "block apply");
-    }
-    return c->hip(hipMemcpyAsync(z, r, 8 * (size_t)n3, hipMemcpyDeviceToDevice, s), "copy");
-  };
   // r = b - K x; z = M r; p = z
-  int cur = 0;  // flexible CG: history slot of the current direction
-  double* p = flexible ? S->ph[0] : S->p;
-  if ((rc = qs::state(c))) return rc;
+  int cur = 0;  // history slot of the current direction
   if ((rc = qs::tangent(c, x, S->q))) return rc;
   hipLaunchKernelGGL(k_sub, dim3(vb), blk, 0, s, n3, b, S->q, S->r);
   rc = c->hip(hipMemsetAsync(S->scal, 0, 8 * kScal, s), "zero scalars");
-  if (!rc) rc = precond_apply(S->r, S->z);
-  if (!rc) rc = c->hip(hipMemcpyAsync(p, S->z, 8 * (size_t)n3, hipMemcpyDeviceToDevice, s), "copy");
+  if (!rc) rc = gnn_apply(c, S->r, S->z);
+  if (!rc) rc = c->hip(hipMemcpyAsync(S->ph[0], S->z, 8 * (size_t)n3, hipMemcpyDeviceToDevice, s), "copy");
   if (rc) return rc;
-  ddot(S->r, S->z, SC_RZN);  // r.z of the first iteration (read by k_cg_step)
   ddot(S->r, S->r, SC_RR);
   auto check = [&](double* relres, bool* brk) -> int {
     int r2 = c->hip(hipMemcpyAsync(S->hscal, S->scal, 8 * kScal, hipMemcpyDeviceToHost, s), "d2h");
@@ -1403,98 +1518,60 @@ int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int ma
   bool stalled = false;
   // The iteration is two fixed launch sequences: A (K p, p.Kp, step, r.r)
   // and B (preconditioner, dots, new direction), split by the host check.
-  // For flexible CG both depend on the history slot `cur`; once the history
-  // is full (nhist = kFcgSlots - 1) they are the same every time that slot
-  // comes round. With graphs on, each (preconditioner, sequence, slot) is
-  // captured once (kept in the solver state until its vectors or the
-  // network's buffers change) and replayed.
+  // Both depend on the history slot `cur`; once the history is full (nhist =
+  // kFcgSlots - 1) they are the same every time that slot comes round. With
+  // graphs on, each (sequence, slot) is captured once (kept in the solver
+  // state until its vectors or the network's buffers change) and replayed.
   // rr: also reduce r.r to its slot (needed only where the host checks it)
   auto seq_a = [&](int cs, bool rr) -> int {
-    double* pp = flexible ? S->ph[cs] : S->p;
-    double* qq = flexible ? S->qh[cs] : S->q;
+    double* pp = S->ph[cs];
+    double* qq = S->qh[cs];
     int r2 = qs::tangent(c, pp, qq);
     if (r2) return r2;
-    double* rrp = S->part;  // r.r partials
-    if (flexible) {
-      ddot(pp, qq, SC_PQH + cs);
-      ddot(pp, S->r, SC_PR);
-      hipLaunchKernelGGL(k_fcg_step, red, blk, 0, s, n3, S->scal, cs, pp, qq, x, S->r, S->part);
-    } else {
-      hipLaunchKernelGGL(k_dot, red, blk, 0, s, n3, pp, qq, S->part);
-      rrp = S->part + S->nblk;
-      hipLaunchKernelGGL(k_cg_step, red, blk, 0, s, n3, S->nblk, S->scal, S->part, pp, qq, x, S->r,
-                         rrp);
-    }
-    if (rr) hipLaunchKernelGGL(k_final, dim3(1), blk, 0, s, S->nblk, rrp, 1, S->scal + SC_RR);
+    ddot(pp, qq, SC_PQH + cs);
+    ddot(pp, S->r, SC_PR);
+    hipLaunchKernelGGL(k_fcg_step, red, blk, 0, s, n3, S->scal, cs, pp, qq, x, S->r, S->part);
+    if (rr) hipLaunchKernelGGL(k_final, dim3(1), blk, 0, s, S->nblk, S->part, 1, S->scal + SC_RR);
     return c->hip(hipGetLastError(), "cg step");
   };
   auto seq_b = [&](int cs, int nh) -> int {
-    int r2 = 0;
-    if (flexible) {
-      r2 = precond_apply(S->r, S->z);
-    } else if (precond == 1) {
-      // z = Dinv r with the r.z partials in the same pass
-      hipLaunchKernelGGL(k_block_apply_dot, red, blk, 0, s, c->N, S->dinv, S->r, S->z, S->part);
-    } else if (precond == 3) {
-      r2 = coarse(S->r);
-      if (!r2) hipLaunchKernelGGL((k_two_level_apply<true>), red, blk, 0, s, c->N, S->dinv, S->cgr,
-                                  S->x, S->fixed, S->cy, S->r, S->z, S->part);
-    } else {
-      r2 = precond_apply(S->r, S->z);
-      if (!r2) hipLaunchKernelGGL(k_dot, red, blk, 0, s, n3, S->r, S->z, S->part);
-    }
+    int r2 = gnn_apply(c, S->r, S->z);
     if (r2) return r2;
-    if (flexible) {
-      FcgHist h{};
-      h.nh = nh;
-      for (int k = 0; k < nh; k++) {
-        const int slot = (cs - k + kFcgSlots) % kFcgSlots;
-        h.p[k] = S->ph[slot];
-        h.slot[k] = slot;
-        ddot(S->z, S->qh[slot], SC_ZQH + slot);
-      }
-      hipLaunchKernelGGL(k_fcg_dir, dim3(vb), blk, 0, s, n3, S->scal, S->z, h,
-                         S->ph[(cs + 1) % kFcgSlots]);
-    } else {
-      hipLaunchKernelGGL(k_cg_dir, red, blk, 0, s, n3, S->nblk, S->scal, S->part, S->z, S->p);
+    FcgHist h{};
+    h.nh = nh;
+    for (int k = 0; k < nh; k++) {
+      const int slot = (cs - k + kFcgSlots) % kFcgSlots;
+      h.p[k] = S->ph[slot];
+      h.slot[k] = slot;
+      ddot(S->z, S->qh[slot], SC_ZQH + slot);
     }
+    hipLaunchKernelGGL(k_fcg_dir, dim3(vb), blk, 0, s, n3, S->scal, S->z, h,
+                       S->ph[(cs + 1) % kFcgSlots]);
     return c->hip(hipGetLastError(), "cg direction");
   };
-  // the damped tangent adds a launch: no graphs while damping
-  const bool graphs = S->graphs && !S->damped && precond < 3;
+  // the damped tangent of an untiled mesh adds a launch: no graphs while damping
+  const bool graphs = S->graphs && !S->damped;
   // graphs captured for other vectors or older network buffers are stale
-  if (graphs && (S->gx != x || S->gb != b || (flexible && S->gepoch != c->gnn_epoch))) {
+  if (graphs && (S->gx != x || S->gb != b || S->gtiled != c->tiled() || S->gepoch != c->gnn_epoch)) {
     qs::drop_graphs(c);
-    S->gx = x; S->gb = b; S->gepoch = c->gnn_epoch;
+    S->gx = x; S->gb = b; S->gtiled = c->tiled(); S->gepoch = c->gnn_epoch;
   }
-  hipGraphExec_t* ga = S->gexec[std::min(precond, 2)][0];
-  hipGraphExec_t* gb = S->gexec[std::min(precond, 2)][1];
-  auto capture = [&](hipGraphExec_t* out, auto&& body) -> int {
-    hipGraph_t g = nullptr;
-    int r2 = c->hip(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
-    if (r2) return r2;
-    const int rb = body();
-    const hipError_t e = hipStreamEndCapture(s, &g);
-    if (rb) { if (g) (void)hipGraphDestroy(g); return rb; }
-    r2 = c->hip(e, "end capture");
-    if (!r2) r2 = c->hip(hipGraphInstantiate(out, g, nullptr, nullptr, 0), "instantiate");
-    if (g) (void)hipGraphDestroy(g);
-    return r2;
-  };
   // runs sequence A or B for slot cs: replayed from a graph when the history
   // is full and graphs are on, otherwise launched directly
   auto run_a = [&](int cs, bool full, bool rr) -> int {
     if (!graphs || !full) return seq_a(cs, rr);
     // a captured sequence is replayed before every check: it reduces r.r
-    if (!ga[cs]) { int r2 = capture(&ga[cs], [&]() { return seq_a(cs, true); }); if (r2) return r2; }
-    return c->hip(hipGraphLaunch(ga[cs], s), "graph launch");
+    hipGraphExec_t& g = S->gexec[0][cs];
+    if (!g) { int r2 = qs::capture(c, &g, [&]() { return seq_a(cs, true); }); if (r2) return r2; }
+    return c->hip(hipGraphLaunch(g, s), "graph launch");
   };
   auto run_b = [&](int cs, int nh, bool full) -> int {
     if (!graphs || !full) return seq_b(cs, nh);
-    if (!gb[cs]) { int r2 = capture(&gb[cs], [&]() { return seq_b(cs, nh); }); if (r2) return r2; }
-    return c->hip(hipGraphLaunch(gb[cs], s), "graph launch");
+    hipGraphExec_t& g = S->gexec[1][cs];
+    if (!g) { int r2 = qs::capture(c, &g, [&]() { return seq_b(cs, nh); }); if (r2) return r2; }
+    return c->hip(hipGraphLaunch(g, s), "graph launch");
   };
-  const int hist_full = flexible ? kFcgSlots - 1 : 0;
+  const int hist_full = kFcgSlots - 1;
   // the host checks the residual after iterations 1-8, every fourth, and the last
   auto checked = [&](int k) { return k <= 8 || k % 4 == 0 || k == maxit; };
   while (relres > tol && it < maxit) {
@@ -1504,19 +1581,15 @@ int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int ma
       if ((rc = check(&relres, &brk))) return rc;
       if (brk) return c->fail(PDG_E_NOCONV, "CG breakdown: p.Kp <= 0");
       if (relres <= tol) break;
-      if (flexible && it % 48 == 0) {
+      if (it % 48 == 0) {
         if (!(relres < 0.5 * watch)) { stalled = true; break; }
         watch = relres;
       }
     }
-    if (flexible) {
-      const int nh = std::min(nhist + 1, kFcgSlots - 1);
-      if ((rc = run_b(cur, nh, nh >= hist_full && nhist >= hist_full))) return rc;
-      nhist = nh;
-      cur = (cur + 1) % kFcgSlots;
-    } else {
-      if ((rc = run_b(0, 0, true))) return rc;
-    }
+    const int nh = std::min(nhist + 1, kFcgSlots - 1);
+    if ((rc = run_b(cur, nh, nh >= hist_full && nhist >= hist_full))) return rc;
+    nhist = nh;
+    cur = (cur + 1) % kFcgSlots;
   }
   if (!stalled && relres > tol) {
     if ((rc = check(&relres, &brk))) return rc;

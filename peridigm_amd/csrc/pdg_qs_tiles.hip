@@ -10,12 +10,12 @@
 // The untiled kernels gather 80 to 112 bytes a bond through L1 and L2 and are
 // bound by those gathers' latency; here HBM and L2 see each halo record once
 // per tile and a 2-byte index a bond. Bound by FP64 issue (about 70
-// instructions a bond in the tangent's force pass) and, on small meshes, by
+// instructions a bond in the tangent's force pass), LDS reads and, on small meshes, by
 // the launch and the two rounds of loads before the bond loop. One tangent
 // product, dilatation + force pass, against the untiled kernels:
-//   3,000-node bar:     6.0 + 6.6 us   (9.5 + 10.5)
-//   24,000-node bar:   11.0 + 14.0 us  (32 + 41)
-//   200,000-node bar:  55 + 77 us      (223 + 313)
+//   3,000-node bar:     5.9 + 6.5 us   (9.5 + 10.5)
+//   24,000-node bar:   11.0 + 13.3 us  (32 + 41)
+//   200,000-node bar:  57 + 76 us      (223 + 313)
 // Records as one 80- to 112-byte structure a node instead of arrays measured
 // 61 + 125 us on the last (each lane's load then touches a line of its own,
 // and 112 bytes leave one workgroup to a CU in the force pass).
@@ -78,21 +78,27 @@ __device__ __forceinline__ double omega64(double z2, double hhat) {
   return exp(z2 * (-1.0 / (hhat * hhat * 0.4 * 0.4)));
 }
 
+// Sum over a node's lanes: its group of G, and with two groups a node the one
+// in the neighbouring row of 16.
 template <int G, int HV>
 __device__ __forceinline__ double lanes_sum(double v) {
-#pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  v = group_sum64<G>(v);
   if (HV == 2) v += __shfl_xor(v, 16);
   return v;
 }
 
-// What a pass does with a bond.
-enum { QP_THETA, QP_DTHETA, QP_FORCE, QP_DFORCE };
+// What a pass does with a bond. QP_CG is QP_DTHETA with a direction that the
+// staging forms.
+enum { QP_THETA, QP_DTHETA, QP_FORCE, QP_DFORCE, QP_CG };
+template <int PASS>
+constexpr bool is_dtheta() { return PASS == QP_DTHETA || PASS == QP_CG; }
+template <int PASS>
+constexpr bool is_dual() { return is_dtheta<PASS>() || PASS == QP_DFORCE; }
 
 // LDS arrays of a pass, 16-byte slots of one halo node each, at compile-time
 // distances (one byte offset addresses all of them): xu[0..2], then
 //   QP_THETA   (V, -)
-//   QP_DTHETA  (w0, w1), (w2, V)
+//   QP_DTHETA, QP_CG  (w0, w1), (w2, V)
 //   QP_FORCE   (alpha, q), (V, -)
 //   QP_DFORCE  (alpha, q), (w0, w1), (w2, dq), and an array of V unless every
 //              node has the same.
@@ -116,7 +122,7 @@ struct Rec {
   __device__ double x(int c) const { return c == 0 ? v[0].x : c == 1 ? v[0].y : v[1].x; }
   __device__ double u(int c) const { return c == 0 ? v[1].y : c == 1 ? v[2].x : v[2].y; }
   __device__ double vol() const {
-    return PASS == QP_THETA ? v[3].x : PASS == QP_DTHETA ? v[units<PASS>() - 1].y
+    return PASS == QP_THETA ? v[3].x : is_dtheta<PASS>() ? v[units<PASS>() - 1].y
            : PASS == QP_FORCE ? v[units<PASS>() - 1].x : vj;
   }
   __device__ double alpha() const { return v[3].x; }  // force passes
@@ -129,37 +135,48 @@ struct Rec {
 };
 
 template <int PASS, bool UNIV>
-__device__ __forceinline__ void rec_read(Rec<PASS>& r, const char* lds, int jb, double vol1) {
+__device__ __forceinline__ void rec_read(Rec<PASS>& r, const char* lds, int jb) {
 #pragma unroll
   for (int k = 0; k < units<PASS>(); k++)
     r.v[k] = *reinterpret_cast<const f64x2*>(lds + 16 * HS * k + jb);
-  if (PASS == QP_DFORCE)
-    r.vj = UNIV ? vol1 : *reinterpret_cast<const double*>(lds + 16 * HS * units<PASS>() + (jb >> 1));
+  if (PASS == QP_DFORCE && !UNIV)
+    r.vj = *reinterpret_cast<const double*>(lds + 16 * HS * units<PASS>() + (jb >> 1));
 }
 
-// One bond of a pass: the sums of the lane (one for the dilatation passes,
-// three for the force passes).
-template <int PASS, int INFL, bool LIN>
+// One bond of a pass, added to the lane's sums s when `ok` (one sum for the
+// dilatation passes, three for the force passes). UNIV: without the volume
+// factor, which the caller applies to the sums. A masked-out bond may give a
+// NaN, so the sums are selected, not the terms.
+template <int PASS, bool UNIV, int INFL, bool LIN>
 __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, double hhat,
-                                     double thermal, double (&b)[3]) {
+                                     double thermal, bool ok, double (&s)[3]) {
   const double X0 = nb.x(0) - me.x(0), X1 = nb.x(1) - me.x(1), X2 = nb.x(2) - me.x(2);
   const double z2 = fma(X2, X2, fma(X1, X1, X0 * X0));
-  const double om = omega64<INFL>(z2, hhat);
+  const double wv = UNIV ? omega64<INFL>(z2, hhat) : omega64<INFL>(z2, hhat) * nb.vol();
   double d0 = 0.0, d1 = 0.0, d2 = 0.0;
-  if (PASS == QP_DTHETA || PASS == QP_DFORCE) {
+  if (is_dual<PASS>()) {
     d0 = nb.w(0) - me.w(0); d1 = nb.w(1) - me.w(1); d2 = nb.w(2) - me.w(2);
   }
   const double D0 = nb.u(0) - me.u(0), D1 = nb.u(1) - me.u(1), D2 = nb.u(2) - me.u(2);
+  auto add1 = [&](double f, double v) {
+    const double n = fma(f, v, s[0]);
+    s[0] = ok ? n : s[0];
+  };
+  auto add3 = [&](double f, double v0, double v1, double v2) {
+    const double n0 = fma(f, v0, s[0]), n1 = fma(f, v1, s[1]), n2 = fma(f, v2, s[2]);
+    s[0] = ok ? n0 : s[0];
+    s[1] = ok ? n1 : s[1];
+    s[2] = ok ? n2 : s[2];
+  };
   if (LIN) {
     // theta and force linear in u, the force along the reference bond
-    const bool dual = PASS == QP_DTHETA || PASS == QP_DFORCE;
+    constexpr bool dual = is_dual<PASS>();
     const double pr = fma(X2, dual ? d2 : D2, fma(X1, dual ? d1 : D1, X0 * (dual ? d0 : D0)));
-    if (PASS == QP_THETA || PASS == QP_DTHETA) {
-      b[0] = om * nb.vol() * pr;
+    if (PASS == QP_THETA || is_dtheta<PASS>()) {
+      add1(wv, pr);
     } else {
       const double qs = PASS == QP_FORCE ? me.q() + nb.q() : me.dq() + nb.dq();
-      const double t = om * nb.vol() * fma(me.alpha() + nb.alpha(), pr * rcp64(z2), qs);
-      b[0] = t * X0; b[1] = t * X1; b[2] = t * X2;
+      add3(wv * fma(me.alpha() + nb.alpha(), pr * rcp64(z2), qs), X0, X1, X2);
     }
     return;
   }
@@ -167,37 +184,45 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
   const double yy = fma(Y2, Y2, fma(Y1, Y1, Y0 * Y0));
   const double t = rsqrt64(z2 * yy);
   double g = z2 * t, ryy = g * t;
-  if (z2 == 0.0) {  // points that coincide in the reference configuration
-    g = 0.0;
-    ryy = rcp64(yy);
+  // points that coincide in the reference configuration (rare: one branch of
+  // the wave, no selects)
+  if (__builtin_amdgcn_ballot_w64(z2 == 0.0)) {
+    if (z2 == 0.0) {
+      g = 0.0;
+      ryy = rcp64(yy);
+    }
   }
   if (PASS == QP_THETA) {
     const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
-    b[0] = om * nb.vol() * (dd * g * rcp64(1.0 + g) - thermal * z2);
-  } else if (PASS == QP_DTHETA) {
-    b[0] = om * nb.vol() * g * fma(Y2, d2, fma(Y1, d1, Y0 * d0));
+    add1(wv, dd * g * rcp64(1.0 + g) - thermal * z2);
+  } else if (is_dtheta<PASS>()) {
+    add1(wv * g, fma(Y2, d2, fma(Y1, d1, Y0 * d0)));
   } else if (PASS == QP_FORCE) {
     const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
     const double ey = dd * ryy * rcp64(1.0 + g);
-    const double s = om * nb.vol() * fma(me.alpha() + nb.alpha(), ey, (me.q() + nb.q()) * g);
-    b[0] = s * Y0; b[1] = s * Y1; b[2] = s * Y2;
+    add3(wv * fma(me.alpha() + nb.alpha(), ey, (me.q() + nb.q()) * g), Y0, Y1, Y2);
   } else {
     const double a = me.alpha() + nb.alpha();
-    const double S = om * fma(a, 1.0 - g, (me.q() + nb.q()) * g);
+    const double S = fma(a, 1.0 - g, (me.q() + nb.q()) * g);  // over w
     const double yd = fma(Y2, d2, fma(Y1, d1, Y0 * d0));
-    const double c = fma(om * g, me.dq() + nb.dq(), (om * a - S) * (yd * ryy)) * nb.vol();
-    const double sv = S * nb.vol();
-    b[0] = fma(sv, d0, c * Y0);
-    b[1] = fma(sv, d1, c * Y1);
-    b[2] = fma(sv, d2, c * Y2);
+    const double c = wv * fma(g, me.dq() + nb.dq(), (a - S) * (yd * ryy));
+    const double sv = wv * S;
+    const double n0 = fma(sv, d0, fma(c, Y0, s[0]));
+    const double n1 = fma(sv, d1, fma(c, Y1, s[1]));
+    const double n2 = fma(sv, d2, fma(c, Y2, s[2]));
+    s[0] = ok ? n0 : s[0];
+    s[1] = ok ? n1 : s[1];
+    s[2] = ok ? n2 : s[2];
   }
 }
 
 // What the pass writes, besides what QsTileArgs holds.
 struct QsOut {
-  const double* w;  // QP_DTHETA: the direction, 3n
+  const double* w;  // QP_DTHETA: the direction, QP_CG: z; 3n
   double* out;      // force passes: 3n
   int all;          // QP_FORCE: prescribed DOFs too
+  QsCgStart start;  // QP_CG; QP_DFORCE: start.cg null outside a solve
+  double* pq_part;  // QP_DFORCE in a solve
 };
 
 // A node group's row: CSR range, then the lane's intact bits (two words,
@@ -240,7 +265,7 @@ __device__ __forceinline__ void slot_load(const QsTileArgs& a, const QsOut& o, u
 #pragma unroll
   for (int k = 0; k < 3; k++) r.v[k] = a.rec.xu[k][i];
   if (PASS == QP_FORCE || PASS == QP_DFORCE) r.v[3] = a.rec.aq[i];
-  if (PASS == QP_DTHETA) {
+  if (is_dtheta<PASS>()) {
     const double* w = o.w + 3u * i;
     r.v[units<PASS>() - 2] = f64x2{w[0], w[1]};
     r.v[units<PASS>() - 1] = f64x2{w[2], a.vol[i]};
@@ -282,8 +307,11 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
   constexpr int T = WG * HV;
   constexpr int GB = G * HV;  // bonds of a node per step
   constexpr int kHaloRounds = (kTileHaloMax + T - 1) / T;
+  __shared__ double sums[PASS == QP_CG ? 2 * T / 64 : PASS == QP_DFORCE ? T / 64 : 1];
   const int tile = tile_of_block(blockIdx.x, a.t.ntiles);
   if (tile >= a.t.ntiles) return;
+  // launches after the end of a solve return at once
+  if ((PASS == QP_CG || PASS == QP_DFORCE) && o.start.cg && o.start.cg->done) return;
   const int n0 = a.t.tile_start[tile], n1 = a.t.tile_start[tile + 1];
   const int h0 = a.t.halo_off[tile], hn = min(a.t.halo_off[tile + 1] - h0, HS);
   const int own = a.t.own_off[tile];
@@ -302,15 +330,28 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
   Row<U> rw;
   row_range(a, n0 + grp, n0, n1, rw);
   row_data<GB, U>(a, l, rw);
+  double beta = 0.0;
 #pragma unroll
   for (int r = 0; r < kHaloRounds; r++) {
     if (r > 0 && r * T >= hn) break;
     Rec<PASS> v;
-    slot_load<PASS, UNIV>(a, o, (unsigned)idx[r], v);
+    const unsigned i = (unsigned)idx[r];
+    slot_load<PASS, UNIV>(a, o, i, v);
+    if (PASS == QP_CG) {
+      const f64x2 p0 = a.rec.wp[0][i], p1 = a.rec.wp[1][i];
+      if (r == 0 && cg_start<T>(o.start, sums, beta)) return;
+      if (beta != 0.0) {  // the first direction is z
+        f64x2 &w0 = v.v[units<PASS>() - 2], &w1 = v.v[units<PASS>() - 1];
+        w0.x = fma(beta, p0.x, w0.x);
+        w0.y = fma(beta, p0.y, w0.y);
+        w1.x = fma(beta, p1.x, w1.x);
+      }
+    }
     const int h = threadIdx.x + r * T;
     if (h < hn) slot_store<PASS, UNIV>(lds, h, v);
   }
   __syncthreads();
+  double pq = 0.0;  // QP_DFORCE: this thread's part of w.Kw
   for (int base = n0; base < n1; base += NG) {
     const int node = base + grp;
     const bool valid = node < n1;
@@ -322,7 +363,7 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
     const int deg = rw.deg;
     const unsigned short* lp = a.t.lcol + (unsigned)(rw.rs + l);
     Rec<PASS> me;
-    rec_read<PASS, UNIV>(me, lds, kLdsSlot * (own + (nd - n0)), a.vol1);
+    rec_read<PASS, UNIV>(me, lds, kLdsSlot * (own + (nd - n0)));
     double thermal = 0.0;
     if (PASS == QP_THETA && a.dT) thermal = a.alphaT * a.dT[(unsigned)nd];
     // nodes of a tile are ordered by descending degree: the wave's first
@@ -337,25 +378,22 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
       for (int k = 0; k < U; k++) ln[k] = np[k * GB];
       const int b0 = c * (GB * U);
       const unsigned long long bits = (b0 < 64 ? rw.in[0] : rw.in[1]) >> (b0 & 63);
+      const unsigned half[2] = {(unsigned)bits, (unsigned)(bits >> 32)};
 #pragma unroll
       for (int k = 0; k < U; k++) {
         Rec<PASS> nb;
-        rec_read<PASS, UNIV>(nb, lds, lj[k], a.vol1);
-        double b[3] = {0.0, 0.0, 0.0};
-        bond<PASS, INFL, LIN>(me, nb, a.hhat, thermal, b);
-        const bool ok = (bits >> (k * GB)) & 1ull;
-#pragma unroll
-        for (int d = 0; d < (PASS == QP_FORCE || PASS == QP_DFORCE ? 3 : 1); d++)
-          s[d] = ok ? s[d] + b[d] : s[d];
+        rec_read<PASS, UNIV>(nb, lds, lj[k]);
+        const bool ok = (half[(k * GB) >> 5] & (1u << ((k * GB) & 31))) != 0u;
+        bond<PASS, UNIV, INFL, LIN>(me, nb, a.hhat, thermal, ok, s);
       }
 #pragma unroll
       for (int k = 0; k < U; k++) lj[k] = ln[k];
     }
-    if (PASS == QP_THETA || PASS == QP_DTHETA) {
+    if (PASS == QP_THETA || is_dtheta<PASS>()) {
       const double sum = lanes_sum<G, HV>(s[0]);
       if (!valid || l != 0) continue;
       const double m = a.m[(unsigned)node];
-      const double c = m > 0.0 ? 3.0 / m : 0.0;
+      const double c = (m > 0.0 ? 3.0 / m : 0.0) * (UNIV ? a.vol1 : 1.0);
       if (PASS == QP_THETA) {
         const double th = c * (a.L * a.L) * sum;
         a.theta[(unsigned)node] = th;
@@ -370,11 +408,28 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
     } else {
       const double f0 = lanes_sum<G, HV>(s[0]), f1 = lanes_sum<G, HV>(s[1]), f2 = lanes_sum<G, HV>(s[2]);
       if (!valid || l >= 3) continue;
-      const double f = (l == 0 ? f0 : (l == 1 ? f1 : f2)) * me.vol();
+      const double f = (l == 0 ? f0 : (l == 1 ? f1 : f2)) * (UNIV ? a.vol1 * a.vol1 : me.vol());
       const unsigned q = 3u * (unsigned)node + (unsigned)l;
       const bool fx = a.fixed[q] != 0;
-      if (PASS == QP_FORCE) o.out[q] = fx && !o.all ? 0.0 : a.L * f;
-      else o.out[q] = fx ? (l == 0 ? me.w(0) : (l == 1 ? me.w(1) : me.w(2))) : -f;
+      if (PASS == QP_FORCE) {
+        o.out[q] = fx && !o.all ? 0.0 : a.L * f;
+      } else {
+        const double w = l == 0 ? me.w(0) : (l == 1 ? me.w(1) : me.w(2));
+        double kw = fx ? w : -f;
+        if (a.damp) kw += a.damp[q] * w;
+        o.out[q] = kw;
+        pq += w * kw;
+      }
+    }
+  }
+  if (PASS == QP_DFORCE && o.start.cg) {
+    pq = wave_sum64(pq);
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = pq;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      for (int k = 0; k < T / 64; k++) t += sums[k];
+      o.pq_part[tile] = t;
     }
   }
 }
@@ -405,7 +460,7 @@ hipError_t launch_g(const QsTileArgs& a, const QsOut& o, int lanes, hipStream_t 
 
 template <int PASS, int INFL, bool LIN>
 hipError_t launch_v(const QsTileArgs& a, const QsOut& o, int lanes, hipStream_t s) {
-  if (PASS == QP_DFORCE && a.vol1 > 0.0) return launch_g<PASS, PASS == QP_DFORCE, INFL, LIN>(a, o, lanes, s);
+  if (a.vol1 > 0.0) return launch_g<PASS, true, INFL, LIN>(a, o, lanes, s);
   return launch_g<PASS, false, INFL, LIN>(a, o, lanes, s);
 }
 
@@ -440,6 +495,17 @@ hipError_t launch_qs_tangent(const QsTileArgs& a, const double* w, double* out, 
   o.w = w;
   o.out = out;
   hipError_t e = launch<QP_DTHETA>(a, o, lanes, s);
+  return e == hipSuccess ? launch<QP_DFORCE>(a, o, lanes, s) : e;
+}
+
+hipError_t launch_qs_tangent_cg(const QsTileArgs& a, const QsCgStart& start, const double* z,
+                                double* out, double* pq_part, int lanes, hipStream_t s) {
+  QsOut o{};
+  o.w = z;
+  o.out = out;
+  o.start = start;
+  o.pq_part = pq_part;
+  hipError_t e = launch<QP_CG>(a, o, lanes, s);
   return e == hipSuccess ? launch<QP_DFORCE>(a, o, lanes, s) : e;
 }
 

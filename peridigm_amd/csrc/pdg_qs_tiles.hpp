@@ -1,7 +1,7 @@
 // LDS-tiled FP64 bond passes of the quasi-static path (pdg_qs_tiles.hip).
 #pragma once
 
-#include "pdg_internal.hpp"
+#include "pdg_qs_cg.hpp"
 
 namespace pdg {
 
@@ -19,6 +19,7 @@ struct QsRecords {
   f64x2* xu[3];
   f64x2* aq;
   f64x2* wd[2];
+  f64x2* wp[2];  // the previous direction of a conjugate-gradient solve
 };
 
 struct QsTileArgs {
@@ -40,6 +41,7 @@ struct QsTileArgs {
   const double* dT;  // temperature change per node, or null
   double alphaT;
   const signed char* fixed;
+  const double* damp;  // 3n, added to the tangent's diagonal, or null
   QsRecords rec;
   double* theta;
 };
@@ -53,5 +55,11 @@ hipError_t launch_qs_residual(const QsTileArgs& a, bool all, double* out, int la
 // out = K w at that state (w on prescribed DOFs); w: 3n.
 hipError_t launch_qs_tangent(const QsTileArgs& a, const double* w, double* out, int lanes,
                              hipStream_t s);
+
+// The same product for a conjugate-gradient iteration: w = z + beta wp (the
+// records wp) with beta and the decision to stop from `start`, w into the
+// records wd; pq_part[t] is tile t's part of w.Kw.
+hipError_t launch_qs_tangent_cg(const QsTileArgs& a, const QsCgStart& start, const double* z,
+                                double* out, double* pq_part, int lanes, hipStream_t s);
 
 }  // namespace pdg

@@ -97,3 +97,69 @@ def test_coincident_points():
             out[variant] = (Q.residual(ctx, u)[0], Q.tangent_apply(ctx, u, w))
     for a, b in zip(out[0], out[1]):
         assert np.isfinite(b).all() and _rel(a, b) <= 1e-11
+
+
+def _bar(n):
+    from peridigm_amd import Context, discretization
+    from peridigm_amd import quasistatic as Q
+    h = 1e-3
+    x, vol = discretization.lattice_centres(n, [0, 0, 0], [k * h for k in n])
+    nl = discretization.radius_search(x, 3.015 * h)
+    i = np.rint(x[:, 0] / h - 0.5).astype(int)
+    ctx = Context(0)
+    ctx.set_topology(nl, len(vol))
+    ctx.set_constants(x, vol, 130e9, 78e9, 3.015 * h, 0, 0.0)
+    fixed = Q.end_dofs(np.nonzero(i <= 1)[0], np.nonzero(i >= n[0] - 2)[0])
+    Q.set_fixed(ctx, fixed)
+    return ctx, x, fixed
+
+
+# 120 nodes (one workgroup of the update), 1,920, and 67,200 (wide workgroups)
+@pytest.mark.parametrize("n", [(8, 5, 3), (20, 12, 8), (42, 40, 40)])
+@pytest.mark.parametrize("precond", ["none", "block_jacobi", "two_level"])
+def test_solve_from_a_guess(n, precond):
+    """Solves from a non-zero guess on tiled and untiled kernels: the residual
+    by the tangent itself is the reported one (1e-8, plus the drift of the
+    recursive residual, far below a tenth of it)."""
+    from peridigm_amd import quasistatic as Q
+    ctx, x, fixed = _bar(n)
+    with ctx:
+        rng = np.random.default_rng(5)
+        u = 2e-4 * x
+        b = rng.standard_normal(x.shape)
+        b.reshape(-1)[fixed] = 0.0
+        x0 = rng.standard_normal(x.shape) * 1e-9
+        x0.reshape(-1)[fixed] = 0.0
+        for variant in (0, 1):
+            ctx.set_kernel_variant(variant)
+            xs, it, rel = Q.solve(ctx, u, b, x0=x0, precond=precond, rel_tol=1e-8)
+            r = np.linalg.norm(b - Q.tangent_apply(ctx, u, xs)) / np.linalg.norm(b)
+            assert it > 0 and rel <= 1e-8 and r <= 1.1e-8
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("precond", ["none", "block_jacobi"])
+def test_iteration_limit(precond, graphs):
+    """A solve cut off after k iterations reports it and leaves the k-th
+    iterate: the same on tiled, untiled and replayed launches (FP64 sums in
+    another order over at most 13 iterations: 1e-10)."""
+    from peridigm_amd import quasistatic as Q
+    from peridigm_amd.learned import _iterate
+    from peridigm_amd._lib import PdgError
+    ctx, x, fixed = _bar((20, 8, 6))
+    with ctx:
+        Q.set_graphs(ctx, graphs)
+        rng = np.random.default_rng(6)
+        u = 2e-4 * x
+        b = rng.standard_normal(x.shape)
+        b.reshape(-1)[fixed] = 0.0
+        with pytest.raises(PdgError) as e:
+            Q.solve(ctx, u, b, precond=precond, max_iter=6)
+        assert e.value.code == -5
+        if precond == "block_jacobi":
+            for k in (0, 1, 4, 7, 9, 13):
+                it = []
+                for variant in (0, 1):
+                    ctx.set_kernel_variant(variant)
+                    it.append(_iterate(ctx, u, b, k, 1e-12))
+                assert np.abs(it[0] - it[1]).max() <= 1e-10 * max(np.abs(it[1]).max(), 1e-300)
