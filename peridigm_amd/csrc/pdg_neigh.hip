@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <climits>
 #include <cmath>
 #include <vector>
 
@@ -88,74 +89,63 @@ __device__ __forceinline__ int cell_coord(double x, double lo, double cs, int nc
   return c < 0 ? 0 : (c >= nc ? nc - 1 : c);
 }
 
-__global__ void k_cell_ids(int n, const double* __restrict__ x, RGrid g, int* __restrict__ cell,
-                           int* __restrict__ idx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int a = cell_coord(x[3 * i], g.lo[0], g.cs, g.nc[0]);
-  const int b = cell_coord(x[3 * i + 1], g.lo[1], g.cs, g.nc[1]);
-  const int c = cell_coord(x[3 * i + 2], g.lo[2], g.cs, g.nc[2]);
-  cell[i] = (c * g.nc[1] + b) * g.nc[0] + a;
-  idx[i] = i;
-}
-
-__global__ void k_cell_start(int n, const int* __restrict__ scell, int* __restrict__ cstart) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int c = scell[q];
-  if (q == 0 || scell[q - 1] != c) cstart[c] = q;
-}
-
-__global__ void k_cell_end(int n, const int* __restrict__ scell, int* __restrict__ cend) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int c = scell[q];
-  if (q == n - 1 || scell[q + 1] != c) cend[c] = q + 1;
-}
-
-// Candidates from the 27 surrounding cells; membership by the predicate only.
-template <bool FILL>
-__global__ __launch_bounds__(256) void k_radius(int n, const double* __restrict__ x, RGrid g,
-                                                const int* __restrict__ cstart,
-                                                const int* __restrict__ cend,
-                                                const int* __restrict__ sidx,
-                                                long long* __restrict__ count,
-                                                const long long* __restrict__ off,
-                                                unsigned long long* __restrict__ keys) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double X0 = x[3 * i], X1 = x[3 * i + 1], X2 = x[3 * i + 2];
-  const int a = cell_coord(X0, g.lo[0], g.cs, g.nc[0]);
-  const int b = cell_coord(X1, g.lo[1], g.cs, g.nc[1]);
-  const int c = cell_coord(X2, g.lo[2], g.cs, g.nc[2]);
-  long long o = FILL ? off[i] : 0;
-  int cnt = 0;
-  for (int dz = -1; dz <= 1; dz++) {
-    const int cz = c + dz;
-    if (cz < 0 || cz >= g.nc[2]) continue;
-    for (int dy = -1; dy <= 1; dy++) {
-      const int cy = b + dy;
-      if (cy < 0 || cy >= g.nc[1]) continue;
-      for (int dx = -1; dx <= 1; dx++) {
-        const int cx = a + dx;
-        if (cx < 0 || cx >= g.nc[0]) continue;
-        const int cc = (cz * g.nc[1] + cy) * g.nc[0] + cx;
-        const int s = cstart[cc], e = cend[cc];
-        for (int q = s; q < e; q++) {
-          const int j = sidx[q];
-          if (j == i) continue;
-          const double ddx = (x[3 * j] - X0);
-          const double ddy = (x[3 * j + 1] - X1);
-          const double ddz = (x[3 * j + 2] - X2);
-          if (ddx * ddx + ddy * ddy + ddz * ddz <= g.R2) {
-            if (FILL) keys[o++] = ((unsigned long long)i << 32) | (unsigned)j;
-            cnt++;
-          }
-        }
-      }
+// Partial bounding boxes (lo, hi per block) of the points; NaNs drop out, as
+// in the comparisons of a host loop.
+constexpr int kBoxBlocks = 64;
+__global__ __launch_bounds__(256) void k_box(int n, const double* __restrict__ x,
+                                             double* __restrict__ part) {
+  __shared__ double sh[4][6];
+  double b[6] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX};
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+    for (int d = 0; d < 3; d++) {
+      b[d] = fmin(b[d], x[3 * (size_t)i + d]);
+      b[3 + d] = fmax(b[3 + d], x[3 * (size_t)i + d]);
     }
+  for (int o = 32; o > 0; o >>= 1)
+    for (int d = 0; d < 3; d++) {
+      b[d] = fmin(b[d], __shfl_xor(b[d], o));
+      b[3 + d] = fmax(b[3 + d], __shfl_xor(b[3 + d], o));
+    }
+  if ((threadIdx.x & 63) == 0)
+    for (int d = 0; d < 6; d++) sh[threadIdx.x >> 6][d] = b[d];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int d = threadIdx.x;
+    double v = sh[0][d];
+    for (int w = 1; w < 4; w++) v = d < 3 ? fmin(v, sh[w][d]) : fmax(v, sh[w][d]);
+    part[6 * blockIdx.x + d] = v;
   }
-  if (!FILL) count[i] = cnt;
+}
+
+__device__ __forceinline__ void cell_of(const RGrid& g, double X0, double X1, double X2, int (&c)[3]) {
+  c[0] = cell_coord(X0, g.lo[0], g.cs, g.nc[0]);
+  c[1] = cell_coord(X1, g.lo[1], g.cs, g.nc[1]);
+  c[2] = cell_coord(X2, g.lo[2], g.cs, g.nc[2]);
+}
+
+// Points of each cell, then (after a scan into `begin`) the points and their
+// positions by cell; the order inside a cell is left to the atomics, since
+// the rows are sorted at the end.
+__global__ void k_cell_count(int n, const double* __restrict__ x, RGrid g, int* __restrict__ cell,
+                             int* __restrict__ count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  int c[3];
+  cell_of(g, x[3 * (size_t)i], x[3 * (size_t)i + 1], x[3 * (size_t)i + 2], c);
+  const int id = (c[2] * g.nc[1] + c[1]) * g.nc[0] + c[0];
+  cell[i] = id;
+  atomicAdd(&count[id], 1);
+}
+
+// count: what is left of each cell (counted down to 0)
+__global__ void k_cell_scatter(int n, const double* __restrict__ x, const int* __restrict__ cell,
+                               const int* __restrict__ begin, int* __restrict__ count,
+                               int* __restrict__ sidx, double* __restrict__ xs) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int q = begin[cell[i]] + atomicSub(&count[cell[i]], 1) - 1;
+  sidx[q] = i;
+  for (int d = 0; d < 3; d++) xs[3 * (size_t)q + d] = x[3 * (size_t)i + d];
 }
 
 // FinitePlane::bondIntersectInfinitePlane + bondIntersect (tolerance 1e-15),
@@ -189,45 +179,156 @@ __device__ bool plane_cuts(const double* pl, const double* p0, const double* p1)
   return -zero < aa && aa / a < one && -zero < bb && bb / b < one;
 }
 
-__global__ void k_plane_flags(long long nb, const unsigned long long* __restrict__ keys,
-                              const double* __restrict__ x, int nplanes,
-                              const double* __restrict__ planes, int* __restrict__ keep) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nb) return;
-  const int i = (int)(keys[q] >> 32), j = (int)(keys[q] & 0xffffffffu);
-  bool cut = false;
-  for (int p = 0; p < nplanes && !cut; p++) cut = plane_cuts(planes + 11 * p, x + 3 * i, x + 3 * j);
-  keep[q] = cut ? 0 : 1;
+// One wave per point, in cell order: candidates from the 27 surrounding cells
+// (nine runs of the cell order, three cells along x each), 64 at a time;
+// membership by the predicate alone. The lanes' hits are packed into the
+// wave's LDS row, the packed row is filtered by the planes, and FILL ranks its
+// ids (unique: an id's place is the number of smaller ones) and writes the
+// row in order. COUNT only counts. Rows that outgrow the LDS row are flushed
+// in pieces: counted, or written unsorted to `spill` for k_spilled_rows.
+// Against a thread per point (whose lanes walk cells of different lengths),
+// a radix sort of 64-bit (row, id) keys and per-bond kernels for the planes
+// and the compaction, 160,000 points with 13.7M bonds and one plane: 0.23 ms
+// to count and 0.33 ms to fill (the kernels before took 1.9 and 2.7 ms). Bound
+// by instruction issue: two in three candidates fail the distance test, and
+// ranking a row of 122 takes 244 broadcast compares a lane.
+constexpr int kRowCap = 512;
+constexpr int kWaves = 4;  // per workgroup
+struct NearArgs {
+  int n;
+  RGrid g;
+  const double* xs;
+  const int* sidx;
+  const int* begin;
+  int nplanes;
+  const double* planes;
+  long long* count;
+  const long long* off;  // FILL: kept bonds of the rows before
+  int* nlist;
+  int* big;              // COUNT: set when any row was flushed
+  int* spill;            // FILL, if so: the flushed rows, unsorted
+  int* flushed;          // FILL, if so: which rows they are
+};
+
+// Orders the wave's LDS accesses before and after it.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ void k_row_count(long long nb, const unsigned long long* __restrict__ keys,
-                            const int* __restrict__ keep, long long* __restrict__ count) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nb || !keep[q]) return;
-  atomicAdd((unsigned long long*)&count[keys[q] >> 32], 1ull);
+template <bool FILL>
+__global__ __launch_bounds__(64 * kWaves) void k_near(NearArgs a) {
+  __shared__ __align__(16) int rows[kWaves][kRowCap + 68];
+  const int lane = threadIdx.x & 63;
+  int* const row = rows[threadIdx.x >> 6];
+  const int t = blockIdx.x * kWaves + (threadIdx.x >> 6);
+  if (t >= a.n) return;  // whole waves: no barrier below
+  const int i = a.sidx[t];
+  const double P[3] = {a.xs[3 * (size_t)t], a.xs[3 * (size_t)t + 1], a.xs[3 * (size_t)t + 2]};
+  int c[3];
+  cell_of(a.g, P[0], P[1], P[2], c);
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int nb = 0;            // entries of the LDS row: sorted positions, then (filtered) ids
+  long long total = 0;   // kept so far (flushed pieces)
+  bool flushed = false;
+  // filters the LDS row by the planes and turns positions into ids
+  auto filter = [&]() {
+    int kept = 0;
+    for (int e0 = 0; e0 < nb; e0 += 64) {
+      const bool have = e0 + lane < nb;
+      const int q = have ? row[e0 + lane] : t;
+      bool keep = have;
+      if (a.nplanes > 0 && have) {
+        const double Q[3] = {a.xs[3 * (size_t)q], a.xs[3 * (size_t)q + 1], a.xs[3 * (size_t)q + 2]};
+        for (int p = 0; p < a.nplanes && keep; p++) keep = !plane_cuts(a.planes + 11 * p, P, Q);
+      }
+      const int id = a.sidx[q];
+      const unsigned long long m = __ballot(keep);
+      wave_sync();
+      if (keep) row[kept + __popcll(m & below)] = id;  // never past what was read
+      wave_sync();
+      kept += __popcll(m);
+    }
+    nb = kept;
+  };
+  auto flush = [&]() {
+    filter();
+    if (FILL)
+      for (int e = lane; e < nb; e += 64) a.spill[a.off[i] + total + e] = row[e];
+    total += nb;
+    nb = 0;
+    flushed = true;
+  };
+  for (int dz = -1; dz <= 1; dz++) {
+    const int cz = c[2] + dz;
+    if (cz < 0 || cz >= a.g.nc[2]) continue;
+    for (int dy = -1; dy <= 1; dy++) {
+      const int cy = c[1] + dy;
+      if (cy < 0 || cy >= a.g.nc[1]) continue;
+      const int first = (cz * a.g.nc[1] + cy) * a.g.nc[0];
+      const int s = a.begin[first + max(c[0] - 1, 0)];
+      const int e = a.begin[first + min(c[0] + 1, a.g.nc[0] - 1) + 1];
+      for (int q0 = s; q0 < e; q0 += 64) {
+        const int q = q0 + lane;
+        bool hit = false;
+        if (q < e && q != t) {
+          const double d0 = a.xs[3 * (size_t)q] - P[0], d1 = a.xs[3 * (size_t)q + 1] - P[1],
+                       d2 = a.xs[3 * (size_t)q + 2] - P[2];
+          hit = d0 * d0 + d1 * d1 + d2 * d2 <= a.g.R2;
+        }
+        const unsigned long long m = __ballot(hit);
+        if (nb > kRowCap) flush();
+        if (hit) row[nb + __popcll(m & below)] = q;
+        wave_sync();
+        nb += __popcll(m);
+      }
+    }
+  }
+  if (flushed) flush();
+  else if (FILL || a.nplanes > 0) filter();
+  if (!FILL) {
+    if (lane == 0) {
+      a.count[i] = total + nb;
+      if (flushed) *a.big = 1;
+    }
+    return;
+  }
+  const long long h = a.off[i] + i;
+  if (lane == 0) a.nlist[h] = (int)(total + nb);
+  if (a.flushed && lane == 0) a.flushed[i] = flushed;
+  if (flushed) return;
+  // pad to whole groups of four that no id ranks above
+  if (lane < 4) row[nb + lane] = INT_MAX;
+  wave_sync();
+  for (int e = lane; e < nb; e += 64) {
+    const int v = row[e];
+    int rank = 0;
+    for (int k = 0; k < nb; k += 4) {
+      const int4 w = *reinterpret_cast<const int4*>(row + k);
+      rank += (w.x < v) + (w.y < v) + (w.z < v) + (w.w < v);
+    }
+    a.nlist[h + 1 + rank] = v;
+  }
 }
 
-__global__ void k_emit(long long nb, const unsigned long long* __restrict__ keys,
-                       const int* __restrict__ keep, const long long* __restrict__ kpos,
-                       const long long* __restrict__ head, int* __restrict__ nlist) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nb || !keep[q]) return;
-  // keys are sorted by (row, col); kpos = exclusive scan of keep, so the
-  // position inside the row is kpos[q] - (kept bonds before this row)
-  const int i = (int)(keys[q] >> 32);
-  const long long before_row = head[i] - i;  // kept bonds of rows < i
-  nlist[head[i] + 1 + (kpos[q] - before_row)] = (int)(keys[q] & 0xffffffffu);
-}
-
-__global__ void k_widen(long long nb, const int* __restrict__ a, long long* __restrict__ b) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < nb) b[q] = a[q];
-}
-
-__global__ void k_emit_counts(int n, const long long* __restrict__ count,
-                              const long long* __restrict__ head, int* __restrict__ nlist) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) nlist[head[i]] = (int)count[i];
+// The flushed rows, ranked from `spill` (a workgroup per point).
+__global__ __launch_bounds__(256) void k_spilled_rows(int n, const long long* __restrict__ count,
+                                                      const long long* __restrict__ off,
+                                                      const int* __restrict__ spill,
+                                                      const int* __restrict__ flushed,
+                                                      int* __restrict__ nlist) {
+  const int i = blockIdx.x;
+  if (!flushed[i]) return;
+  const long long m = count[i];
+  const int* r = spill + off[i];
+  int* out = nlist + off[i] + i + 1;
+  for (long long e = threadIdx.x; e < m; e += 256) {
+    const int v = r[e];
+    long long rank = 0;
+    for (long long k = 0; k < m; k++) rank += r[k] < v;
+    out[rank] = v;
+  }
 }
 
 template <class T>
@@ -322,13 +423,24 @@ int pdg_radius_search(int N, const double* x, double R, int nplanes, const doubl
                       int* nlist, long long* listSize) {
   if (N <= 0 || !x || !(R > 0.0) || !listSize || nplanes < 0 || (nplanes > 0 && !planes))
     return PDG_E_ARG;
+  hipStream_t s = nullptr;
+  const unsigned nb = (unsigned)((N + 255) / 256);
+  DevBuf<double> dx, dpl;
+  PDG_CK(dx.alloc(6 * (size_t)N + 6 * kBoxBlocks));  // x, sorted positions, boxes
+  double* const xs = dx.p + 3 * (size_t)N;
+  double* const dbox = xs + 3 * (size_t)N;
+  PDG_CK(hipMemcpyAsync(dx.p, x, 24 * (size_t)N, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_box, dim3(kBoxBlocks), dim3(256), 0, s, N, dx.p, dbox);
+  double box[6 * kBoxBlocks];
+  PDG_CK(hipMemcpy(box, dbox, sizeof(box), hipMemcpyDeviceToHost));
   double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  for (int i = 0; i < N; i++)
+  for (int b = 0; b < kBoxBlocks; b++)
     for (int d = 0; d < 3; d++) {
-      lo[d] = std::min(lo[d], x[3 * (size_t)i + d]);
-      hi[d] = std::max(hi[d], x[3 * (size_t)i + d]);
+      lo[d] = std::min(lo[d], box[6 * b + d]);
+      hi[d] = std::max(hi[d], box[6 * b + 3 + d]);
     }
-  RGrid g;
+  NearArgs a{};
+  RGrid& g = a.g;
   g.cs = R * 1.0000001;
   long long ncell = 1;
   for (int d = 0; d < 3; d++) {
@@ -338,82 +450,63 @@ int pdg_radius_search(int N, const double* x, double R, int nplanes, const doubl
   }
   if (ncell > (1ll << 30)) return PDG_E_UNSUPPORTED;
   g.R2 = R * R;
-  hipStream_t s = nullptr;
-  DevBuf<double> dx;
-  DevBuf<int> cell, idx, scell, sidx, cstart, cend;
-  PDG_CK(dx.alloc(3 * (size_t)N));
-  PDG_CK(hipMemcpy(dx.p, x, 24 * (size_t)N, hipMemcpyHostToDevice));
-  PDG_CK(cell.alloc(N)); PDG_CK(idx.alloc(N)); PDG_CK(scell.alloc(N)); PDG_CK(sidx.alloc(N));
-  PDG_CK(cstart.alloc(ncell)); PDG_CK(cend.alloc(ncell));
-  const unsigned nb = (unsigned)((N + 255) / 256);
-  hipLaunchKernelGGL(k_cell_ids, dim3(nb), dim3(256), 0, s, N, dx.p, g, cell.p, idx.p);
-  {
-    size_t bytes = 0;
-    PDG_CK(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, cell.p, scell.p, idx.p, sidx.p, N, 0, 32, s));
-    DevBuf<char> tmp;
-    PDG_CK(tmp.alloc(bytes));
-    PDG_CK(hipcub::DeviceRadixSort::SortPairs(tmp.p, bytes, cell.p, scell.p, idx.p, sidx.p, N, 0, 32, s));
-  }
-  PDG_CK(hipMemsetAsync(cstart.p, 0, 4 * ncell, s));
-  PDG_CK(hipMemsetAsync(cend.p, 0, 4 * ncell, s));
-  hipLaunchKernelGGL(k_cell_start, dim3(nb), dim3(256), 0, s, N, scell.p, cstart.p);
-  hipLaunchKernelGGL(k_cell_end, dim3(nb), dim3(256), 0, s, N, scell.p, cend.p);
-  DevBuf<long long> cnt, off;
-  PDG_CK(cnt.alloc(N)); PDG_CK(off.alloc(N));
-  hipLaunchKernelGGL((k_radius<false>), dim3(nb), dim3(256), 0, s, N, dx.p, g, cstart.p, cend.p,
-                     sidx.p, cnt.p, nullptr, nullptr);
-  PDG_CK(hipGetLastError());
-  int rc = exclusive_scan(cnt.p, off.p, N, s);
-  if (rc) return rc;
-  long long lastc = 0, lasto = 0;
-  PDG_CK(hipMemcpy(&lastc, cnt.p + N - 1, 8, hipMemcpyDeviceToHost));
-  PDG_CK(hipMemcpy(&lasto, off.p + N - 1, 8, hipMemcpyDeviceToHost));
-  const long long B0 = lasto + lastc;
-  DevBuf<unsigned long long> keys, skeys;
-  PDG_CK(keys.alloc(B0)); PDG_CK(skeys.alloc(B0));
-  hipLaunchKernelGGL((k_radius<true>), dim3(nb), dim3(256), 0, s, N, dx.p, g, cstart.p, cend.p,
-                     sidx.p, nullptr, off.p, keys.p);
-  PDG_CK(hipGetLastError());
-  {
-    size_t bytes = 0;
-    PDG_CK(hipcub::DeviceRadixSort::SortKeys(nullptr, bytes, keys.p, skeys.p, (int)B0, 0, 64, s));
-    DevBuf<char> tmp;
-    PDG_CK(tmp.alloc(bytes));
-    PDG_CK(hipcub::DeviceRadixSort::SortKeys(tmp.p, bytes, keys.p, skeys.p, (int)B0, 0, 64, s));
-  }
-  // plane filter, per-row counts of kept bonds, compaction
-  DevBuf<int> keep;
-  DevBuf<double> dpl;
-  PDG_CK(keep.alloc(B0));
+  // cells: counts (one more, 0, for the scan) and first points; points: cell
+  // and cell order; the flush flag
+  const size_t nc1 = (size_t)ncell + 1, n1 = (size_t)N + 1;
+  DevBuf<int> ints;
+  PDG_CK(ints.alloc(2 * nc1 + 2 * (size_t)N + 1));
+  int* const ccount = ints.p;
+  int* const begin = ccount + nc1;
+  int* const cell = begin + nc1;
+  int* const sidx = cell + N;
+  int* const big = sidx + N;
+  DevBuf<long long> sums;  // bonds of each row (a 0 after the last) and of the rows before
+  PDG_CK(sums.alloc(2 * n1));
+  long long* const count = sums.p;
+  long long* const off = count + n1;
+  // one workspace for both scans
+  size_t bytes = 0, b2 = 0;
+  PDG_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, ccount, begin, (int)nc1, s));
+  PDG_CK(hipcub::DeviceScan::ExclusiveSum(nullptr, b2, count, off, (int)n1, s));
+  bytes = std::max(bytes, b2);
+  DevBuf<char> tmp;
+  PDG_CK(tmp.alloc(bytes));
   PDG_CK(dpl.alloc(std::max(1, 11 * nplanes)));
-  if (nplanes > 0) PDG_CK(hipMemcpy(dpl.p, planes, 88 * (size_t)nplanes, hipMemcpyHostToDevice));
-  const unsigned bb = (unsigned)((B0 + 255) / 256);
-  if (B0 > 0)
-    hipLaunchKernelGGL(k_plane_flags, dim3(bb), dim3(256), 0, s, B0, skeys.p, dx.p, nplanes, dpl.p, keep.p);
-  PDG_CK(hipMemsetAsync(cnt.p, 0, 8 * (size_t)N, s));
-  if (B0 > 0) hipLaunchKernelGGL(k_row_count, dim3(bb), dim3(256), 0, s, B0, skeys.p, keep.p, cnt.p);
-  rc = exclusive_scan(cnt.p, off.p, N, s);
-  if (rc) return rc;
-  PDG_CK(hipMemcpy(&lastc, cnt.p + N - 1, 8, hipMemcpyDeviceToHost));
-  PDG_CK(hipMemcpy(&lasto, off.p + N - 1, 8, hipMemcpyDeviceToHost));
-  const long long B = lasto + lastc;
+  if (nplanes > 0) PDG_CK(hipMemcpyAsync(dpl.p, planes, 88 * (size_t)nplanes, hipMemcpyHostToDevice, s));
+  PDG_CK(hipMemsetAsync(ccount, 0, 4 * nc1, s));
+  PDG_CK(hipMemsetAsync(big, 0, 4, s));
+  PDG_CK(hipMemsetAsync(count + N, 0, 8, s));
+  hipLaunchKernelGGL(k_cell_count, dim3(nb), dim3(256), 0, s, N, dx.p, g, cell, ccount);
+  PDG_CK(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, ccount, begin, (int)nc1, s));
+  hipLaunchKernelGGL(k_cell_scatter, dim3(nb), dim3(256), 0, s, N, dx.p, cell, begin, ccount, sidx, xs);
+  a.n = N; a.xs = xs; a.sidx = sidx; a.begin = begin; a.nplanes = nplanes; a.planes = dpl.p;
+  a.count = count; a.off = off; a.big = big;
+  const unsigned nw = (unsigned)((N + kWaves - 1) / kWaves);
+  hipLaunchKernelGGL(k_near<false>, dim3(nw), dim3(64 * kWaves), 0, s, a);
+  PDG_CK(hipGetLastError());
+  PDG_CK(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, count, off, (int)n1, s));
+  long long B = 0;
+  int hbig = 0;
+  PDG_CK(hipMemcpyAsync(&hbig, big, 4, hipMemcpyDeviceToHost, s));
+  PDG_CK(hipMemcpy(&B, off + N, 8, hipMemcpyDeviceToHost));
+  PDG_CK(hipStreamSynchronize(s));
   const long long size = B + N;
   const long long cap = *listSize;
   *listSize = size;
   if (!nlist) return PDG_OK;
   if (cap < size) return PDG_E_ARG;
-  DevBuf<long long> head, keep64, kpos;
-  PDG_CK(head.alloc(N)); PDG_CK(keep64.alloc(B0)); PDG_CK(kpos.alloc(B0));
-  hipLaunchKernelGGL(k_head, dim3(nb), dim3(256), 0, s, (long long)N, off.p, head.p);
-  // kpos: exclusive scan of keep (as 64-bit)
-  if (B0 > 0) hipLaunchKernelGGL(k_widen, dim3(bb), dim3(256), 0, s, B0, keep.p, keep64.p);
-  if (B0 > 0) { rc = exclusive_scan(keep64.p, kpos.p, B0, s); if (rc) return rc; }
-  DevBuf<int> dl;
-  PDG_CK(dl.alloc(size));
-  hipLaunchKernelGGL(k_emit_counts, dim3(nb), dim3(256), 0, s, N, cnt.p, head.p, dl.p);
-  if (B0 > 0) hipLaunchKernelGGL(k_emit, dim3(bb), dim3(256), 0, s, B0, skeys.p, keep.p, kpos.p, head.p, dl.p);
+  DevBuf<int> list, spill;
+  PDG_CK(list.alloc(size));
+  if (hbig) PDG_CK(spill.alloc((size_t)B + (size_t)N));
+  a.nlist = list.p;
+  a.spill = spill.p;
+  a.flushed = hbig ? spill.p + B : nullptr;
+  hipLaunchKernelGGL(k_near<true>, dim3(nw), dim3(64 * kWaves), 0, s, a);
+  if (hbig)
+    hipLaunchKernelGGL(k_spilled_rows, dim3((unsigned)N), dim3(256), 0, s, N, count, off, spill.p,
+                       a.flushed, list.p);
   PDG_CK(hipGetLastError());
-  PDG_CK(hipMemcpy(nlist, dl.p, 4 * size, hipMemcpyDeviceToHost));
+  PDG_CK(hipMemcpy(nlist, list.p, 4 * size, hipMemcpyDeviceToHost));
   return PDG_OK;
 }
 
