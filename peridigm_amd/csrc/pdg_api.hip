@@ -37,6 +37,69 @@ __global__ void k_set_u_disp(int n, const double* __restrict__ u, const int* __r
   rec[k].u[c] = u[3 * perm[k] + c] * (1.0 / uq);
 }
 
+// Node vectors and scalars between the reference order (host arrays) and the
+// internal order, a component or node per thread: the reordering runs here at
+// memory speed and the host copies whole arrays (a host loop over 640,000
+// nodes took 5 to 10 ms a vector). The scattered side is a node's 24 or 8
+// bytes.
+__global__ void k_vec3_in(int n, const double* __restrict__ ref, const int* __restrict__ perm,
+                          double* __restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 3 * n) return;
+  const int k = t / 3, c = t - 3 * k;
+  out[t] = ref[3 * (size_t)perm[k] + c];
+}
+
+__global__ void k_vec3_out(int n, const double* __restrict__ in, const int* __restrict__ perm,
+                           double* __restrict__ ref) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 3 * n) return;
+  const int k = t / 3, c = t - 3 * k;
+  ref[3 * (size_t)perm[k] + c] = in[t];
+}
+
+__global__ void k_scalar_out(int n, const double* __restrict__ in, const int* __restrict__ perm,
+                             double* __restrict__ ref) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) ref[perm[k]] = in[k];
+}
+
+__global__ void k_disp_out(int n, const NodeRec* __restrict__ rec, const int* __restrict__ perm,
+                           double uq, double* __restrict__ ref) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 3 * n) return;
+  const int k = t / 3, c = t - 3 * k;
+  ref[3 * (size_t)perm[k] + c] = rec[k].u[c] * uq;
+}
+
+__global__ void k_theta_out(int n, const float* __restrict__ theta, const int* __restrict__ perm,
+                            double* __restrict__ ref) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) ref[perm[k]] = (double)theta[k];
+}
+
+// broken bonds over all bonds of the node (0 without bonds, or `none`)
+__global__ void k_damage_out(int n, const int* __restrict__ nbroken, const int* __restrict__ row,
+                             const int* __restrict__ perm, int none, double* __restrict__ ref) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int deg = row[k + 1] - row[k];
+  ref[perm[k]] = !none && deg > 0 ? (double)nbroken[k] / deg : 0.0;
+}
+
+// the records' displacement set to zero
+__global__ void k_zero_u(int n, NodeRec* __restrict__ rec) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 3 * n) rec[t / 3].u[t - 3 * (t / 3)] = 0.0;
+}
+
+// Staging bytes of the node fields of a state: four vectors and two scalars.
+inline size_t state_stage_bytes(int n) {
+  return 4 * (24 * (size_t)n + 64) + 2 * (8 * (size_t)n + 64);
+}
+
+inline dim3 blocks_of(long long n) { return dim3((unsigned)((n + 255) / 256)); }
+
 // Hilbert index of a 21-bit cell triple (Skilling's transpose algorithm:
 // undo excess work, Gray-encode, then interleave with axis 0 most significant).
 uint64_t spread3(uint64_t v);
@@ -348,31 +411,23 @@ char* Ctx::stage(size_t bytes) {
     return nullptr;
   }
   h_stage_bytes = bytes;
+  // its pages are mapped here, not under the first copy
+  parallel_for((long long)bytes, [&](long long lo, long long hi) {
+    std::memset(h_stage + lo, 0, (size_t)(hi - lo));
+  }, 4 << 20);
   return h_stage;
 }
 
-// Current positions y (reference order, host) -> the records' u = y - x,
-// through the pinned staging buffer when it is available. The stream is
-// synchronised first: a call that failed after its upload (a rejected bond
-// field) returns without waiting, and its copy may still read the buffer.
-// Such a call leaves u set to its y.
+// Current positions y (reference order, host) -> the records' u = y - x. The
+// copy reads the caller's array (37 GB/s; through the staging buffer, whose
+// filling takes a thread as long, it is no faster), so the caller synchronises
+// before it returns. A call that fails after this leaves u set to its y.
 int Ctx::upload_y(const double* y) {
   if (N <= 0) return PDG_OK;
-  const size_t vbytes = 24 * (size_t)N;
-  int rc = hip(hipStreamSynchronize(stream), "sync");
-  if (rc) return rc;
-  char* st = stage(vbytes + 4 * (size_t)N);
-  if (st) {
-    parallel_for(3 * (long long)N, [&](long long q0, long long q1) {
-      std::memcpy(st + 8 * q0, y + q0, 8 * (size_t)(q1 - q0));
-    });
-    rc = hip(hipMemcpyAsync(d_y, st, vbytes, hipMemcpyHostToDevice, stream), "h2d y");
-  } else {
-    rc = hip(hipMemcpyAsync(d_y, y, vbytes, hipMemcpyHostToDevice, stream), "h2d y");
-  }
+  int rc = hip(hipMemcpyAsync(d_y, y, 24 * (size_t)N, hipMemcpyHostToDevice, stream), "h2d y");
   if (!rc)
-    hipLaunchKernelGGL(k_set_u, dim3((3 * N + 255) / 256), dim3(256), 0, stream, N, d_y, d_perm,
-                       d_x, d_rec[cur], q);
+    hipLaunchKernelGGL(k_set_u, blocks_of(3ll * N), dim3(256), 0, stream, N, d_y, d_perm, d_x,
+                       d_rec[cur], q);
   return rc;
 }
 
@@ -433,29 +488,82 @@ int Ctx::download_mask(double* bd) {
   return PDG_OK;
 }
 
-// internal-order 3-vectors (device) -> reference order (host)
-int Ctx::download_vec3(const double* dsrc, double* out) {
-  std::vector<double> tmp(3 * (size_t)N);
-  int rc = hip(hipMemcpyAsync(tmp.data(), dsrc, tmp.size() * 8, hipMemcpyDeviceToHost, stream), "d2h");
+int HostOut::add(void* dst, const void* dev, size_t bytes) {
+  if (!bytes) return PDG_OK;
+  Part& p = part_[n_];
+  p = Part{(char*)dst, at_ ? at_ + used_ : nullptr, bytes};
+  int rc = c_->hip(hipMemcpyAsync(at_ ? at_ + used_ : (char*)dst, dev, bytes, hipMemcpyDeviceToHost,
+                                  c_->stream), "d2h");
+  hipEvent_t& e = c_->oev[n_];
+  if (!rc && !e) rc = c_->hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+  if (!rc) rc = c_->hip(hipEventRecord(e, c_->stream), "event");
   if (rc) return rc;
-  rc = hip(hipStreamSynchronize(stream), "sync");
-  if (rc) return rc;
-  parallel_for(N, [&](long long k0, long long k1) {
-    for (int k = (int)k0; k < (int)k1; k++)
-      for (int c = 0; c < 3; c++) out[3 * (size_t)perm[k] + c] = tmp[3 * (size_t)k + c];
-  });
+  used_ += (bytes + 63) & ~(size_t)63;
+  total_ += bytes;
+  n_++;
   return PDG_OK;
 }
 
-int Ctx::upload_vec3(const double* in, double* ddst) {
-  std::vector<double> tmp(3 * (size_t)N);
-  parallel_for(N, [&](long long k0, long long k1) {
-    for (int k = (int)k0; k < (int)k1; k++)
-      for (int c = 0; c < 3; c++) tmp[3 * (size_t)k + c] = in ? in[3 * (size_t)perm[k] + c] : 0.0;
+int HostOut::finish() {
+  const unsigned nt = total_ < (2u << 20) ? 1 : total_ < (32u << 20) ? 4 : 8;
+  std::atomic<int> bad{0};
+  on_threads(at_ ? nt : 1, [&](unsigned t) {
+    for (int k = 0; k < n_; k++) {
+      if (hipEventSynchronize(c_->oev[k]) != hipSuccess) { bad = 1; return; }
+      const Part& p = part_[k];
+      if (!p.src) continue;
+      const size_t lo = (p.bytes / 64 * t / nt) * 64;
+      const size_t hi = t + 1 == nt ? p.bytes : (p.bytes / 64 * (t + 1) / nt) * 64;
+      std::memcpy(p.dst + lo, p.src + lo, hi - lo);
+    }
   });
-  int rc = hip(hipMemcpyAsync(ddst, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, stream), "h2d");
-  if (rc) return rc;
-  return hip(hipStreamSynchronize(stream), "sync");
+  int rc = c_->hip(hipStreamSynchronize(c_->stream), "sync");
+  if (!rc && bad) rc = c_->fail(PDG_E_HIP, "waiting for a result failed");
+  return rc;
+}
+
+int Ctx::download_vec3(const double* dsrc, double* out) {
+  if (N <= 0) return PDG_OK;
+  HostOut o(this, 24 * (size_t)N);
+  hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, stream, N, dsrc, d_perm, d_y);
+  int rc = o.add(out, d_y, 24 * (size_t)N);
+  return rc ? rc : o.finish();
+}
+
+int Ctx::download_scalar(const double* dsrc, double* out) {
+  if (N <= 0) return PDG_OK;
+  HostOut o(this, 8 * (size_t)N);
+  hipLaunchKernelGGL(k_scalar_out, blocks_of(N), dim3(256), 0, stream, N, dsrc, d_perm, d_y);
+  int rc = o.add(out, d_y, 8 * (size_t)N);
+  return rc ? rc : o.finish();
+}
+
+int Ctx::queue_vec3(const double* in, double* ddst, int slot) {
+  if (N <= 0) return PDG_OK;
+  const size_t bytes = 24 * (size_t)N;
+  if (!in) return hip(hipMemsetAsync(ddst, 0, bytes, stream), "zero vector");
+  // small vectors through the staging buffer: a copy from pageable memory
+  // takes up to 250 us to set up
+  constexpr size_t small = 2u << 20;
+  constexpr int slots = 4;
+  const double* src = in;
+  char* st = bytes <= small ? stage(slots * bytes) : nullptr;
+  if (st) {
+    std::memcpy(st + slot * bytes, in, bytes);
+    src = reinterpret_cast<const double*>(st + slot * bytes);
+  }
+  int rc = hip(hipMemcpyAsync(d_y, src, bytes, hipMemcpyHostToDevice, stream), "h2d");
+  if (!rc)
+    hipLaunchKernelGGL(k_vec3_in, blocks_of(3ll * N), dim3(256), 0, stream, N, d_y, d_perm, ddst);
+  // a copy that reads the caller's array is over when this returns
+  if (!rc && !st) rc = hip(hipStreamSynchronize(stream), "sync");
+  return rc;
+}
+
+int Ctx::upload_vec3(const double* in, double* ddst) {
+  int rc = hip(hipStreamSynchronize(stream), "sync");
+  if (!rc) rc = queue_vec3(in, ddst);
+  return rc ? rc : hip(hipStreamSynchronize(stream), "sync");
 }
 
 }  // namespace pdg
@@ -493,6 +601,7 @@ int pdg_ctx_destroy(pdg_ctx* h) {
   c->free_device();
   c->free_extra();
   if (c->h_stage) (void)hipHostFree(c->h_stage);
+  for (hipEvent_t e : c->oev) if (e) (void)hipEventDestroy(e);
   for (int i = 0; i < 4; i++) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
   (void)hipStreamDestroy(c->stream);
   delete c;
@@ -847,6 +956,10 @@ int pdg_set_constants(pdg_ctx* h, const double* x, const double* vol, double K, 
   if (rc) return rc;
   c->cur = 0;
   c->have_consts = true;
+  // the staging buffer of a whole state (u, v, a, force, damage, dilatation),
+  // now rather than in the first call that needs it: pinning and mapping it
+  // take 0.1 to 0.3 ms per MB
+  (void)c->stage(state_stage_bytes(N));
   return PDG_OK;
 }
 
@@ -937,20 +1050,21 @@ int pdg_compute_damage(pdg_ctx* h, const double* y, const double* bdN, double* b
   if (!rc) rc = c->upload_mask(bdN, false);
   if (!rc) rc = c->hip(hipMemsetAsync(c->d_near, 0, 8, s), "zero near");
   if (!rc) rc = c->hip(c->pass1(c->d_rec[c->cur], c->d_nbroken, true, nearCritical != nullptr), "pass1");
-  if (!rc) rc = c->download_mask(bdNP1);
-  if (rc) return rc;
-  std::vector<int> nb(N);
-  rc = c->hip(hipMemcpyAsync(nb.data(), c->d_nbroken, 4 * (size_t)N, hipMemcpyDeviceToHost, s), "d2h nb");
   unsigned long long near = 0;
   if (!rc && nearCritical)
     rc = c->hip(hipMemcpyAsync(&near, c->d_near, 8, hipMemcpyDeviceToHost, s), "d2h near");
-  if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-  if (rc) return rc;
-  for (int k = 0; k < N; k++) {
-    const int deg = c->row[k + 1] - c->row[k];
-    double t = (double)nb[k];
-    damage[c->perm[k]] = deg > 0 ? t / deg : 0.0;
+  if (!rc) rc = c->download_mask(bdNP1);
+  if (rc) {
+    (void)hipStreamSynchronize(s);  // the copy of y reads the caller's array
+    return rc;
   }
+  HostOut o(c, 8 * (size_t)N);
+  if (N > 0)
+    hipLaunchKernelGGL(k_damage_out, blocks_of(N), dim3(256), 0, s, N, c->d_nbroken, c->d_row,
+                       c->d_perm, 0, c->d_y);
+  rc = o.add(damage, c->d_y, 8 * (size_t)N);
+  if (!rc) rc = o.finish();
+  if (rc) return rc;
   if (nearCritical) *nearCritical = (long long)near;
   return PDG_OK;
 }
@@ -965,52 +1079,29 @@ int pdg_compute_force(pdg_ctx* h, double dt, const double* y, const double* bdNP
     // the linearized model and thermal strains through the FP64
     // quasi-static kernels at u = y - x
     int r = c->upload_mask(bdNP1, true);
-    if (r) return r;
-    std::vector<double> u(3 * (size_t)c->N);
-    for (size_t q = 0; q < u.size(); q++) u[q] = y[q] - c->x[q];
-    return pdg_qs_force_dilatation(h, u.data(), force, dilatation);
+    return r ? r : qs_force_at(c, y, force, dilatation);
   }
   hipStream_t s = c->stream;
   const int N = c->N;
-  // y in and f, theta out go through one pinned buffer (PCIe at full rate);
-  // the stream orders the copies, and the call ends synchronised
-  const size_t vbytes = 24 * (size_t)N, tbytes = 4 * (size_t)N;
   int rc = c->upload_y(y);
-  char* st = N > 0 ? c->stage(vbytes + tbytes) : nullptr;  // the buffer upload_y used
   if (!rc) rc = c->upload_mask(bdNP1, true);
   if (!rc) rc = c->hip(c->pass1(c->d_rec[c->cur], nullptr, false, false), "pass1");
   if (!rc) rc = c->hip(c->tiled() ? launch_pass2_tiled_force(c->bond_args(), c->tile_args(), c->d_rec[c->cur], c->d_fout, c->tile_lanes(), c->pipe(), s)
                                   : launch_pass2_force(c->bond_args(), c->d_rec[c->cur], c->d_fout, c->lanes, s),
                        "pass2");
-  if (rc) return rc;
-  if (!st) {
-    rc = c->download_vec3(c->d_fout, force);
-    if (rc) return rc;
-    if (dilatation) {
-      std::vector<float> th(N);
-      rc = c->hip(hipMemcpyAsync(th.data(), c->d_theta, tbytes, hipMemcpyDeviceToHost, s), "d2h theta");
-      if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-      if (rc) return rc;
-      for (int k = 0; k < N; k++) dilatation[c->perm[k]] = (double)th[k];
-    }
-    return PDG_OK;
+  if (rc || N == 0) {
+    (void)hipStreamSynchronize(s);  // the copy of y reads the caller's array
+    return rc;
   }
-  rc = c->hip(hipMemcpyAsync(st, c->d_fout, vbytes, hipMemcpyDeviceToHost, s), "d2h force");
-  if (!rc && dilatation)
-    rc = c->hip(hipMemcpyAsync(st + vbytes, c->d_theta, tbytes, hipMemcpyDeviceToHost, s), "d2h theta");
-  if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-  if (rc) return rc;
-  const double* fs = reinterpret_cast<const double*>(st);
-  const float* ts = reinterpret_cast<const float*>(st + vbytes);
-  const int* perm = c->perm.data();
-  parallel_for(N, [&](long long k0, long long k1) {
-    for (int k = (int)k0; k < (int)k1; k++) {
-      const size_t p = (size_t)perm[k];
-      for (int d = 0; d < 3; d++) force[3 * p + d] = fs[3 * (size_t)k + d];
-      if (dilatation) dilatation[p] = (double)ts[k];
-    }
-  });
-  return PDG_OK;
+  HostOut o(c, 32 * (size_t)N + 128);
+  hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_fout, c->d_perm, c->d_y);
+  rc = o.add(force, c->d_y, 24 * (size_t)N);
+  if (!rc && dilatation) {
+    hipLaunchKernelGGL(k_theta_out, blocks_of(N), dim3(256), 0, s, N, c->d_theta, c->d_perm, c->d_y);
+    rc = o.add(dilatation, c->d_y, 8 * (size_t)N);
+  }
+  const int rc2 = o.finish();
+  return rc ? rc : rc2;
 }
 
 int pdg_state_upload(pdg_ctx* h, const double* u, const double* v, const double* a,
@@ -1020,22 +1111,21 @@ int pdg_state_upload(pdg_ctx* h, const double* u, const double* v, const double*
   (void)hipSetDevice(c->device);
   hipStream_t s = c->stream;
   const int N = c->N;
-  int rc = 0;
-  if (u) {
-    rc = c->hip(hipMemcpyAsync(c->d_y, u, 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d u");
-    if (!rc && N > 0)
-      hipLaunchKernelGGL(k_set_u_disp, dim3((3 * N + 255) / 256), dim3(256), 0, s, N, c->d_y,
-                         c->d_perm, c->d_rec[c->cur], c->q);
-  } else if (N > 0) {
-    std::vector<double> z(3 * (size_t)N, 0.0);
-    rc = c->hip(hipMemcpyAsync(c->d_y, z.data(), 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d u");
-    if (!rc)
-      hipLaunchKernelGGL(k_set_u_disp, dim3((3 * N + 255) / 256), dim3(256), 0, s, N, c->d_y,
-                         c->d_perm, c->d_rec[c->cur], c->q);
-    if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
+  int rc = c->hip(hipStreamSynchronize(s), "sync");
+  if (!rc && N > 0) {
+    if (u) {
+      rc = c->hip(hipMemcpyAsync(c->d_y, u, 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d u");
+      if (!rc)
+        hipLaunchKernelGGL(k_set_u_disp, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_y, c->d_perm,
+                           c->d_rec[c->cur], c->q);
+    } else {
+      hipLaunchKernelGGL(k_zero_u, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_rec[c->cur]);
+    }
   }
-  if (!rc) rc = c->upload_vec3(v, c->d_v);
-  if (!rc) rc = c->upload_vec3(a, c->d_a);
+  if (!rc) rc = c->queue_vec3(v, c->d_v, 0);
+  if (!rc) rc = c->queue_vec3(a, c->d_a, 1);
+  const int rc2 = c->hip(hipStreamSynchronize(s), "sync");
+  if (!rc) rc = rc2;
   if (!rc) rc = c->upload_mask(bd, true);
   if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
   return rc;
@@ -1221,33 +1311,39 @@ int pdg_state_download(pdg_ctx* h, double* u, double* v, double* a, double* bd, 
   (void)hipSetDevice(c->device);
   hipStream_t s = c->stream;
   const int N = c->N;
-  int rc = 0;
-  if (u) {
-    std::vector<NodeRec> rec(N);
-    rc = c->hip(hipMemcpyAsync(rec.data(), c->d_rec[c->cur], N * sizeof(NodeRec), hipMemcpyDeviceToHost, s), "d2h rec");
-    if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-    if (rc) return rc;
-    for (int k = 0; k < N; k++)
-      for (int d = 0; d < 3; d++) u[3 * (size_t)c->perm[k] + d] = rec[k].u[d] * c->q;
-  }
-  if (v && (rc = c->download_vec3(c->d_v, v))) return rc;
-  if (a && (rc = c->download_vec3(c->d_a, a))) return rc;
-  if (force && (rc = c->download_vec3(c->d_f, force))) return rc;
-  if (bd && (rc = c->download_mask(bd))) return rc;
-  if (damage || dilatation) {
-    std::vector<int> nb(N);
-    std::vector<float> th(N);
-    rc = c->hip(hipMemcpyAsync(nb.data(), c->d_nbroken, 4 * (size_t)N, hipMemcpyDeviceToHost, s), "d2h nb");
-    if (!rc) rc = c->hip(hipMemcpyAsync(th.data(), c->d_theta, 4 * (size_t)N, hipMemcpyDeviceToHost, s), "d2h th");
-    if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-    if (rc) return rc;
-    for (int k = 0; k < N; k++) {
-      const int deg = c->row[k + 1] - c->row[k];
-      if (damage) damage[c->perm[k]] = (c->sc > 0.0 && deg > 0) ? (double)nb[k] / deg : 0.0;
-      if (dilatation) dilatation[c->perm[k]] = (double)th[k];
+  const size_t vec = 24 * (size_t)N, sca = 8 * (size_t)N;
+  int rc = PDG_OK;
+  if (N > 0) {
+    // every node field through one scratch vector, each copied out before the
+    // next overwrites it (stream order)
+    HostOut o(c, state_stage_bytes(N));
+    auto vec3 = [&](const double* d, double* out) {
+      if (rc || !out) return;
+      hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, d, c->d_perm, c->d_y);
+      rc = o.add(out, c->d_y, vec);
+    };
+    if (u) {
+      hipLaunchKernelGGL(k_disp_out, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_rec[c->cur],
+                         c->d_perm, c->q, c->d_y);
+      rc = o.add(u, c->d_y, vec);
     }
+    vec3(c->d_v, v);
+    vec3(c->d_a, a);
+    vec3(c->d_f, force);
+    if (!rc && damage) {
+      hipLaunchKernelGGL(k_damage_out, blocks_of(N), dim3(256), 0, s, N, c->d_nbroken, c->d_row,
+                         c->d_perm, c->sc > 0.0 ? 0 : 1, c->d_y);
+      rc = o.add(damage, c->d_y, sca);
+    }
+    if (!rc && dilatation) {
+      hipLaunchKernelGGL(k_theta_out, blocks_of(N), dim3(256), 0, s, N, c->d_theta, c->d_perm, c->d_y);
+      rc = o.add(dilatation, c->d_y, sca);
+    }
+    const int rc2 = o.finish();
+    if (!rc) rc = rc2;
   }
-  return PDG_OK;
+  if (!rc && bd) rc = c->download_mask(bd);
+  return rc;
 }
 
 int pdg_last_timing(const pdg_ctx* h, double* total, double* p1, double* p2) {

@@ -564,6 +564,12 @@ __global__ __launch_bounds__(RB) void k_sub(int n, const double* a, const double
   if (i < n) c[i] = a[i] - b[i];
 }
 
+// v /= the node's volume
+__global__ __launch_bounds__(RB) void k_per_volume(int n, const double* vol, double* v) {
+  const int i = blockIdx.x * RB + threadIdx.x;
+  if (i < n) v[i] /= vol[i / 3];
+}
+
 // out += s * w (damped-Newton diagonal shift)
 __global__ __launch_bounds__(RB) void k_damp_add(int n, const double* sdiag, const double* w,
                                                  double* out) {
@@ -959,13 +965,21 @@ static int ensure(Ctx* c) {
   return rc;
 }
 
-// reference-order 3N host vector -> internal-order device vector
-static int to_dev(Ctx* c, const double* h, double* d) {
-  std::vector<double> t(3 * (size_t)c->N);
-  for (int k = 0; k < c->N; k++)
-    for (int q = 0; q < 3; q++) t[3 * (size_t)k + q] = h[3 * (size_t)c->perm[k] + q];
-  int rc = c->hip(hipMemcpyAsync(d, t.data(), t.size() * 8, hipMemcpyHostToDevice, c->stream), "h2d");
-  if (!rc) rc = c->hip(hipStreamSynchronize(c->stream), "sync");
+// Reference-order 3N host vector -> internal-order device vector, queued; a
+// call's first has slot 0 and waits for what an earlier call left behind. The
+// caller synchronises before it returns (to_host does).
+static int to_dev(Ctx* c, const double* h, double* d, int slot = 0) {
+  int rc = slot == 0 ? c->hip(hipStreamSynchronize(c->stream), "sync") : PDG_OK;
+  return rc ? rc : c->queue_vec3(h, d, slot);
+}
+
+// Positions y (reference order, host) -> S->u = y - x.
+static int u_from_y(Ctx* c, const double* y) {
+  const int n3 = 3 * c->N;
+  int rc = to_dev(c, y, c->qs->u);
+  if (!rc)
+    hipLaunchKernelGGL(k_sub, dim3((n3 + RB - 1) / RB), dim3(RB), 0, c->stream, n3, c->qs->u,
+                       c->qs->x, c->qs->u);
   return rc;
 }
 
@@ -1255,6 +1269,18 @@ static int reaction_norm(Ctx* c, double* norm) {
   return rc;
 }
 
+// Force density and dilatation (optional) at S->u into host arrays.
+static int force_dilatation(Ctx* c, double* force, double* dilatation) {
+  QsState* S = c->qs;
+  int rc = residual(c, true);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_per_volume, dim3((3 * c->N + RB - 1) / RB), dim3(RB), 0, c->stream, 3 * c->N,
+                     S->vol, S->out);
+  rc = to_host(c, S->out, force);
+  if (!rc && dilatation) rc = c->download_scalar(S->theta, dilatation);
+  return rc;
+}
+
 // Destroys the cached iteration graphs (after the stream has drained).
 static void drop_graphs(Ctx* c) {
   QsState* S = c->qs;
@@ -1277,6 +1303,12 @@ static void drop_graphs(Ctx* c) {
 
 int qs_tangent_apply(Ctx* c, const double* w, double* out) { return qs::tangent(c, w, out); }
 int qs_dot(Ctx* c, const double* x, const double* y, double* out) { return qs::dot(c, x, y, out); }
+
+int qs_force_at(Ctx* c, const double* y, double* force, double* dilatation) {
+  int rc = qs::ensure(c);
+  if (!rc) rc = qs::u_from_y(c, y);
+  return rc ? rc : qs::force_dilatation(c, force, dilatation);
+}
 
 double* Ctx::qs_dinv() { return qs ? qs->dinv : nullptr; }
 const signed char* Ctx::qs_fixed() { return qs ? qs->fixed : nullptr; }
@@ -1638,16 +1670,11 @@ int pdg_qs_residual(pdg_ctx* h, const double* u, double* residual, double* norm)
   if (!c || !c->have_consts || !u) return PDG_E_ARG;
   int rc = qs::ensure(c);
   if (!rc) rc = qs::to_dev(c, u, c->qs->u);
-  if (!rc) rc = qs::residual(c);
-  if (rc) return rc;
-  std::vector<double> r(3 * (size_t)c->N);
-  rc = qs::to_host(c, c->qs->out, r.data());
-  if (rc) return rc;
-  double n2 = 0.0, ninf = 0.0;
-  for (double v : r) { n2 += v * v; ninf = std::max(ninf, std::fabs(v)); }
-  if (residual) std::copy(r.begin(), r.end(), residual);
-  if (norm) *norm = std::sqrt(n2) + 20.0 * ninf;
-  return PDG_OK;
+  double rnorm = 0.0;
+  if (!rc) rc = qs::residual_norm(c, &rnorm);
+  if (!rc && residual) rc = qs::to_host(c, c->qs->out, residual);
+  if (!rc && norm) *norm = rnorm;
+  return rc;
 }
 
 int pdg_qs_set_graphs(pdg_ctx* h, int enable) {
@@ -1670,7 +1697,7 @@ int pdg_qs_tangent_apply(pdg_ctx* h, const double* u, const double* w, double* K
   if (!c || !c->have_consts || !u || !w || !Kw) return PDG_E_ARG;
   int rc = qs::ensure(c);
   if (!rc) rc = qs::to_dev(c, u, c->qs->u);
-  if (!rc) rc = qs::to_dev(c, w, c->qs->w);
+  if (!rc) rc = qs::to_dev(c, w, c->qs->w, 1);
   if (!rc) rc = qs::state(c);
   if (!rc) rc = qs::tangent(c, c->qs->w, c->qs->out);
   if (!rc) rc = qs::to_host(c, c->qs->out, Kw);
@@ -1702,8 +1729,8 @@ int pdg_qs_solve(pdg_ctx* h, const double* u, const double* rhs, double* x, int 
   if (!rc) rc = qs::to_dev(c, u, S->u);
   if (!rc && precond >= 1) rc = qs::block_jacobi(c);
   if (!rc && precond == 3 && !S->coarse_ok) rc = qs::coarse_build(c);
-  if (!rc) rc = qs::to_dev(c, rhs, S->b);
-  if (!rc) rc = qs::to_dev(c, x, S->xs);
+  if (!rc) rc = qs::to_dev(c, rhs, S->b, 1);
+  if (!rc) rc = qs::to_dev(c, x, S->xs, 2);
   if (rc) return rc;
   int it = 0;
   double rel = 0.0;
@@ -1734,31 +1761,12 @@ int pdg_qs_newton(pdg_ctx* h, double* u, double tol, int maxNewton, int precond,
   int nit = 0, lit = 0;
   bool converged = false;
   double rnorm = 0.0;
-  std::vector<double> hr(n3);
   double multiplier = 1.0;
-  if (!c->qs_abs_tol) {
-    // reactions: the residual with no rows zeroed, read on the kinematic DOFs
-    std::vector<double> hreac(n3);
-    std::vector<signed char> none(n3, 0);
-    rc = c->hip(hipMemcpyAsync(S->fixed, none.data(), n3, hipMemcpyHostToDevice, c->stream), "h2d");
-    if (!rc) rc = qs::residual(c);
-    if (!rc) rc = c->hip(hipMemcpyAsync(hreac.data(), S->out, 8 * (size_t)n3, hipMemcpyDeviceToHost, c->stream), "d2h");
-    if (!rc) rc = c->hip(hipMemcpyAsync(S->fixed, S->hfixed.data(), n3, hipMemcpyHostToDevice, c->stream), "h2d");
-    if (!rc) rc = c->hip(hipStreamSynchronize(c->stream), "sync");
-    if (rc) return rc;
-    double reac = 0.0;
-    for (int q = 0; q < n3; q++) if (S->hfixed[q]) reac += hreac[q] * hreac[q];
-    multiplier = std::sqrt(reac);
-  }
+  // reactions: f V on the kinematic DOFs
+  if (!c->qs_abs_tol && (rc = qs::reaction_norm(c, &multiplier))) return rc;
   c->qs_tol_multiplier = multiplier;
   for (;; nit++) {
-    if ((rc = qs::residual(c))) return rc;
-    rc = c->hip(hipMemcpyAsync(hr.data(), S->out, 8 * (size_t)n3, hipMemcpyDeviceToHost, c->stream), "d2h");
-    if (!rc) rc = c->hip(hipStreamSynchronize(c->stream), "sync");
-    if (rc) return rc;
-    double n2 = 0.0, ninf = 0.0;
-    for (double v : hr) { n2 += v * v; ninf = std::max(ninf, std::fabs(v)); }
-    rnorm = std::sqrt(n2) + 20.0 * ninf;
+    if ((rc = qs::residual_norm(c, &rnorm))) return rc;
     if (rnorm <= tol * multiplier) { converged = true; break; }
     if (nit == maxNewton) break;
     // the learned and two-level preconditioners use the diagonal blocks too
@@ -1788,23 +1796,8 @@ int pdg_qs_force_dilatation(pdg_ctx* h, const double* u, double* force, double* 
   if (!c || !c->have_consts || !u || !force) return PDG_E_ARG;
   (void)hipSetDevice(c->device);
   int rc = qs::ensure(c);
-  QsState* S = c->qs;
-  if (!rc) rc = qs::to_dev(c, u, S->u);
-  if (rc) return rc;
-  hipStream_t s = c->stream;
-  rc = qs::residual(c, true);
-  if (!rc) rc = qs::to_host(c, S->out, force);
-  if (rc) return rc;
-  for (int p = 0; p < c->N; p++)
-    for (int d = 0; d < 3; d++) force[3 * (size_t)p + d] /= c->vol[p];
-  if (dilatation) {
-    std::vector<double> th(c->N);
-    rc = c->hip(hipMemcpyAsync(th.data(), S->theta, 8 * (size_t)c->N, hipMemcpyDeviceToHost, s), "d2h");
-    if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-    if (rc) return rc;
-    for (int k = 0; k < c->N; k++) dilatation[c->perm[k]] = th[k];
-  }
-  return PDG_OK;
+  if (!rc) rc = qs::to_dev(c, u, c->qs->u);
+  return rc ? rc : qs::force_dilatation(c, force, dilatation);
 }
 
 int pdg_set_thermal_expansion(pdg_ctx* h, double coefficient) {
@@ -1857,9 +1850,7 @@ int pdg_compute_partial_stress(pdg_ctx* h, const double* y, const double* bondDa
   if (!S->ps && (rc = c->hip(hipMalloc((void**)&S->ps, std::max<size_t>(72 * (size_t)N, 64)), "qs alloc")))
     return rc;
   if ((rc = c->upload_mask(bondDamage, true))) return rc;
-  std::vector<double> u(3 * (size_t)N);
-  for (size_t q = 0; q < u.size(); q++) u[q] = y[q] - c->x[q];
-  if ((rc = qs::to_dev(c, u.data(), S->u))) return rc;
+  if ((rc = qs::u_from_y(c, y))) return rc;
   QsArgs a = qs::args(c);
   hipStream_t s = c->stream;
   qs_theta<false, false>(a, s);
