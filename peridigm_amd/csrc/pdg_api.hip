@@ -154,6 +154,7 @@ int Ctx::hip(hipError_t e, const char* what) {
 }
 
 void Ctx::free_device() {
+  free_bond_maps();
   auto F = [](void* p) { if (p) (void)hipFree(p); };
   F(d_row); F(d_col); F(d_mw); F(d_mask); F(d_nc); F(d_rec[0]); F(d_rec[1]); F(d_theta);
   F(d_nbroken); F(d_v); F(d_a); F(d_f); F(d_inv_rho); F(d_bcslot); F(d_bcs); F(d_err); F(d_near);
@@ -429,63 +430,6 @@ int Ctx::upload_y(const double* y) {
     hipLaunchKernelGGL(k_set_u, blocks_of(3ll * N), dim3(256), 0, stream, N, d_y, d_perm, d_x,
                        d_rec[cur], q);
   return rc;
-}
-
-// Host list (reference order) -> device mask words (internal order).
-int Ctx::upload_mask(const double* bd, bool check_symmetric) {
-  if (!bd)  // no field: every bond intact
-    return hip(hipMemsetAsync(d_mask, 0, (size_t)mw.back() * 8, stream), "zero mask");
-  std::vector<unsigned long long> words(mw.back(), 0ull);
-  std::atomic<int> bad_value{0}, asym{0};
-  // each node writes only its own words; a node's bonds are one contiguous
-  // run of the list-order field
-  parallel_for(N, [&](long long i0, long long i1) {
-    for (int i = (int)i0; i < (int)i1; i++) {
-      const int rs = row[i], deg = row[i + 1] - rs;
-      for (int k = 0; k < deg; k++) {
-        const double d = bd[src[rs + k]];
-        if (d != 0.0 && d != 1.0) bad_value = 1;
-        if (d == 1.0) words[mw[i] + (k >> 6)] |= 1ull << (k & 63);
-      }
-    }
-  });
-  if (check_symmetric && !bad_value) {
-    // d_ij == d_ji, checked on the bit words (a few MB) rather than on the
-    // list-order field
-    auto bit = [&](int node, int k) {
-      return (words[mw[node] + (k >> 6)] >> (k & 63)) & 1ull;
-    };
-    parallel_for(N, [&](long long i0, long long i1) {
-      for (int i = (int)i0; i < (int)i1; i++)
-        for (int b = row[i]; b < row[i + 1]; b++) {
-          const int j = col[b];
-          if (bit(i, b - row[i]) != bit(j, rev[b] - row[j])) { asym = 1; return; }
-        }
-    });
-  }
-  if (bad_value) return fail(PDG_E_UNSUPPORTED, "bond damage values must be 0 or 1");
-  if (asym) return fail(PDG_E_UNSUPPORTED, "bond damage must be symmetric (d_ij == d_ji)");
-  int rc = hip(hipMemcpyAsync(d_mask, words.data(), words.size() * 8, hipMemcpyHostToDevice, stream),
-               "upload mask");
-  if (!rc) rc = hip(hipStreamSynchronize(stream), "sync");
-  return rc;
-}
-
-int Ctx::download_mask(double* bd) {
-  std::vector<unsigned long long> words(mw.back());
-  int rc = hip(hipMemcpyAsync(words.data(), d_mask, words.size() * 8, hipMemcpyDeviceToHost, stream),
-               "download mask");
-  if (rc) return rc;
-  rc = hip(hipStreamSynchronize(stream), "sync");
-  if (rc) return rc;
-  parallel_for(N, [&](long long i0, long long i1) {
-    for (int i = (int)i0; i < (int)i1; i++) {
-      const int rs = row[i], deg = row[i + 1] - rs;
-      for (int k = 0; k < deg; k++)
-        bd[src[rs + k]] = ((words[mw[i] + (k >> 6)] >> (k & 63)) & 1ull) ? 1.0 : 0.0;
-    }
-  });
-  return PDG_OK;
 }
 
 int HostOut::add(void* dst, const void* dev, size_t bytes) {

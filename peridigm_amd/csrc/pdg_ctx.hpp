@@ -185,6 +185,17 @@ struct Ctx {
   void free_extra();
   BondArgs bond_args() const;
   hipError_t pass1(NodeRec* rec, int* nbroken, bool damage, bool count_near);
+  // bond fields (pdg_bondfield.hip): maps between the list order and the
+  // internal rows on the device, made by the first call that needs them, bits
+  // in list order, internal words awaiting their check, a chunk of a field
+  int* d_src = nullptr;  // B: list-order index of each internal bond
+  int* d_rev = nullptr;  // B: the reverse bond
+  unsigned long long* d_lbits = nullptr;
+  unsigned long long* d_words = nullptr;
+  double* d_chunk = nullptr;
+  int* d_bad = nullptr;  // 2: a value other than 0 and 1, an asymmetric bond
+  int bond_maps(bool reverse);
+  void free_bond_maps();
   int upload_mask(const double* bd, bool check_symmetric);
   int download_mask(double* bd);
   // node vectors (3n) between the host (reference order) and the device

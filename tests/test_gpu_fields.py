@@ -49,3 +49,38 @@ def _heads(nl, n):
         out.append(p)
         p += nl[p] + 1
     return out
+
+
+# 24 nodes (rows of up to 23 bonds), rows past 64 bonds, and 5.3M bonds (two
+# chunks of the bond field, several threads)
+@pytest.mark.parametrize("n", [(4, 3, 2), (9, 8, 7), (60, 30, 30)])
+def test_bond_field_round_trip(n):
+    from peridigm_amd import Context
+    from peridigm_amd._lib import PdgError
+    from peridigm_amd.core import list_to_csr
+    from peridigm_amd.discretization import lattice_centres, radius_search
+    h = 1e-3
+    x, vol = lattice_centres(n, [0, 0, 0], [k * h for k in n])
+    rng = np.random.default_rng(2)
+    x = x[rng.permutation(len(vol))]
+    N = len(vol)
+    nl = radius_search(x, 3.015 * h)
+    rp, col = list_to_csr(nl, N)
+    i = np.repeat(np.arange(N), np.diff(rp))
+    key = rng.random(N)
+    with Context(0) as ctx:
+        ctx.set_topology(nl, N)
+        ctx.set_constants(x, vol, 130e9, 78e9, 3.015 * h, 0, 1e-2)
+        for share in (0.0, 0.3, 1.0):
+            bd = ((key[np.minimum(i, col)] + key[np.maximum(i, col)]) % 1.0 < share).astype(float)
+            ctx.upload_state(bond_damage=bd)
+            assert np.array_equal(ctx.download_state()["bond_damage"], bd)
+        # a rejected field (one value, or one end only, in the last chunk) leaves
+        # the state as it was
+        for value in (0.5, np.nan, 1.0 - bd[-1]):
+            wrong = bd.copy()
+            wrong[-1] = value
+            with pytest.raises(PdgError) as e:
+                ctx.upload_state(bond_damage=wrong)
+            assert e.value.code == -3
+            assert np.array_equal(ctx.download_state()["bond_damage"], bd)
