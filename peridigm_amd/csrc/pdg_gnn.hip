@@ -66,7 +66,8 @@ struct GnnState {
   float* out = nullptr;       // N x 3
   float* gbuf[2] = {};        // N x 32 fp32 gradients
   float* gagg = nullptr;      // N x 32
-  float* part = nullptr;      // per-tile partial dW/db
+  float* part[gnn::NL] = {};  // per-tile partial dW/db of each layer
+  unsigned short* mean[gnn::NL] = {};  // neighbour means of the last forward pass with `keep`
   float* scales = nullptr;    // [s_r, s_z, loss]
   double* z0 = nullptr;       // D^-1 r (3N)
   double* dz = nullptr;       // z - e (3N), training
@@ -106,111 +107,136 @@ __device__ __forceinline__ f32x4 mfma_block(const unsigned short* A, int lda,
   return acc;
 }
 
-// Builds the [self, mean over neighbours] bf16 input rows of a 64-node tile.
+// Workgroups of the forward layers: 16 threads per node of a 32-node tile (64 nodes
+// and 1,024 threads took 22.8, 20.8 and 17.6 us for the three layers on 24,000
+// nodes, this 22.3, 20.4 and 14.8).
+constexpr int FTILE = 32;
+constexpr int FT = 16 * FTILE;
+
+// Builds the [self, mean over neighbours] bf16 input rows of a 32-node tile
+// and, with `mean`, keeps the means for the backward pass. 16 threads per
+// node: thread (u, q) sums feature chunk q (D/4 features, one 8- or 16-byte
+// vector a neighbour) of the neighbours u, u + 4, u + 8, ... (the last, partial
+// group of four all in u = 0), kAhead of them in flight; the four sums combine
+// as (0 + 1) + (2 + 3). The sums are those of one thread that keeps four
+// accumulators (this kernel before, 27 to 29 us a layer on 24,000 nodes: 27
+// dependent rounds of loads a node), in the same order, so the BF16 means are
+// the same bit for bit. Now 15 to 22 us a layer, bound by L1: 2.5M row reads
+// of 64 bytes at 7.4 TB/s.
+constexpr int kAhead = 8;
 template <int D>
 __device__ void build_inputs(int n, const int* __restrict__ row, const int* __restrict__ col,
                              const unsigned short* __restrict__ hin, int node0,
-                             unsigned short* X, int ldx) {
+                             unsigned short* X, int ldx, unsigned short* __restrict__ mean) {
   // self part
-  for (int q = threadIdx.x; q < gnn::TILE * D; q += 256) {
+  for (int q = threadIdx.x; q < FTILE * D; q += FT) {
     const int r = q / D, c = q - r * D;
     const int node = node0 + r;
     X[r * ldx + c] = node < n ? hin[(size_t)node * D + c] : (unsigned short)0;
   }
-  // mean over neighbours: 4 threads per node, D/4 features each, read as one
-  // 8- or 16-byte vector per neighbour; four neighbours are loaded per round
-  // (independent partial sums, combined in a fixed order) so their loads
-  // overlap
   constexpr int CH = D / 4;
   constexpr int NW = CH / 2;  // 32-bit words (two bf16 each) per chunk
-  const int r = threadIdx.x >> 2, q = threadIdx.x & 3;
+  const int r = threadIdx.x >> 4, u = (threadIdx.x >> 2) & 3, q = threadIdx.x & 3;
   const int node = node0 + r;
-  float acc[4][CH];
+  float acc[CH];
 #pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int c = 0; c < CH; c++) acc[u][c] = 0.0f;
-  int deg = 0;
-  auto add_row = [&](float (&a)[CH], int j) {
-    const unsigned* w = reinterpret_cast<const unsigned*>(hin + (size_t)j * D + q * CH);
-    unsigned v[NW];
+  for (int c = 0; c < CH; c++) acc[c] = 0.0f;
+  const int rs = node < n ? row[node] : 0, deg = node < n ? row[node + 1] - rs : 0;
+  auto load = [&](int b, unsigned (&v)[NW]) {
+    const unsigned* w = reinterpret_cast<const unsigned*>(hin + (size_t)col[b] * D + q * CH);
 #pragma unroll
     for (int k = 0; k < NW; k++) v[k] = w[k];
+  };
+  auto add = [&](const unsigned (&v)[NW]) {
 #pragma unroll
     for (int k = 0; k < NW; k++) {
-      a[2 * k] += __uint_as_float(v[k] << 16);
-      a[2 * k + 1] += __uint_as_float(v[k] & 0xffff0000u);
+      acc[2 * k] += __uint_as_float(v[k] << 16);
+      acc[2 * k + 1] += __uint_as_float(v[k] & 0xffff0000u);
     }
   };
-  if (node < n) {
-    const int rs = row[node], re = row[node + 1];
-    deg = re - rs;
-    int b = rs;
-    for (; b + 4 <= re; b += 4) {
-      const int j0 = col[b], j1 = col[b + 1], j2 = col[b + 2], j3 = col[b + 3];
-      add_row(acc[0], j0);
-      add_row(acc[1], j1);
-      add_row(acc[2], j2);
-      add_row(acc[3], j3);
-    }
-    for (; b < re; b++) add_row(acc[0], col[b]);
-  }
+  const int m = deg >> 2;  // neighbours of this thread in whole groups of four
+  int g = 0;
+  for (; g + kAhead <= m; g += kAhead) {
+    unsigned v[kAhead][NW];
 #pragma unroll
-  for (int c = 0; c < CH; c++) acc[0][c] = (acc[0][c] + acc[1][c]) + (acc[2][c] + acc[3][c]);
+    for (int k = 0; k < kAhead; k++) load(rs + 4 * (g + k) + u, v[k]);
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) add(v[k]);
+  }
+  for (; g < m; g++) {
+    unsigned v[NW];
+    load(rs + 4 * g + u, v);
+    add(v);
+  }
+  if (u == 0)
+    for (int b = rs + 4 * m; b < rs + deg; b++) {
+      unsigned v[NW];
+      load(b, v);
+      add(v);
+    }
   const float inv = deg > 0 ? 1.0f / (float)deg : 0.0f;
 #pragma unroll
-  for (int c = 0; c < CH; c++) X[r * ldx + D + q * CH + c] = f2bf(acc[0][c] * inv);
+  for (int c = 0; c < CH; c++) {
+    // a + b is commutative bit for bit, so lanes 0 and 1 (2 and 3) agree
+    const float pair = acc[c] + __shfl_xor(acc[c], 4);
+    const float other = __shfl_xor(pair, 8);
+    if (u != 0) continue;
+    const unsigned short b = f2bf((pair + other) * inv);
+    X[r * ldx + D + q * CH + c] = b;
+    if (mean && node < n) mean[(size_t)node * D + q * CH + c] = b;
+  }
 }
 
-// Forward of one layer over 64-node tiles.
+// Forward of one layer over 32-node tiles.
 template <int DI, int DO, bool ACT>
-__global__ __launch_bounds__(256) void k_fwd(int n, const int* __restrict__ row,
-                                             const int* __restrict__ col,
-                                             const unsigned short* __restrict__ hin,
-                                             const unsigned short* __restrict__ wt,
-                                             const float* __restrict__ bias,
-                                             unsigned short* __restrict__ hout,
-                                             float* __restrict__ out3) {
+__global__ __launch_bounds__(FT) void k_fwd(int n, const int* __restrict__ row,
+                                            const int* __restrict__ col,
+                                            const unsigned short* __restrict__ hin,
+                                            const unsigned short* __restrict__ wt,
+                                            const float* __restrict__ bias,
+                                            unsigned short* __restrict__ hout,
+                                            float* __restrict__ out3,
+                                            unsigned short* __restrict__ mean) {
   constexpr int K = 2 * DI;
   constexpr int LD = K + 4;
-  __shared__ __align__(16) unsigned short X[gnn::TILE * LD];
+  __shared__ __align__(16) unsigned short X[FTILE * LD];
   __shared__ __align__(16) unsigned short W[DO * LD];
-  const int node0 = blockIdx.x * gnn::TILE;
-  for (int q = threadIdx.x; q < DO * K; q += 256) {
+  const int node0 = blockIdx.x * FTILE;
+  for (int q = threadIdx.x; q < DO * K; q += FT) {
     const int o = q / K, k = q - o * K;
     W[o * LD + k] = wt[o * K + k];
   }
-  build_inputs<DI>(n, row, col, hin, node0, X, LD);
+  build_inputs<DI>(n, row, col, hin, node0, X, LD, mean);
   __syncthreads();
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  // wave w: rows 16 (w & 1).., outputs 16 (w >> 1)..
+  const int w = (threadIdx.x >> 6) & 1, nb = threadIdx.x >> 7, l = threadIdx.x & 63;
+  if (nb >= DO / 16) return;
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  acc = mfma_block<K>(X + (16 * w) * LD, LD, W + (16 * nb) * LD, LD, acc);
+  const int cc = 16 * nb + (l & 15);
+  const float bb = bias[cc];
 #pragma unroll
-  for (int nb = 0; nb < DO / 16; nb++) {
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    acc = mfma_block<K>(X + (16 * w) * LD, LD, W + (16 * nb) * LD, LD, acc);
-    const int cc = 16 * nb + (l & 15);
-    const float bb = bias[cc];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int node = node0 + 16 * w + 4 * (l >> 4) + i;
-      if (node >= n) continue;
-      float z = acc[i] + bb;
-      if (ACT) {
-        hout[(size_t)node * DO + cc] = f2bf(tanhf(z));
-      } else if (cc < 3) {
-        out3[(size_t)node * 3 + cc] = z;
-      }
+  for (int i = 0; i < 4; i++) {
+    const int node = node0 + 16 * w + 4 * (l >> 4) + i;
+    if (node >= n) continue;
+    float z = acc[i] + bb;
+    if (ACT) {
+      hout[(size_t)node * DO + cc] = f2bf(tanhf(z));
+    } else if (cc < 3) {
+      out3[(size_t)node * 3 + cc] = z;
     }
   }
 }
 
-// Backward of one layer: given g (gradient w.r.t. the layer output, fp32,
+// Backward of one layer from the inputs and means that the forward pass left:
+// given g (gradient w.r.t. the layer output, fp32,
 // N x DOG where DOG = DO for hidden layers, 3 for the last), writes per-tile
 // partials of dW (2DI x DO) and db (DO), and gX split into gself (N x DI) and
 // gagg (N x DI, already divided by the node degree).
 template <int DI, int DO, bool ACT, int DOG>
 __global__ __launch_bounds__(256) void k_bwd(int n, const int* __restrict__ row,
-                                             const int* __restrict__ col,
                                              const unsigned short* __restrict__ hin,
+                                             const unsigned short* __restrict__ mean,
                                              const unsigned short* __restrict__ hout,
                                              const float* __restrict__ g,
                                              const unsigned short* __restrict__ wn,
@@ -231,7 +257,12 @@ __global__ __launch_bounds__(256) void k_bwd(int n, const int* __restrict__ row,
     const int k = q / DO, o = q - k * DO;
     Wn[k * LDG + o] = wn[k * DO + o];
   }
-  build_inputs<DI>(n, row, col, hin, node0, X, LDX);
+  for (int q = threadIdx.x; q < gnn::TILE * DI; q += 256) {
+    const int r = q / DI, c = q - r * DI;
+    const int node = node0 + r;
+    X[r * LDX + c] = node < n ? hin[(size_t)node * DI + c] : (unsigned short)0;
+    X[r * LDX + DI + c] = node < n ? mean[(size_t)node * DI + c] : (unsigned short)0;
+  }
   // gz = g * act'(z)
   for (int q = threadIdx.x; q < gnn::TILE * DO; q += 256) {
     const int r = q / DO, o = q - r * DO;
@@ -300,68 +331,151 @@ __global__ __launch_bounds__(256) void k_bwd(int n, const int* __restrict__ row,
   }
 }
 
-// g_in_j = gself_j + sum_{i in N(j)} gagg_i
+// g_in_j = gself_j + sum_{i in N(j)} gagg_i. DI threads per node: thread
+// (u, q) sums four features (one 16-byte vector a neighbour) of the neighbours
+// u, u + 4, ..., kAhead in flight, as build_inputs does, so the sums are those
+// of a thread per feature with four accumulators (41.8 us on 24,000 nodes, now
+// 21.6).
 template <int DI>
 __global__ __launch_bounds__(256) void k_bwd_gather(int n, const int* __restrict__ row,
                                                     const int* __restrict__ col,
                                                     const float* __restrict__ gself,
                                                     const float* __restrict__ gagg,
                                                     float* __restrict__ gin) {
+  constexpr int CH = DI / 4;  // feature chunks, and threads per accumulator
   const int t = blockIdx.x * 256 + threadIdx.x;
-  const int node = t / DI, c = t - (t / DI) * DI;
-  if (node >= n) return;
-  float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-  const int re = row[node + 1];
-  int b = row[node];
-  for (; b + 4 <= re; b += 4) {  // four independent loads in flight
-    s0 += gagg[(size_t)col[b] * DI + c];
-    s1 += gagg[(size_t)col[b + 1] * DI + c];
-    s2 += gagg[(size_t)col[b + 2] * DI + c];
-    s3 += gagg[(size_t)col[b + 3] * DI + c];
+  const int node = t / DI, u = (t & (DI - 1)) / CH, q = t & (CH - 1);
+  const bool valid = node < n;
+  const int rs = valid ? row[node] : 0, deg = valid ? row[node + 1] - rs : 0;
+  f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto load = [&](int b) {
+    return *reinterpret_cast<const f32x4*>(gagg + (size_t)col[b] * DI + 4 * q);
+  };
+  const int m = deg >> 2;
+  int g = 0;
+  for (; g + kAhead <= m; g += kAhead) {
+    f32x4 v[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) v[k] = load(rs + 4 * (g + k) + u);
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) s += v[k];
   }
-  for (; b < re; b++) s0 += gagg[(size_t)col[b] * DI + c];
-  gin[(size_t)node * DI + c] = gself[(size_t)node * DI + c] + ((s0 + s1) + (s2 + s3));
+  for (; g < m; g++) s += load(rs + 4 * g + u);
+  if (u == 0)
+    for (int b = rs + 4 * m; b < rs + deg; b++) s += load(b);
+  f32x4 sum;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const float pair = s[c] + __shfl_xor(s[c], CH);
+    sum[c] = pair + __shfl_xor(pair, 2 * CH);
+  }
+  if (valid && u == 0) {
+    const f32x4 self = *reinterpret_cast<const f32x4*>(gself + (size_t)node * DI + 4 * q);
+    *reinterpret_cast<f32x4*>(gin + (size_t)node * DI + 4 * q) = self + sum;
+  }
 }
 
-// Deterministic sum of per-tile partials into the master gradient layout.
-__global__ __launch_bounds__(256) void k_reduce_layer(int ntiles, const float* __restrict__ part,
-                                                      int di, int dip, int dout, int doutp,
-                                                      float* __restrict__ grad) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  const int np = 2 * di * dout + dout;
-  if (q >= np) return;
-  int src;
-  if (q < 2 * di * dout) {
-    const int half = q / (di * dout);      // 0: self rows, 1: neighbour rows
-    const int rem = q - half * di * dout;
-    const int k = rem / dout, o = rem - (rem / dout) * dout;
-    src = (half * dip + k) * doutp + o;
-  } else {
-    src = 2 * dip * doutp + (q - 2 * di * dout);
-  }
-  const int stride = 2 * dip * doutp + doutp;
+// Deterministic sums of every layer's per-tile partials into the master
+// gradient layout, one launch for all layers. A workgroup takes 16 consecutive
+// parameters; each is summed by 16 threads over a sixteenth of the tiles, four
+// loads in flight, then the 16 sums in order. (A thread per parameter over all
+// tiles in turn, a launch per layer: 92 us each on 375 tiles, now 5 for all.)
+struct ReduceLayer {
+  const float* part;
+  float* grad;
+  int di, dip, dout, doutp, first;  // first: the layer's first workgroup
+};
+struct ReduceArgs {
+  ReduceLayer l[gnn::NL];
+};
+constexpr int kReducePer = 16;
+__global__ __launch_bounds__(256) void k_reduce(int ntiles, ReduceArgs a) {
+  __shared__ float sh[kReducePer][17];
+  int layer = 0;
+  for (int l = 1; l < gnn::NL; l++)
+    if ((int)blockIdx.x >= a.l[l].first) layer = l;
+  const ReduceLayer L = a.l[layer];
+  const int p = threadIdx.x & 15, sl = threadIdx.x >> 4;
+  const int q = (blockIdx.x - L.first) * kReducePer + p;
+  const int np = 2 * L.di * L.dout + L.dout;
+  const int stride = 2 * L.dip * L.doutp + L.doutp;
   float s = 0.0f;
-  for (int t = 0; t < ntiles; t++) s += part[(size_t)t * stride + src];
-  grad[q] = s;
+  if (q < np) {
+    int src;
+    if (q < 2 * L.di * L.dout) {
+      const int half = q / (L.di * L.dout);  // 0: self rows, 1: neighbour rows
+      const int rem = q - half * L.di * L.dout;
+      const int k = rem / L.dout, o = rem - k * L.dout;
+      src = (half * L.dip + k) * L.doutp + o;
+    } else {
+      src = 2 * L.dip * L.doutp + (q - 2 * L.di * L.dout);
+    }
+    const int t0 = ntiles * sl / 16, t1 = ntiles * (sl + 1) / 16;
+    const float* v = L.part + src;
+    float s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+    int t = t0;
+    for (; t + 4 <= t1; t += 4) {
+      s += v[(size_t)t * stride];
+      s1 += v[(size_t)(t + 1) * stride];
+      s2 += v[(size_t)(t + 2) * stride];
+      s3 += v[(size_t)(t + 3) * stride];
+    }
+    for (; t < t1; t++) s += v[(size_t)t * stride];
+    s = (s + s1) + (s2 + s3);
+  }
+  sh[p][sl] = s;
+  __syncthreads();
+  if (sl == 0 && q < np) {
+    float r = 0.0f;
+    for (int k = 0; k < 16; k++) r += sh[p][k];
+    L.grad[q] = r;
+  }
 }
 
-// Packs master FP32 params of a layer into the padded bf16 forward/backward
+// Packs the layers' master FP32 params into the padded bf16 forward/backward
 // weight layouts and the padded bias.
-__global__ void k_pack(const float* __restrict__ p, int di, int dip, int dout, int doutp,
-                       unsigned short* __restrict__ wt, unsigned short* __restrict__ wn,
-                       float* __restrict__ bias) {
+struct PackLayer {
+  const float* p;
+  int di, dip, dout, doutp;
+  unsigned short *wt, *wn;
+  float* bias;
+};
+struct PackArgs {
+  PackLayer l[gnn::NL];
+};
+__global__ void k_pack(PackArgs a) {  // blockIdx.y: the layer
+  const PackLayer L = a.l[blockIdx.y];
   const int q = blockIdx.x * 256 + threadIdx.x;
-  const int K = 2 * dip;
-  if (q < K * doutp) {
-    const int k = q / doutp, o = q - (q / doutp) * doutp;
-    const int half = k / dip, kk = k - half * dip;
+  const int K = 2 * L.dip;
+  if (q < K * L.doutp) {
+    const int k = q / L.doutp, o = q - k * L.doutp;
+    const int half = k / L.dip, kk = k - half * L.dip;
     float v = 0.0f;
-    if (kk < di && o < dout) v = p[half * di * dout + kk * dout + o];
+    if (kk < L.di && o < L.dout) v = L.p[half * L.di * L.dout + kk * L.dout + o];
     const unsigned short b = f2bf(v);
-    wn[k * doutp + o] = b;
-    wt[o * K + k] = b;
+    L.wn[k * L.doutp + o] = b;
+    L.wt[o * K + k] = b;
   }
-  if (q < doutp) bias[q] = q < dout ? p[2 * di * dout + q] : 0.0f;
+  if (q < L.doutp) L.bias[q] = q < L.dout ? L.p[2 * L.di * L.dout + q] : 0.0f;
+}
+
+// Features (8) and 3-vectors between the reference order and the internal one.
+__global__ void k_feat_in(int n, const float* __restrict__ ref, const int* __restrict__ perm,
+                          unsigned short* __restrict__ x) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= 16 * n) return;
+  const int k = t >> 4, q = t & 15;
+  x[t] = q < 8 ? f2bf(ref[8 * (size_t)perm[k] + q]) : (unsigned short)0;
+}
+template <bool IN>
+__global__ void k_vec3f(int n, const float* __restrict__ a, const int* __restrict__ perm,
+                        float* __restrict__ b) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= 3 * n) return;
+  const int k = t / 3, c = t - 3 * k;
+  const size_t r = 3 * (size_t)perm[k] + c;
+  if (IN) b[t] = a[r];
+  else b[r] = a[t];
 }
 
 __global__ void k_adam(int np, float* __restrict__ p, const float* __restrict__ g,
@@ -531,7 +645,10 @@ static int ensure(Ctx* c, unsigned seed) {
   if (!rc) rc = A((void**)&G->gbuf[0], 4 * (size_t)N * 32);
   if (!rc) rc = A((void**)&G->gbuf[1], 4 * (size_t)N * 32);
   if (!rc) rc = A((void**)&G->gagg, 4 * (size_t)N * 32);
-  if (!rc) rc = A((void**)&G->part, 4 * (size_t)G->ntiles * (2 * 32 * 32 + 32));
+  for (int l = 0; l < NL && !rc; l++) {
+    rc = A((void**)&G->part[l], 4 * (size_t)G->ntiles * (2 * DINP[l] * DOUTP[l] + DOUTP[l]));
+    if (!rc) rc = A((void**)&G->mean[l], 2 * (size_t)N * DINP[l]);
+  }
   if (!rc) rc = A((void**)&G->scales, 64);
   if (!rc) rc = A((void**)&G->z0, 24 * (size_t)N);
   if (!rc) rc = A((void**)&G->dz, 24 * (size_t)N);
@@ -558,22 +675,28 @@ static int ensure(Ctx* c, unsigned seed) {
 
 static int pack(Ctx* c) {
   GnnState* G = c->gnn;
+  PackArgs a{};
+  long long most = 0;
   for (int l = 0; l < NL; l++) {
-    const long long cnt = (long long)2 * DINP[l] * DOUTP[l];
-    hipLaunchKernelGGL(k_pack, dim3(nblk(cnt)), dim3(256), 0, c->stream, G->params + param_off(l),
-                       DIN[l], DINP[l], DOUT[l], DOUTP[l], G->wt[l], G->wn[l], G->bias[l]);
+    a.l[l] = PackLayer{G->params + param_off(l), DIN[l], DINP[l], DOUT[l], DOUTP[l],
+                       G->wt[l], G->wn[l], G->bias[l]};
+    most = std::max(most, (long long)2 * DINP[l] * DOUTP[l]);
   }
+  hipLaunchKernelGGL(k_pack, dim3(nblk(most), NL), dim3(256), 0, c->stream, a);
   return c->hip(hipGetLastError(), "gnn pack");
 }
 
-// features already in G->h[0]; runs the three layers into G->out
-static int forward(Ctx* c) {
+// features already in G->h[0]; runs the three layers into G->out (`keep`: a
+// backward pass follows)
+static int forward(Ctx* c, bool keep) {
   GnnState* G = c->gnn;
   const int N = c->N;
-  const dim3 grid(G->ntiles), blk(256);
-  hipLaunchKernelGGL((k_fwd<16, 32, true>), grid, blk, 0, c->stream, N, c->d_row, c->d_col, G->h[0], G->wt[0], G->bias[0], G->h[1], nullptr);
-  hipLaunchKernelGGL((k_fwd<32, 32, true>), grid, blk, 0, c->stream, N, c->d_row, c->d_col, G->h[1], G->wt[1], G->bias[1], G->h[2], nullptr);
-  hipLaunchKernelGGL((k_fwd<32, 16, false>), grid, blk, 0, c->stream, N, c->d_row, c->d_col, G->h[2], G->wt[2], G->bias[2], nullptr, G->out);
+  const dim3 grid((N + FTILE - 1) / FTILE), blk(FT);
+  unsigned short* m[NL];
+  for (int l = 0; l < NL; l++) m[l] = keep ? G->mean[l] : nullptr;
+  hipLaunchKernelGGL((k_fwd<16, 32, true>), grid, blk, 0, c->stream, N, c->d_row, c->d_col, G->h[0], G->wt[0], G->bias[0], G->h[1], nullptr, m[0]);
+  hipLaunchKernelGGL((k_fwd<32, 32, true>), grid, blk, 0, c->stream, N, c->d_row, c->d_col, G->h[1], G->wt[1], G->bias[1], G->h[2], nullptr, m[1]);
+  hipLaunchKernelGGL((k_fwd<32, 16, false>), grid, blk, 0, c->stream, N, c->d_row, c->d_col, G->h[2], G->wt[2], G->bias[2], nullptr, G->out, m[2]);
   return c->hip(hipGetLastError(), "gnn forward");
 }
 
@@ -581,21 +704,25 @@ static int forward(Ctx* c) {
 static int backward(Ctx* c) {
   GnnState* G = c->gnn;
   const int N = c->N;
-  const dim3 grid(G->ntiles), blk(256);
+  const dim3 grid(G->ntiles), blk(256), gat(nblk((long long)N * 32));
   float* g_out = G->gbuf[1];
   float* g_next = G->gbuf[0];
   hipStream_t s = c->stream;
   // layer 3 (identity)
-  hipLaunchKernelGGL((k_bwd<32, 16, false, 3>), grid, blk, 0, s, N, c->d_row, c->d_col, G->h[2], nullptr, g_out, G->wn[2], G->part, g_next, G->gagg, 1);
-  hipLaunchKernelGGL(k_reduce_layer, dim3(nblk(layer_params(2))), blk, 0, s, G->ntiles, G->part, DIN[2], DINP[2], DOUT[2], DOUTP[2], G->grads + param_off(2));
-  hipLaunchKernelGGL((k_bwd_gather<32>), dim3(nblk((long long)N * 32)), blk, 0, s, N, c->d_row, c->d_col, g_next, G->gagg, g_out);
+  hipLaunchKernelGGL((k_bwd<32, 16, false, 3>), grid, blk, 0, s, N, c->d_row, G->h[2], G->mean[2], nullptr, g_out, G->wn[2], G->part[2], g_next, G->gagg, 1);
+  hipLaunchKernelGGL((k_bwd_gather<32>), gat, blk, 0, s, N, c->d_row, c->d_col, g_next, G->gagg, g_out);
   // layer 2
-  hipLaunchKernelGGL((k_bwd<32, 32, true, 32>), grid, blk, 0, s, N, c->d_row, c->d_col, G->h[1], G->h[2], g_out, G->wn[1], G->part, g_next, G->gagg, 1);
-  hipLaunchKernelGGL(k_reduce_layer, dim3(nblk(layer_params(1))), blk, 0, s, G->ntiles, G->part, DIN[1], DINP[1], DOUT[1], DOUTP[1], G->grads + param_off(1));
-  hipLaunchKernelGGL((k_bwd_gather<32>), dim3(nblk((long long)N * 32)), blk, 0, s, N, c->d_row, c->d_col, g_next, G->gagg, g_out);
+  hipLaunchKernelGGL((k_bwd<32, 32, true, 32>), grid, blk, 0, s, N, c->d_row, G->h[1], G->mean[1], G->h[2], g_out, G->wn[1], G->part[1], g_next, G->gagg, 1);
+  hipLaunchKernelGGL((k_bwd_gather<32>), gat, blk, 0, s, N, c->d_row, c->d_col, g_next, G->gagg, g_out);
   // layer 1 (no gradient w.r.t. the features)
-  hipLaunchKernelGGL((k_bwd<16, 32, true, 32>), grid, blk, 0, s, N, c->d_row, c->d_col, G->h[0], G->h[1], g_out, G->wn[0], G->part, g_next, G->gagg, 0);
-  hipLaunchKernelGGL(k_reduce_layer, dim3(nblk(layer_params(0))), blk, 0, s, G->ntiles, G->part, DIN[0], DINP[0], DOUT[0], DOUTP[0], G->grads + param_off(0));
+  hipLaunchKernelGGL((k_bwd<16, 32, true, 32>), grid, blk, 0, s, N, c->d_row, G->h[0], G->mean[0], G->h[1], g_out, G->wn[0], G->part[0], g_next, G->gagg, 0);
+  ReduceArgs a{};
+  int first = 0;
+  for (int l = 0; l < NL; l++) {
+    a.l[l] = ReduceLayer{G->part[l], G->grads + param_off(l), DIN[l], DINP[l], DOUT[l], DOUTP[l], first};
+    first += (layer_params(l) + kReducePer - 1) / kReducePer;
+  }
+  hipLaunchKernelGGL(k_reduce, dim3(first), blk, 0, s, G->ntiles, a);
   return c->hip(hipGetLastError(), "gnn backward");
 }
 
@@ -616,12 +743,14 @@ void Ctx::free_gnn() {
   if (!gnn) return;
   GnnState* G = gnn;
   void* ptrs[] = {G->params, G->grads, G->adam_m, G->adam_v, G->h[0], G->h[1], G->h[2], G->out,
-                  G->gbuf[0], G->gbuf[1], G->gagg, G->part, G->scales, G->z0, G->red, G->dz, G->kdz};
+                  G->gbuf[0], G->gbuf[1], G->gagg, G->scales, G->z0, G->red, G->dz, G->kdz};
   for (void* p : ptrs) if (p) (void)hipFree(p);
   for (int l = 0; l < gnn::NL; l++) {
     if (G->wt[l]) (void)hipFree(G->wt[l]);
     if (G->wn[l]) (void)hipFree(G->wn[l]);
     if (G->bias[l]) (void)hipFree(G->bias[l]);
+    if (G->part[l]) (void)hipFree(G->part[l]);
+    if (G->mean[l]) (void)hipFree(G->mean[l]);
   }
   delete G;
   gnn = nullptr;
@@ -631,7 +760,7 @@ int gnn_apply(Ctx* c, const double* r, double* z) {
   if (!c->gnn || !c->gnn->trained) return c->fail(PDG_E_ARG, "learned preconditioner not trained");
   GnnState* G = c->gnn;
   int rc = gnnh::features(c, r);
-  if (!rc) rc = gnnh::forward(c);
+  if (!rc) rc = gnnh::forward(c, false);
   if (rc) return rc;
   hipLaunchKernelGGL(k_output, dim3(nblk(3LL * c->N)), dim3(256), 0, c->stream, 3 * c->N, G->z0, G->out, c->qs_fixed(), G->scales, z);
   return c->hip(hipGetLastError(), "gnn output");
@@ -682,36 +811,42 @@ int pdg_gnn_forward_backward(pdg_ctx* h, const float* feat, const float* gout, f
   if (!c || !c->gnn || !feat) return PDG_E_ARG;
   GnnState* G = c->gnn;
   const int N = c->N;
-  std::vector<unsigned short> x((size_t)N * 16, 0);
-  auto tobf = [](float f) {
-    unsigned u;
-    std::memcpy(&u, &f, 4);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-  };
-  for (int k = 0; k < N; k++)
-    for (int q = 0; q < 8; q++) x[(size_t)k * 16 + q] = tobf(feat[(size_t)c->perm[k] * 8 + q]);
-  int rc = c->hip(hipMemcpyAsync(G->h[0], x.data(), 2 * x.size(), hipMemcpyHostToDevice, c->stream), "h2d");
-  if (!rc) rc = gnnh::pack(c);
-  if (!rc) rc = gnnh::forward(c);
-  if (rc) return rc;
-  std::vector<float> o((size_t)N * 3);
-  rc = c->hip(hipMemcpyAsync(o.data(), G->out, 4 * o.size(), hipMemcpyDeviceToHost, c->stream), "d2h");
-  if (!rc) rc = c->hip(hipStreamSynchronize(c->stream), "sync");
-  if (rc) return rc;
-  if (out)
-    for (int k = 0; k < N; k++)
-      for (int q = 0; q < 3; q++) out[(size_t)c->perm[k] * 3 + q] = o[(size_t)k * 3 + q];
-  if (gout && dparams) {
-    std::vector<float> g((size_t)N * 3);
-    for (int k = 0; k < N; k++)
-      for (int q = 0; q < 3; q++) g[(size_t)k * 3 + q] = gout[(size_t)c->perm[k] * 3 + q];
-    rc = c->hip(hipMemcpyAsync(G->gbuf[1], g.data(), 4 * g.size(), hipMemcpyHostToDevice, c->stream), "h2d");
-    if (!rc) rc = gnnh::backward(c);
-    if (!rc) rc = c->hip(hipMemcpyAsync(dparams, G->grads, 4 * (size_t)gnn::total_params(), hipMemcpyDeviceToHost, c->stream), "d2h");
-    if (!rc) rc = c->hip(hipStreamSynchronize(c->stream), "sync");
+  hipStream_t s = c->stream;
+  const bool grad = gout && dparams;
+  const size_t fb = 32 * (size_t)N, gb = 12 * (size_t)N, pb = 4 * (size_t)gnn::total_params();
+  // both inputs through the staging buffer when it is there (small copies from
+  // pageable memory take up to 250 us to set up)
+  int rc = c->hip(hipStreamSynchronize(s), "sync");
+  char* st = c->stage(fb + gb + pb + 256);
+  const void *fsrc = feat, *gsrc = gout;
+  if (st) {
+    std::memcpy(st, feat, fb);
+    fsrc = st;
+    if (grad) {
+      std::memcpy(st + fb, gout, gb);
+      gsrc = st + fb;
+    }
   }
-  return rc;
+  if (!rc && N > 0) {
+    rc = c->hip(hipMemcpyAsync(G->gbuf[0], fsrc, fb, hipMemcpyHostToDevice, s), "h2d");
+    hipLaunchKernelGGL(k_feat_in, dim3(nblk(16ll * N)), dim3(256), 0, s, N, G->gbuf[0], c->d_perm, G->h[0]);
+  }
+  if (!rc) rc = gnnh::pack(c);
+  if (!rc) rc = gnnh::forward(c, grad);
+  if (!rc && grad) {
+    rc = c->hip(hipMemcpyAsync(G->gbuf[0], gsrc, gb, hipMemcpyHostToDevice, s), "h2d");
+    if (N > 0)
+      hipLaunchKernelGGL(k_vec3f<true>, dim3(nblk(3ll * N)), dim3(256), 0, s, N, G->gbuf[0], c->d_perm, G->gbuf[1]);
+    if (!rc) rc = gnnh::backward(c);
+  }
+  HostOut o(c, gb + pb + 256);
+  if (!rc && out && N > 0) {
+    hipLaunchKernelGGL(k_vec3f<false>, dim3(nblk(3ll * N)), dim3(256), 0, s, N, G->out, c->d_perm, G->gbuf[0]);
+    rc = o.add(out, G->gbuf[0], gb);
+  }
+  if (!rc && grad) rc = o.add(dparams, G->grads, pb);
+  const int rc2 = o.finish();
+  return rc ? rc : rc2;
 }
 
 // Trains on (r, e = K^-1 r) pairs, vectors in reference order (nsamples x 3N),
@@ -765,7 +900,7 @@ int pdg_gnn_train(pdg_ctx* h, const double* u, int nsamples, const double* r, co
       const double* es = de + (size_t)order[q] * n3;
       rc = gnnh::pack(c);
       if (!rc) rc = gnnh::features(c, rs);
-      if (!rc) rc = gnnh::forward(c);
+      if (!rc) rc = gnnh::forward(c, true);
       if (rc) break;
       hipLaunchKernelGGL(k_step_error, dim3(nblk(n3)), dim3(256), 0, s, n3, es, G->z0, G->out, c->qs_fixed(), G->scales, G->dz);
       rc = qs_tangent_apply(c, G->dz, G->kdz);
