@@ -242,6 +242,13 @@ int pdg_last_timing(const pdg_ctx* ctx, double* totalMs, double* pass1Ms, double
  * synchronisation, only the total time is recorded. */
 int pdg_set_per_pass_timing(pdg_ctx* ctx, int on);
 
+/* Longest time (s, 0 to 10; 0.2 by default) that a tile of a resident explicit
+ * run waits for another. A pdg_verlet_run of 16 or more steps on a small mesh
+ * keeps every tile on the GPU for all of them; when a wait ends in vain, as it
+ * soon does with 0, the run is repeated with two launches a step, as later
+ * ones are until this is called again. The results are the same. */
+int pdg_set_resident_wait(pdg_ctx* ctx, double seconds);
+
 /* Near-critical count of the last pdg_verlet_run / pdg_verlet_run_persistent
  * (or of the last pdg_compute_damage that asked for one): the number of
  * (bond, damage evaluation) pairs in which an intact bond's FP32 stretch lay

@@ -272,6 +272,9 @@ class Context:
     def set_per_pass_timing(self, on=True):
         self.check(self.lib.pdg_set_per_pass_timing(self.h, int(bool(on))))
 
+    def set_resident_wait(self, seconds=0.2):
+        self.check(self.lib.pdg_set_resident_wait(self.h, seconds))
+
     def last_timing(self):
         t = C.c_double(); a = C.c_double(); b = C.c_double()
         self.check(self.lib.pdg_last_timing(self.h, C.byref(t), C.byref(a), C.byref(b)))

@@ -159,6 +159,9 @@ void Ctx::free_device() {
   F(d_row); F(d_col); F(d_mw); F(d_mask); F(d_nc); F(d_rec[0]); F(d_rec[1]); F(d_theta);
   F(d_nbroken); F(d_v); F(d_a); F(d_f); F(d_inv_rho); F(d_bcslot); F(d_bcs); F(d_err); F(d_near);
   F(d_perm); F(d_fout); F(d_y); F(d_vol); F(d_x);
+  F(d_xch); F(d_mask_old);
+  d_xch = d_mask_old = nullptr;
+  resident_max = -1;
   F(d_tile_start); F(d_halo_off); F(d_halo); F(d_own_off); F(d_lcol);
   d_tile_start = d_halo_off = d_halo = d_own_off = nullptr;
   d_lcol = nullptr;
@@ -429,6 +432,72 @@ int Ctx::upload_y(const double* y) {
   if (!rc)
     hipLaunchKernelGGL(k_set_u, blocks_of(3ll * N), dim3(256), 0, stream, N, d_y, d_perm, d_x,
                        d_rec[cur], q);
+  return rc;
+}
+
+// Whether an explicit run of nsteps is resident: tiles of 32 nodes (meshes of
+// up to 16,384 nodes give at most 512, two to a CU) and enough steps to pay for
+// the copies of v and the mask and the cooperative launch (they add 45 to 60
+// us, and a step saves 3 to 5; at 16 steps both take the same).
+bool Ctx::resident_run(int nsteps) const {
+  return variant == 0 && ntiles > 0 && tile_nodes == 32 && tile_lanes() == 16 && !resident_off &&
+         !per_pass_timing && sc_t.empty() && nsteps >= 16;
+}
+
+// Evaluations first..nsteps of an explicit run from the displacement in
+// d_rec[cur], resident. *done is false when the mesh has too many tiles for
+// it, when its memory or launch is refused, or when a tile waited in vain: the
+// state is then as before.
+int Ctx::run_resident(const VerletArgs& va, int first, int nsteps, double t0, bool damage,
+                      bool* done) {
+  *done = false;
+  const BondArgs ba = bond_args();
+  if (resident_max < 0) resident_max = resident_tiles(ba.influence, damage);
+  if (ntiles > resident_max) return PDG_OK;
+  const size_t n = (size_t)N, words = 13 * n + 1, vb = 24 * n, mb = 8 * (size_t)mw.back();
+  int rc = PDG_OK;
+  if (!d_xch) {
+    if (hipMalloc((void**)&d_xch, 8 * words) != hipSuccess ||
+        hipMalloc((void**)&d_mask_old, std::max<size_t>(mb, 64)) != hipSuccess) {
+      (void)hipGetLastError();
+      (void)hipFree(d_xch);
+      d_xch = d_mask_old = nullptr;
+      resident_off = true;
+      return PDG_OK;
+    }
+    xch_tag = 0xffffffffu;  // clear the words
+  }
+  if (!rc && xch_tag > 0xffffffffu - (unsigned)nsteps - 2u) {
+    rc = hip(hipMemsetAsync(d_xch, 0, 8 * words, stream), "clear exchange");
+    xch_tag = 1;
+  }
+  int* const stuck = reinterpret_cast<int*>(d_xch + 13 * n);
+  if (!rc) rc = hip(hipMemcpyAsync(d_fout, d_v, vb, hipMemcpyDeviceToDevice, stream), "copy v");
+  if (!rc && damage) rc = hip(hipMemcpyAsync(d_mask_old, d_mask, mb, hipMemcpyDeviceToDevice, stream), "copy mask");
+  if (rc) return rc;
+  ResidentArgs x{d_xch, d_xch + 12 * n, xch_tag, stuck, resident_wait};
+  if (launch_resident(ba, tile_args(), x, d_rec[cur], d_rec[cur ^ 1], d_theta, d_nbroken, va,
+                      first, nsteps, t0, damage, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    resident_off = true;
+    return PDG_OK;
+  }
+  xch_tag += (unsigned)nsteps + 2u;
+  int bad = 0;
+  if (!rc) rc = hip(hipMemcpyAsync(&bad, stuck, 4, hipMemcpyDeviceToHost, stream), "d2h");
+  if (!rc) rc = hip(hipStreamSynchronize(stream), "sync");
+  if (rc) return rc;
+  if (!bad) {
+    cur ^= 1;
+    *done = true;
+    return PDG_OK;
+  }
+  resident_off = true;
+  rc = hip(hipMemsetAsync(stuck, 0, 4, stream), "clear flag");
+  if (!rc) rc = hip(hipMemcpyAsync(d_v, d_fout, vb, hipMemcpyDeviceToDevice, stream), "restore v");
+  if (!rc && damage) rc = hip(hipMemcpyAsync(d_mask, d_mask_old, mb, hipMemcpyDeviceToDevice, stream), "restore mask");
+  if (!rc) rc = hip(hipMemsetAsync(d_err, 0, 4, stream), "zero err");
+  if (!rc) rc = hip(hipMemsetAsync(d_near, 0, 8, stream), "zero near");
   return rc;
 }
 
@@ -1165,16 +1234,25 @@ int pdg_verlet_run(pdg_ctx* h, int nsteps, double dt, double t0, int initialEval
     c->cur ^= 1;
     return r;
   };
+  bool resident = !contact && c->resident_run(nsteps);
   if (initialEval) {
-    rc = eval(0, false);
+    if (resident) {
+      c->sc_cur = c->sc_value;
+      rc = c->run_resident(va, 0, nsteps, t0, damage, &resident);
+    }
+    if (!rc && !resident) rc = eval(0, false);
   } else if (nsteps > 0) {
     va.t_cur = step_time(1);
     va.t_prev = step_time(0);
     va.inv_dtbc = 1.0 / (va.t_cur - va.t_prev);
     rc = c->hip(launch_verlet_prologue(c->N, c->d_rec[c->cur], c->d_rec[c->cur ^ 1], va, s), "prologue");
     c->cur ^= 1;
+    if (!rc && resident) {
+      c->sc_cur = c->sc_value;
+      rc = c->run_resident(va, 1, nsteps, t0, damage, &resident);
+    }
   }
-  for (int k = 1; k <= nsteps && !rc; k++) rc = eval(k, true);
+  for (int k = 1; k <= nsteps && !rc && !resident; k++) rc = eval(k, true);
   c->sc_cur = c->sc_value;
   if (rc) return rc;
   rc = c->hip(hipEventRecord(c->ev[3], s), "event");
@@ -1303,6 +1381,14 @@ int pdg_set_per_pass_timing(pdg_ctx* h, int on) {
   Ctx* c = reinterpret_cast<Ctx*>(h);
   if (!c) return PDG_E_ARG;
   c->per_pass_timing = on != 0;
+  return PDG_OK;
+}
+
+int pdg_set_resident_wait(pdg_ctx* h, double seconds) {
+  Ctx* c = reinterpret_cast<Ctx*>(h);
+  if (!c || !(seconds >= 0.0) || seconds > 10.0) return PDG_E_ARG;
+  c->resident_wait = (unsigned long long)(1e8 * seconds);
+  c->resident_off = false;
   return PDG_OK;
 }
 

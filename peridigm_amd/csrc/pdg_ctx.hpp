@@ -119,6 +119,17 @@ struct Ctx {
   double* d_fout = nullptr;
   double* d_y = nullptr;
   double* d_inv_rho = nullptr;  // n: 1 / density (internal order)
+  // resident explicit runs: exchange words, the next number to use, copies of
+  // v and the mask from before the run, and whether a run got stuck (later
+  // ones then launch their steps)
+  unsigned long long* d_xch = nullptr;  // 13n + 1 (the last: the stuck flag)
+  unsigned xch_tag = 1;
+  int resident_max = -1;  // most tiles (-1: not asked yet)
+  unsigned long long* d_mask_old = nullptr;
+  bool resident_off = false;
+  unsigned long long resident_wait = 20000000ull;  // 100 MHz ticks
+  bool resident_run(int nsteps) const;
+  int run_resident(const VerletArgs& va, int first, int nsteps, double t0, bool damage, bool* done);
   int* d_bcslot = nullptr;
   BcSlot* d_bcs = nullptr;
   int* d_err = nullptr;

@@ -133,6 +133,26 @@ hipError_t launch_persistent(const BondArgs& a, const TileArgs& t, NodeRec* rec0
                              double t0, int initial_eval, bool damage, int lanes, int* grid_out,
                              hipStream_t s);
 
+// Resident explicit run (pdg_tiles.hip): evaluations first..nsteps of a small
+// mesh with 32-node tiles and 16 lanes per node in one cooperative launch, the
+// tiles exchanging displacements (x.u, 12n words, two buffers) and dilatation
+// terms (x.p, n words) numbered x.tag + evaluation; numbers must not repeat.
+// Reads u from rec, ends with it in rec_end. *x.stuck is set, and the state
+// left half-way, if a tile waited in vain.
+struct ResidentArgs {
+  unsigned long long* u;
+  unsigned long long* p;
+  unsigned tag;
+  int* stuck;
+  unsigned long long wait;  // 100 MHz ticks a workgroup waits for another
+};
+// Most tiles that are resident together (0: no cooperative launch).
+int resident_tiles(int influence, bool damage);
+hipError_t launch_resident(const BondArgs& a, const TileArgs& t, const ResidentArgs& x,
+                           const NodeRec* rec, NodeRec* rec_end, float* theta, int* nbroken,
+                           const VerletArgs& va, int first, int nsteps, double t0, bool damage,
+                           hipStream_t s);
+
 // Launchers (pdg_bonds.hip). `lanes` = lanes per node (16, 32 or 64; smaller
 // values run as 16).
 hipError_t launch_pass1(const BondArgs& a, NodeRec* rec, float* theta, int* nbroken,

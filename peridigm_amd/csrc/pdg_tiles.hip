@@ -773,6 +773,263 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_persistent(BondArgs a, T
   }
 }
 
+// Resident explicit run of a small mesh: one workgroup per tile, all of them
+// on the GPU at once, for every step of the run. A small mesh is bound by
+// latency: two launches a step, each with three rounds of dependent loads
+// before its bond loop (10,000 nodes, 313 tiles: 5.7 + 6.0 us a step, of which
+// the bond loops take about 2.5). Here a tile keeps its rows, mask words,
+// constants, halo positions and Verlet state in registers and LDS, and only
+// displacements and dilatation terms travel: a node's are stored as 8-byte
+// words of 32 bits of data and the 32-bit number of the evaluation they belong
+// to, and whoever needs them reads the words until the numbers match. A word
+// is valid by itself, so there is no flag, no fence and no barrier between
+// workgroups; an exchange costs one store and one load past the L2s. (Grid
+// barriers cost 3 to 5 us here, more than a launch.)
+//
+// Measured a step, against two launches: 980 nodes 5.5 us (10.5), 3,840 nodes
+// 5.8 (11), 10,000 nodes 8.4 (11.7), 16,000 nodes 9.0; above 256 tiles some CUs
+// run two. Words of one kind lie together (node by node: a wave reads runs of
+// them; 48 bytes a node instead took 9.9 us at 10,000 nodes), and the
+// dilatation terms are first waited for by one thread per neighbouring tile
+// (8.4 us; all threads polling 8.9, the same for displacements 8.9). Half a
+// tile per workgroup, for evener CUs, took 9.4: twice the halo reads.
+//
+// A tile that is one exchange ahead of another never writes what that one
+// still reads: displacements alternate between two buffers, and the dilatation
+// words of evaluation k + 1 are stored after its displacements have arrived,
+// which their owners send after reading those of k.
+//
+// Every wait ends: after x.wait ticks of the 100 MHz clock a workgroup sets
+// *stuck and leaves, and the host repeats the run with two launches a step
+// from its copy of the state. The same arithmetic as those, bit for bit.
+constexpr int RG = 16;  // lanes per node (32-node tiles)
+
+__device__ __forceinline__ void word_put(unsigned long long* p, unsigned data, unsigned tag) {
+  __hip_atomic_store(p, (unsigned long long)tag << 32 | data, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long word_get(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Reads the NW words p[0], p[stride], ... until all carry `tag`; false after
+// `limit` ticks (looked at every 64 reads; 0: after the first).
+template <int NW>
+__device__ __forceinline__ bool words_wait(const unsigned long long* p, int stride, unsigned tag,
+                                           unsigned long long limit, unsigned (&v)[NW]) {
+  unsigned long long began = 0ull;
+  for (int tries = 0;; tries++) {
+    unsigned long long w[NW];
+#pragma unroll
+    for (int k = 0; k < NW; k++) w[k] = word_get(p + (size_t)k * stride);
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < NW; k++) {
+      ok = ok && (unsigned)(w[k] >> 32) == tag;
+      v[k] = (unsigned)w[k];
+    }
+    if (ok) return true;
+    if ((tries & 63) == 63 || limit == 0ull) {
+      const unsigned long long now = wall_clock64();
+      if (!began) began = now;
+      if (now - began >= limit) return false;
+    }
+  }
+}
+
+template <bool DAMAGE, int INFL>
+__global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
+    BondArgs a, TileArgs t, ResidentArgs x, const NodeRec* __restrict__ rec,
+    NodeRec* __restrict__ rec_end, float* __restrict__ theta, int* __restrict__ nbroken,
+    VerletArgs va, int first, int nsteps, double t0) {
+  __shared__ TileLds L;
+  __shared__ int bad;
+  const int tile = blockIdx.x;
+  const int n0 = t.tile_start[tile], n1 = t.tile_start[tile + 1];
+  const int h0 = t.halo_off[tile], hn = min(t.halo_off[tile + 1] - h0, HMAX);
+  const int own = t.own_off[tile];
+  const int grp = threadIdx.x / RG, g = (threadIdx.x & 63) / RG, l = threadIdx.x & (RG - 1);
+  const int node = n0 + grp;
+  const bool valid = node < n1;
+  if (threadIdx.x == 0) bad = 0;
+  // the start, as in the passes
+  HaloStage hs;
+  halo_idx(hs, t, h0, hn);
+  RowData<RG> rd;
+  row_scalars<RG>(a, node, valid, n0, rd);
+  const int q = threadIdx.x, qk = q / 3, ql = q - 3 * qk;
+  const bool has_q = q < 3 * (n1 - n0);
+  const VerletPre vp = verlet_pre(va, n0 + (has_q ? qk : 0), has_q ? ql : 0);
+  double v_own = vp.v;
+  double u_own = rec[(unsigned)(n0 + (has_q ? qk : 0))].u[has_q ? ql : 0];
+  const bool bc = has_q && va.bc_slot[n0 + qk] >= 0;
+  const BcSlot* const bcs = va.bcs + (bc ? va.bc_slot[n0 + qk] : 0);
+  halo_load(hs, rec);
+  row_arrays<RG>(a, t, l, valid, rd);
+  halo_write<false>(L, hs);
+  float hvol[kSlotsPerThread], halpha[kSlotsPerThread];
+  bool last[kSlotsPerThread];  // the halo's last slot of its tile
+#pragma unroll
+  for (int r = 0; r < kSlotsPerThread; r++) {
+    hvol[r] = hs.v[r].vol;
+    halpha[r] = hs.v[r].alpha;
+    const int h = threadIdx.x + r * WG;
+    last[r] = false;
+    if (h < hn) {
+      int lo = 0;  // the tile of node idx
+      for (int step = 1 << 15; step > 0; step >>= 1)
+        if (lo + step < t.ntiles && t.tile_start[lo + step] <= hs.idx[r]) lo += step;
+      last[r] = h + 1 == hn || t.halo[h0 + h + 1] >= t.tile_start[lo + 1];
+    }
+  }
+  __syncthreads();
+  const int deg = rd.deg, nmax = wave_trips<RG>(deg);
+  const float scz = (a.sc_now > 0.0f && rd.c.sc > 0.0f) ? a.sc_now : rd.c.sc;
+  const float nlim = a.near_rel * scz;
+  const int me = kLdsSlot * (valid ? own + grp : 0);
+  unsigned long long near = 0ull;
+  for (int k = first; k <= nsteps; k++) {
+    const unsigned tag = x.tag + (unsigned)k;
+    if (k > first) {
+      // the halo's displacements
+      const unsigned long long* src = x.u + (size_t)(k & 1) * 6 * a.n;
+#pragma unroll
+      for (int r = 0; r < kSlotsPerThread; r++) {
+        const int h = threadIdx.x + r * WG;
+        if (r > 0 && r * WG >= hn) break;
+        unsigned w[6] = {0, 0, 0, 0, 0, 0};
+        if (h < hn && !words_wait<6>(src + hs.idx[r], a.n, tag, x.wait, w)) bad = 1;
+        if (h < hn) {
+          lds_put(lds_b(L), h, make_uint4(w[0], w[1], w[2], w[3]));
+          lds_put(lds_c(L), h, make_uint2(w[4], w[5]));
+        }
+      }
+      __syncthreads();
+      if (bad) break;
+    }
+    // damage and dilatation
+    Nb nb{};
+    if (valid) nb = nb_load(L, me);
+    unsigned ih[2 * NWORDS];
+    lane_intact<RG>(rd.m, l, ih);
+    P1Loop<RG, DAMAGE, DAMAGE, INFL == kPairModelPmb ? 0 : INFL> p1{
+        L, rd.lj, ih, nmax, nb.x0, nb.x1, nb.x2, nb.u0, nb.u1, nb.u2, scz, nlim, rd.c.hhat, {}, {}};
+#pragma unroll
+    for (int it = 0; it < MAXDEG / RG; ++it) p1.balv[it] = 0ull;
+    p1.nb[0] = nb_load(L, rd.lj[0]);
+    p1.nb[1] = nb_load(L, rd.lj[1]);
+    p1.template step<0>();
+    if (DAMAGE) {
+      near += p1.nnear_w;
+#pragma unroll
+      for (int it = 0; it < MAXDEG / RG; ++it) {
+        if (p1.balv[it] == 0ull) continue;
+        const unsigned long long gb = (p1.balv[it] >> (g * RG)) & ((1ull << RG) - 1ull);
+        rd.m[(it * RG) >> 6] |= gb << ((it * RG) & 63);
+      }
+    }
+    const float acc = group_sum<RG>(p1.acc);
+    if (valid && l == 0) {
+      word_put(x.p + node, __float_as_uint(rd.c.kp * acc), tag);
+      if (k == nsteps) {
+        theta[node] = rd.c.ctheta * acc;
+        if (DAMAGE) {
+          const int nw = (deg + 63) >> 6;
+          int nbr = 0;
+#pragma unroll
+          for (int w = 0; w < NWORDS; w++) {
+            const unsigned long long m = rd.m[w] & valid_bits(deg, w);
+            if (w < nw) a.mask[(unsigned)(rd.w0 + w)] = m;
+            nbr += __popcll(m);
+          }
+          nbroken[node] = nbr;
+        }
+      }
+    }
+    // the halo's dilatation terms, next to the displacements in array c (the
+    // dilatation loop reads the other half of its slots)
+#pragma unroll
+    for (int r = 0; r < kSlotsPerThread; r++) {
+      unsigned w[1];
+      if (last[r] && !words_wait<1>(x.p + hs.idx[r], 0, tag, x.wait, w)) bad = 1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSlotsPerThread; r++) {
+      const int h = threadIdx.x + r * WG;
+      if (r > 0 && r * WG >= hn) break;
+      unsigned w[1] = {0};
+      if (h < hn && !words_wait<1>(x.p + hs.idx[r], 0, tag, x.wait, w)) bad = 1;
+      if (h < hn) {
+        const float p = __uint_as_float(w[0]);
+        const float dp[2] = {hvol[r] * (halpha[r] - p), hvol[r] * p};
+        *reinterpret_cast<float2*>(lds_c(L) + kLdsSlot * h + 8) = make_float2(dp[0], dp[1]);
+      }
+    }
+    __syncthreads();
+    if (bad) break;
+    // force
+    Nb2 n2{};
+    float d_i = 0.0f, p_i = 0.0f;
+    if (valid) {
+      n2 = nb2_load(L, me);
+      const float rv = n2.vol > 0.0f ? __builtin_amdgcn_rcpf(n2.vol) : 0.0f;
+      d_i = n2.vd * rv;
+      p_i = n2.vp * rv;
+    }
+    lane_intact<RG>(rd.m, l, ih);
+    P2Loop<RG, INFL> p2{L, rd.lj, ih, nmax, n2.x0, n2.x1, n2.x2, n2.u0, n2.u1, n2.u2,
+                        p_i, d_i, rd.c.hhat, a.pmb_c, {}};
+    p2.nb[0] = nb2_load(L, rd.lj[0]);
+    p2.nb[1] = nb2_load(L, rd.lj[1]);
+    p2.template step<0>();
+    const float f0 = group_sum<RG>(p2.f0), f1 = group_sum<RG>(p2.f1), f2 = group_sum<RG>(p2.f2);
+    if (valid && l < 3) L.sf[3 * grp + l] = (l == 0 ? f0 : (l == 1 ? f1 : f2)) * a.fq;
+    __syncthreads();
+    // velocity Verlet of this thread's component, as verlet_epilogue
+    if (has_q) {
+      const double tot = (double)L.sf[q];
+      if (!isfinite(tot)) *va.err = 1;
+      double ac = tot;
+      ac += 0.0;
+      ac *= vp.inv_rho;
+      const double dt2 = va.dt / 2.0;
+      double u = u_own * va.uq;
+      if (k > 0) v_own = v_own + dt2 * ac;
+      if (k < nsteps) {
+        v_own = v_own + dt2 * ac;
+        if (bc && ((bcs->mask >> ql) & 1)) {
+          const double t_cur = t0 + ((k + 1) * va.dt), t_prev = t0 + (k * va.dt);
+          const double inv_dtbc = 1.0 / (t_cur - t_prev);
+          const double c0 = bcs->c0[ql], c1 = bcs->c1[ql];
+          const double cur = c1 * t_cur + c0;
+          double prev = c1 * t_prev + c0;
+          if (cur - prev == 0.0) prev = u;
+          v_own = 0.0 * (cur - prev) + 1.0 * (cur - prev) * inv_dtbc;
+        }
+        u = u + va.dt * v_own;
+      } else {
+        va.a[3 * (n0 + qk) + ql] = ac;
+        va.f[3 * (n0 + qk) + ql] = tot;
+        va.v[3 * (n0 + qk) + ql] = v_own;
+      }
+      u_own = u * va.inv_uq;
+      if (k < nsteps) {
+        unsigned long long* dst = x.u + (size_t)(((k + 1) & 1) * 6 + 2 * ql) * a.n + (n0 + qk);
+        word_put(dst, (unsigned)__double2loint(u_own), tag + 1u);
+        word_put(dst + a.n, (unsigned)__double2hiint(u_own), tag + 1u);
+      } else {
+        rec_end[n0 + qk].u[ql] = u_own;
+      }
+    }
+  }
+  if (bad) {
+    if (threadIdx.x == 0) *x.stuck = 1;
+    return;
+  }
+  if (DAMAGE && near && (threadIdx.x & 63) == 0) atomicAdd(a.near_ctr, near);
+}
+
 // pipe: the pipelined branch-free bond loops (default); the plain loops are
 // kept for G = 16 as a measured alternative.
 template <int G, int INFL, bool PIPE>
@@ -870,6 +1127,41 @@ hipError_t launch_persistent(const BondArgs& a, const TileArgs& t, NodeRec* rec0
   VerletArgs vv = va;
   void* args[] = {&aa, &tt, &rec0, &rec1, &theta, &nbroken, &vv, &nsteps, &t0, &initial_eval};
   return hipLaunchCooperativeKernel(fn, dim3(nb), dim3(WG), args, 0, s);
+}
+
+namespace {
+const void* resident_fn(int influence, bool damage) {
+  if (influence == kPairModelPmb)
+    return damage ? (const void*)k_resident<true, kPairModelPmb> : (const void*)k_resident<false, kPairModelPmb>;
+  if (influence == PDG_INFLUENCE_ONE)
+    return damage ? (const void*)k_resident<true, 0> : (const void*)k_resident<false, 0>;
+  if (influence == PDG_INFLUENCE_PARABOLIC_DECAY)
+    return damage ? (const void*)k_resident<true, 1> : (const void*)k_resident<false, 1>;
+  return damage ? (const void*)k_resident<true, 2> : (const void*)k_resident<false, 2>;
+}
+}  // namespace
+
+int resident_tiles(int influence, bool damage) {
+  int dev = 0, ncu = 0, per_cu = 0, coop = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, resident_fn(influence, damage), WG, 0) != hipSuccess)
+    return 0;
+  return per_cu * ncu;
+}
+
+hipError_t launch_resident(const BondArgs& a, const TileArgs& t, const ResidentArgs& x,
+                           const NodeRec* rec, NodeRec* rec_end, float* theta, int* nbroken,
+                           const VerletArgs& va, int first, int nsteps, double t0, bool damage,
+                           hipStream_t s) {
+  BondArgs aa = a;
+  TileArgs tt = t;
+  ResidentArgs xx = x;
+  VerletArgs vv = va;
+  vv.start_step = 1;  // boundary-condition slots are loaded
+  void* args[] = {&aa, &tt, &xx, &rec, &rec_end, &theta, &nbroken, &vv, &first, &nsteps, &t0};
+  return hipLaunchCooperativeKernel(resident_fn(a.influence, damage), dim3(t.ntiles), dim3(WG), args, 0, s);
 }
 
 hipError_t launch_pass1_tiled(const BondArgs& a, const TileArgs& t, NodeRec* rec, float* theta,
