@@ -38,6 +38,7 @@ struct CoarseGrid {
   double o[3] = {0.0, 0.0, 0.0};
   double H = 1.0;
   int points() const { return d[0] * d[1] * d[2]; }
+  int cells() const { return (d[0] - 1) * (d[1] - 1) * (d[2] - 1); }
 };
 
 struct QsState {
@@ -100,12 +101,14 @@ struct QsState {
   CoarseGrid cgr;
   int nc = 0;
   bool coarse_ok = false;
-  int* cstart = nullptr;  // grid points + 1: each point's nodes in clist
-  int* clist = nullptr;   // 8n: nodes of the cells around each grid point
-  double* wlist = nullptr;  // 8n: the grid point's weight at each entry of clist
-  double* cpart = nullptr;  // 3 kCoarseSplit points: restriction partials
-  double* cinv = nullptr;    // nc x nc inverse of P^T K P (dropped functions: zero)
-  double* cmat = nullptr;    // nc x nc build buffer
+  bool grid_ok = false;     // the grid and the lists below hold (they depend on x alone)
+  int* cstart = nullptr;    // cells + 1: each cell's nodes in clist
+  int* clist = nullptr;     // n: nodes by cell, in order
+  double* ct = nullptr;     // 3n: local coordinates at each entry of clist
+  double* cpart = nullptr;  // 3 x 24 per block of k_restrict
+  double* cinv = nullptr;   // nc x nc inverse of P^T K P (dropped functions: zero)
+  double* cmat = nullptr;   // nc x nc build buffer
+  double* cdmax = nullptr;  // largest diagonal entry of P^T K P
   double* cy = nullptr;      // nc: coarse solution
 };
 
@@ -667,87 +670,250 @@ __device__ __forceinline__ int corner_id(const CoarseGrid& G, const int c[3], in
   return (c[0] + (q & 1)) + G.d[0] * ((c[1] + ((q >> 1) & 1)) + G.d[1] * (c[2] + ((q >> 2) & 1)));
 }
 
-// Weight of grid point g at node i (0 when g is not a corner of i's cell)
-__device__ __forceinline__ double point_w(const CoarseGrid& G, const double* p, int g) {
+// Local coordinates at the entries of the cells' lists
+__global__ __launch_bounds__(RB) void k_coarse_local(int n, CoarseGrid G, const int* __restrict__ list,
+                                                     const double* __restrict__ x,
+                                                     double* __restrict__ ct) {
+  const int e = blockIdx.x * RB + threadIdx.x;
+  if (e >= n) return;
   int c[3];
   double t[3];
-  coarse_cell(G, p, c, t);
-  double w = 0.0;
-  for (int q = 0; q < 8; q++) w += corner_id(G, c, q) == g ? corner_w(q, t) : 0.0;
-  return w;
+  coarse_cell(G, x + 3 * (size_t)list[e], c, t);
+  for (int k = 0; k < 3; k++) ct[3 * (size_t)e + k] = t[k];
 }
 
-// Weights of the restriction lists: wlist[e] = weight of grid point pt at
-// node clist[e], for the entries e of pt's list (one block per point, once
-// per set-up)
-__global__ __launch_bounds__(RB) void k_coarse_weights(CoarseGrid G, const int* __restrict__ start,
-                                                       const int* __restrict__ list,
-                                                       const double* __restrict__ x,
-                                                       double* __restrict__ wlist) {
-  const int pt = blockIdx.x;
-  for (int e = start[pt] + threadIdx.x; e < start[pt + 1]; e += RB)
-    wlist[e] = point_w(G, x + 3 * (size_t)list[e], pt);
-}
-
-constexpr int kCoarseSplit = 8;  // blocks per grid point in the restriction
-
-// Restriction partials: block (pt, sp) sums phi_(pt,k) . r over the sp-th
-// eighth of pt's list into part[3 (pt kCoarseSplit + sp) + k]
-__global__ __launch_bounds__(RB) void k_coarse_partial(const int* __restrict__ start,
-                                                       const int* __restrict__ list,
-                                                       const double* __restrict__ wlist,
-                                                       const signed char* __restrict__ fixed,
-                                                       const double* __restrict__ r,
-                                                       double* __restrict__ part) {
-  __shared__ double sh[RB / 64];
-  const int pt = blockIdx.x / kCoarseSplit, sp = blockIdx.x - kCoarseSplit * pt;
-  const int e0 = start[pt], len = start[pt + 1] - e0;
-  const int b0 = e0 + (int)((long long)len * sp / kCoarseSplit);
-  const int b1 = e0 + (int)((long long)len * (sp + 1) / kCoarseSplit);
-  double acc[3] = {0.0, 0.0, 0.0};
-  for (int e = b0 + threadIdx.x; e < b1; e += RB) {
+// Restriction P^T r by cells: a node adds to the 8 corners of its cell, so a
+// block takes a share of one cell's nodes, each node once, and leaves the 24
+// sums of the corners in part[24 block + 3 corner + k]. (A list of nodes per
+// grid point instead, with stored weights, read every node's r 8 times: 20 us
+// against 7 on the 200,000-node bar.) blockIdx.y picks one of three vectors
+// (the set-up's probes); launches after the end of a solve return at once.
+constexpr int kCellSplit = 2;  // blocks per cell
+constexpr int kRestrictThreads = 1024;
+__global__ __launch_bounds__(kRestrictThreads) void k_restrict(
+    const QsCg* cg, const int* __restrict__ start, const int* __restrict__ list,
+    const double* __restrict__ ct, const signed char* __restrict__ fixed, const double* r0,
+    const double* r1, const double* r2, double* __restrict__ part) {
+  constexpr int NW = kRestrictThreads / 64;
+  __shared__ double sh[NW][24];
+  if (cg && cg->done) return;
+  const double* __restrict__ r = blockIdx.y == 0 ? r0 : blockIdx.y == 1 ? r1 : r2;
+  const int cell = blockIdx.x / kCellSplit, sp = blockIdx.x - kCellSplit * cell;
+  const int e0 = start[cell], len = start[cell + 1] - e0;
+  const int b0 = e0 + (int)((long long)len * sp / kCellSplit);
+  const int b1 = e0 + (int)((long long)len * (sp + 1) / kCellSplit);
+  double acc[24];
+#pragma unroll
+  for (int k = 0; k < 24; k++) acc[k] = 0.0;
+  const int active = min(NW, (b1 - b0 + 63) >> 6);  // waves with nodes
+  for (int e = b0 + threadIdx.x; e < b1; e += kRestrictThreads) {
     const int i = list[e];
-    const double w = wlist[e];
-    for (int k = 0; k < 3; k++) acc[k] += fixed[3 * i + k] ? 0.0 : w * r[3 * i + k];
+    const double t[3] = {ct[3 * (size_t)e], ct[3 * (size_t)e + 1], ct[3 * (size_t)e + 2]};
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) v[k] = fixed[3 * (size_t)i + k] ? 0.0 : r[3 * (size_t)i + k];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const double w = corner_w(q, t);
+#pragma unroll
+      for (int k = 0; k < 3; k++) acc[3 * q + k] += w * v[k];
+    }
   }
-  for (int k = 0; k < 3; k++) {
-    const double t = block_sum(acc[k], sh);
-    if (threadIdx.x == 0) part[3 * (size_t)blockIdx.x + k] = t;
+  // the wave's sums: three exchanges halve the values that a lane holds, which
+  // leaves 3 to each group of 8 lanes
+  if ((int)(threadIdx.x >> 6) < active) {
+    int first = 0;
+#pragma unroll
+    for (int h = 0; h < 3; h++) {
+      const int xr = 32 >> h, half = 12 >> h;
+      const bool up = (threadIdx.x & xr) != 0;
+      if (up) first += half;
+#pragma unroll
+      for (int k = 0; k < half; k++) {
+        const double send = up ? acc[k] : acc[k + half], keep = up ? acc[k + half] : acc[k];
+        acc[k] = keep + __shfl_xor(send, xr);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double v = group_sum64<8>(acc[k]);
+      if ((threadIdx.x & 7) == 0) sh[threadIdx.x >> 6][first + k] = v;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 24) {
+    double v = 0.0;
+    for (int w = 0; w < active; w++) v += sh[w][threadIdx.x];
+    part[24 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x) + threadIdx.x] = v;
   }
 }
 
-// g = P^T r from the partials (fixed order), then, when SOLVE, y = Cinv g:
-// every block forms g in LDS and its waves take rows (lanes over a row);
-// without SOLVE block 0 writes g to `out` (a column of the coarse matrix at
-// set-up)
-template <bool SOLVE>
-__global__ __launch_bounds__(RB) void k_coarse_finish(int nc, const double* __restrict__ part,
-                                                      const double* __restrict__ cinv,
-                                                      double* __restrict__ out) {
-  __shared__ double gl[3 * kCoarsePointsMax];
-  if (!SOLVE && blockIdx.x > 0) return;
-  for (int t = threadIdx.x; t < nc; t += RB) {
-    const int pt = t / 3, k = t - 3 * pt;
-    double v = 0.0;
-    for (int sp = 0; sp < kCoarseSplit; sp++) v += part[3 * (size_t)(pt * kCoarseSplit + sp) + k];
-    if (SOLVE) gl[t] = v;
-    else out[t] = v;
+// Function j = 3 point + k of P^T r: the point's corner in the up to 8 cells
+// around it, in a fixed order
+__device__ __forceinline__ double restricted(const CoarseGrid& G, const double* __restrict__ part,
+                                             int j) {
+  const int pt = j / 3, k = j - 3 * pt;
+  const int p0 = pt % G.d[0], p1 = (pt / G.d[0]) % G.d[1], p2 = pt / (G.d[0] * G.d[1]);
+  double v = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int c0 = p0 - (q & 1), c1 = p1 - ((q >> 1) & 1), c2 = p2 - ((q >> 2) & 1);
+    if (c0 < 0 || c1 < 0 || c2 < 0 || c0 >= G.d[0] - 1 || c1 >= G.d[1] - 1 || c2 >= G.d[2] - 1) continue;
+    const int cell = c0 + (G.d[0] - 1) * (c1 + (G.d[1] - 1) * c2);
+#pragma unroll
+    for (int sp = 0; sp < kCellSplit; sp++)
+      v += part[24 * (size_t)(cell * kCellSplit + sp) + 3 * q + k];
   }
-  if (!SOLVE) return;
+  return v;
+}
+
+// y = Cinv P^T r: every block forms P^T r in LDS and its waves take rows
+// (lanes over a row)
+__global__ __launch_bounds__(RB) void k_coarse_solve(const QsCg* cg, CoarseGrid G, int nc,
+                                                     const double* __restrict__ part,
+                                                     const double* __restrict__ cinv,
+                                                     double* __restrict__ y) {
+  __shared__ double gl[3 * kCoarsePointsMax];
+  if (cg->done) return;
+  for (int t = threadIdx.x; t < nc; t += RB) gl[t] = restricted(G, part, t);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   for (int row = blockIdx.x * (RB / 64) + (threadIdx.x >> 6); row < nc; row += gridDim.x * (RB / 64)) {
     const double* c = cinv + (size_t)row * nc;
     double v = 0.0;
     for (int k = lane; k < nc; k += 64) v += c[k] * gl[k];
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) out[row] = v;
+    v = wave_sum64(v);
+    if (lane == 0) y[row] = v;
   }
 }
 
-// Probe vector of the coarse set-up: the sum of the coarse functions (g, k0)
-// over the grid points g of one colour (gx, gy, gz congruent to cx, cy, cz
-// modulo `stride`)
+// P^T of three probes' images (one block each) into rows of R
+__global__ __launch_bounds__(RB) void k_coarse_columns(CoarseGrid G, int nc, int blocks,
+                                                       const double* __restrict__ part,
+                                                       double* __restrict__ R) {
+  for (int t = threadIdx.x; t < nc; t += RB)
+    R[(size_t)blockIdx.x * nc + t] = restricted(G, part + 24 * (size_t)blockIdx.x * blocks, t);
+}
+
+// M = P^T K P, symmetrised, from the probes' rows of R: entry (target t,
+// source g) stands in the row of g's colour when t and g are within reach on
+// every axis, and is 0 otherwise
+struct ProbeColours {
+  int reach, stride, d[3];  // colours per axis
+};
+__global__ __launch_bounds__(RB) void k_coarse_matrix(CoarseGrid G, ProbeColours pc, int nc,
+                                                      const double* __restrict__ R,
+                                                      double* __restrict__ M) {
+  const int e = blockIdx.x * RB + threadIdx.x;
+  if (e >= nc * nc) return;
+  const int i = e / nc, j = e - nc * i;
+  const int pi = i / 3, pj = j / 3;
+  const int a[3] = {pi % G.d[0], (pi / G.d[0]) % G.d[1], pi / (G.d[0] * G.d[1])};
+  const int b[3] = {pj % G.d[0], (pj / G.d[0]) % G.d[1], pj / (G.d[0] * G.d[1])};
+  bool near = true;
+  for (int d = 0; d < 3; d++) near = near && abs(a[d] - b[d]) <= pc.reach;
+  auto row = [&](const int g[3], int k) {
+    return (((g[2] % pc.stride) * pc.d[1] + g[1] % pc.stride) * pc.d[0] + g[0] % pc.stride) * 3 + k;
+  };
+  M[e] = near ? 0.5 * (R[(size_t)row(a, i - 3 * pi) * nc + j] + R[(size_t)row(b, j - 3 * pj) * nc + i])
+              : 0.0;
+}
+
+__global__ __launch_bounds__(RB) void k_coarse_dmax(int nc, const double* __restrict__ M, double* dmax) {
+  __shared__ double sh[RB];
+  double m = 0.0;
+  for (int i = threadIdx.x; i < nc; i += RB) m = fmax(m, M[(size_t)i * nc + i]);
+  sh[threadIdx.x] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < RB; k++) m = fmax(m, sh[k]);
+    *dmax = m;
+  }
+}
+
+// One step of the block Gauss-Jordan inversion of a symmetric positive matrix
+// (no pivoting needed): rows and columns p0 .. p0 + kGj - 1 leave. With the
+// pivot block's inverse P, out = in - in(:, K) P in(K, :) outside the pivots'
+// rows and columns, P in(K, :) in the rows, -in(:, K) P in the columns and P
+// where they meet. Every block inverts the pivot block itself and takes a tile
+// of the matrix; steps alternate between two buffers. A pivot at or below
+// 1e-12 of the largest diagonal entry of the start (or a NaN) is dropped: its
+// row and column become 0. Latency of the pivots' serial chain bounds it: 30
+// steps of 13 us at 480 functions, where factorising on the host took 30 ms.
+constexpr int kGj = 16;
+constexpr int kGjTile = 48;
+__global__ __launch_bounds__(RB) void k_gj_step(int nc, int p0, const double* __restrict__ in,
+                                                const double* __restrict__ dmax,
+                                                double* __restrict__ out) {
+  __shared__ double P[kGj][kGj + 1];
+  __shared__ double rows[kGj][kGjTile + 1];   // in(K, tile columns), then P times it
+  __shared__ double cols[kGjTile][kGj + 1];   // in(tile rows, K)
+  const int b = min(kGj, nc - p0);
+  const int i0 = blockIdx.y * kGjTile, j0 = blockIdx.x * kGjTile;
+  const int pi = threadIdx.x / kGj, pj = threadIdx.x % kGj;
+  const double cut = 1e-12 * *dmax;
+  P[pi][pj] = pi < b && pj < b ? in[(size_t)(p0 + pi) * nc + p0 + pj] : 0.0;
+  for (int e = threadIdx.x; e < kGj * kGjTile; e += RB) {
+    const int k = e / kGjTile, j = e - kGjTile * k;
+    rows[k][j] = k < b && j0 + j < nc ? in[(size_t)(p0 + k) * nc + j0 + j] : 0.0;
+    const int r = e / kGj, q = e - kGj * r;
+    cols[r][q] = q < b && i0 + r < nc ? in[(size_t)(i0 + r) * nc + p0 + q] : 0.0;
+  }
+  __syncthreads();
+  unsigned dropped = 0u;
+  for (int p = 0; p < b; p++) {
+    const double d = P[p][p], rp = P[p][pj], cp = P[pi][p], v = P[pi][pj];
+    __syncthreads();
+    if (!(d > cut)) {
+      dropped |= 1u << p;
+      continue;
+    }
+    const double id = 1.0 / d;
+    P[pi][pj] = pi == p ? (pj == p ? id : rp * id) : (pj == p ? -cp * id : v - cp * (rp * id));
+    __syncthreads();
+  }
+  if (dropped >> pi & 1u || dropped >> pj & 1u) P[pi][pj] = 0.0;
+  for (int e = threadIdx.x; e < kGj * kGjTile; e += RB) {
+    const int k = e / kGjTile, r = e / kGj, q = e - kGj * r;
+    if (dropped >> k & 1u) rows[k][e - kGjTile * k] = 0.0;
+    if (dropped >> q & 1u) cols[r][q] = 0.0;
+  }
+  __syncthreads();
+  double t[kGj * kGjTile / RB];
+#pragma unroll
+  for (int m = 0; m < kGj * kGjTile / RB; m++) {
+    const int e = threadIdx.x + m * RB, k = e / kGjTile, j = e - kGjTile * k;
+    const int jk = j0 + j - p0;  // pivot column
+    double v = 0.0;
+    for (int q = 0; q < kGj; q++) v += P[k][q] * rows[q][j];
+    t[m] = jk >= 0 && jk < b ? P[k][jk] : v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < kGj * kGjTile / RB; m++) {
+    const int e = threadIdx.x + m * RB, k = e / kGjTile;
+    rows[k][e - kGjTile * k] = t[m];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < kGjTile * kGjTile; e += RB) {
+    const int r = e / kGjTile, j = e - kGjTile * r;
+    if (i0 + r >= nc || j0 + j >= nc) continue;
+    const int ik = i0 + r - p0, jk = j0 + j - p0;
+    double v;
+    if (ik >= 0 && ik < b) {
+      v = rows[ik][j];
+    } else {
+      double s = 0.0;
+      for (int q = 0; q < kGj; q++) s += cols[r][q] * rows[q][j];
+      v = (jk >= 0 && jk < b ? 0.0 : in[(size_t)(i0 + r) * nc + j0 + j]) - s;
+    }
+    out[(size_t)(i0 + r) * nc + j0 + j] = v;
+  }
+}
+
+// Probe vector of the coarse set-up: the sum of the coarse functions (g, k0),
+// or with k0 < 0 of all three of a point, over the grid points g of one colour
+// (gx, gy, gz congruent to cx, cy, cz modulo `stride`)
 __global__ __launch_bounds__(RB) void k_coarse_probe(int n, CoarseGrid G, int stride, int cx, int cy,
                                                      int cz, int k0, const double* __restrict__ x,
                                                      const signed char* __restrict__ fixed,
@@ -763,11 +929,11 @@ __global__ __launch_bounds__(RB) void k_coarse_probe(int n, CoarseGrid G, int st
                     (c[2] + ((q >> 2) & 1)) % stride == cz;
     w += in ? corner_w(q, t) : 0.0;
   }
-  for (int k = 0; k < 3; k++) v[3 * i + k] = (k == k0 && !fixed[3 * i + k]) ? w : 0.0;
+  for (int k = 0; k < 3; k++) v[3 * i + k] = ((k0 < 0 || k == k0) && !fixed[3 * i + k]) ? w : 0.0;
 }
 
-// Linear index of each node's cell (the lists of the restriction are built
-// from it on the host, so they follow the device's cell assignment)
+// Index of each node's cell (the lists of the restriction are built from it on
+// the host, so they follow the device's cell assignment)
 __global__ __launch_bounds__(RB) void k_coarse_cells(int n, CoarseGrid G, const double* __restrict__ x,
                                                      int* __restrict__ cell) {
   const int i = blockIdx.x * RB + threadIdx.x;
@@ -775,12 +941,13 @@ __global__ __launch_bounds__(RB) void k_coarse_cells(int n, CoarseGrid G, const 
   int c[3];
   double t[3];
   coarse_cell(G, x + 3 * (size_t)i, c, t);
-  cell[i] = c[0] + G.d[0] * (c[1] + G.d[1] * c[2]);
+  cell[i] = c[0] + (G.d[0] - 1) * (c[1] + (G.d[1] - 1) * c[2]);
 }
 
 // z = Dinv r + P y (the two-level preconditioner), with the partial sums of
 // r.z (grid-stride over nodes, one partial per block, like k_dot)
-__global__ __launch_bounds__(RB) void k_two_level_apply(int n, const double* __restrict__ dinv,
+__global__ __launch_bounds__(RB) void k_two_level_apply(const QsCg* cg, int n,
+                                                        const double* __restrict__ dinv,
                                                         CoarseGrid G, const double* __restrict__ x,
                                                         const signed char* __restrict__ fixed,
                                                         const double* __restrict__ y,
@@ -788,6 +955,7 @@ __global__ __launch_bounds__(RB) void k_two_level_apply(int n, const double* __r
                                                         double* __restrict__ z,
                                                         double* __restrict__ part) {
   __shared__ double sh[RB / 64];
+  if (cg->done) return;
   double s = 0.0;
   for (int i = blockIdx.x * RB + threadIdx.x; i < n; i += gridDim.x * RB) {
     const double* D = dinv + 9 * i;
@@ -1049,31 +1217,24 @@ static int block_jacobi(Ctx* c) {
   return c->hip(hipGetLastError(), "qs block jacobi");
 }
 
-// Two-level preconditioner set-up at the current state: the coarse grid
-// (at most coarse_points_cap(n) points, spacing equal on all axes, centred on
-// the bounding box), the node lists of the restriction, and the inverse of
-// the coarse matrix A_c = P^T K P, column by column from one tangent apply
-// per coarse function. A_c is inverted on the host by Cholesky
-// factorisation; a function whose pivot falls below 1e-12 of the largest
-// diagonal entry (a grid point whose nodes' DOFs are all prescribed, or none
-// at all) is dropped: its row and column of the inverse are 0.
-static int coarse_build(Ctx* c) {
+// The two-level preconditioner's grid (at most coarse_points_cap(n) points,
+// spacing equal on all axes, centred on the bounding box) and the node lists
+// of the restriction, which depend on the positions alone.
+static int coarse_grid(Ctx* c) {
   QsState* S = c->qs;
   const int N = c->N;
   hipStream_t s = c->stream;
-  auto A = [&](void** p, size_t bytes) { return c->hip(hipMalloc(p, std::max<size_t>(bytes, 64)), "qs coarse alloc"); };
-  int rc = 0;
+  auto A = [&](void** p, size_t bytes) { return *p ? PDG_OK : c->hip(hipMalloc(p, std::max<size_t>(bytes, 64)), "qs coarse alloc"); };
   const size_t mc = 3 * (size_t)kCoarsePointsMax;
-  if (!S->clist) {
-    rc = A((void**)&S->clist, 32 * (size_t)N);
-    if (!rc) rc = A((void**)&S->wlist, 64 * (size_t)N);
-    if (!rc) rc = A((void**)&S->cpart, 24 * (size_t)kCoarseSplit * kCoarsePointsMax);
-    if (!rc) rc = A((void**)&S->cstart, 4 * (size_t)(kCoarsePointsMax + 1));
-    if (!rc) rc = A((void**)&S->cinv, 8 * mc * mc);
-    if (!rc) rc = A((void**)&S->cmat, 8 * mc * mc);
-    if (!rc) rc = A((void**)&S->cy, 8 * mc);
-    if (rc) return rc;
-  }
+  int rc = A((void**)&S->clist, 4 * (size_t)N);
+  if (!rc) rc = A((void**)&S->ct, 24 * (size_t)N);
+  if (!rc) rc = A((void**)&S->cpart, 3 * 24 * 8 * (size_t)kCellSplit * kCoarsePointsMax);
+  if (!rc) rc = A((void**)&S->cstart, 4 * (size_t)(kCoarsePointsMax + 1));
+  if (!rc) rc = A((void**)&S->cinv, 8 * mc * mc);
+  if (!rc) rc = A((void**)&S->cmat, 8 * mc * mc);
+  if (!rc) rc = A((void**)&S->cy, 8 * mc);
+  if (!rc) rc = A((void**)&S->cdmax, 8);
+  if (rc) return rc;
   // grid over the bounding box
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
   for (int k = 0; k < N; k++)
@@ -1095,132 +1256,89 @@ static int coarse_build(Ctx* c) {
     for (int d = 0; d < 3; d++) T.o[d] = lo[d] - 0.5 * ((T.d[d] - 1) * H - E[d]);
     G = T;
   }
-  const int np = G.points(), nc = 3 * np;
   S->cgr = G;
-  S->nc = nc;
-  // node lists of each grid point (the nodes of the up to 8 cells around it)
-  std::vector<int> cell(N);
+  S->nc = 3 * G.points();
+  // nodes by cell
+  std::vector<int> cell(N), cnt(G.cells() + 1, 0), list(N);
   const unsigned nb = (unsigned)((N + RB - 1) / RB);
-  int* dcell = S->clist;  // scratch until the lists are written
-  hipLaunchKernelGGL(k_coarse_cells, dim3(nb), dim3(RB), 0, s, N, G, S->x, dcell);
-  rc = c->hip(hipMemcpyAsync(cell.data(), dcell, 4 * (size_t)N, hipMemcpyDeviceToHost, s), "d2h");
+  hipLaunchKernelGGL(k_coarse_cells, dim3(nb), dim3(RB), 0, s, N, G, S->x, S->clist);
+  rc = c->hip(hipMemcpyAsync(cell.data(), S->clist, 4 * (size_t)N, hipMemcpyDeviceToHost, s), "d2h");
   if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
   if (rc) return rc;
-  std::vector<int> cnt(np + 1, 0), list(8 * (size_t)N);
-  auto corner = [&](int cl, int q) {
-    const int cx = cl % G.d[0], cy = (cl / G.d[0]) % G.d[1], cz = cl / (G.d[0] * G.d[1]);
-    return (cx + (q & 1)) + G.d[0] * ((cy + ((q >> 1) & 1)) + G.d[1] * (cz + ((q >> 2) & 1)));
-  };
-  for (int i = 0; i < N; i++)
-    for (int q = 0; q < 8; q++) cnt[corner(cell[i], q) + 1]++;
-  for (int g = 0; g < np; g++) cnt[g + 1] += cnt[g];
+  for (int i = 0; i < N; i++) cnt[cell[i] + 1]++;
+  for (int g = 0; g < G.cells(); g++) cnt[g + 1] += cnt[g];
   std::vector<int> fill(cnt.begin(), cnt.end() - 1);
-  for (int i = 0; i < N; i++)
-    for (int q = 0; q < 8; q++) list[fill[corner(cell[i], q)]++] = i;
-  rc = c->hip(hipMemcpyAsync(S->cstart, cnt.data(), 4 * (size_t)(np + 1), hipMemcpyHostToDevice, s), "h2d");
-  if (!rc) rc = c->hip(hipMemcpyAsync(S->clist, list.data(), 32 * (size_t)N, hipMemcpyHostToDevice, s), "h2d");
+  for (int i = 0; i < N; i++) list[fill[cell[i]]++] = i;
+  rc = c->hip(hipMemcpyAsync(S->cstart, cnt.data(), 4 * cnt.size(), hipMemcpyHostToDevice, s), "h2d");
+  if (!rc) rc = c->hip(hipMemcpyAsync(S->clist, list.data(), 4 * (size_t)N, hipMemcpyHostToDevice, s), "h2d");
   if (rc) return rc;
-  hipLaunchKernelGGL(k_coarse_weights, dim3(np), dim3(RB), 0, s, G, S->cstart, S->clist, S->x,
-                     S->wlist);
-  // A_c by probing: the tangent couples nodes at most 2 bond lengths apart
-  // (the dilatation term reaches the neighbours' neighbours), so phi_g' . K
-  // phi_g vanishes unless g and g' are within `reach` grid steps on every
-  // axis (supports H either side of a point, bond components at most
-  // bond_cmax). Points of one colour (indices congruent modulo 2 reach + 1 on
-  // every axis) then never meet the same target, and one tangent apply of
-  // their summed functions gives all their columns at once. S->z holds the
-  // probe, S->q its image; probe p's restriction goes to column p of S->cmat.
-  const double bc = c->bond_cmax;
-  const int reach = std::max(1, (int)std::ceil((2.0 * G.H + 2.0 * bc) / G.H - 1e-12) - 1);
-  const int stride = 2 * reach + 1;
-  const int sc[3] = {std::min(stride, G.d[0]), std::min(stride, G.d[1]), std::min(stride, G.d[2])};
-  if ((rc = state(c))) return rc;
-  std::vector<int> pcol;  // probe -> colour code (cx, cy, cz, k0)
-  for (int cz = 0; cz < sc[2]; cz++)
-    for (int cy = 0; cy < sc[1]; cy++)
-      for (int cx = 0; cx < sc[0]; cx++)
-        for (int k0 = 0; k0 < 3; k0++) {
-          const int pr = (int)pcol.size();
-          pcol.push_back(((cz * sc[1] + cy) * sc[0] + cx) * 3 + k0);
-          hipLaunchKernelGGL(k_coarse_probe, dim3(nb), dim3(RB), 0, s, N, G, stride, cx, cy, cz, k0,
-                             S->x, S->fixed, S->z);
-          if ((rc = tangent(c, S->z, S->q))) return rc;
-          hipLaunchKernelGGL(k_coarse_partial, dim3(np * kCoarseSplit), dim3(RB), 0, s, S->cstart,
-                             S->clist, S->wlist, S->fixed, S->q, S->cpart);
-          hipLaunchKernelGGL(k_coarse_finish<false>, dim3(1), dim3(RB), 0, s, nc, S->cpart, nullptr,
-                             S->cmat + (size_t)pr * nc);
+  hipLaunchKernelGGL(k_coarse_local, dim3(nb), dim3(RB), 0, s, N, G, S->clist, S->x, S->ct);
+  rc = c->hip(hipStreamSynchronize(s), "sync");  // the lists leave the host
+  S->grid_ok = rc == 0;
+  return rc;
+}
+
+// Two-level preconditioner set-up at the current state: the inverse of the
+// coarse matrix A_c = P^T K P, whose columns come from tangent products of
+// probe vectors.
+//
+// The tangent couples nodes at most 2 bond lengths apart (the dilatation term
+// reaches the neighbours' neighbours), so phi_g' . K phi_g vanishes unless g
+// and g' are within `reach` grid steps on every axis (supports H either side
+// of a point, bond components at most bond_cmax). Points of one colour
+// (indices congruent modulo 2 reach + 1 on every axis) then never meet the
+// same target, and one product of their summed functions gives all their
+// columns at once; on a tiled mesh one pair of passes gives those of all three
+// axes. S->z holds the probe, S->r, S->p and S->q the images, row p of S->cmat
+// probe p's restriction.
+//
+// 200,000-node bar, 480 functions, 80 colours: 25 ms in all, of which the probes
+// take 17 (70 with a product per function and the factorisation on the host).
+static int coarse_build(Ctx* c) {
+  QsState* S = c->qs;
+  const int N = c->N;
+  hipStream_t s = c->stream;
+  int rc = S->grid_ok ? PDG_OK : coarse_grid(c);
+  if (!rc) rc = state(c);
+  if (rc) return rc;
+  const CoarseGrid& G = S->cgr;
+  const int nc = S->nc, blocks = G.cells() * kCellSplit;
+  const unsigned nb = (unsigned)((N + RB - 1) / RB);
+  ProbeColours pc;
+  pc.reach = std::max(1, (int)std::ceil((2.0 * G.H + 2.0 * c->bond_cmax) / G.H - 1e-12) - 1);
+  pc.stride = 2 * pc.reach + 1;
+  for (int d = 0; d < 3; d++) pc.d[d] = std::min(pc.stride, G.d[d]);
+  double* const img[3] = {S->r, S->p, S->q};
+  int pr = 0;  // probes so far: at most nc, so S->cmat holds every row
+  for (int cz = 0; cz < pc.d[2]; cz++)
+    for (int cy = 0; cy < pc.d[1]; cy++)
+      for (int cx = 0; cx < pc.d[0]; cx++, pr += 3) {
+        if (c->tiled()) {
+          hipLaunchKernelGGL(k_coarse_probe, dim3(nb), dim3(RB), 0, s, N, G, pc.stride, cx, cy, cz,
+                             -1, S->x, S->fixed, S->z);
+          rc = c->hip(launch_qs_tangent3(tile_args(c), S->z, img, c->tile_lanes(), s), "qs probes");
+        } else {
+          for (int k = 0; k < 3 && !rc; k++) {
+            hipLaunchKernelGGL(k_coarse_probe, dim3(nb), dim3(RB), 0, s, N, G, pc.stride, cx, cy, cz,
+                               k, S->x, S->fixed, S->z);
+            rc = tangent(c, S->z, img[k]);
+          }
         }
-  const int nprobe = (int)pcol.size();  // <= nc, so S->cmat holds every probe
-  std::vector<double> R((size_t)nprobe * nc), M((size_t)nc * nc, 0.0);
-  rc = c->hip(hipGetLastError(), "qs coarse build");
-  if (!rc) rc = c->hip(hipMemcpyAsync(R.data(), S->cmat, 8 * R.size(), hipMemcpyDeviceToHost, s), "d2h");
-  if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-  if (rc) return rc;
-  // entry (target t, source g): the source of the target's colour within
-  // reach on every axis, if any (M[col * nc + row] = A_c[row][col])
-  for (int pr = 0; pr < nprobe; pr++) {
-    const int k0 = pcol[pr] % 3, code = pcol[pr] / 3;
-    const int cx = code % sc[0], cy = (code / sc[0]) % sc[1], cz = code / (sc[0] * sc[1]);
-    const int cc[3] = {cx, cy, cz};
-    for (int t = 0; t < np; t++) {
-      const int tp[3] = {t % G.d[0], (t / G.d[0]) % G.d[1], t / (G.d[0] * G.d[1])};
-      int gp[3];
-      bool ok = true;
-      for (int d = 0; d < 3 && ok; d++) {
-        int delta = ((cc[d] - tp[d]) % stride + stride) % stride;
-        if (delta > reach) delta -= stride;
-        gp[d] = tp[d] + delta;
-        ok = gp[d] >= 0 && gp[d] < G.d[d] && gp[d] % stride == cc[d];
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_restrict, dim3(blocks, 3), dim3(kRestrictThreads), 0, s, nullptr,
+                           S->cstart, S->clist, S->ct, S->fixed, img[0], img[1], img[2], S->cpart);
+        hipLaunchKernelGGL(k_coarse_columns, dim3(3), dim3(RB), 0, s, G, nc, blocks, S->cpart,
+                           S->cmat + (size_t)pr * nc);
       }
-      if (!ok) continue;
-      const int g = gp[0] + G.d[0] * (gp[1] + G.d[1] * gp[2]);
-      for (int k = 0; k < 3; k++) M[(size_t)(3 * g + k0) * nc + 3 * t + k] = R[(size_t)pr * nc + 3 * t + k];
-    }
+  hipLaunchKernelGGL(k_coarse_matrix, dim3((unsigned)((nc * nc + RB - 1) / RB)), dim3(RB), 0, s, G, pc,
+                     nc, S->cmat, S->cinv);
+  hipLaunchKernelGGL(k_coarse_dmax, dim3(1), dim3(RB), 0, s, nc, S->cinv, S->cdmax);
+  const unsigned nt = (unsigned)((nc + kGjTile - 1) / kGjTile);
+  for (int p0 = 0; p0 < nc; p0 += kGj) {
+    hipLaunchKernelGGL(k_gj_step, dim3(nt, nt), dim3(RB), 0, s, nc, p0, S->cinv, S->cdmax, S->cmat);
+    std::swap(S->cinv, S->cmat);
   }
-  // symmetrise, factor L L^T with dropped functions, invert
-  for (int i = 0; i < nc; i++)
-    for (int j = 0; j < i; j++) {
-      const double v = 0.5 * (M[(size_t)i * nc + j] + M[(size_t)j * nc + i]);
-      M[(size_t)i * nc + j] = M[(size_t)j * nc + i] = v;
-    }
-  double dmax = 0.0;
-  for (int i = 0; i < nc; i++) dmax = std::max(dmax, M[(size_t)i * nc + i]);
-  std::vector<double> L((size_t)nc * nc, 0.0);
-  std::vector<char> drop(nc, 0);
-  for (int j = 0; j < nc; j++) {
-    double d = M[(size_t)j * nc + j];
-    for (int k = 0; k < j; k++) d -= L[(size_t)j * nc + k] * L[(size_t)j * nc + k];
-    if (!(d > 1e-12 * dmax)) { drop[j] = 1; continue; }
-    const double ljj = std::sqrt(d);
-    L[(size_t)j * nc + j] = ljj;
-    for (int i = j + 1; i < nc; i++) {
-      double v = M[(size_t)i * nc + j];
-      for (int k = 0; k < j; k++) v -= L[(size_t)i * nc + k] * L[(size_t)j * nc + k];
-      L[(size_t)i * nc + j] = v / ljj;
-    }
-  }
-  std::vector<double> inv((size_t)nc * nc, 0.0);
-  parallel_for(nc, [&](long long e0, long long e1) {  // columns on host threads
-  std::vector<double> y(nc);
-  for (int e = (int)e0; e < (int)e1; e++) {
-    if (drop[e]) continue;
-    for (int i = 0; i < nc; i++) {  // L y = e_e
-      if (drop[i]) { y[i] = 0.0; continue; }
-      double v = i == e ? 1.0 : 0.0;
-      for (int k = 0; k < i; k++) v -= L[(size_t)i * nc + k] * y[k];
-      y[i] = v / L[(size_t)i * nc + i];
-    }
-    for (int i = nc - 1; i >= 0; i--) {  // L^T x = y
-      if (drop[i]) { y[i] = 0.0; continue; }
-      double v = y[i];
-      for (int k = i + 1; k < nc; k++) v -= L[(size_t)k * nc + i] * y[k];
-      y[i] = v / L[(size_t)i * nc + i];
-    }
-    for (int i = 0; i < nc; i++) inv[(size_t)i * nc + e] = y[i];
-  }
-  }, 64);
-  rc = c->hip(hipMemcpyAsync(S->cinv, inv.data(), 8 * inv.size(), hipMemcpyHostToDevice, s), "h2d");
-  if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
+  rc = c->hip(hipGetLastError(), "qs coarse build");
   S->coarse_ok = rc == 0;
   return rc;
 }
@@ -1332,7 +1450,7 @@ void Ctx::free_extra() {
                       S->dampv, S->dT,   S->ps};
     for (double* p : ptrs) if (p) (void)hipFree(p);
     for (double* p : S->rv) if (p) (void)hipFree(p);
-    double* cptrs[] = {S->cinv, S->cmat, S->cy, S->wlist, S->cpart};
+    double* cptrs[] = {S->cinv, S->cmat, S->cy, S->ct, S->cpart, S->cdmax};
     for (double* p : cptrs) if (p) (void)hipFree(p);
     if (S->clist) (void)hipFree(S->clist);
     if (S->cstart) (void)hipFree(S->cstart);
@@ -1414,11 +1532,11 @@ static int cg_solve(Ctx* c, double* x, const double* b, double bnorm, int precon
     } else if (precond == 3) {
       if (init) wide ? go(k_cg_update<256, 3, true>) : go(k_cg_update<128, 3, true>);
       else wide ? go(k_cg_update<256, 3, false>) : go(k_cg_update<128, 3, false>);
-      hipLaunchKernelGGL(k_coarse_partial, dim3(S->cgr.points() * kCoarseSplit), dim3(RB), 0, s,
-                         S->cstart, S->clist, S->wlist, S->fixed, S->r, S->cpart);
-      hipLaunchKernelGGL(k_coarse_finish<true>, dim3((S->nc + RB / 64 - 1) / (RB / 64)), dim3(RB),
-                         0, s, S->nc, S->cpart, S->cinv, S->cy);
-      hipLaunchKernelGGL(k_two_level_apply, dim3(S->nblk), dim3(RB), 0, s, N, S->dinv, S->cgr,
+      hipLaunchKernelGGL(k_restrict, dim3(S->cgr.cells() * kCellSplit), dim3(kRestrictThreads), 0, s,
+                         S->cg, S->cstart, S->clist, S->ct, S->fixed, S->r, S->r, S->r, S->cpart);
+      hipLaunchKernelGGL(k_coarse_solve, dim3((S->nc + RB / 64 - 1) / (RB / 64)), dim3(RB), 0, s,
+                         S->cg, S->cgr, S->nc, S->cpart, S->cinv, S->cy);
+      hipLaunchKernelGGL(k_two_level_apply, dim3(S->nblk), dim3(RB), 0, s, S->cg, N, S->dinv, S->cgr,
                          S->x, S->fixed, S->cy, S->r, S->z, S->rz_part);
     } else {
       if (init) wide ? go(k_cg_update<256, 0, true>) : go(k_cg_update<128, 0, true>);

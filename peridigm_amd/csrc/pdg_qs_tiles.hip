@@ -88,12 +88,19 @@ __device__ __forceinline__ double lanes_sum(double v) {
 }
 
 // What a pass does with a bond. QP_CG is QP_DTHETA with a direction that the
-// staging forms.
-enum { QP_THETA, QP_DTHETA, QP_FORCE, QP_DFORCE, QP_CG };
+// staging forms. QP_DTHETA3 and QP_DFORCE3 take three directions at once, the
+// k-th of them w's component k along axis k (0 along the others): the probes
+// of the two-level preconditioner's set-up. They share the geometry and the
+// records of one direction; only the sums differ, three and nine.
+enum { QP_THETA, QP_DTHETA, QP_FORCE, QP_DFORCE, QP_CG, QP_DTHETA3, QP_DFORCE3 };
 template <int PASS>
-constexpr bool is_dtheta() { return PASS == QP_DTHETA || PASS == QP_CG; }
+constexpr bool is_dtheta() { return PASS == QP_DTHETA || PASS == QP_CG || PASS == QP_DTHETA3; }
 template <int PASS>
-constexpr bool is_dual() { return is_dtheta<PASS>() || PASS == QP_DFORCE; }
+constexpr bool is_dforce() { return PASS == QP_DFORCE || PASS == QP_DFORCE3; }
+template <int PASS>
+constexpr bool is_dual() { return is_dtheta<PASS>() || is_dforce<PASS>(); }
+template <int PASS>
+constexpr int nsums() { return PASS == QP_DFORCE3 ? 9 : 3; }
 
 // LDS arrays of a pass, 16-byte slots of one halo node each, at compile-time
 // distances (one byte offset addresses all of them): xu[0..2], then
@@ -101,16 +108,20 @@ constexpr bool is_dual() { return is_dtheta<PASS>() || PASS == QP_DFORCE; }
 //   QP_DTHETA, QP_CG  (w0, w1), (w2, V)
 //   QP_FORCE   (alpha, q), (V, -)
 //   QP_DFORCE  (alpha, q), (w0, w1), (w2, dq), and an array of V unless every
-//              node has the same.
+//              node has the same
+//   QP_DFORCE3 as QP_DFORCE, with (dq1, dq2) after (w2, dq0).
 constexpr int HS = kTileHaloMax;
 template <int PASS>
-constexpr int units() { return PASS == QP_THETA ? 4 : PASS == QP_DFORCE ? 6 : 5; }
+constexpr int units() {
+  return PASS == QP_THETA ? 4 : PASS == QP_DFORCE ? 6 : PASS == QP_DFORCE3 ? 7 : 5;
+}
 template <int PASS, bool UNIV>
-constexpr int lds_bytes() { return 16 * HS * units<PASS>() + (PASS == QP_DFORCE && !UNIV ? 8 * HS : 0); }
+constexpr int lds_bytes() { return 16 * HS * units<PASS>() + (is_dforce<PASS>() && !UNIV ? 8 * HS : 0); }
 
 // Workgroups of 512 threads, two to a CU (at most 80 KB of LDS each). The
-// tangent's force pass with a volume array takes 83 KB: one workgroup to a CU
-// then, of 1,024 threads, each node's bonds shared by two lane groups.
+// tangent's force pass with a volume array takes 83 KB, that of three
+// directions 90 or 96: one workgroup to a CU then, of 1,024 threads, each
+// node's bonds shared by two lane groups.
 template <int PASS, bool UNIV>
 constexpr int halves() { return lds_bytes<PASS, UNIV>() > 81920 ? 2 : 1; }
 
@@ -118,7 +129,7 @@ constexpr int halves() { return lds_bytes<PASS, UNIV>() > 81920 ? 2 : 1; }
 template <int PASS>
 struct Rec {
   f64x2 v[units<PASS>()];
-  double vj;  // QP_DFORCE: V
+  double vj;  // tangent's force passes: V
   __device__ double x(int c) const { return c == 0 ? v[0].x : c == 1 ? v[0].y : v[1].x; }
   __device__ double u(int c) const { return c == 0 ? v[1].y : c == 1 ? v[2].x : v[2].y; }
   __device__ double vol() const {
@@ -128,10 +139,12 @@ struct Rec {
   __device__ double alpha() const { return v[3].x; }  // force passes
   __device__ double q() const { return v[3].y; }      // force passes
   __device__ double w(int c) const {                  // tangent passes
-    constexpr int k = units<PASS>() - 2;
+    constexpr int k = is_dforce<PASS>() ? 4 : units<PASS>() - 2;
     return c == 0 ? v[k].x : c == 1 ? v[k].y : v[k + 1].x;
   }
-  __device__ double dq() const { return v[units<PASS>() - 1].y; }
+  __device__ double dq(int k = 0) const {             // tangent's force passes
+    return k == 0 ? v[5].y : k == 1 ? v[units<PASS>() - 1].x : v[units<PASS>() - 1].y;
+  }
 };
 
 template <int PASS, bool UNIV>
@@ -139,17 +152,18 @@ __device__ __forceinline__ void rec_read(Rec<PASS>& r, const char* lds, int jb) 
 #pragma unroll
   for (int k = 0; k < units<PASS>(); k++)
     r.v[k] = *reinterpret_cast<const f64x2*>(lds + 16 * HS * k + jb);
-  if (PASS == QP_DFORCE && !UNIV)
+  if (is_dforce<PASS>() && !UNIV)
     r.vj = *reinterpret_cast<const double*>(lds + 16 * HS * units<PASS>() + (jb >> 1));
 }
 
 // One bond of a pass, added to the lane's sums s when `ok` (one sum for the
-// dilatation passes, three for the force passes). UNIV: without the volume
-// factor, which the caller applies to the sums. A masked-out bond may give a
-// NaN, so the sums are selected, not the terms.
+// dilatation passes, three for the force passes, and as many for each of three
+// directions). UNIV: without the volume factor, which the caller applies to
+// the sums. A masked-out bond may give a NaN, so the sums are selected, or the
+// factors of all terms (three directions).
 template <int PASS, bool UNIV, int INFL, bool LIN>
 __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, double hhat,
-                                     double thermal, bool ok, double (&s)[3]) {
+                                     double thermal, bool ok, double (&s)[nsums<PASS>()]) {
   const double X0 = nb.x(0) - me.x(0), X1 = nb.x(1) - me.x(1), X2 = nb.x(2) - me.x(2);
   const double z2 = fma(X2, X2, fma(X1, X1, X0 * X0));
   const double wv = UNIV ? omega64<INFL>(z2, hhat) : omega64<INFL>(z2, hhat) * nb.vol();
@@ -171,6 +185,25 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
   if (LIN) {
     // theta and force linear in u, the force along the reference bond
     constexpr bool dual = is_dual<PASS>();
+    if (PASS == QP_DTHETA3) {
+      const double f = ok ? wv : 0.0;
+      s[0] = fma(f, X0 * d0, s[0]);
+      s[1] = fma(f, X1 * d1, s[1]);
+      s[2] = fma(f, X2 * d2, s[2]);
+      return;
+    }
+    if (PASS == QP_DFORCE3) {
+      const double ar = (me.alpha() + nb.alpha()) * rcp64(z2);
+      const double pr[3] = {X0 * d0, X1 * d1, X2 * d2};
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const double c = ok ? wv * fma(ar, pr[k], me.dq(k) + nb.dq(k)) : 0.0;
+        s[(3 * k) % nsums<PASS>()] = fma(c, X0, s[(3 * k) % nsums<PASS>()]);
+        s[(3 * k + 1) % nsums<PASS>()] = fma(c, X1, s[(3 * k + 1) % nsums<PASS>()]);
+        s[(3 * k + 2) % nsums<PASS>()] = fma(c, X2, s[(3 * k + 2) % nsums<PASS>()]);
+      }
+      return;
+    }
     const double pr = fma(X2, dual ? d2 : D2, fma(X1, dual ? d1 : D1, X0 * (dual ? d0 : D0)));
     if (PASS == QP_THETA || is_dtheta<PASS>()) {
       add1(wv, pr);
@@ -195,12 +228,33 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
   if (PASS == QP_THETA) {
     const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
     add1(wv, dd * g * rcp64(1.0 + g) - thermal * z2);
+  } else if (PASS == QP_DTHETA3) {
+    const double f = ok ? wv * g : 0.0;
+    s[0] = fma(f, Y0 * d0, s[0]);
+    s[1] = fma(f, Y1 * d1, s[1]);
+    s[2] = fma(f, Y2 * d2, s[2]);
   } else if (is_dtheta<PASS>()) {
     add1(wv * g, fma(Y2, d2, fma(Y1, d1, Y0 * d0)));
   } else if (PASS == QP_FORCE) {
     const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
     const double ey = dd * ryy * rcp64(1.0 + g);
     add3(wv * fma(me.alpha() + nb.alpha(), ey, (me.q() + nb.q()) * g), Y0, Y1, Y2);
+  } else if (PASS == QP_DFORCE3) {
+    const double a = me.alpha() + nb.alpha();
+    const double S = fma(a, 1.0 - g, (me.q() + nb.q()) * g);  // over w
+    const double sv = ok ? wv * S : 0.0, wo = ok ? wv : 0.0, gw = ok ? g : 0.0;
+    const double ar = ok ? (a - S) * ryy : 0.0;
+    const double Y[3] = {Y0, Y1, Y2}, d[3] = {d0, d1, d2};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double c = wo * fma(gw, me.dq(k) + nb.dq(k), ar * (Y[k] * d[k]));
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        double& t = s[(3 * k + j) % nsums<PASS>()];
+        t = fma(c, Y[j], t);
+        if (j == k) t = fma(sv, d[k], t);
+      }
+    }
   } else {
     const double a = me.alpha() + nb.alpha();
     const double S = fma(a, 1.0 - g, (me.q() + nb.q()) * g);  // over w
@@ -220,6 +274,7 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
 struct QsOut {
   const double* w;  // QP_DTHETA: the direction, QP_CG: z; 3n
   double* out;      // force passes: 3n
+  double* out3[2];  // QP_DFORCE3: the second and third direction's
   int all;          // QP_FORCE: prescribed DOFs too
   QsCgStart start;  // QP_CG; QP_DFORCE: start.cg null outside a solve
   double* pq_part;  // QP_DFORCE in a solve
@@ -264,14 +319,15 @@ __device__ __forceinline__ void slot_load(const QsTileArgs& a, const QsOut& o, u
                                           Rec<PASS>& r) {
 #pragma unroll
   for (int k = 0; k < 3; k++) r.v[k] = a.rec.xu[k][i];
-  if (PASS == QP_FORCE || PASS == QP_DFORCE) r.v[3] = a.rec.aq[i];
+  if (PASS == QP_FORCE || is_dforce<PASS>()) r.v[3] = a.rec.aq[i];
   if (is_dtheta<PASS>()) {
     const double* w = o.w + 3u * i;
     r.v[units<PASS>() - 2] = f64x2{w[0], w[1]};
     r.v[units<PASS>() - 1] = f64x2{w[2], a.vol[i]};
-  } else if (PASS == QP_DFORCE) {
-    r.v[units<PASS>() - 2] = a.rec.wd[0][i];
-    r.v[units<PASS>() - 1] = a.rec.wd[1][i];
+  } else if (is_dforce<PASS>()) {
+    r.v[4 % units<PASS>()] = a.rec.wd[0][i];
+    r.v[5 % units<PASS>()] = a.rec.wd[1][i];
+    if (PASS == QP_DFORCE3) r.v[6 % units<PASS>()] = a.rec.wp[0][i];
     if (!UNIV) r.vj = a.vol[i];
   } else {
     r.v[units<PASS>() - 1] = f64x2{a.vol[i], 0.0};
@@ -283,7 +339,7 @@ __device__ __forceinline__ void slot_store(char* lds, int h, const Rec<PASS>& r)
 #pragma unroll
   for (int k = 0; k < units<PASS>(); k++)
     *reinterpret_cast<f64x2*>(lds + 16 * (HS * k + h)) = r.v[k];
-  if (PASS == QP_DFORCE && !UNIV)
+  if (is_dforce<PASS>() && !UNIV)
     *reinterpret_cast<double*>(lds + 16 * HS * units<PASS>() + 8 * h) = r.vj;
 }
 
@@ -369,7 +425,9 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
     // nodes of a tile are ordered by descending degree: the wave's first
     // group has the largest
     const int rounds = (__builtin_amdgcn_readfirstlane(deg) + GB * U - 1) / (GB * U);
-    double s[3] = {0.0, 0.0, 0.0};
+    double s[nsums<PASS>()];
+#pragma unroll
+    for (int k = 0; k < nsums<PASS>(); k++) s[k] = 0.0;
     int (&lj)[U] = rw.lj;
     for (int c = 0; c < rounds; c++) {
       int ln[U];
@@ -389,7 +447,34 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
 #pragma unroll
       for (int k = 0; k < U; k++) lj[k] = ln[k];
     }
-    if (PASS == QP_THETA || is_dtheta<PASS>()) {
+    if (PASS == QP_DTHETA3) {
+      const double s0 = lanes_sum<G, HV>(s[0]), s1 = lanes_sum<G, HV>(s[1]), s2 = lanes_sum<G, HV>(s[2]);
+      if (!valid || l != 0) continue;
+      const double m = a.m[(unsigned)node];
+      const double c = (m > 0.0 ? 3.0 / m : 0.0) * (UNIV ? a.vol1 : 1.0);
+      const double f = a.L * a.beta[(unsigned)node] * (c * a.L);
+      a.rec.wd[0][(unsigned)node] = f64x2{me.w(0), me.w(1)};
+      a.rec.wd[1][(unsigned)node] = f64x2{me.w(2), f * s0};
+      a.rec.wp[0][(unsigned)node] = f64x2{f * s1, f * s2};
+    } else if (PASS == QP_DFORCE3) {
+      double f[3];  // lane l's: direction l
+#pragma unroll
+      for (int k = 0; k < nsums<PASS>(); k++) {
+        const double v = lanes_sum<G, HV>(s[k]);
+        f[k % 3] = k < 3 || k / 3 == l ? v : f[k % 3];
+      }
+      if (!valid || l >= 3) continue;
+      const double w = l == 0 ? me.w(0) : (l == 1 ? me.w(1) : me.w(2));
+      double* const out = l == 0 ? o.out : o.out3[l - 1];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const unsigned q = 3u * (unsigned)node + (unsigned)k;
+        const double wk = k == l ? w : 0.0;
+        double kw = a.fixed[q] ? wk : -f[k] * (UNIV ? a.vol1 * a.vol1 : me.vol());
+        if (a.damp) kw += a.damp[q] * wk;
+        out[q] = kw;
+      }
+    } else if (PASS == QP_THETA || is_dtheta<PASS>()) {
       const double sum = lanes_sum<G, HV>(s[0]);
       if (!valid || l != 0) continue;
       const double m = a.m[(unsigned)node];
@@ -496,6 +581,17 @@ hipError_t launch_qs_tangent(const QsTileArgs& a, const double* w, double* out, 
   o.out = out;
   hipError_t e = launch<QP_DTHETA>(a, o, lanes, s);
   return e == hipSuccess ? launch<QP_DFORCE>(a, o, lanes, s) : e;
+}
+
+hipError_t launch_qs_tangent3(const QsTileArgs& a, const double* w, double* const (&out)[3],
+                              int lanes, hipStream_t s) {
+  QsOut o{};
+  o.w = w;
+  o.out = out[0];
+  o.out3[0] = out[1];
+  o.out3[1] = out[2];
+  hipError_t e = launch<QP_DTHETA3>(a, o, lanes, s);
+  return e == hipSuccess ? launch<QP_DFORCE3>(a, o, lanes, s) : e;
 }
 
 hipError_t launch_qs_tangent_cg(const QsTileArgs& a, const QsCgStart& start, const double* z,

@@ -56,6 +56,11 @@ hipError_t launch_qs_residual(const QsTileArgs& a, bool all, double* out, int la
 hipError_t launch_qs_tangent(const QsTileArgs& a, const double* w, double* out, int lanes,
                              hipStream_t s);
 
+// out[k] = K (w's component k along axis k) for the three axes; uses the
+// records wp.
+hipError_t launch_qs_tangent3(const QsTileArgs& a, const double* w, double* const (&out)[3],
+                              int lanes, hipStream_t s);
+
 // The same product for a conjugate-gradient iteration: w = z + beta wp (the
 // records wp) with beta and the decision to stop from `start`, w into the
 // records wd; pq_part[t] is tile t's part of w.Kw.
