@@ -1211,15 +1211,23 @@ int pdg_verlet_run(pdg_ctx* h, int nsteps, double dt, double t0, int initialEval
   int nevals = 0;
   const bool contact = contact_on(c);
   va.fadd = contact ? contact_force_ptr(c) : nullptr;
+  // the contact force goes with pass 1's launch, except where the passes are
+  // timed each by itself
+  const bool joint_gather = contact && c->tiled() && c->pipe() && c->tile_lanes() <= 16 && !nev;
   // pass1 + pass2 of one force evaluation, finishing step `k` (k=0: initial)
   auto eval = [&](int k, bool end_kick) -> int {
     int r = 0;
     // contact force at the evaluation's positions and half-step velocities
-    if (contact) r = contact_step(c, k, dt, c->d_rec[c->cur ^ 1], c->d_rec[c->cur]);
+    ContactGather g{};
+    if (contact) r = contact_step(c, k, dt, c->d_rec[c->cur ^ 1], c->d_rec[c->cur], &g);
+    const bool joint = joint_gather && g.nact > 0;
+    if (contact && !r && !joint) r = c->hip(launch_contact_gather(g, s), "contact force");
     if (!r && nev) r = c->hip(hipEventRecord(c->tev[3 * nevals], s), "event");
     // a time-dependent critical stretch at the time this evaluation ends
     c->sc_cur = c->sc_at(step_time(k));
-    if (!r) r = c->hip(c->pass1(c->d_rec[c->cur], c->d_nbroken, damage, damage), "pass1");
+    if (!r) r = c->hip(joint ? launch_pass1_contact(c->bond_args(), c->tile_args(), c->d_rec[c->cur], c->d_theta, c->d_nbroken, damage, c->tile_lanes(), g, s)
+                             : c->pass1(c->d_rec[c->cur], c->d_nbroken, damage, damage),
+                       "pass1");
     if (!r && nev) r = c->hip(hipEventRecord(c->tev[3 * nevals + 1], s), "event");
     va.end_kick = end_kick ? 1 : 0;
     va.start_step = k < nsteps ? 1 : 0;

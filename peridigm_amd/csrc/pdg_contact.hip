@@ -34,6 +34,7 @@
 #include <cmath>
 #include <vector>
 
+#include "pdg_contact_dev.hpp"
 #include "pdg_ctx.hpp"
 
 namespace pdg {
@@ -75,10 +76,6 @@ struct ContactState {
 };
 
 namespace {
-
-struct PairParams {
-  double rc, rc2, c, horizon, mu;
-};
 
 // Cell coordinate of one position component; huge or non-finite values are
 // clamped (clamping keeps cells of points within one cell size of each other
@@ -313,53 +310,6 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_contact_rows(
   }
 }
 
-// One pair of the short-range force model seen from `cur` (position X,
-// velocity V, volume vc) with neighbour `nb` (y, v, vn); returns false beyond
-// the contact radius. fc: the force density on cur; fn (BOTH only): on nb.
-// Expressions in the reference's order.
-template <bool BOTH>
-__device__ __forceinline__ bool contact_pair(const PairParams& P, const double X[3],
-                                             const double V[3], double vc, const double y[3],
-                                             const double v[3], double vn, double fc[3],
-                                             double fn[3]) {
-  const double d0 = y[0] - X[0], d1 = y[1] - X[1], d2 = y[2] - X[2];
-  const double dsq = d0 * d0 + d1 * d1 + d2 * d2;
-  if (!(dsq < P.rc2)) return false;
-  const double d = sqrt(dsq);
-  const double temp = P.c * (P.rc - d) / P.horizon;
-  const double cf0 = -(temp * vn * d0 / d), cf1 = -(temp * vn * d1 / d), cf2 = -(temp * vn * d2 / d);
-  const double nf0 = temp * vc * d0 / d, nf1 = temp * vc * d1 / d, nf2 = temp * vc * d2 / d;
-  fc[0] = cf0; fc[1] = cf1; fc[2] = cf2;
-  if (BOTH) { fn[0] = nf0; fn[1] = nf1; fn[2] = nf2; }
-  if (P.mu != 0.0) {
-    const double n0 = d0 / d, n1 = d1 / d, n2 = d2 / d;
-    const double cn = V[0] * n0 + V[1] * n1 + V[2] * n2;
-    const double nbn = v[0] * n0 + v[1] * n1 + v[2] * n2;
-    const double cp0 = V[0] - cn * n0, cp1 = V[1] - cn * n1, cp2 = V[2] - cn * n2;
-    const double np0 = v[0] - nbn * n0, np1 = v[1] - nbn * n1, np2 = v[2] - nbn * n2;
-    const double m0 = 0.5 * (cp0 + np0), m1 = 0.5 * (cp1 + np1), m2 = 0.5 * (cp2 + np2);
-    const double cr0 = cp0 - m0, cr1 = cp1 - m1, cr2 = cp2 - m2;
-    const double ncr = sqrt(cr0 * cr0 + cr1 * cr1 + cr2 * cr2);
-    const double ncf = sqrt(cf0 * cf0 + cf1 * cf1 + cf2 * cf2);
-    if (ncr != 0.0) {
-      fc[0] = cf0 + -P.mu * ncf * cr0 / ncr;
-      fc[1] = cf1 + -P.mu * ncf * cr1 / ncr;
-      fc[2] = cf2 + -P.mu * ncf * cr2 / ncr;
-    }
-    if (BOTH) {
-      const double nr0 = np0 - m0, nr1 = np1 - m1, nr2 = np2 - m2;
-      const double nnr = sqrt(nr0 * nr0 + nr1 * nr1 + nr2 * nr2);
-      const double nnf = sqrt(nf0 * nf0 + nf1 * nf1 + nf2 * nf2);
-      if (nnr != 0.0) {
-        fn[0] = nf0 + -P.mu * nnf * nr0 / nnr;
-        fn[1] = nf1 + -P.mu * nnf * nr1 / nnr;
-        fn[2] = nf2 + -P.mu * nnf * nr2 / nnr;
-      }
-    }
-  }
-  return true;
-}
-
 // Points with a non-empty contact list, appended in any order (each point's
 // force is computed on its own, so the order does not reach the results).
 __global__ void k_contact_active(int n, const long long* __restrict__ cnt, int* __restrict__ nact,
@@ -369,49 +319,9 @@ __global__ void k_contact_active(int n, const long long* __restrict__ cnt, int* 
   act[atomicAdd(nact, 1)] = i;
 }
 
-constexpr int kGatherLanes = 16;  // lanes per point of the contact gather
-
-// Explicit-run contact force (internal order) of the points with contacts
-// (the others keep the zero written at the search): each point gathers twice
-// its own side of every pair of its (symmetric) list, kGatherLanes lanes per
-// point, lane l taking entries l, l + kGatherLanes, ..., then a lane-tree sum.
-// Positions as the reference forms them, y = (x + u) + dt v, from the record
-// of the step's start (u) and the half-step velocity v (dt = 0 at the
-// initial evaluation).
-__global__ __launch_bounds__(256) void k_contact_gather(
-    int nact, const int* __restrict__ act, const NodeRec* __restrict__ rec,
-    const double* __restrict__ x, double q, double dt, const double* __restrict__ v,
-    const double* __restrict__ vol, const long long* __restrict__ off,
-    const int* __restrict__ list, PairParams P, double* __restrict__ fout) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int a = t / kGatherLanes, lane = t % kGatherLanes;
-  const bool valid = a < nact;
-  const int i = valid ? act[a] : 0;
-  double f[3] = {0.0, 0.0, 0.0};
-  if (valid) {
-    const long long e0 = off[i], e1 = off[i + 1];
-    double X[3], V[3];
-    for (int l = 0; l < 3; l++) {
-      V[l] = v[3 * i + l];
-      X[l] = (x[3 * i + l] + rec[i].u[l] * q) + dt * V[l];
-    }
-    const double vc = vol[i];
-    for (long long e = e0 + lane; e < e1; e += kGatherLanes) {
-      const int j = list[e];
-      double Y[3], W[3], fc[3], fn[3];
-      for (int l = 0; l < 3; l++) {
-        W[l] = v[3 * j + l];
-        Y[l] = (x[3 * j + l] + rec[j].u[l] * q) + dt * W[l];
-      }
-      if (contact_pair<false>(P, X, V, vc, Y, W, vol[j], fc, fn))
-        for (int l = 0; l < 3; l++) f[l] += fc[l];
-    }
-  }
-  // every lane takes part in the shuffles (the group of a point is aligned)
-  for (int m = kGatherLanes / 2; m >= 1; m >>= 1)
-    for (int l = 0; l < 3; l++) f[l] += __shfl_xor(f[l], m, kGatherLanes);
-  if (valid && lane == 0)
-    for (int l = 0; l < 3; l++) fout[3 * i + l] = 2.0 * f[l];
+// The explicit run's contact force by itself (untiled runs, per-pass timing).
+__global__ __launch_bounds__(256) void k_contact_gather(ContactGather a) {
+  dev::contact_gather(a, blockIdx.x * 256 + threadIdx.x);
 }
 
 // Drop-in contact force (reference order, any list): both sides of every
@@ -433,7 +343,7 @@ __global__ __launch_bounds__(256) void k_contact_scatter(
     const int j = list[h + 1 + k];
     double Y[3], W[3], fc[3], fn[3];
     for (int l = 0; l < 3; l++) { Y[l] = y[3 * j + l]; W[l] = v[3 * j + l]; }
-    if (contact_pair<true>(P, X, V, vc, Y, W, vol[j], fc, fn)) {
+    if (dev::contact_pair<true>(P, X, V, vc, Y, W, vol[j], fc, fn)) {
       for (int l = 0; l < 3; l++) {
         f[l] += fc[l];
         unsafeAtomicAdd(fout + 3 * (size_t)j + l, fn[l]);
@@ -557,39 +467,34 @@ bool contact_on(const Ctx* c) { return c->contact != nullptr && c->N > 0; }
 
 const double* contact_force_ptr(const Ctx* c) { return c->contact ? c->contact->fc : nullptr; }
 
-// One explicit evaluation's contact force at y = x + u + dt v (u from `rec`),
-// after a search in the configuration x + u of `rec_search` when that is not
-// null.
-int contact_eval(Ctx* c, const NodeRec* rec_search, const NodeRec* rec, double dt) {
+// Step bookkeeping of an explicit run: evaluation k (0: initial) of a run.
+// rec_prev holds the displacement at the start of step k (the previous
+// evaluation's), rec the initial one at k = 0. Searches, when one is due, in
+// the configuration x + u of that displacement; g is the evaluation's contact
+// force at y = x + u + dt v, for a launch of either kind.
+int contact_step(Ctx* c, int k, double dt, const NodeRec* rec_prev, const NodeRec* rec,
+                 ContactGather* g) {
   ContactState* S = c->contact;
   const int N = c->N;
   hipStream_t s = c->stream;
-  int rc = PDG_OK;
-  if (rec_search) {
-    hipLaunchKernelGGL(k_contact_y, dim3(blocks_for(3ll * N)), dim3(256), 0, s, N, rec_search,
-                       c->d_x, c->q, S->y);
-    rc = search(c, true);
+  const NodeRec* const u = k == 0 ? rec : rec_prev;
+  S->step = k == 0 ? 0 : S->step + 1;
+  if (k == 0 || !S->built || S->step % S->freq == 0) {
+    hipLaunchKernelGGL(k_contact_y, dim3(blocks_for(3ll * N)), dim3(256), 0, s, N, u, c->d_x, c->q,
+                       S->y);
+    int rc = search(c, true);
     if (rc) return rc;
   }
-  if (S->nact == 0) return PDG_OK;  // all zero since the search
-  hipLaunchKernelGGL(k_contact_gather, dim3(blocks_for((long long)S->nact * kGatherLanes)),
-                     dim3(256), 0, s, S->nact, S->act, rec, c->d_x, c->q, dt, c->d_v, c->d_vol,
-                     S->off, S->list, pair_params(c), S->fc);
-  return c->hip(hipGetLastError(), "contact force");
+  *g = ContactGather{S->nact, S->act, u, c->d_x, c->q, k == 0 ? 0.0 : dt, c->d_v, c->d_vol,
+                     S->off, S->list, pair_params(c), S->fc};
+  return PDG_OK;
 }
 
-// Step bookkeeping of an explicit run: evaluation k (0: initial) of a run.
-// rec_prev holds the displacement at the start of step k (the previous
-// evaluation's), rec the initial one at k = 0.
-int contact_step(Ctx* c, int k, double dt, const NodeRec* rec_prev, const NodeRec* rec) {
-  ContactState* S = c->contact;
-  if (k == 0) {
-    S->step = 0;
-    return contact_eval(c, rec, rec, 0.0);
-  }
-  S->step++;
-  const bool search_now = !S->built || S->step % S->freq == 0;
-  return contact_eval(c, search_now ? rec_prev : nullptr, rec_prev, dt);
+hipError_t launch_contact_gather(const ContactGather& g, hipStream_t s) {
+  if (g.nact == 0) return hipSuccess;  // all zero since the search
+  hipLaunchKernelGGL(k_contact_gather, dim3(blocks_for((long long)g.nact * kGatherLanes)), dim3(256),
+                     0, s, g);
+  return hipGetLastError();
 }
 
 }  // namespace pdg

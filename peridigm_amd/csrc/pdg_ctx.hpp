@@ -251,12 +251,13 @@ class HostOut {
 // short-range contact (pdg_contact.hip): whether a contact model is set, its
 // force density of the last explicit evaluation (device, internal order), and
 // evaluation k (0: initial) of an explicit run with step dt: a search in the
-// configuration of rec_prev (the step's start) when one is due, then the
+// configuration of rec_prev (the step's start) when one is due, and in *g the
 // force at y = x + u_prev + dt v with the context's half-step velocities v
-// (at k = 0: search and force at rec).
+// (at k = 0: search and force at rec), for the caller to launch.
 bool contact_on(const Ctx* c);
 const double* contact_force_ptr(const Ctx* c);
-int contact_step(Ctx* c, int k, double dt, const NodeRec* rec_prev, const NodeRec* rec);
+int contact_step(Ctx* c, int k, double dt, const NodeRec* rec_prev, const NodeRec* rec,
+                 ContactGather* g);
 
 // quasi-static solver (pdg_qs.hip) and learned preconditioner (pdg_gnn.hip)
 int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int maxit, int* iters,

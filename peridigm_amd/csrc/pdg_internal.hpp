@@ -116,9 +116,36 @@ struct TileArgs {
   const unsigned short* lcol; // B
 };
 
+// Parameters of the short-range contact force of a pair, and the contact force
+// of one explicit evaluation on the nact points `act` with contacts, from their
+// rows list[off[i] .. off[i + 1]) (see contact_gather, pdg_contact_dev.hpp).
+struct PairParams {
+  double rc, rc2, c, horizon, mu;
+};
+constexpr int kGatherLanes = 16;  // lanes per point
+struct ContactGather {
+  int nact;
+  const int* act;
+  const NodeRec* rec;
+  const double* x;
+  double q, dt;
+  const double* v;
+  const double* vol;
+  const long long* off;
+  const int* list;
+  PairParams P;
+  double* fout;
+};
+hipError_t launch_contact_gather(const ContactGather& g, hipStream_t s);  // pdg_contact.hip
+
 hipError_t launch_pass1_tiled(const BondArgs& a, const TileArgs& t, NodeRec* rec, float* theta,
                               int* nbroken, bool damage, bool count_near, int lanes, bool pipe,
                               hipStream_t s);
+// Pass 1 of an explicit evaluation with contact, the contact force computed by
+// workgroups of its own in the same launch (4, 8 or 16 lanes per node).
+hipError_t launch_pass1_contact(const BondArgs& a, const TileArgs& t, NodeRec* rec, float* theta,
+                                int* nbroken, bool damage, int lanes, const ContactGather& g,
+                                hipStream_t s);
 hipError_t launch_pass2_tiled_force(const BondArgs& a, const TileArgs& t, const NodeRec* rec,
                                     double* f, int lanes, bool pipe, hipStream_t s);
 hipError_t launch_pass2_tiled_verlet(const BondArgs& a, const TileArgs& t, const NodeRec* rec,
