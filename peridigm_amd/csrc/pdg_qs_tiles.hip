@@ -159,8 +159,9 @@ __device__ __forceinline__ void rec_read(Rec<PASS>& r, const char* lds, int jb) 
 // One bond of a pass, added to the lane's sums s when `ok` (one sum for the
 // dilatation passes, three for the force passes, and as many for each of three
 // directions). UNIV: without the volume factor, which the caller applies to
-// the sums. A masked-out bond may give a NaN, so the sums are selected, or the
-// factors of all terms (three directions).
+// the sums. A masked-out bond may address a slot that was never written, and
+// give a NaN, so the sums are selected; with three directions the factors are,
+// and the caller passes the node itself as such a bond's neighbour.
 template <int PASS, bool UNIV, int INFL, bool LIN>
 __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, double hhat,
                                      double thermal, bool ok, double (&s)[nsums<PASS>()]) {
@@ -440,8 +441,11 @@ __global__ __launch_bounds__((WG * halves<PASS, UNIV>()), 4) void k_qs_tile(QsTi
 #pragma unroll
       for (int k = 0; k < U; k++) {
         Rec<PASS> nb;
-        rec_read<PASS, UNIV>(nb, lds, lj[k]);
         const bool ok = (half[(k * GB) >> 5] & (1u << ((k * GB) & 31))) != 0u;
+        // where not the sums but the factors are selected, a masked-out bond
+        // must read finite values: its node's own slot
+        constexpr bool own_slot = PASS == QP_DTHETA3 || PASS == QP_DFORCE3;
+        rec_read<PASS, UNIV>(nb, lds, own_slot && !ok ? kLdsSlot * (own + (nd - n0)) : lj[k]);
         bond<PASS, UNIV, INFL, LIN>(me, nb, a.hhat, thermal, ok, s);
       }
 #pragma unroll
