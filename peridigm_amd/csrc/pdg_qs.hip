@@ -1193,9 +1193,9 @@ static int residual(Ctx* c, bool all = false) {
 }
 
 // K w for device w, output in `out`; needs state() at the current u
-static int tangent(Ctx* c, const double* w, double* out) {
+static int tangent(Ctx* c, const double* w, double* out, bool tiled = true) {
   hipStream_t s = c->stream;
-  if (c->tiled())
+  if (tiled && c->tiled())
     return c->hip(launch_qs_tangent(tile_args(c), w, out, c->tile_lanes(), s), "qs tangent");
   QsArgs a = args(c);
   a.w = w;
@@ -1811,14 +1811,20 @@ int pdg_qs_fallback_count(pdg_ctx* h, int* count) {
   return PDG_OK;
 }
 
+// One product on a small mesh takes the untiled kernels: two, which read u
+// itself, against four (records, dilatation, its derivative, force) of which
+// the first two pay only where several products share a state. Device time
+// at 3,000 nodes 20 us against 21 and two more gaps, at 24,000 73 against 40.
+constexpr int kTangentTiledMin = 6000;
+
 int pdg_qs_tangent_apply(pdg_ctx* h, const double* u, const double* w, double* Kw) {
   Ctx* c = reinterpret_cast<Ctx*>(h);
   if (!c || !c->have_consts || !u || !w || !Kw) return PDG_E_ARG;
   int rc = qs::ensure(c);
   if (!rc) rc = qs::to_dev(c, u, c->qs->u);
   if (!rc) rc = qs::to_dev(c, w, c->qs->w, 1);
-  if (!rc) rc = qs::state(c);
-  if (!rc) rc = qs::tangent(c, c->qs->w, c->qs->out);
+  if (!rc && c->tiled() && c->N > kTangentTiledMin) rc = qs::state(c);
+  if (!rc) rc = qs::tangent(c, c->qs->w, c->qs->out, c->N > kTangentTiledMin);
   if (!rc) rc = qs::to_host(c, c->qs->out, Kw);
   return rc;
 }
