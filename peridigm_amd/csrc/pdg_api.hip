@@ -431,9 +431,9 @@ char* Ctx::stage(size_t bytes) {
 constexpr int kHostOrderMax = 32768;
 
 // Current positions y (reference order, host) -> the records' u = y - x. The
-// copy reads the caller's array (37 GB/s; through the staging buffer, whose
-// filling takes a thread as long, it is no faster), so the caller synchronises
-// before it returns. A call that fails after this leaves u set to its y.
+// copy of a large mesh reads the caller's array (37 GB/s; through the staging
+// buffer, whose filling takes a thread as long, it is no faster), so the caller
+// synchronises before it returns. A call that fails after this leaves u set to its y.
 int Ctx::upload_y(const double* y) {
   if (N <= 0) return PDG_OK;
   const void* src = y;
