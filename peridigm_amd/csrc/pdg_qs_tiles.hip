@@ -228,7 +228,10 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
   }
   if (PASS == QP_THETA) {
     const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
-    add1(wv, dd * g * rcp64(1.0 + g) - thermal * z2);
+    double ez = dd * g * rcp64(1.0 + g);  // e |X|
+    // points that the deformation brings to one place, where g has no value
+    if (__builtin_amdgcn_ballot_w64(z2 * yy == 0.0)) ez = z2 * yy == 0.0 ? -z2 : ez;
+    add1(wv, ez - thermal * z2);
   } else if (PASS == QP_DTHETA3) {
     const double f = ok ? wv * g : 0.0;
     s[0] = fma(f, Y0 * d0, s[0]);
