@@ -1572,9 +1572,12 @@ static int cg_solve(Ctx* c, double* x, const double* b, double bnorm, int precon
     drop_graphs(c);
     S->gx = x; S->gb = b; S->gtiled = tiled;
   }
-  volatile const QsCgStatus* st = S->hstat;
-  for (int chunk = 0; !st->done; chunk++) {
-    if (chunk > std::max(maxit, 0) / kCgChunk + 2) return c->fail(PDG_E_HIP, "CG did not report its end");
+  const QsCgStatus* const st = S->hstat;
+  // launches of a solve that failed half-way must not write the next one's status
+  auto drained = [&](int r2) { (void)hipStreamSynchronize(s); return r2; };
+  for (int chunk = 0; !cg_status_ended(st); chunk++) {
+    if (chunk > std::max(maxit, 0) / kCgChunk + 2)
+      return drained(c->fail(PDG_E_HIP, "CG did not report its end"));
     hipEvent_t ev = S->cev[chunk & 1];
     if (graphs) {
       hipGraphExec_t* g = &S->gchunk[precond];
@@ -1598,7 +1601,7 @@ static int cg_solve(Ctx* c, double* x, const double* b, double bnorm, int precon
       }
       if (!rc) rc = c->hip(hipEventSynchronize(ev), "sync");
     }
-    if (rc) return rc;
+    if (rc) return drained(rc);
   }
   if (st->brk) return c->fail(PDG_E_NOCONV, "CG breakdown: p.Kp <= 0");
   const double relres = std::sqrt(st->rr) / bnorm;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "pdg_device.hpp"
+#include "pdg_qs_status.hpp"
 
 namespace pdg {
 
@@ -12,12 +13,6 @@ namespace pdg {
 struct QsCg {
   int done, brk, it, maxit;
   double rz, rz2[2], bnorm, tol;
-};
-
-// What the host reads of a stopped solve (pinned memory).
-struct QsCgStatus {
-  int done, brk, it, pad;
-  double rr;
 };
 
 // Arguments of the kernel that starts an iteration: the scalars, the partial
@@ -96,10 +91,7 @@ __device__ __forceinline__ bool cg_start(const QsCgStart& s, double* sh, double&
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (stop) {
       s.cg->done = 1;
-      s.status->brk = brk;
-      s.status->it = it;
-      s.status->rr = rr;
-      s.status->done = 1;
+      cg_status_publish(s.status, brk, it, rr);
     } else {
       s.cg->rz = rz;
       s.cg->rz2[it & 1] = rz;
