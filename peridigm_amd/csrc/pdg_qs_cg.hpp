@@ -69,13 +69,11 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
   }
 }
 
-// Start of iteration cg->it + 1: decides whether the solve stops (every
-// workgroup alike, from the same sums in the same order) and gives the new
-// direction's beta. It stops after a breakdown (p.Kp <= 0), at the last
-// iteration, and where the residual is looked at (iterations 0 to 8 and every
-// fourth) unless it is above the tolerance (a NaN stops it too). Workgroup 0
-// stores what the iteration's other kernels and the host read; rz2 alternates
-// by parity, so no workgroup reads what another writes.
+// Start of iteration cg->it + 1: decides whether the solve stops (cg_next;
+// every workgroup alike, from the same sums in the same order) and gives the
+// new direction's beta. Workgroup 0 stores what the iteration's other kernels
+// and the host read; rz2 alternates by parity, so no workgroup reads what
+// another writes.
 template <int T>
 __device__ __forceinline__ bool cg_start(const QsCgStart& s, double* sh, double& beta) {
   double rz = 0.0, rr = 0.0;
@@ -84,14 +82,13 @@ __device__ __forceinline__ bool cg_start(const QsCgStart& s, double* sh, double&
   const int it = s.cg->it, brk = s.cg->brk;
   const double before = s.cg->rz2[(it + 1) & 1];
   block_sum2<T>(rz, rr, sh);
-  const bool look = it <= 8 || it % 4 == 0 || it >= s.cg->maxit;
-  const bool stop = brk || it >= s.cg->maxit ||
-                    (look && !(sqrt(rr) / s.cg->bnorm > s.cg->tol));
+  const int next = cg_next(it, s.cg->maxit, brk, rr, s.cg->bnorm, s.cg->tol);
+  const bool stop = next != CG_GO;
   beta = it > 0 ? rz / before : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (stop) {
       s.cg->done = 1;
-      cg_status_publish(s.status, brk, it, rr);
+      cg_status_publish(s.status, next == CG_BREAKS_DOWN, it, rr);
     } else {
       s.cg->rz = rz;
       s.cg->rz2[it & 1] = rz;

@@ -26,3 +26,8 @@ def test_status_is_handed_over_in_order(tmp_path):
     if "FATAL: ThreadSanitizer" in r.stdout:
         pytest.skip("the sanitizer does not run on this kernel: " + r.stdout[:200])
     assert r.returncode == 0 and "0 wrong" in r.stdout and "data race" not in r.stdout, r.stdout[:3000]
+
+
+def test_end_of_a_solve_is_the_host_loops(tmp_path):
+    r = subprocess.run([_build(tmp_path, "test_cg_next")], stdout=subprocess.PIPE, text=True, timeout=60)
+    assert r.returncode == 0 and " 0 wrong" in r.stdout, r.stdout
