@@ -824,7 +824,9 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_persistent(BondArgs a, T
 //
 // Every wait ends: after x.wait ticks of the 100 MHz clock a workgroup sets
 // *stuck and leaves, and the host repeats the run with two launches a step
-// from its copy of the state. The same arithmetic as those, bit for bit.
+// from its copy of the state. Its waves leave together: each of a step's two
+// waits has a flag of its own, read behind that wait's barrier and not written
+// again before every wave has passed another one. The same arithmetic as those, bit for bit.
 constexpr int RG = 16;  // lanes per node (32-node tiles)
 
 __device__ __forceinline__ void word_put(unsigned long long* p, unsigned data, unsigned tag) {
@@ -866,7 +868,7 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
     NodeRec* __restrict__ rec_end, float* __restrict__ theta, int* __restrict__ nbroken,
     VerletArgs va, int first, int nsteps, double t0) {
   __shared__ TileLds L;
-  __shared__ int bad;
+  __shared__ int bad[2];
   const int tile = blockIdx.x;
   const int n0 = t.tile_start[tile], n1 = t.tile_start[tile + 1];
   const int h0 = t.halo_off[tile], hn = min(t.halo_off[tile + 1] - h0, HMAX);
@@ -874,7 +876,7 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
   const int grp = threadIdx.x / RG, g = (threadIdx.x & 63) / RG, l = threadIdx.x & (RG - 1);
   const int node = n0 + grp;
   const bool valid = node < n1;
-  if (threadIdx.x == 0) bad = 0;
+  if (threadIdx.x < 2) bad[threadIdx.x] = 0;
   // the start, as in the passes
   HaloStage hs;
   halo_idx(hs, t, h0, hn);
@@ -921,14 +923,14 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
         const int h = threadIdx.x + r * WG;
         if (r > 0 && r * WG >= hn) break;
         unsigned w[6] = {0, 0, 0, 0, 0, 0};
-        if (h < hn && !words_wait<6>(src + hs.idx[r], a.n, tag, x.wait, w)) bad = 1;
+        if (h < hn && !words_wait<6>(src + hs.idx[r], a.n, tag, x.wait, w)) bad[0] = 1;
         if (h < hn) {
           lds_put(lds_b(L), h, make_uint4(w[0], w[1], w[2], w[3]));
           lds_put(lds_c(L), h, make_uint2(w[4], w[5]));
         }
       }
       __syncthreads();
-      if (bad) break;
+      if (bad[0]) break;
     }
     // damage and dilatation
     Nb nb{};
@@ -974,7 +976,7 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
 #pragma unroll
     for (int r = 0; r < kSlotsPerThread; r++) {
       unsigned w[1];
-      if (last[r] && !words_wait<1>(x.p + hs.idx[r], 0, tag, x.wait, w)) bad = 1;
+      if (last[r] && !words_wait<1>(x.p + hs.idx[r], 0, tag, x.wait, w)) bad[1] = 1;
     }
     __syncthreads();
 #pragma unroll
@@ -982,7 +984,7 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
       const int h = threadIdx.x + r * WG;
       if (r > 0 && r * WG >= hn) break;
       unsigned w[1] = {0};
-      if (h < hn && !words_wait<1>(x.p + hs.idx[r], 0, tag, x.wait, w)) bad = 1;
+      if (h < hn && !words_wait<1>(x.p + hs.idx[r], 0, tag, x.wait, w)) bad[1] = 1;
       if (h < hn) {
         const float p = __uint_as_float(w[0]);
         const float dp[2] = {hvol[r] * (halpha[r] - p), hvol[r] * p};
@@ -990,7 +992,7 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
       }
     }
     __syncthreads();
-    if (bad) break;
+    if (bad[1]) break;
     // force
     Nb2 n2{};
     float d_i = 0.0f, p_i = 0.0f;
@@ -1046,7 +1048,7 @@ __global__ __launch_bounds__(WG, WAVES_PER_SIMD) void k_resident(
       }
     }
   }
-  if (bad) {
+  if (bad[0] || bad[1]) {
     if (threadIdx.x == 0) *x.stuck = 1;
     return;
   }
