@@ -248,6 +248,11 @@ int pdg_set_per_pass_timing(pdg_ctx* ctx, int on);
  * soon does with 0, the run is repeated with two launches a step, as later
  * ones are until this is called again. The results are the same. */
 int pdg_set_resident_wait(pdg_ctx* ctx, double seconds);
+/* How the steps of the last pdg_verlet_run were taken. */
+#define PDG_ROUTE_LAUNCHED 0 /* launches for every step */
+#define PDG_ROUTE_RESIDENT 1 /* every tile on the GPU for the whole run */
+#define PDG_ROUTE_REPEATED 2 /* resident, given up, repeated with launches */
+int pdg_last_run_route(const pdg_ctx* ctx, int* route);
 
 /* Near-critical count of the last pdg_verlet_run / pdg_verlet_run_persistent
  * (or of the last pdg_compute_damage that asked for one): the number of

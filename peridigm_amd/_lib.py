@@ -102,6 +102,7 @@ SIGNATURES = {
     "pdg_last_timing": (_i, [_vp, C.POINTER(_d), C.POINTER(_d), C.POINTER(_d)]),
     "pdg_set_per_pass_timing": (_i, [_vp, _i]),
     "pdg_set_resident_wait": (_i, [_vp, _d]),
+    "pdg_last_run_route": (_i, [_vp, C.POINTER(_i)]),
     "pdg_near_critical_count": (_i, [_vp, C.POINTER(_ll)]),
     "pdg_qs_set_fixed": (_i, [_vp, _vp, _i]),
     "pdg_qs_residual": (_i, [_vp, _vp, _vp, C.POINTER(_d)]),

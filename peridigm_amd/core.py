@@ -275,6 +275,13 @@ class Context:
     def set_resident_wait(self, seconds=0.2):
         self.check(self.lib.pdg_set_resident_wait(self.h, seconds))
 
+    def last_run_route(self):
+        """How the last verlet_run took its steps: "launched", "resident", or
+        "repeated" (resident, given up after a wait in vain, launched)."""
+        r = C.c_int()
+        self.check(self.lib.pdg_last_run_route(self.h, C.byref(r)))
+        return ("launched", "resident", "repeated")[r.value]
+
     def last_timing(self):
         t = C.c_double(); a = C.c_double(); b = C.c_double()
         self.check(self.lib.pdg_last_timing(self.h, C.byref(t), C.byref(a), C.byref(b)))

@@ -500,6 +500,7 @@ int Ctx::run_resident(const VerletArgs& va, int first, int nsteps, double t0, bo
   if (!rc) rc = hip(hipMemcpyAsync(&bad, stuck, 4, hipMemcpyDeviceToHost, stream), "d2h");
   if (!rc) rc = hip(hipStreamSynchronize(stream), "sync");
   if (rc) return rc;
+  run_route = bad ? PDG_ROUTE_REPEATED : PDG_ROUTE_RESIDENT;
   if (!bad) {
     cur ^= 1;
     *done = true;
@@ -1285,6 +1286,7 @@ int pdg_verlet_run(pdg_ctx* h, int nsteps, double dt, double t0, int initialEval
     c->cur ^= 1;
     return r;
   };
+  c->run_route = PDG_ROUTE_LAUNCHED;
   bool resident = !contact && c->resident_run(nsteps);
   if (initialEval) {
     if (resident) {
@@ -1440,6 +1442,13 @@ int pdg_set_resident_wait(pdg_ctx* h, double seconds) {
   if (!c || !(seconds >= 0.0) || seconds > 10.0) return PDG_E_ARG;
   c->resident_wait = (unsigned long long)(1e8 * seconds);
   c->resident_off = false;
+  return PDG_OK;
+}
+
+int pdg_last_run_route(const pdg_ctx* h, int* route) {
+  const Ctx* c = reinterpret_cast<const Ctx*>(h);
+  if (!c || !route) return PDG_E_ARG;
+  *route = c->run_route;
   return PDG_OK;
 }
 
