@@ -44,8 +44,9 @@ __global__ __launch_bounds__(256) void k_rows_from_bits(int n, const int* __rest
                                                         const int* __restrict__ src,
                                                         const unsigned long long* __restrict__ bits,
                                                         unsigned long long* __restrict__ words) {
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (i >= n) return;
+  const long long t = wave_index();
+  if (t >= n) return;
+  const int i = (int)t, lane = threadIdx.x & 63;
   const int rs = row[i], deg = row[i + 1] - rs, w0 = mw[i];
   for (int k0 = 0; k0 < deg; k0 += 64) {
     bool broken = false;
@@ -65,8 +66,9 @@ __global__ __launch_bounds__(256) void k_check_ends(int n, const int* __restrict
                                                     const int* __restrict__ rev,
                                                     const unsigned long long* __restrict__ words,
                                                     int* __restrict__ bad) {
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (i >= n) return;
+  const long long t = wave_index();
+  if (t >= n) return;
+  const int i = (int)t, lane = threadIdx.x & 63;
   const int rs = row[i], deg = row[i + 1] - rs, w0 = mw[i];
   bool wrong = false;
   for (int k = lane; k < deg; k += 64) {
@@ -97,8 +99,9 @@ __global__ __launch_bounds__(256) void k_bits_from_rows(int n, const int* __rest
                                                         const int* __restrict__ src,
                                                         const unsigned long long* __restrict__ mask,
                                                         unsigned long long* __restrict__ bits) {
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (i >= n) return;
+  const long long t = wave_index();
+  if (t >= n) return;
+  const int i = (int)t, lane = threadIdx.x & 63;
   const int rs = row[i], deg = row[i + 1] - rs, w0 = mw[i];
   for (int k0 = 0; k0 < deg; k0 += 64) {
     const unsigned long long w = mask[w0 + (k0 >> 6)];
@@ -157,7 +160,7 @@ int Ctx::upload_mask(const double* bd, bool check_symmetric) {
     hipLaunchKernelGGL(k_pack_bits, dim3(blocks_for(n)), dim3(256), 0, stream, n, d_chunk,
                        d_lbits + b / 64, d_bad);
   }
-  const dim3 per_node((unsigned)((N + 3) / 4));
+  const dim3 per_node = wave_grid(N);
   hipLaunchKernelGGL(k_rows_from_bits, per_node, dim3(256), 0, stream, N, d_row, d_mw, d_src,
                      d_lbits, d_words);
   if (check_symmetric)
@@ -180,7 +183,7 @@ int Ctx::download_mask(double* bd) {
   if (rc) return rc;
   const long long nw = (B + 63) / 64;
   hipLaunchKernelGGL(k_zero_words, dim3(blocks_for(nw)), dim3(256), 0, stream, nw, d_lbits);
-  hipLaunchKernelGGL(k_bits_from_rows, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, stream, N,
+  hipLaunchKernelGGL(k_bits_from_rows, wave_grid(N), dim3(256), 0, stream, N,
                      d_row, d_mw, d_src, d_mask, d_lbits);
   rc = hip(hipGetLastError(), "bond field");
   if (rc) return rc;

@@ -241,17 +241,16 @@ __global__ __launch_bounds__(256) void k_contact_count(
 // thread per point left the GPU to a handful of waves, each walking some 300
 // candidates: 469 us on the notch of a 160,000-node plate, now 15.
 constexpr int kRowLds = 256;
-constexpr int kRowWaves = 4;
-__global__ __launch_bounds__(64 * kRowWaves) void k_contact_rows(
+__global__ __launch_bounds__(64 * kGroupWaves) void k_contact_rows(
     const int* __restrict__ npts, const int* __restrict__ pts, const double* __restrict__ y,
     const double* __restrict__ ys, double R2, double inv_cs, unsigned mask,
     const int* __restrict__ bstart, const int* __restrict__ bend, const int* __restrict__ sidx,
     const int* __restrict__ brow, const int* __restrict__ bcol, const long long* __restrict__ off,
     int* __restrict__ list) {
-  __shared__ int rows[kRowWaves][kRowLds];
-  __shared__ int first[kRowWaves][28], base[kRowWaves][28];
+  __shared__ int rows[kGroupWaves][kRowLds];
+  __shared__ int first[kGroupWaves][28], base[kGroupWaves][28];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * kRowWaves + w;
+  const long long t = wave_index();
   if (t >= *npts) return;  // whole waves: no barrier below
   const int i = pts[t];
   const double Y0 = y[3 * (size_t)i], Y1 = y[3 * (size_t)i + 1], Y2 = y[3 * (size_t)i + 2];
@@ -440,8 +439,7 @@ int search(Ctx* c, bool run) {
   // the rows of the points with contacts (their number stays on the device:
   // threads past it return at once)
   if (total > 0)
-    hipLaunchKernelGGL(k_contact_rows, dim3((unsigned)((N + kRowWaves - 1) / kRowWaves)),
-                       dim3(64 * kRowWaves), 0, s, S->nover_d, S->over, S->y,
+    hipLaunchKernelGGL(k_contact_rows, wave_grid(N), dim3(64 * kGroupWaves), 0, s, S->nover_d, S->over, S->y,
                        S->ys, R2, S->inv_cs, mask, S->bstart, S->bend, S->sidx, c->d_row, S->bcol, S->off,
                        S->list);
   rc = c->hip(hipGetLastError(), "contact fill");

@@ -180,6 +180,25 @@ hipError_t launch_resident(const BondArgs& a, const TileArgs& t, const ResidentA
                            const VerletArgs& va, int first, int nsteps, double t0, bool damage,
                            hipStream_t s);
 
+// Launches of a workgroup, or of a wave, for each of n points. A launch counts
+// its threads along an axis in 32 bits and drops the rest without an error (a
+// search of 2^26 + 5 points with a wave each ran for 5 of them), so from 2^20
+// workgroups on they go on along y.
+inline dim3 group_grid(long long groups) {
+  constexpr long long kAxis = 1ll << 20;
+  return dim3((unsigned)(groups < kAxis ? groups : kAxis), (unsigned)((groups + kAxis - 1) / kAxis));
+}
+constexpr int kGroupWaves = 4;  // waves of a workgroup
+inline dim3 wave_grid(long long n) { return group_grid((n + kGroupWaves - 1) / kGroupWaves); }
+#ifdef __HIPCC__
+__device__ __forceinline__ long long group_index() {
+  return (long long)blockIdx.y * gridDim.x + blockIdx.x;
+}
+__device__ __forceinline__ long long wave_index() {
+  return kGroupWaves * group_index() + (threadIdx.x >> 6);
+}
+#endif
+
 // Launchers (pdg_bonds.hip). `lanes` = lanes per node (16, 32 or 64; smaller
 // values run as 16).
 hipError_t launch_pass1(const BondArgs& a, NodeRec* rec, float* theta, int* nbroken,

@@ -193,7 +193,7 @@ __device__ bool plane_cuts(const double* pl, const double* p0, const double* p1)
 // by instruction issue: two in three candidates fail the distance test, and
 // ranking a row of 122 takes 244 broadcast compares a lane.
 constexpr int kRowCap = 512;
-constexpr int kWaves = 4;  // per workgroup
+using pdg::kGroupWaves;
 struct NearArgs {
   int n;
   RGrid g;
@@ -218,12 +218,13 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 template <bool FILL>
-__global__ __launch_bounds__(64 * kWaves) void k_near(NearArgs a) {
-  __shared__ __align__(16) int rows[kWaves][kRowCap + 68];
+__global__ __launch_bounds__(64 * kGroupWaves) void k_near(NearArgs a) {
+  __shared__ __align__(16) int rows[kGroupWaves][kRowCap + 68];
   const int lane = threadIdx.x & 63;
   int* const row = rows[threadIdx.x >> 6];
-  const int t = blockIdx.x * kWaves + (threadIdx.x >> 6);
-  if (t >= a.n) return;  // whole waves: no barrier below
+  const long long at = pdg::wave_index();
+  if (at >= a.n) return;  // whole waves: no barrier below
+  const int t = (int)at;
   const int i = a.sidx[t];
   const double P[3] = {a.xs[3 * (size_t)t], a.xs[3 * (size_t)t + 1], a.xs[3 * (size_t)t + 2]};
   int c[3];
@@ -318,8 +319,9 @@ __global__ __launch_bounds__(256) void k_spilled_rows(int n, const long long* __
                                                       const int* __restrict__ spill,
                                                       const int* __restrict__ flushed,
                                                       int* __restrict__ nlist) {
-  const int i = blockIdx.x;
-  if (!flushed[i]) return;
+  const long long at = pdg::group_index();
+  if (at >= n || !flushed[at]) return;
+  const int i = (int)at;
   const long long m = count[i];
   const int* r = spill + off[i];
   int* out = nlist + off[i] + i + 1;
@@ -481,8 +483,8 @@ int pdg_radius_search(int N, const double* x, double R, int nplanes, const doubl
   hipLaunchKernelGGL(k_cell_scatter, dim3(nb), dim3(256), 0, s, N, dx.p, cell, begin, ccount, sidx, xs);
   a.n = N; a.xs = xs; a.sidx = sidx; a.begin = begin; a.nplanes = nplanes; a.planes = dpl.p;
   a.count = count; a.off = off; a.big = big;
-  const unsigned nw = (unsigned)((N + kWaves - 1) / kWaves);
-  hipLaunchKernelGGL(k_near<false>, dim3(nw), dim3(64 * kWaves), 0, s, a);
+  const dim3 nw = pdg::wave_grid(N);
+  hipLaunchKernelGGL(k_near<false>, nw, dim3(64 * kGroupWaves), 0, s, a);
   PDG_CK(hipGetLastError());
   PDG_CK(hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, count, off, (int)n1, s));
   long long B = 0;
@@ -501,9 +503,9 @@ int pdg_radius_search(int N, const double* x, double R, int nplanes, const doubl
   a.nlist = list.p;
   a.spill = spill.p;
   a.flushed = hbig ? spill.p + B : nullptr;
-  hipLaunchKernelGGL(k_near<true>, dim3(nw), dim3(64 * kWaves), 0, s, a);
+  hipLaunchKernelGGL(k_near<true>, nw, dim3(64 * kGroupWaves), 0, s, a);
   if (hbig)
-    hipLaunchKernelGGL(k_spilled_rows, dim3((unsigned)N), dim3(256), 0, s, N, count, off, spill.p,
+    hipLaunchKernelGGL(k_spilled_rows, pdg::group_grid(N), dim3(256), 0, s, N, count, off, spill.p,
                        a.flushed, list.p);
   PDG_CK(hipGetLastError());
   PDG_CK(hipMemcpy(nlist, list.p, 4 * size, hipMemcpyDeviceToHost));
