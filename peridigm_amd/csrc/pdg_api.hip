@@ -211,7 +211,7 @@ TileArgs Ctx::tile_args() const {
 }
 
 // Internal CSR from perm: rows sorted by internal neighbour id, src = list-order
-// bond index, rev = reverse bond, mw = first mask word of each row.
+// bond index, mw = first mask word of each row.
 int Ctx::build_csr() {
   iperm.resize(N);
   for (int k = 0; k < N; k++) iperm[perm[k]] = k;
@@ -244,8 +244,7 @@ int Ctx::build_csr() {
     }
   });
   if (dup) return fail(PDG_E_UNSUPPORTED, "duplicate neighbour in neighbourhood list");
-  // Reverse bonds; the gather-only force needs a symmetric list.
-  rev.resize(B);
+  // The gather-only force needs a symmetric list.
   parallel_for(N, [&](long long k0, long long k1) {
     for (int k = (int)k0; k < (int)k1; k++)
       for (int b = row[k]; b < row[k + 1]; b++) {
@@ -253,8 +252,7 @@ int Ctx::build_csr() {
         const int* s = col.data() + row[j];
         const int* e = col.data() + row[j + 1];
         const int* it = std::lower_bound(s, e, k);
-        if (it == e || *it != k) { asym = 1; rev[b] = b; continue; }
-        rev[b] = (int)(it - col.data());
+        if (it == e || *it != k) asym = 1;
       }
   });
   if (asym) return fail(PDG_E_UNSUPPORTED, "neighbourhood list is not symmetric");
@@ -349,7 +347,7 @@ int Ctx::build_tiles(const std::vector<int>& bounds) {
 
 // Bond order inside the rows of the tiled CSR for conflict-free LDS reads
 // (pdg_sched.hpp), for the current lanes per node; col, src and lcol are
-// permuted together and the reverse-bond index rebuilt.
+// permuted together.
 void Ctx::order_bonds() {
   std::vector<int> slot(B), order(B);
   for (long long b = 0; b < B; b++) slot[b] = lcol[b] / kLdsSlot;
@@ -379,24 +377,6 @@ void Ctx::order_bonds() {
     src.swap(s2);
     lcol.swap(l2);
   }
-  // reverse bonds: rows are no longer sorted, so look up through a sorted
-  // copy of each row
-  std::vector<std::pair<int, int>> srt(B);
-  parallel_for(N, [&](long long k0, long long k1) {
-    for (int k = (int)k0; k < (int)k1; k++) {
-      for (int b = row[k]; b < row[k + 1]; b++) srt[b] = {col[b], b};
-      std::sort(srt.begin() + row[k], srt.begin() + row[k + 1]);
-    }
-  });
-  parallel_for(N, [&](long long k0, long long k1) {
-    for (int k = (int)k0; k < (int)k1; k++)
-      for (int b = row[k]; b < row[k + 1]; b++) {
-        const int j = col[b];
-        auto it = std::lower_bound(srt.begin() + row[j], srt.begin() + row[j + 1],
-                                   std::make_pair(k, -1));
-        rev[b] = it->second;
-      }
-  });
 }
 
 // Pinned host buffer of at least `bytes` (hipHostMalloc), kept for later
@@ -427,8 +407,7 @@ char* Ctx::stage(size_t bytes) {
 // as do copies from and to pageable memory and the events of HostOut. Calls
 // with host vectors, by kernels and so: drop-in force of 2,040 nodes 93 and 60
 // us, 12,000 127 and 88, 32,000 158 and 139; tangent product of 24,000 nodes
-// 184 and 145, 16,000 nodes 158 and 116.
-constexpr int kHostOrderMax = 32768;
+// 184 and 145, 16,000 nodes 158 and 116. The line: kHostOrderMax.
 
 // Current positions y (reference order, host) -> the records' u = y - x. The
 // copy of a large mesh reads the caller's array (37 GB/s; through the staging
@@ -726,6 +705,7 @@ int pdg_set_topology(pdg_ctx* h, int numOwned, const int* ownedIDs, const int* n
   c->nlist.assign(nlist, nlist + listSize);
   c->head.assign(numOwned, 0);
   long long li = 0, B = 0;
+  c->list_ascends = true;
   for (int i = 0; i < numOwned; i++) {
     if (li >= listSize) return c->fail(PDG_E_ARG, "neighbourhood list too short");
     c->head[i] = li;
@@ -736,6 +716,7 @@ int pdg_set_topology(pdg_ctx* h, int numOwned, const int* ownedIDs, const int* n
       if (j < 0 || j >= numOwned)
         return c->fail(PDG_E_UNSUPPORTED, "neighbour id outside the owned points (ghosts unsupported)");
       if (j == i) return c->fail(PDG_E_UNSUPPORTED, "self bond in neighbourhood list");
+      if (k > 0 && j < nlist[li + k]) c->list_ascends = false;
     }
     li += nn + 1;
     B += nn;

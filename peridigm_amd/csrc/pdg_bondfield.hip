@@ -1,17 +1,20 @@
 // Bond fields across the boundary: Bond_Damage, FP64 in list order on the host
 // and one bit a bond in the internal rows on the device.
 //
-// A field of zeros and ones goes up in chunks, each packed into bits in list
-// order as it arrives; one kernel then gathers the internal rows' words from
-// those bits through the bond index map, and one checks that both ends of
-// every bond agree. Coming back, the broken bonds' bits are set in list order
-// (few, so atomics are cheap) and the host threads only widen bits to doubles,
-// front to back. A host that gathers and scatters single bonds through the
-// index maps took 5 to 8 ms a call for 3M bonds; here the copy over PCIe, 24
-// MB at 30 GB/s, and the caller's pages bound it: 3.1M bonds 1.0 ms up and
-// 0.9 ms down.
+// Host threads pack a field of zeros and ones into bits in list order, front to
+// back, and a 64th of it goes up; one kernel then gathers the internal rows'
+// words from those bits through the bond index map, and one checks the other
+// end of every broken bond. Coming back, the broken bonds' bits are set in list
+// order (few, so atomics are cheap) and the host threads only widen bits to
+// doubles, front to back. Bound by host memory: the field is read once.
+// The whole field over PCIe, packed by a kernel, was bound by the copy from
+// pageable memory (drop-in force with a field: 640,000 nodes, 55M bonds, 16.1
+// ms, 980 nodes 354 us; host threads that gather single bonds through the map
+// 13.4 ms and 193 us; now 4.7 ms and 94 us).
 
 #include <algorithm>
+#include <atomic>
+#include <climits>
 #include <cstring>
 
 #include "pdg_ctx.hpp"
@@ -19,23 +22,59 @@
 namespace pdg {
 namespace {
 
-constexpr long long kChunk = 1ll << 22;  // doubles (32 MB), a multiple of 64
-
 inline unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 
-// Bits of n field values in list order (a wave per word); bad[0] is set by a
-// value that is neither 0 nor 1.
-__global__ __launch_bounds__(256) void k_pack_bits(long long n, const double* __restrict__ bd,
-                                                   unsigned long long* __restrict__ bits,
-                                                   int* __restrict__ bad) {
-  const long long b = (long long)blockIdx.x * 256 + threadIdx.x;
-  const double d = b < n ? bd[b] : 0.0;
-  const unsigned long long m = __ballot(d == 1.0);
-  const bool wrong = __ballot(d != 0.0 && d != 1.0) != 0ull;
-  if ((threadIdx.x & 63) == 0 && b < n) {
-    bits[b >> 6] = m;
-    if (wrong) bad[0] = 1;
+// Threads that pack or widen a field of nb bonds (starting one takes as long as
+// a core takes for some 50,000 bonds).
+inline unsigned field_threads(long long nb) { return nb < (1ll << 18) ? 1 : nb < (1ll << 22) ? 4 : 8; }
+
+// Bits of m <= 64 field values; `wrong` is set by a value other than 0 and 1.
+inline unsigned long long pack_bits(const double* v, int m, bool& wrong) {
+  constexpr unsigned long long kOne = 0x3ff0000000000000ull;
+  unsigned long long x[64];
+  std::memcpy(x, v, 8 * (size_t)m);
+  unsigned long long any = 0ull;
+  for (int k = 0; k < m; k++) any |= x[k];
+  if ((any << 1) == 0ull) return 0ull;  // zeros of either sign: most of a field
+  unsigned long long bits = 0ull;
+  bool bad = false;
+  for (int k = 0; k < m; k++) {
+    const bool one = x[k] == kOne;
+    bad |= !one && (x[k] << 1) != 0ull;
+    bits |= (unsigned long long)one << k;
   }
+  wrong |= bad;
+  return bits;
+}
+
+// List-order index of every internal bond where the list's rows ascend and
+// have at most 128 entries: the row's first index plus the number of smaller
+// ids in the row. A wave per node. (Computed, the map is there in 0.2 ms at 55M
+// bonds; the copy of the host's took 8.)
+__global__ __launch_bounds__(256) void k_src_by_rank(int n, const int* __restrict__ row,
+                                                     const int* __restrict__ col,
+                                                     const int* __restrict__ perm,
+                                                     const int* __restrict__ first,
+                                                     int* __restrict__ src) {
+  const long long t = wave_index();
+  if (t >= n) return;
+  const int i = (int)t, lane = threadIdx.x & 63;
+  const int rs = row[i], deg = row[i + 1] - rs;
+  const int a = lane < deg ? perm[col[rs + lane]] : INT_MAX;
+  const int b = lane + 64 < deg ? perm[col[rs + lane + 64]] : INT_MAX;
+  int ra = 0, rb = 0;
+  for (int k = 0; k < min(deg, 64); k++) {
+    const int v = __shfl(a, k);
+    ra += v < a;
+    rb += v < b;
+  }
+  for (int k = 0; k < deg - 64; k++) {
+    const int v = __shfl(b, k);
+    ra += v < a;
+    rb += v < b;
+  }
+  if (lane < deg) src[rs + lane] = first[i] + ra;
+  if (lane + 64 < deg) src[rs + lane + 64] = first[i] + rb;
 }
 
 // Mask words of the internal rows from the list-order bits: a wave per node.
@@ -59,11 +98,11 @@ __global__ __launch_bounds__(256) void k_rows_from_bits(int n, const int* __rest
   }
 }
 
-// bad[1] is set by a bond that only one end has broken: a wave per node.
+// *bad is set by a broken bond whose other end is intact: a wave per node, which
+// looks the node up in the other end's row for each of its broken bonds.
 __global__ __launch_bounds__(256) void k_check_ends(int n, const int* __restrict__ row,
                                                     const int* __restrict__ mw,
                                                     const int* __restrict__ col,
-                                                    const int* __restrict__ rev,
                                                     const unsigned long long* __restrict__ words,
                                                     int* __restrict__ bad) {
   const long long t = wave_index();
@@ -71,13 +110,15 @@ __global__ __launch_bounds__(256) void k_check_ends(int n, const int* __restrict
   const int i = (int)t, lane = threadIdx.x & 63;
   const int rs = row[i], deg = row[i + 1] - rs, w0 = mw[i];
   bool wrong = false;
-  for (int k = lane; k < deg; k += 64) {
-    const int j = col[rs + k], r = rev[rs + k] - row[j];
-    const unsigned long long a = words[w0 + (k >> 6)] >> (k & 63);
-    const unsigned long long b = words[mw[j] + (r >> 6)] >> (r & 63);
-    wrong |= ((a ^ b) & 1ull) != 0ull;
+  for (int k0 = 0; k0 < deg; k0 += 64) {
+    for (unsigned long long m = words[w0 + (k0 >> 6)]; m != 0ull; m &= m - 1ull) {
+      const int j = col[rs + k0 + __ffsll(m) - 1];
+      const int rj = row[j], dj = row[j + 1] - rj;
+      for (int q = lane; q < dj; q += 64)
+        if (col[rj + q] == i) wrong = wrong || !((words[mw[j] + (q >> 6)] >> (q & 63)) & 1ull);
+    }
   }
-  if (__ballot(wrong) && lane == 0) bad[1] = 1;
+  if (__ballot(wrong) && lane == 0) *bad = 1;
 }
 
 // The checked words become the mask (an accepted field only).
@@ -85,7 +126,7 @@ __global__ __launch_bounds__(256) void k_take_words(long long n, const unsigned 
                                                     const int* __restrict__ bad,
                                                     unsigned long long* __restrict__ mask) {
   const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (t < n && !bad[0] && !bad[1]) mask[t] = words[t];
+  if (t < n && !*bad) mask[t] = words[t];
 }
 
 __global__ __launch_bounds__(256) void k_zero_words(long long n, unsigned long long* __restrict__ w) {
@@ -116,29 +157,40 @@ __global__ __launch_bounds__(256) void k_bits_from_rows(int n, const int* __rest
 }  // namespace
 
 void Ctx::free_bond_maps() {
-  void* p[] = {d_src, d_rev, d_lbits, d_words, d_chunk, d_bad};
-  for (void* q : p) if (q) (void)hipFree(q);
-  d_src = d_rev = d_bad = nullptr;
+  if (d_src) (void)hipFree(d_src);
+  d_src = d_bad = nullptr;
   d_lbits = d_words = nullptr;
-  d_chunk = nullptr;
 }
 
-int Ctx::bond_maps(bool reverse) {
-  auto A = [&](void** p, size_t bytes) { return hip(hipMalloc(p, std::max<size_t>(bytes, 64)), "alloc bond maps"); };
-  const size_t nb = (size_t)B;
-  int rc = PDG_OK;
-  if (!d_bad) {
-    rc = A((void**)&d_src, 4 * nb);
-    if (!rc) rc = A((void**)&d_lbits, 8 * ((nb + 63) / 64));
-    if (!rc) rc = A((void**)&d_words, 8 * (size_t)mw.back());
-    if (!rc) rc = A((void**)&d_chunk, 8 * (size_t)std::min<long long>(B, kChunk));
-    if (!rc) rc = A((void**)&d_bad, 8);
-    if (!rc && nb) rc = hip(hipMemcpyAsync(d_src, src.data(), 4 * nb, hipMemcpyHostToDevice, stream), "h2d bond map");
-    if (rc) { free_bond_maps(); return rc; }
+// Device memory of the fields and the bond index map. `first` is a place in
+// memory that copies may read until the stream is synchronised (n ints).
+int Ctx::bond_maps(int* first) {
+  if (d_src) return PDG_OK;
+  auto up = [](size_t bytes) { return (bytes + 63) & ~(size_t)63; };
+  const size_t sb = up(4 * (size_t)B), wb = up(8 * (size_t)mw.back()), lw = ((size_t)B + 63) / 64;
+  char* p = nullptr;
+  int rc = hip(hipMalloc((void**)&p, sb + wb + 8 * (lw + 1)), "alloc bond maps");
+  if (rc) {
+    (void)hipGetLastError();
+    return rc;
   }
-  if (reverse && !d_rev) {
-    rc = A((void**)&d_rev, 4 * nb);
-    if (!rc && nb) rc = hip(hipMemcpyAsync(d_rev, rev.data(), 4 * nb, hipMemcpyHostToDevice, stream), "h2d bond map");
+  d_src = reinterpret_cast<int*>(p);
+  d_words = reinterpret_cast<unsigned long long*>(p + sb);
+  d_lbits = reinterpret_cast<unsigned long long*>(p + sb + wb);
+  d_bad = reinterpret_cast<int*>(d_lbits + lw);  // cleared with the bits' copy
+  if (list_ascends && ntiles > 0) {
+    for (int k = 0; k < N; k++) first[k] = (int)(head[perm[k]] - perm[k]);
+    int* const d_first = reinterpret_cast<int*>(d_y);
+    rc = hip(hipMemcpyAsync(d_first, first, 4 * (size_t)N, hipMemcpyHostToDevice, stream), "h2d rows");
+    if (!rc)
+      hipLaunchKernelGGL(k_src_by_rank, wave_grid(N), dim3(256), 0, stream, N, d_row, d_col, d_perm,
+                         d_first, d_src);
+  } else {
+    rc = hip(hipMemcpyAsync(d_src, src.data(), 4 * (size_t)B, hipMemcpyHostToDevice, stream), "h2d bond map");
+  }
+  if (rc) {
+    (void)hipStreamSynchronize(stream);
+    free_bond_maps();
   }
   return rc;
 }
@@ -146,57 +198,74 @@ int Ctx::bond_maps(bool reverse) {
 // Host field (list order) -> mask words. A rejected field leaves the mask as
 // it was.
 int Ctx::upload_mask(const double* bd, bool check_symmetric) {
-  const long long nw = mw.back();
+  const long long nw = mw.back(), lw = (B + 63) / 64;
   if (!bd)  // no field: every bond intact
     return hip(hipMemsetAsync(d_mask, 0, (size_t)nw * 8, stream), "zero mask");
   if (B == 0) return PDG_OK;
-  int rc = bond_maps(check_symmetric);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(256), 0, stream, 1ll, (unsigned long long*)d_bad);
-  for (long long b = 0; b < B; b += kChunk) {
-    const long long n = std::min(kChunk, B - b);
-    rc = hip(hipMemcpyAsync(d_chunk, bd + b, 8 * (size_t)n, hipMemcpyHostToDevice, stream), "h2d bond field");
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_pack_bits, dim3(blocks_for(n)), dim3(256), 0, stream, n, d_chunk,
-                       d_lbits + b / 64, d_bad);
+  // bits and rows behind the place of a small mesh's positions, which may be
+  // on their way
+  const size_t at = N <= kHostOrderMax ? (24 * (size_t)N + 63) & ~(size_t)63 : 0;
+  const size_t bytes = 8 * (size_t)(lw + 1) + 4 * (size_t)N + 8;
+  std::vector<char> own;
+  char* st = stage(at + bytes);
+  if (st) {
+    st += at;
+  } else {
+    own.resize(bytes);
+    st = own.data();
   }
-  const dim3 per_node = wave_grid(N);
-  hipLaunchKernelGGL(k_rows_from_bits, per_node, dim3(256), 0, stream, N, d_row, d_mw, d_src,
+  unsigned long long* const w = reinterpret_cast<unsigned long long*>(st);
+  int* const first = reinterpret_cast<int*>(w + lw + 1);
+  int* const bad = first + N;
+  w[lw] = 0ull;
+  std::atomic<bool> wrong{false};
+  const unsigned nt = field_threads(B);
+  on_threads(nt, [&](unsigned t) {
+    bool bad_value = false;
+    for (long long q = lw * t / nt; q < lw * (t + 1) / nt; q++)
+      w[q] = pack_bits(bd + 64 * q, (int)std::min<long long>(64, B - 64 * q), bad_value);
+    if (bad_value) wrong = true;
+  });
+  if (wrong) return fail(PDG_E_UNSUPPORTED, "bond damage values must be 0 or 1");
+  int rc = bond_maps(first);
+  if (rc) return rc;
+  rc = hip(hipMemcpyAsync(d_lbits, w, 8 * (size_t)(lw + 1), hipMemcpyHostToDevice, stream), "h2d bond bits");
+  hipLaunchKernelGGL(k_rows_from_bits, wave_grid(N), dim3(256), 0, stream, N, d_row, d_mw, d_src,
                      d_lbits, d_words);
   if (check_symmetric)
-    hipLaunchKernelGGL(k_check_ends, per_node, dim3(256), 0, stream, N, d_row, d_mw, d_col, d_rev,
+    hipLaunchKernelGGL(k_check_ends, wave_grid(N), dim3(256), 0, stream, N, d_row, d_mw, d_col,
                        d_words, d_bad);
   hipLaunchKernelGGL(k_take_words, dim3(blocks_for(nw)), dim3(256), 0, stream, nw, d_words, d_bad, d_mask);
-  rc = hip(hipGetLastError(), "bond field");
-  int bad[2] = {0, 0};
-  if (!rc) rc = hip(hipMemcpyAsync(bad, d_bad, 8, hipMemcpyDeviceToHost, stream), "d2h");
+  if (!rc) rc = hip(hipGetLastError(), "bond field");
+  *bad = 0;
+  if (!rc && check_symmetric)
+    rc = hip(hipMemcpyAsync(bad, d_bad, 4, hipMemcpyDeviceToHost, stream), "d2h");
   const int rc2 = hip(hipStreamSynchronize(stream), "sync");
   if (rc || rc2) return rc ? rc : rc2;
-  if (bad[0]) return fail(PDG_E_UNSUPPORTED, "bond damage values must be 0 or 1");
-  if (bad[1]) return fail(PDG_E_UNSUPPORTED, "bond damage must be symmetric (d_ij == d_ji)");
-  return PDG_OK;
+  return *bad ? fail(PDG_E_UNSUPPORTED, "bond damage must be symmetric (d_ij == d_ji)") : PDG_OK;
 }
 
 int Ctx::download_mask(double* bd) {
   if (B == 0) return hip(hipStreamSynchronize(stream), "sync");
-  int rc = bond_maps(false);
-  if (rc) return rc;
   const long long nw = (B + 63) / 64;
+  std::vector<char> own;
+  char* st = stage(8 * (size_t)nw + 4 * (size_t)N);
+  if (!st) {
+    own.resize(8 * (size_t)nw + 4 * (size_t)N);
+    st = own.data();
+  }
+  unsigned long long* const w = reinterpret_cast<unsigned long long*>(st);
+  int rc = bond_maps(reinterpret_cast<int*>(st + 8 * nw));
+  if (rc) return rc;
   hipLaunchKernelGGL(k_zero_words, dim3(blocks_for(nw)), dim3(256), 0, stream, nw, d_lbits);
   hipLaunchKernelGGL(k_bits_from_rows, wave_grid(N), dim3(256), 0, stream, N,
                      d_row, d_mw, d_src, d_mask, d_lbits);
   rc = hip(hipGetLastError(), "bond field");
   if (rc) return rc;
-  std::vector<unsigned long long> own;
-  unsigned long long* w = reinterpret_cast<unsigned long long*>(stage(8 * (size_t)nw));
-  if (!w) {
-    own.resize(nw);
-    w = own.data();
-  }
   rc = hip(hipMemcpyAsync(w, d_lbits, 8 * (size_t)nw, hipMemcpyDeviceToHost, stream), "d2h bond bits");
   if (!rc) rc = hip(hipStreamSynchronize(stream), "sync");
   if (rc) return rc;
-  const unsigned nt = B < (1ll << 18) ? 1 : B < (1ll << 22) ? 4 : 8;
+  const unsigned nt = field_threads(B);
   on_threads(nt, [&](unsigned t) {
     for (long long q = nw * t / nt; q < nw * (t + 1) / nt; q++) {
       double* out = bd + 64 * q;

@@ -58,6 +58,10 @@ struct QsState;   // quasi-static solver workspace (pdg_qs.hip)
 struct GnnState;  // learned preconditioner (pdg_gnn.hip)
 struct ContactState;  // short-range contact (pdg_contact.hip)
 
+// Meshes of at most this many nodes have their vectors reordered on the host
+// (pdg_api.hip says why).
+constexpr int kHostOrderMax = 32768;
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -75,12 +79,12 @@ struct Ctx {
   long long B = 0;
   std::vector<int> nlist;
   std::vector<long long> head;
+  bool list_ascends = false;  // every row's neighbours in ascending order
 
   // Hilbert order and internal CSR
   std::vector<int> perm, iperm;  // perm[k]: original id of internal node k
   std::vector<int> row, col;     // CSR over internal ids (tiled: rows in LDS-schedule order)
   std::vector<int> src;          // internal bond -> list-order bond index
-  std::vector<int> rev;          // internal bond (i->j) -> internal bond (j->i)
   std::vector<int> mw;           // first mask word of each node
 
   // constants
@@ -197,16 +201,14 @@ struct Ctx {
   void free_extra();
   BondArgs bond_args() const;
   hipError_t pass1(NodeRec* rec, int* nbroken, bool damage, bool count_near);
-  // bond fields (pdg_bondfield.hip): maps between the list order and the
-  // internal rows on the device, made by the first call that needs them, bits
-  // in list order, internal words awaiting their check, a chunk of a field
+  // bond fields (pdg_bondfield.hip), in one piece of device memory made by the
+  // first call that needs it: the bond index map, bits in list order, internal
+  // words awaiting their check, whether they failed it
   int* d_src = nullptr;  // B: list-order index of each internal bond
-  int* d_rev = nullptr;  // B: the reverse bond
   unsigned long long* d_lbits = nullptr;
   unsigned long long* d_words = nullptr;
-  double* d_chunk = nullptr;
-  int* d_bad = nullptr;  // 2: a value other than 0 and 1, an asymmetric bond
-  int bond_maps(bool reverse);
+  int* d_bad = nullptr;
+  int bond_maps(int* first);
   void free_bond_maps();
   int upload_mask(const double* bd, bool check_symmetric);
   int download_mask(double* bd);
