@@ -149,6 +149,7 @@ int Ctx::fail(int code, const std::string& msg) {
 
 int Ctx::hip(hipError_t e, const char* what) {
   if (e == hipSuccess) return PDG_OK;
+  (void)hipGetLastError();  // reported here, not by the next launch's check too
   err = std::string(what) + ": " + hipGetErrorString(e);
   return PDG_E_HIP;
 }
@@ -391,6 +392,7 @@ char* Ctx::stage(size_t bytes) {
   h_stage = nullptr;
   h_stage_bytes = 0;
   if (hipHostMalloc((void**)&h_stage, bytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch would be taken to have failed
     h_stage = nullptr;
     return nullptr;
   }
