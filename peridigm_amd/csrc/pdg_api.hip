@@ -98,6 +98,8 @@ inline size_t state_stage_bytes(int n) {
   return 4 * (24 * (size_t)n + 64) + 2 * (8 * (size_t)n + 64);
 }
 
+constexpr size_t kStageAheadMax = 128u << 20;
+
 inline dim3 blocks_of(long long n) { return dim3((unsigned)((n + 255) / 256)); }
 
 // Hilbert index of a 21-bit cell triple (Skilling's transpose algorithm:
@@ -983,8 +985,9 @@ int pdg_set_constants(pdg_ctx* h, const double* x, const double* vol, double K, 
   c->have_consts = true;
   // the staging buffer of a whole state (u, v, a, force, damage, dilatation),
   // now rather than in the first call that needs it: pinning and mapping it
-  // take 0.1 to 0.3 ms per MB
-  (void)c->stage(state_stage_bytes(N));
+  // take 0.1 to 0.3 ms per MB. Contexts for which that is more than 128 MB (1.2M
+  // nodes) get theirs in the call that needs one, of the size it needs.
+  if (state_stage_bytes(N) <= kStageAheadMax) (void)c->stage(state_stage_bytes(N));
   return PDG_OK;
 }
 
@@ -1374,7 +1377,10 @@ int pdg_state_download(pdg_ctx* h, double* u, double* v, double* a, double* bd, 
   if (N > 0) {
     // every node field through one scratch vector, each copied out before the
     // next overwrites it (stream order)
-    HostOut o(c, state_stage_bytes(N));
+    size_t bytes = 0;
+    for (const double* f : {u, v, a, force}) bytes += f ? vec + 64 : 0;
+    for (const double* f : {damage, dilatation}) bytes += f ? sca + 64 : 0;
+    HostOut o(c, bytes);
     auto vec3 = [&](const double* d, double* out) {
       if (rc || !out) return;
       hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, d, c->d_perm, c->d_y);

@@ -14,6 +14,8 @@ SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 static int refuse;
+static size_t pinned;
+extern "C" long long pinned_bytes() { return (long long)pinned; }
 extern "C" void set_refuse(int on) { refuse = on; }
 extern "C" int hipHostMalloc(void** p, size_t n, unsigned flags) {
   typedef int (*fn)(void**, size_t, unsigned);
@@ -23,6 +25,7 @@ extern "C" int hipHostMalloc(void** p, size_t n, unsigned flags) {
     real(nullptr, n, flags);
     return 2;  // hipErrorOutOfMemory
   }
+  pinned += n;
   return real(p, n, flags);
 }
 """
@@ -65,14 +68,58 @@ print("same", flush=True)
 """
 
 
-@pytest.mark.parametrize("nx", [20, 450])  # 1,600 and 36,000 nodes
-def test_calls_without_the_staging_buffer(tmp_path, nx):
+LARGE = r"""
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+shim.pinned_bytes.restype = ctypes.c_longlong
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from peridigm_amd import Context
+n = int(sys.argv[3])
+x = np.zeros((n, 3))
+x[:, 0] = np.arange(n)
+i = np.arange(n, dtype=np.int32)
+nl = np.empty(3 * n - 2, np.int32)
+nl[:2], nl[-2:] = (1, 1), (1, n - 2)
+nl[2:-2].reshape(-1, 3)[:] = np.stack([np.full(n - 2, 2, np.int32), i[:-2], i[2:]], axis=1)
+with Context(0) as c:
+    c.set_topology(nl, n)
+    c.set_constants(x, np.ones(n), 130e9, 60e9, 1.1, 0, 1e-2)
+    ahead = shim.pinned_bytes()
+    assert ahead <= 128 << 20, ahead
+    assert (ahead > 100 * n) == (112 * n + 384 <= 128 << 20), ahead
+    c.set_density(7800.0)
+    v = np.random.default_rng(1).standard_normal(x.shape)
+    c.upload_state(v=v)
+    out = np.zeros((n, 3))
+    p = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    c.check(c.lib.pdg_state_download(c.h, None, p(out), None, None, None, None, None))
+    assert np.array_equal(out, v)
+    # what the download needed: its one field
+    assert shim.pinned_bytes() - ahead <= 24 * n + 4096, shim.pinned_bytes()
+print("same", flush=True)
+"""
+
+
+def _run(tmp_path, program, *args):
     import os
     src, so, prog = tmp_path / "shim.cpp", tmp_path / "shim.so", tmp_path / "prog.py"
     src.write_text(SHIM)
-    prog.write_text(textwrap.dedent(PROGRAM))
+    prog.write_text(textwrap.dedent(program))
     subprocess.run(["g++", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl"], check=True, timeout=60)
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    r = subprocess.run([sys.executable, str(prog), str(so), root, str(nx)], timeout=100,
+    r = subprocess.run([sys.executable, str(prog), str(so), root, *map(str, args)], timeout=100,
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert r.returncode == 0 and r.stdout.strip().endswith("same"), r.stdout[-2000:]
+
+
+@pytest.mark.parametrize("nx", [20, 450])  # 1,600 and 36,000 nodes
+def test_calls_without_the_staging_buffer(tmp_path, nx):
+    _run(tmp_path, PROGRAM, nx)
+
+
+@pytest.mark.parametrize("n", [100000, 1300000])
+def test_set_up_pins_a_bounded_buffer(tmp_path, n):
+    """Set-up pins a whole state's buffer up to 128 MB; larger contexts pin what
+    their calls need."""
+    _run(tmp_path, LARGE, n)
