@@ -502,12 +502,14 @@ int HostOut::add(void* dst, const void* dev, size_t bytes) {
   if (!bytes) return PDG_OK;
   Part& p = part_[n_];
   p = Part{(char*)dst, at_ ? at_ + used_ : nullptr, bytes};
-  int rc = c_->hip(hipMemcpyAsync(at_ ? at_ + used_ : (char*)dst, dev, bytes, hipMemcpyDeviceToHost,
-                                  c_->stream), "d2h");
-  hipEvent_t& e = c_->oev[n_];
-  if (!rc && !e) rc = c_->hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
-  if (!rc) rc = c_->hip(hipEventRecord(e, c_->stream), "event");
-  if (rc) return rc;
+  if (!together_) {
+    int rc = c_->hip(hipMemcpyAsync(at_ ? at_ + used_ : (char*)dst, dev, bytes, hipMemcpyDeviceToHost,
+                                    c_->stream), "d2h");
+    hipEvent_t& e = c_->oev[n_];
+    if (!rc && !e) rc = c_->hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
+    if (!rc) rc = c_->hip(hipEventRecord(e, c_->stream), "event");
+    if (rc) return rc;
+  }
   used_ += (bytes + 63) & ~(size_t)63;
   total_ += bytes;
   n_++;
@@ -517,9 +519,14 @@ int HostOut::add(void* dst, const void* dev, size_t bytes) {
 int HostOut::finish() {
   const unsigned nt = total_ < (2u << 20) ? 1 : total_ < (32u << 20) ? 4 : 8;
   std::atomic<int> bad{0};
+  if (together_ && n_ > 0) {
+    int rc = c_->hip(hipMemcpyAsync(at_, c_->d_y, used_, hipMemcpyDeviceToHost, c_->stream), "d2h");
+    const int rc2 = c_->hip(hipStreamSynchronize(c_->stream), "sync");
+    if (rc || rc2) return rc ? rc : rc2;
+  }
   on_threads(at_ ? nt : 1, [&](unsigned t) {
     for (int k = 0; k < n_; k++) {
-      if (hipEventSynchronize(c_->oev[k]) != hipSuccess) { bad = 1; return; }
+      if (!together_ && hipEventSynchronize(c_->oev[k]) != hipSuccess) { bad = 1; return; }
       const Part& p = part_[k];
       if (!p.src) continue;
       const size_t lo = (p.bytes / 64 * t / nt) * 64;
@@ -527,6 +534,7 @@ int HostOut::finish() {
       std::memcpy(p.dst + lo, p.src + lo, hi - lo);
     }
   });
+  if (together_ && n_ > 0) return PDG_OK;
   int rc = c_->hip(hipStreamSynchronize(c_->stream), "sync");
   if (!rc && bad) rc = c_->fail(PDG_E_HIP, "waiting for a result failed");
   return rc;
@@ -543,16 +551,16 @@ int Ctx::download_vec3(const double* dsrc, double* out) {
       for (int c = 0; c < 3; c++) out[3 * (size_t)perm[k] + c] = st[3 * (size_t)k + c];
     return PDG_OK;
   }
-  HostOut o(this, 24 * (size_t)N);
-  hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, stream, N, dsrc, d_perm, d_y);
+  HostOut o(this, 24 * (size_t)N, true);
+  hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, stream, N, dsrc, d_perm, o.next());
   int rc = o.add(out, d_y, 24 * (size_t)N);
   return rc ? rc : o.finish();
 }
 
 int Ctx::download_scalar(const double* dsrc, double* out) {
   if (N <= 0) return PDG_OK;
-  HostOut o(this, 8 * (size_t)N);
-  hipLaunchKernelGGL(k_scalar_out, blocks_of(N), dim3(256), 0, stream, N, dsrc, d_perm, d_y);
+  HostOut o(this, 8 * (size_t)N, true);
+  hipLaunchKernelGGL(k_scalar_out, blocks_of(N), dim3(256), 0, stream, N, dsrc, d_perm, o.next());
   int rc = o.add(out, d_y, 8 * (size_t)N);
   return rc ? rc : o.finish();
 }
@@ -863,7 +871,8 @@ int pdg_set_constants(pdg_ctx* h, const double* x, const double* vol, double K, 
   if ((rc = A((void**)&c->d_a, (size_t)N * 24, "alloc a"))) return rc;
   if ((rc = A((void**)&c->d_f, (size_t)N * 24, "alloc f"))) return rc;
   if ((rc = A((void**)&c->d_fout, (size_t)N * 24, "alloc fout"))) return rc;
-  if ((rc = A((void**)&c->d_y, (size_t)N * 24, "alloc y"))) return rc;
+  // small meshes: room for a whole state (HostOut)
+  if ((rc = A((void**)&c->d_y, N <= kHostOrderMax ? state_stage_bytes(N) : (size_t)N * 24, "alloc y"))) return rc;
   if ((rc = A((void**)&c->d_inv_rho, (size_t)N * 8, "alloc rho"))) return rc;
   if ((rc = A((void**)&c->d_bcslot, (size_t)N * 4, "alloc bcslot"))) return rc;
   if ((rc = A((void**)&c->d_bcs, sizeof(BcSlot), "alloc bcs"))) return rc;
@@ -1086,10 +1095,10 @@ int pdg_compute_damage(pdg_ctx* h, const double* y, const double* bdN, double* b
     (void)hipStreamSynchronize(s);  // the copy of y reads the caller's array
     return rc;
   }
-  HostOut o(c, 8 * (size_t)N);
+  HostOut o(c, 8 * (size_t)N, true);
   if (N > 0)
     hipLaunchKernelGGL(k_damage_out, blocks_of(N), dim3(256), 0, s, N, c->d_nbroken, c->d_row,
-                       c->d_perm, 0, c->d_y);
+                       c->d_perm, 0, o.next());
   rc = o.add(damage, c->d_y, 8 * (size_t)N);
   if (!rc) rc = o.finish();
   if (rc) return rc;
@@ -1136,11 +1145,11 @@ int pdg_compute_force(pdg_ctx* h, double dt, const double* y, const double* bdNP
     }
     return PDG_OK;
   }
-  HostOut o(c, 32 * (size_t)N + 128);
-  hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_fout, c->d_perm, c->d_y);
+  HostOut o(c, 32 * (size_t)N + 128, true);
+  hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_fout, c->d_perm, o.next());
   rc = o.add(force, c->d_y, 24 * (size_t)N);
   if (!rc && dilatation) {
-    hipLaunchKernelGGL(k_theta_out, blocks_of(N), dim3(256), 0, s, N, c->d_theta, c->d_perm, c->d_y);
+    hipLaunchKernelGGL(k_theta_out, blocks_of(N), dim3(256), 0, s, N, c->d_theta, c->d_perm, o.next());
     rc = o.add(dilatation, c->d_y, 8 * (size_t)N);
   }
   const int rc2 = o.finish();
@@ -1157,7 +1166,10 @@ int pdg_state_upload(pdg_ctx* h, const double* u, const double* v, const double*
   int rc = c->hip(hipStreamSynchronize(s), "sync");
   if (!rc && N > 0) {
     if (u) {
-      rc = c->hip(hipMemcpyAsync(c->d_y, u, 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d u");
+      const void* src = u;
+      if (char* st = N <= kHostOrderMax ? c->stage(state_stage_bytes(N)) : nullptr)
+        src = std::memcpy(st + 48 * (size_t)N, u, 24 * (size_t)N);  // behind v and a
+      rc = c->hip(hipMemcpyAsync(c->d_y, src, 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d u");
       if (!rc)
         hipLaunchKernelGGL(k_set_u_disp, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_y, c->d_perm,
                            c->d_rec[c->cur], c->q);
@@ -1375,20 +1387,20 @@ int pdg_state_download(pdg_ctx* h, double* u, double* v, double* a, double* bd, 
   const size_t vec = 24 * (size_t)N, sca = 8 * (size_t)N;
   int rc = PDG_OK;
   if (N > 0) {
-    // every node field through one scratch vector, each copied out before the
-    // next overwrites it (stream order)
+    // large meshes: every node field through one scratch vector, each copied out
+    // before the next overwrites it (stream order)
     size_t bytes = 0;
     for (const double* f : {u, v, a, force}) bytes += f ? vec + 64 : 0;
     for (const double* f : {damage, dilatation}) bytes += f ? sca + 64 : 0;
-    HostOut o(c, bytes);
+    HostOut o(c, bytes, true);
     auto vec3 = [&](const double* d, double* out) {
       if (rc || !out) return;
-      hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, d, c->d_perm, c->d_y);
+      hipLaunchKernelGGL(k_vec3_out, blocks_of(3ll * N), dim3(256), 0, s, N, d, c->d_perm, o.next());
       rc = o.add(out, c->d_y, vec);
     };
     if (u) {
       hipLaunchKernelGGL(k_disp_out, blocks_of(3ll * N), dim3(256), 0, s, N, c->d_rec[c->cur],
-                         c->d_perm, c->q, c->d_y);
+                         c->d_perm, c->q, o.next());
       rc = o.add(u, c->d_y, vec);
     }
     vec3(c->d_v, v);
@@ -1396,11 +1408,11 @@ int pdg_state_download(pdg_ctx* h, double* u, double* v, double* a, double* bd, 
     vec3(c->d_f, force);
     if (!rc && damage) {
       hipLaunchKernelGGL(k_damage_out, blocks_of(N), dim3(256), 0, s, N, c->d_nbroken, c->d_row,
-                         c->d_perm, c->sc > 0.0 ? 0 : 1, c->d_y);
+                         c->d_perm, c->sc > 0.0 ? 0 : 1, o.next());
       rc = o.add(damage, c->d_y, sca);
     }
     if (!rc && dilatation) {
-      hipLaunchKernelGGL(k_theta_out, blocks_of(N), dim3(256), 0, s, N, c->d_theta, c->d_perm, c->d_y);
+      hipLaunchKernelGGL(k_theta_out, blocks_of(N), dim3(256), 0, s, N, c->d_theta, c->d_perm, o.next());
       rc = o.add(dilatation, c->d_y, sca);
     }
     const int rc2 = o.finish();
