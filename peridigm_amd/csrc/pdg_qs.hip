@@ -169,11 +169,13 @@ struct QsArgs {
   const double* dT;  // temperature change per node (thermal strains), or null
   double alphaT;     // thermal expansion coefficient
   double* ps;        // partial stress, 9 per node (force<3>)
+  const int* done;   // tangent passes of a solve: its end, after which they return at once
 };
 
 // dilatation (+ its directional derivative, + d theta_i / d u_i)
 template <int QG, bool DUAL, bool DIAG, bool GEN>
 __global__ __launch_bounds__(256) void k_qs_theta(QsArgs a) {
+  if (DUAL && a.done && *a.done) return;
   const int lane = threadIdx.x & 63;
   const int gi = lane / QG, l = lane & (QG - 1);
   const int node = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / QG) + gi;
@@ -240,6 +242,7 @@ __global__ __launch_bounds__(256) void k_qs_theta(QsArgs a) {
 // allowed 4), with no spills
 template <int QG, int MODE, bool GEN>
 __global__ __launch_bounds__(256, 5) void k_qs_force(QsArgs a) {
+  if (MODE == 1 && a.done && *a.done) return;
   const int lane = threadIdx.x & 63;
   const int gi = lane / QG, l = lane & (QG - 1);
   const int node = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / QG) + gi;
@@ -421,8 +424,10 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
   return t;
 }
 
-__global__ __launch_bounds__(RB) void k_dot(int n, const double* a, const double* b, double* part) {
+__global__ __launch_bounds__(RB) void k_dot(int n, const double* a, const double* b, double* part,
+                                            const int* done) {
   __shared__ double sh[RB / 64];
+  if (done && *done) return;
   double s = 0.0;
   for (int i = blockIdx.x * RB + threadIdx.x; i < n; i += gridDim.x * RB) s += a[i] * b[i];
   s = block_sum(s, sh);
@@ -575,9 +580,9 @@ __global__ __launch_bounds__(RB) void k_per_volume(int n, const double* vol, dou
 
 // out += s * w (damped-Newton diagonal shift)
 __global__ __launch_bounds__(RB) void k_damp_add(int n, const double* sdiag, const double* w,
-                                                 double* out) {
+                                                 double* out, const int* done) {
   const int i = blockIdx.x * RB + threadIdx.x;
-  if (i < n) out[i] += sdiag[i] * w[i];
+  if (i < n && !(done && *done)) out[i] += sdiag[i] * w[i];
 }
 
 // s = (f - 1) d + g: the change of the diagonal d scaled by f and shifted by g
@@ -1192,19 +1197,22 @@ static int residual(Ctx* c, bool all = false) {
   return c->hip(hipGetLastError(), "qs residual");
 }
 
-// K w for device w, output in `out`; needs state() at the current u
-static int tangent(Ctx* c, const double* w, double* out, bool tiled = true) {
+// K w for device w, output in `out`; needs state() at the current u. done: see
+// QsArgs (untiled meshes).
+static int tangent(Ctx* c, const double* w, double* out, bool tiled = true,
+                   const int* done = nullptr) {
   hipStream_t s = c->stream;
   if (tiled && c->tiled())
     return c->hip(launch_qs_tangent(tile_args(c), w, out, c->tile_lanes(), s), "qs tangent");
   QsArgs a = args(c);
   a.w = w;
   a.out = out;
+  a.done = done;
   qs_theta<true, false>(a, s);
   qs_force<1>(a, s);
   if (c->qs->damped) {
     const int n3 = 3 * c->N;
-    hipLaunchKernelGGL(k_damp_add, dim3((n3 + RB - 1) / RB), dim3(RB), 0, s, n3, c->qs->dampv, w, out);
+    hipLaunchKernelGGL(k_damp_add, dim3((n3 + RB - 1) / RB), dim3(RB), 0, s, n3, c->qs->dampv, w, out, done);
   }
   return c->hip(hipGetLastError(), "qs tangent");
 }
@@ -1347,7 +1355,7 @@ static int coarse_build(Ctx* c) {
 static int dot(Ctx* c, const double* x, const double* y, double* out) {
   QsState* S = c->qs;
   const int n = 3 * c->N;
-  hipLaunchKernelGGL(k_dot, dim3(S->nblk), dim3(RB), 0, c->stream, n, x, y, S->part);
+  hipLaunchKernelGGL(k_dot, dim3(S->nblk), dim3(RB), 0, c->stream, n, x, y, S->part, nullptr);
   hipLaunchKernelGGL(k_final, dim3(1), dim3(RB), 0, c->stream, S->nblk, S->part, 1, S->scal);
   int rc = c->hip(hipMemcpyAsync(out, S->scal, 8, hipMemcpyDeviceToHost, c->stream), "d2h");
   if (!rc) rc = c->hip(hipStreamSynchronize(c->stream), "sync");
@@ -1552,9 +1560,9 @@ static int cg_solve(Ctx* c, double* x, const double* b, double bnorm, int precon
       return c->hip(launch_qs_tangent_cg(ta[k & 1], start, z, S->q, S->pq_part, c->tile_lanes(), s),
                     "cg product");
     hipLaunchKernelGGL(k_cg_dir, dim3(S->nblk), dim3(RB), 0, s, n3, start, z, S->p);
-    int r2 = tangent(c, S->p, S->q);
+    int r2 = tangent(c, S->p, S->q, false, &S->cg->done);
     if (r2) return r2;
-    hipLaunchKernelGGL(k_dot, dim3(S->nblk), dim3(RB), 0, s, n3, S->p, S->q, S->pq_part);
+    hipLaunchKernelGGL(k_dot, dim3(S->nblk), dim3(RB), 0, s, n3, S->p, S->q, S->pq_part, &S->cg->done);
     return c->hip(hipGetLastError(), "cg product");
   };
   int rc = tangent(c, x, S->q);
@@ -1594,10 +1602,12 @@ static int cg_solve(Ctx* c, double* x, const double* b, double bnorm, int precon
       if (!rc) rc = c->hip(hipEventRecord(ev, s), "event");
       if (!rc && chunk > 0) rc = c->hip(hipEventSynchronize(S->cev[(chunk - 1) & 1]), "sync");
     } else {
-      for (int k = 0; k < kCgChunk && !rc; k++) {
+      // none past the limit: the product of iteration `last` only decides
+      const int last = std::max(maxit, 0) - std::min(chunk, std::max(maxit, 0) / kCgChunk) * kCgChunk;
+      for (int k = 0; k < kCgChunk && k <= last && !rc; k++) {
         rc = product(k);
-        if (!rc && k == 0) rc = c->hip(hipEventRecord(ev, s), "event");
-        if (!rc) rc = update(k, false);
+        if (!rc && (k == 0 || k == last)) rc = c->hip(hipEventRecord(ev, s), "event");
+        if (!rc && k < last) rc = update(k, false);
       }
       if (!rc) rc = c->hip(hipEventSynchronize(ev), "sync");
     }
@@ -1643,7 +1653,7 @@ int qs_solve(Ctx* c, double* x, const double* b, int precond, double tol, int ma
   if (precond != 2) return qs::cg_solve(c, x, b, bnorm, precond, tol, maxit, iters, rel);
   // device dot product into scalar slot k
   auto ddot = [&](const double* u, const double* v, int k) {
-    hipLaunchKernelGGL(k_dot, red, blk, 0, s, n3, u, v, S->part);
+    hipLaunchKernelGGL(k_dot, red, blk, 0, s, n3, u, v, S->part, nullptr);
     hipLaunchKernelGGL(k_final, dim3(1), blk, 0, s, S->nblk, S->part, 1, S->scal + k);
   };
   // r = b - K x; z = M r; p = z
