@@ -313,23 +313,63 @@ __global__ __launch_bounds__(64 * kGroupWaves) void k_near(NearArgs a) {
   }
 }
 
-// The flushed rows, ranked from `spill` (a workgroup per point).
-__global__ __launch_bounds__(256) void k_spilled_rows(int n, const long long* __restrict__ count,
-                                                      const long long* __restrict__ off,
-                                                      const int* __restrict__ spill,
-                                                      const int* __restrict__ flushed,
-                                                      int* __restrict__ nlist) {
+// The flushed rows, sorted from `spill` (a workgroup per row): pieces of up to
+// kSortPiece ids in LDS (bitonic, padded to a power of two), and where a row has
+// more than one, each id then goes to its place in its piece plus the number of
+// smaller ids in the others (ids are unique). Work per row of m ids is about
+// m log^2 m; counting the smaller ones for every id took m^2: lists of 22,000
+// points that are all in each other's radius 1.82 s, with this 0.30 (a radix sort
+// of all bonds, before, 0.64).
+constexpr int kSortPiece = 4096;
+constexpr int kSortThreads = 256;
+__global__ __launch_bounds__(kSortThreads) void k_spilled_rows(
+    int n, const long long* __restrict__ count, const long long* __restrict__ off, int* spill,
+    const int* __restrict__ flushed, int* __restrict__ nlist) {
+  __shared__ int a[kSortPiece];
   const long long at = pdg::group_index();
   if (at >= n || !flushed[at]) return;
-  const int i = (int)at;
-  const long long m = count[i];
-  const int* r = spill + off[i];
-  int* out = nlist + off[i] + i + 1;
-  for (long long e = threadIdx.x; e < m; e += 256) {
+  const long long m = count[at];
+  int* const r = spill + off[at];
+  int* const out = nlist + off[at] + at + 1;
+  for (long long p0 = 0; p0 < m; p0 += kSortPiece) {
+    const int len = (int)min((long long)kSortPiece, m - p0);
+    int size = 64;
+    while (size < len) size *= 2;
+    for (int e = threadIdx.x; e < size; e += kSortThreads) a[e] = e < len ? r[p0 + e] : INT_MAX;
+    for (int k = 2; k <= size; k *= 2)
+      for (int j = k / 2; j > 0; j /= 2) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < size / 2; t += kSortThreads) {
+          const int e = 2 * t - (t & (j - 1));  // e's bit j is clear
+          const int x = a[e], y = a[e + j];
+          if ((x > y) == ((e & k) == 0)) {
+            a[e] = y;
+            a[e + j] = x;
+          }
+        }
+      }
+    __syncthreads();
+    int* const to = m <= kSortPiece ? out : r + p0;
+    for (int e = threadIdx.x; e < len; e += kSortThreads) to[e] = a[e];
+    __syncthreads();
+  }
+  if (m <= kSortPiece) return;
+  for (long long e = threadIdx.x; e < m; e += kSortThreads) {
     const int v = r[e];
-    long long rank = 0;
-    for (long long k = 0; k < m; k++) rank += r[k] < v;
-    out[rank] = v;
+    const long long own = e / kSortPiece;
+    long long place = e - own * kSortPiece;
+    for (long long p = 0; p * kSortPiece < m; p++) {
+      if (p == own) continue;
+      const int* const s = r + p * kSortPiece;
+      int lo = 0;  // ids of the piece below v
+      for (int hi = (int)min((long long)kSortPiece, m - p * kSortPiece); lo < hi;) {
+        const int mid = (lo + hi) / 2;
+        if (s[mid] < v) lo = mid + 1;
+        else hi = mid;
+      }
+      place += lo;
+    }
+    out[place] = v;
   }
 }
 
@@ -505,7 +545,7 @@ int pdg_radius_search(int N, const double* x, double R, int nplanes, const doubl
   a.flushed = hbig ? spill.p + B : nullptr;
   hipLaunchKernelGGL(k_near<true>, nw, dim3(64 * kGroupWaves), 0, s, a);
   if (hbig)
-    hipLaunchKernelGGL(k_spilled_rows, pdg::group_grid(N), dim3(256), 0, s, N, count, off, spill.p,
+    hipLaunchKernelGGL(k_spilled_rows, pdg::group_grid(N), dim3(kSortThreads), 0, s, N, count, off, spill.p,
                        a.flushed, list.p);
   PDG_CK(hipGetLastError());
   PDG_CK(hipMemcpy(nlist, list.p, 4 * size, hipMemcpyDeviceToHost));
