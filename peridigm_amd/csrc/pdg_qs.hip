@@ -1844,9 +1844,10 @@ int pdg_qs_fallback_count(pdg_ctx* h, int* count) {
 
 // One product on a small mesh takes the untiled kernels: two, which read u
 // itself, against four (records, dilatation, its derivative, force) of which
-// the first two pay only where several products share a state. Device time
-// at 3,000 nodes 20 us against 21 and two more gaps, at 24,000 73 against 40.
-constexpr int kTangentTiledMin = 6000;
+// the first two pay only where several products share a state. Whole calls,
+// untiled and tiled: 2,000 nodes 59 and 64 us, 3,000 66 and 68, 4,000 71 and 72,
+// 5,000 76 and 72, 6,000 79 and 75, 8,000 89 and 82, 24,000 181 and 141.
+constexpr int kTangentTiledMin = 4500;
 
 int pdg_qs_tangent_apply(pdg_ctx* h, const double* u, const double* w, double* Kw) {
   Ctx* c = reinterpret_cast<Ctx*>(h);

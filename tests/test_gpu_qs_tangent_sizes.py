@@ -1,4 +1,4 @@
-"""One tangent product on both sides of the size (6,000 nodes) from which it
+"""One tangent product on both sides of the size (4,500 nodes) from which it
 takes the tiled passes, and the tiled passes themselves in every form they have:
 influence functions, linearized model, thermal strains, volumes that differ
 (1,024 threads a tile), 4, 8 and 16 lanes a node, damage, prescribed DOFs. Against
@@ -72,8 +72,8 @@ def test_tiled_product(influence, model, uniform, tile, lanes):
             assert np.array_equal(k0.ravel()[fixed], w.ravel()[fixed])
 
 
-@pytest.mark.parametrize("n,tiled", [((20, 20, 15), False), ((6001, 1, 1), True), ((25, 20, 12), False),
-                                     ((6000, 1, 1), False), ((47, 32, 4), True)])
+@pytest.mark.parametrize("n,tiled", [((20, 15, 15), False), ((4501, 1, 1), True), ((30, 15, 10), False),
+                                     ((4500, 1, 1), False), ((43, 35, 3), True)])
 def test_size_from_which_one_product_is_tiled(n, tiled):
     from peridigm_amd import Context
     from peridigm_amd import quasistatic as Q
@@ -81,7 +81,7 @@ def test_size_from_which_one_product_is_tiled(n, tiled):
     x, vol, nl, hz = _problem(n, True, rng)
     u = 1e-3 * x + 2e-7 * rng.standard_normal(x.shape)
     w = rng.standard_normal(x.shape)
-    assert (len(vol) > 6000) == tiled
+    assert (len(vol) > 4500) == tiled
     with Context(0) as ctx:
         ctx.set_topology(nl, len(vol))
         ctx.set_constants(x, vol, 130e9, 60e9, hz, 0, 0.0)
