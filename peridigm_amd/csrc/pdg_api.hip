@@ -433,11 +433,28 @@ int Ctx::upload_y(const double* y) {
 
 // Whether an explicit run of nsteps is resident: tiles of 32 nodes (meshes of
 // up to 16,384 nodes give at most 512, two to a CU) and enough steps to pay for
-// the copies of v and the mask and the cooperative launch (they add 45 to 60
-// us, and a step saves 3 to 5; at 16 steps both take the same).
+// the copies of v and the mask and the cooperative launch. Runs of 16, 20 and 50
+// steps, launched and resident: 980 nodes 192 and 188, 231 and 212, 516 and 378
+// us; 8,000 nodes 208 and 224, 248 and 256, 557 and 480; 16,000 nodes 257 and
+// 275, 309 and 313, 692 and 617: all gain from 24 steps on.
+constexpr int kResidentSteps = 24;
 bool Ctx::resident_run(int nsteps) const {
   return variant == 0 && ntiles > 0 && tile_nodes == 32 && tile_lanes() == 16 && !resident_off &&
-         !per_pass_timing && sc_t.empty() && nsteps >= 16;
+         !per_pass_timing && sc_t.empty() && nsteps >= kResidentSteps;
+}
+
+// Memory of the resident runs; false when it is refused.
+bool Ctx::resident_memory() {
+  if (d_xch) return true;
+  if (hipMalloc((void**)&d_xch, 8 * (13 * (size_t)N + 1)) != hipSuccess ||
+      hipMalloc((void**)&d_mask_old, std::max<size_t>(8 * (size_t)mw.back(), 64)) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFree(d_xch);
+    d_xch = d_mask_old = nullptr;
+    return false;
+  }
+  xch_tag = 0xffffffffu;  // clear the words
+  return true;
 }
 
 // Evaluations first..nsteps of an explicit run from the displacement in
@@ -452,18 +469,11 @@ int Ctx::run_resident(const VerletArgs& va, int first, int nsteps, double t0, bo
   if (ntiles > resident_max) return PDG_OK;
   const size_t n = (size_t)N, words = 13 * n + 1, vb = 24 * n, mb = 8 * (size_t)mw.back();
   int rc = PDG_OK;
-  if (!d_xch) {
-    if (hipMalloc((void**)&d_xch, 8 * words) != hipSuccess ||
-        hipMalloc((void**)&d_mask_old, std::max<size_t>(mb, 64)) != hipSuccess) {
-      (void)hipGetLastError();
-      (void)hipFree(d_xch);
-      d_xch = d_mask_old = nullptr;
-      resident_off = true;
-      return PDG_OK;
-    }
-    xch_tag = 0xffffffffu;  // clear the words
+  if (!resident_memory()) {
+    resident_off = true;
+    return PDG_OK;
   }
-  if (!rc && xch_tag > 0xffffffffu - (unsigned)nsteps - 2u) {
+  if (xch_tag > 0xffffffffu - (unsigned)nsteps - 2u) {
     rc = hip(hipMemsetAsync(d_xch, 0, 8 * words, stream), "clear exchange");
     xch_tag = 1;
   }
@@ -997,6 +1007,8 @@ int pdg_set_constants(pdg_ctx* h, const double* x, const double* vol, double K, 
   // take 0.1 to 0.3 ms per MB. Contexts for which that is more than 128 MB (1.2M
   // nodes) get theirs in the call that needs one, of the size it needs.
   if (state_stage_bytes(N) <= kStageAheadMax) (void)c->stage(state_stage_bytes(N));
+  // so too the memory of resident runs (1.7 MB at most; 50 to 200 us in the first)
+  if (c->resident_run(kResidentSteps)) (void)c->resident_memory();
   return PDG_OK;
 }
 

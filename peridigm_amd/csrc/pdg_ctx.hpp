@@ -134,6 +134,7 @@ struct Ctx {
   unsigned long long resident_wait = 20000000ull;  // 100 MHz ticks
   int run_route = 0;  // PDG_ROUTE_* of the last run
   bool resident_run(int nsteps) const;
+  bool resident_memory();
   int run_resident(const VerletArgs& va, int first, int nsteps, double t0, bool damage, bool* done);
   int* d_bcslot = nullptr;
   BcSlot* d_bcs = nullptr;
