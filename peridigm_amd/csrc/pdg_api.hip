@@ -603,12 +603,6 @@ int Ctx::queue_vec3(const double* in, double* ddst, int slot) {
   return rc;
 }
 
-int Ctx::upload_vec3(const double* in, double* ddst) {
-  int rc = hip(hipStreamSynchronize(stream), "sync");
-  if (!rc) rc = queue_vec3(in, ddst);
-  return rc ? rc : hip(hipStreamSynchronize(stream), "sync");
-}
-
 }  // namespace pdg
 
 extern "C" {

@@ -213,13 +213,12 @@ struct Ctx {
   void free_bond_maps();
   int upload_mask(const double* bd, bool check_symmetric);
   int download_mask(double* bd);
-  // node vectors (3n) between the host (reference order) and the device
-  // (internal order), reordered on the device; both wait for the copy
+  // node vectors (3n) between the device (internal order) and the host
+  // (reference order); the downloads wait for the copy, an upload does for large
+  // vectors, and small ones go through place `slot` of the staging buffer (the
+  // caller synchronises between uses of a place)
   int download_vec3(const double* dsrc, double* out);
   int download_scalar(const double* dsrc, double* out);  // n
-  int upload_vec3(const double* in, double* ddst);
-  // the same without the wait for small vectors, which go through place `slot`
-  // of the staging buffer (the caller synchronises between uses of a place)
   int queue_vec3(const double* in, double* ddst, int slot = 0);
 };
 
