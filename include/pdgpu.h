@@ -246,7 +246,9 @@ int pdg_set_per_pass_timing(pdg_ctx* ctx, int on);
  * run waits for another. A pdg_verlet_run of 24 or more steps on a small mesh
  * keeps every tile on the GPU for all of them; when a wait ends in vain, as it
  * soon does with 0, the run is repeated with two launches a step, as later
- * ones are until this is called again. The results are the same. */
+ * ones are until this is called again. A run that starts while another context
+ * of the process has one under way on the device, or has had within a tenth of
+ * a second, is launched too. The results are the same. */
 int pdg_set_resident_wait(pdg_ctx* ctx, double seconds);
 /* How the steps of the last pdg_verlet_run were taken. */
 #define PDG_ROUTE_LAUNCHED 0 /* launches for every step */

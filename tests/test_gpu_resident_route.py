@@ -67,3 +67,31 @@ def test_a_wait_in_vain_is_reported():
         ctx.set_resident_wait(0.2)
         ctx.verlet_run(40, p["dt"])
         assert ctx.last_run_route() == "resident"
+
+
+def test_runs_on_several_threads_are_launched():
+    """A run that another accompanies shares the GPU in launches; the fields are
+    those of the run alone, bit for bit."""
+    import threading
+    import time
+    (long, p), (other, _) = _context((50, 50, 4)), _context((50, 50, 4))
+    with long, other:
+        for c in (long, other):
+            c.upload_state()
+            c.verlet_run(40, p["dt"])
+            assert c.last_run_route() == "resident"
+        alone = other.download_state()
+        thread = threading.Thread(target=lambda: long.verlet_run(40000, p["dt"]))  # 0.3 s
+        thread.start()
+        time.sleep(0.05)
+        other.upload_state()
+        other.verlet_run(40, p["dt"])
+        route, under_way = other.last_run_route(), thread.is_alive()
+        together = other.download_state()
+        thread.join()
+        assert route == "launched" or not under_way
+        for k, v in alone.items():
+            assert np.array_equal(v, together[k]), k
+        time.sleep(0.2)  # runs that met are remembered for a tenth of a second
+        other.verlet_run(40, p["dt"])
+        assert other.last_run_route() == "resident"
