@@ -432,13 +432,13 @@ int Ctx::upload_y(const double* y) {
   return rc;
 }
 
-// Explicit runs under way on a device, from any context, and when two last met:
-// cooperative launches run one after the other, where the launches of several
-// runs share the GPU, and the two kinds side by side are slower than either. 300
-// steps of 10,000 nodes on 1, 2 and 4 threads: launched 4.0, 4.3 and 5.8 ms,
-// resident 2.5, 4.9 and 9.6, mixed (only the runs that start alone resident) 2.5,
-// 5.2 and 18. So runs are launched while others are under way and for a tenth of
-// a second after, which contexts on several threads keep renewing.
+// Explicit runs under way on a device, from any context, and when two last met.
+// Two resident runs could each hold a part of the GPU and wait for the rest, and
+// one takes places that the launches of other runs would share. 300 steps of
+// 10,000 nodes on 1, 2 and 4 threads: launched 4.0, 4.3 and 5.4 ms, resident one
+// after the other 2.5, 4.9 and 9.6. So runs are launched while others are under
+// way and for a tenth of a second after, which contexts on several threads keep
+// renewing (2.5, 4.0 and 5.2 ms).
 class RunUnderWay {
  public:
   explicit RunUnderWay(int device) : d_(devices_[device & (kDevices - 1)]) {
@@ -465,7 +465,7 @@ RunUnderWay::Device RunUnderWay::devices_[RunUnderWay::kDevices];
 
 // Whether an explicit run of nsteps is resident: tiles of 32 nodes (meshes of
 // up to 16,384 nodes give at most 512, two to a CU) and enough steps to pay for
-// the copies of v and the mask and the cooperative launch. Runs of 16, 20 and 50
+// the copies of v and the mask and a larger launch. Runs of 16, 20 and 50
 // steps, launched and resident: 980 nodes 192 and 188, 231 and 212, 516 and 378
 // us; 8,000 nodes 208 and 224, 248 and 256, 557 and 480; 16,000 nodes 257 and
 // 275, 309 and 313, 692 and 617: all gain from 24 steps on.

@@ -161,7 +161,7 @@ hipError_t launch_persistent(const BondArgs& a, const TileArgs& t, NodeRec* rec0
                              hipStream_t s);
 
 // Resident explicit run (pdg_tiles.hip): evaluations first..nsteps of a small
-// mesh with 32-node tiles and 16 lanes per node in one cooperative launch, the
+// mesh with 32-node tiles and 16 lanes per node in one launch, the
 // tiles exchanging displacements (x.u, 12n words, two buffers) and dilatation
 // terms (x.p, n words) numbered x.tag + evaluation; numbers must not repeat.
 // Reads u from rec, ends with it in rec_end. *x.stuck is set, and the state
@@ -173,7 +173,7 @@ struct ResidentArgs {
   int* stuck;
   unsigned long long wait;  // 100 MHz ticks a workgroup waits for another
 };
-// Most tiles that are resident together (0: no cooperative launch).
+// Most tiles that are resident together (0: not known).
 int resident_tiles(int influence, bool damage);
 hipError_t launch_resident(const BondArgs& a, const TileArgs& t, const ResidentArgs& x,
                            const NodeRec* rec, NodeRec* rec_end, float* theta, int* nbroken,
