@@ -69,7 +69,7 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* sh) {
   }
 }
 
-// Start of iteration cg->it + 1: decides whether the solve stops (cg_next;
+// Start of iteration cg->it + 1: decides whether the solve stops (cg_ends;
 // every workgroup alike, from the same sums in the same order) and gives the
 // new direction's beta. Workgroup 0 stores what the iteration's other kernels
 // and the host read; rz2 alternates by parity, so no workgroup reads what
@@ -82,13 +82,12 @@ __device__ __forceinline__ bool cg_start(const QsCgStart& s, double* sh, double&
   const int it = s.cg->it, brk = s.cg->brk;
   const double before = s.cg->rz2[(it + 1) & 1];
   block_sum2<T>(rz, rr, sh);
-  const int next = cg_next(it, s.cg->maxit, brk, rr, s.cg->bnorm, s.cg->tol);
-  const bool stop = next != CG_GO;
+  const bool stop = cg_ends(s.cg, it, brk, rr);
   beta = it > 0 ? rz / before : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (stop) {
       s.cg->done = 1;
-      cg_status_publish(s.status, next == CG_BREAKS_DOWN, it, rr);
+      cg_status_publish(s.status, cg_broke_down(s.cg, it, brk, rr), it, rr);
     } else {
       s.cg->rz = rz;
       s.cg->rz2[it & 1] = rz;

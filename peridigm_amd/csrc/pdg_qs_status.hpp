@@ -36,17 +36,21 @@ PDG_BOTH bool cg_status_ended(const QsCgStatus* s) {
   return __atomic_load_n(&s->done, __ATOMIC_ACQUIRE) != 0;
 }
 
-// What happens after `it` iterations with squared residual rr, `brk` set when
-// an iteration so far had p.Kp <= 0. The residual is looked at for it up to 8,
-// every fourth and the last one; a solve whose residual is found within the
-// tolerance there has converged, also when p.Kp came out as 0 because nothing
-// was left to correct (a NaN ends it as well). Otherwise a breakdown ends it.
-enum { CG_GO = 0, CG_ENDS = 1, CG_BREAKS_DOWN = 2 };
-PDG_BOTH int cg_next(int it, int maxit, int brk, double rr, double bnorm, double tol) {
-  const bool look = it <= 8 || it % 4 == 0 || it >= maxit;
-  if (look && !(sqrt(rr) / bnorm > tol)) return CG_ENDS;
-  if (brk) return CG_BREAKS_DOWN;
-  return it >= maxit ? CG_ENDS : CG_GO;
+// The end of a solve after `it` iterations with squared residual rr, `brk` set
+// when an iteration so far had p.Kp <= 0. The residual is looked at for it up to
+// 8, every fourth and the last one (a NaN ends the solve). A solve whose residual
+// is found within the tolerance there has converged, also when p.Kp came out as 0
+// because nothing was left to correct; otherwise a breakdown ends it.
+// S holds maxit, bnorm and tol.
+template <class S>
+PDG_BOTH bool cg_ends(const S* c, int it, int brk, double rr) {
+  const bool look = it <= 8 || it % 4 == 0 || it >= c->maxit;
+  return brk || it >= c->maxit || (look && !(sqrt(rr) / c->bnorm > c->tol));
+}
+template <class S>
+PDG_BOTH bool cg_broke_down(const S* c, int it, int brk, double rr) {
+  const bool look = it <= 8 || it % 4 == 0 || it >= c->maxit;
+  return brk && !(look && !(sqrt(rr) / c->bnorm > c->tol));
 }
 
 }  // namespace pdg

@@ -216,7 +216,9 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
   }
   const double Y0 = X0 + D0, Y1 = X1 + D1, Y2 = X2 + D2;
   const double yy = fma(Y2, Y2, fma(Y1, Y1, Y0 * Y0));
-  const double t = rsqrt64(z2 * yy);
+  // points that the deformation brings to one place: e is -|X| (g then is so
+  // large that g / (1 + g) is 1), where the force of such a bond has no direction
+  const double t = rsqrt64(PASS == QP_THETA ? fmax(z2 * yy, 1e-300) : z2 * yy);
   double g = z2 * t, ryy = g * t;
   // points that coincide in the reference configuration (rare: one branch of
   // the wave, no selects)
@@ -228,10 +230,7 @@ __device__ __forceinline__ void bond(const Rec<PASS>& me, const Rec<PASS>& nb, d
   }
   if (PASS == QP_THETA) {
     const double dd = fma(D2, X2 + Y2, fma(D1, X1 + Y1, D0 * (X0 + Y0)));
-    double ez = dd * g * rcp64(1.0 + g);  // e |X|
-    // points that the deformation brings to one place, where g has no value
-    if (__builtin_amdgcn_ballot_w64(z2 * yy == 0.0)) ez = z2 * yy == 0.0 ? -z2 : ez;
-    add1(wv, ez - thermal * z2);
+    add1(wv, dd * g * rcp64(1.0 + g) - thermal * z2);
   } else if (PASS == QP_DTHETA3) {
     const double f = ok ? wv * g : 0.0;
     s[0] = fma(f, Y0 * d0, s[0]);

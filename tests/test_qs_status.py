@@ -29,5 +29,5 @@ def test_status_is_handed_over_in_order(tmp_path):
 
 
 def test_end_of_a_solve_is_the_host_loops(tmp_path):
-    r = subprocess.run([_build(tmp_path, "test_cg_next")], stdout=subprocess.PIPE, text=True, timeout=60)
+    r = subprocess.run([_build(tmp_path, "test_cg_end")], stdout=subprocess.PIPE, text=True, timeout=60)
     assert r.returncode == 0 and " 0 wrong" in r.stdout, r.stdout
