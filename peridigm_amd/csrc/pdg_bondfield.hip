@@ -8,9 +8,12 @@
 // order (few, so atomics are cheap) and the host threads only widen bits to
 // doubles, front to back. Bound by host memory: the field is read once.
 // The whole field over PCIe, packed by a kernel, was bound by the copy from
-// pageable memory (drop-in force with a field: 640,000 nodes, 55M bonds, 16.1
-// ms, 980 nodes 354 us; host threads that gather single bonds through the map
-// 13.4 ms and 193 us; now 4.7 ms and 94 us).
+// pageable memory, host threads that gather single bonds through the map by
+// those. Drop-in force with a field, 640,000 nodes, 55M bonds, none, a fifth and
+// all of them broken: gather 13.4, 19.1, 15.9 ms, whole field 16.1 in each, now
+// 4.1, 5.2, 8.2; 980 nodes: 196, 307, 233 us, 355 (130 repeated), now 82, 92, 118.
+
+#include <emmintrin.h>
 
 #include <algorithm>
 #include <atomic>
@@ -29,21 +32,33 @@ inline unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 inline unsigned field_threads(long long nb) { return nb < (1ll << 18) ? 1 : nb < (1ll << 22) ? 4 : 8; }
 
 // Bits of m <= 64 field values; `wrong` is set by a value other than 0 and 1.
+// Whole words with SSE2, 21 ns each on one core whatever they hold (a value at a
+// time takes 64 to 75).
 inline unsigned long long pack_bits(const double* v, int m, bool& wrong) {
-  constexpr unsigned long long kOne = 0x3ff0000000000000ull;
-  unsigned long long x[64];
-  std::memcpy(x, v, 8 * (size_t)m);
-  unsigned long long any = 0ull;
-  for (int k = 0; k < m; k++) any |= x[k];
-  if ((any << 1) == 0ull) return 0ull;  // zeros of either sign: most of a field
   unsigned long long bits = 0ull;
-  bool bad = false;
-  for (int k = 0; k < m; k++) {
-    const bool one = x[k] == kOne;
-    bad |= !one && (x[k] << 1) != 0ull;
-    bits |= (unsigned long long)one << k;
+  if (m < 64) {
+    for (int k = 0; k < m; k++) {
+      wrong |= v[k] != 0.0 && v[k] != 1.0;
+      bits |= (unsigned long long)(v[k] == 1.0) << k;
+    }
+    return bits;
   }
-  wrong |= bad;
+  const __m128d one = _mm_set1_pd(1.0), zero = _mm_setzero_pd();
+  __m128d ok = _mm_cmpeq_pd(zero, zero);
+  for (int k = 0; k < 64; k += 16) {
+    __m128i c[8];  // two comparisons each, 16 values
+    for (int q = 0; q < 8; q++) {
+      const __m128d x = _mm_loadu_pd(v + k + 2 * q), o = _mm_cmpeq_pd(x, one);
+      ok = _mm_and_pd(ok, _mm_or_pd(o, _mm_cmpeq_pd(x, zero)));
+      c[q] = _mm_castpd_si128(o);
+    }
+    // narrowed to a byte each
+    for (int q = 0; q < 8; q += 2) c[q] = _mm_packs_epi32(c[q], c[q + 1]);
+    c[0] = _mm_packs_epi32(c[0], c[2]);
+    c[4] = _mm_packs_epi32(c[4], c[6]);
+    bits |= (unsigned long long)(unsigned)_mm_movemask_epi8(_mm_packs_epi16(c[0], c[4])) << k;
+  }
+  wrong |= _mm_movemask_pd(ok) != 3;
   return bits;
 }
 
@@ -99,23 +114,48 @@ __global__ __launch_bounds__(256) void k_rows_from_bits(int n, const int* __rest
 }
 
 // *bad is set by a broken bond whose other end is intact: a wave per node, which
-// looks the node up in the other end's row for each of its broken bonds.
+// looks the node up in the other end's row for each of its broken bonds, four
+// rows in flight.
 __global__ __launch_bounds__(256) void k_check_ends(int n, const int* __restrict__ row,
                                                     const int* __restrict__ mw,
                                                     const int* __restrict__ col,
                                                     const unsigned long long* __restrict__ words,
                                                     int* __restrict__ bad) {
+  constexpr int U = 4;
   const long long t = wave_index();
   if (t >= n) return;
   const int i = (int)t, lane = threadIdx.x & 63;
   const int rs = row[i], deg = row[i + 1] - rs, w0 = mw[i];
   bool wrong = false;
   for (int k0 = 0; k0 < deg; k0 += 64) {
-    for (unsigned long long m = words[w0 + (k0 >> 6)]; m != 0ull; m &= m - 1ull) {
-      const int j = col[rs + k0 + __ffsll(m) - 1];
-      const int rj = row[j], dj = row[j + 1] - rj;
-      for (int q = lane; q < dj; q += 64)
-        if (col[rj + q] == i) wrong = wrong || !((words[mw[j] + (q >> 6)] >> (q & 63)) & 1ull);
+    unsigned long long m = words[w0 + (k0 >> 6)];
+    if (m == 0ull) continue;
+    int rj = 0, dj = 0, wj = 0;  // lane k's bond's other end
+    if (k0 + lane < deg) {
+      const int j = col[rs + k0 + lane];
+      rj = row[j];
+      dj = row[j + 1] - rj;
+      wj = mw[j];
+    }
+    while (m != 0ull) {
+      int d[U], w[U], c0[U], c1[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int b = m != 0ull ? __ffsll(m) - 1 : 0;  // past the last: no row
+        const int r = __shfl(rj, b);
+        d[u] = m != 0ull ? __shfl(dj, b) : 0;
+        w[u] = __shfl(wj, b);
+        m &= m - 1ull;
+        c0[u] = lane < d[u] ? col[r + lane] : -1;
+        c1[u] = lane + 64 < d[u] ? col[r + lane + 64] : -1;
+        for (int q = lane + 128; q < d[u]; q += 64)
+          if (col[r + q] == i) wrong = wrong || !((words[w[u] + (q >> 6)] >> (q & 63)) & 1ull);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (c0[u] == i) wrong = wrong || !((words[w[u]] >> lane) & 1ull);
+        if (c1[u] == i) wrong = wrong || !((words[w[u] + 1] >> lane) & 1ull);
+      }
     }
   }
   if (__ballot(wrong) && lane == 0) *bad = 1;
