@@ -243,7 +243,7 @@ int pdg_last_timing(const pdg_ctx* ctx, double* totalMs, double* pass1Ms, double
 int pdg_set_per_pass_timing(pdg_ctx* ctx, int on);
 
 /* Longest time (s, 0 to 10; 0.2 by default) that a tile of a resident explicit
- * run waits for another. A pdg_verlet_run of 24 or more steps on a small mesh
+ * run waits for another. A pdg_verlet_run of 16 or more steps on a small mesh
  * keeps every tile on the GPU for all of them; when a wait ends in vain, as it
  * soon does with 0, the run is repeated with two launches a step, as later
  * ones are until this is called again. A run that starts while another context

@@ -465,11 +465,11 @@ RunUnderWay::Device RunUnderWay::devices_[RunUnderWay::kDevices];
 
 // Whether an explicit run of nsteps is resident: tiles of 32 nodes (meshes of
 // up to 16,384 nodes give at most 512, two to a CU) and enough steps to pay for
-// the copies of v and the mask and a larger launch. Runs of 16, 20 and 50
-// steps, launched and resident: 980 nodes 192 and 188, 231 and 212, 516 and 378
-// us; 8,000 nodes 208 and 224, 248 and 256, 557 and 480; 16,000 nodes 257 and
-// 275, 309 and 313, 692 and 617: all gain from 24 steps on.
-constexpr int kResidentSteps = 24;
+// the copies of v and the mask and a larger launch. 16 steps, launched and
+// resident: 980 nodes 185 and 148 us, 8,000 196 and 178, 16,000 236 and 224; with
+// damage, whose mask is copied, 194 and 178, 207 and 211, 251 and 253 (20 steps:
+// 247 and 243, 303 and 296).
+constexpr int kResidentSteps = 16;
 bool Ctx::resident_run(int nsteps) const {
   return variant == 0 && ntiles > 0 && tile_nodes == 32 && tile_lanes() == 16 && !resident_off &&
          !per_pass_timing && sc_t.empty() && nsteps >= kResidentSteps;

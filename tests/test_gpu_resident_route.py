@@ -42,7 +42,7 @@ def test_few_steps_large_meshes_and_other_kernels_are_launched():
     ctx, p = _context((40, 40, 4))
     with ctx:
         ctx.upload_state()
-        for steps, route in ((23, "launched"), (24, "resident")):
+        for steps, route in ((15, "launched"), (16, "resident")):
             ctx.verlet_run(steps, p["dt"])
             assert ctx.last_run_route() == route
         ctx.set_critical_stretch_function([0.0, 1.0], [5e-4, 5e-4])
