@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "pdg_contact_dev.hpp"
@@ -639,18 +640,31 @@ int pdg_contact_compute_force(pdg_ctx* h, double dt, const double* y, const doub
   if (!rc && !S->dfc) rc = c->hip(hipMalloc((void**)&S->dfc, 24 * (size_t)N), "alloc contact f");
   if (!rc && !S->dhead) rc = c->hip(hipMalloc((void**)&S->dhead, 8 * (size_t)N), "alloc contact heads");
   if (!rc) rc = grow(c, S->dlist, S->dcap, p, "alloc contact list");
-  if (!rc) rc = c->hip(hipMemcpyAsync(c->d_y, y, 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d y");
-  if (!rc) rc = c->hip(hipMemcpyAsync(S->dv, v, 24 * (size_t)N, hipMemcpyHostToDevice, s), "h2d v");
-  if (!rc) rc = c->hip(hipMemcpyAsync(S->dhead, head.data(), 8 * (size_t)N, hipMemcpyHostToDevice, s), "h2d heads");
-  if (!rc) rc = c->hip(hipMemcpyAsync(S->dlist, contactList, 4 * (size_t)p, hipMemcpyHostToDevice, s), "h2d list");
-  if (rc) return rc;
+  // small meshes: everything through the staging buffer as set-up made it, but
+  // for a list that does not fit (14 contacts a node)
+  const size_t vb = 24 * (size_t)N, hb = 8 * (size_t)N, lb = 4 * (size_t)p;
+  char* st = !rc && N <= kHostOrderMax ? c->stage(2 * vb + hb) : nullptr;
+  auto up = [&](void* dev, const void* host, size_t bytes, size_t at, const char* what) {
+    if (rc) return;
+    const void* from = st && at + bytes <= c->h_stage_bytes ? std::memcpy(st + at, host, bytes) : host;
+    rc = c->hip(hipMemcpyAsync(dev, from, bytes, hipMemcpyHostToDevice, s), what);
+  };
+  up(c->d_y, y, vb, 0, "h2d y");
+  up(S->dv, v, vb, vb, "h2d v");
+  up(S->dhead, head.data(), hb, 2 * vb, "h2d heads");
+  up(S->dlist, contactList, lb, 2 * vb + hb, "h2d list");
+  if (rc) {
+    (void)hipStreamSynchronize(s);
+    return rc;
+  }
   hipLaunchKernelGGL(k_fill_f64, dim3(blocks_for(3ll * N)), dim3(256), 0, s, 3ll * N, S->dfc);
   hipLaunchKernelGGL(k_contact_scatter, dim3(blocks_for(N)), dim3(256), 0, s, N, c->d_y, S->dv,
                      S->vref, S->dhead, S->dlist, pair_params(c), S->dfc);
   rc = c->hip(hipGetLastError(), "contact force");
-  if (!rc) rc = c->hip(hipMemcpyAsync(contactForce, S->dfc, 24 * (size_t)N, hipMemcpyDeviceToHost, s), "d2h f");
-  if (!rc) rc = c->hip(hipStreamSynchronize(s), "sync");
-  if (rc) return rc;
+  if (!rc) rc = c->hip(hipMemcpyAsync(st ? (void*)st : contactForce, S->dfc, vb, hipMemcpyDeviceToHost, s), "d2h f");
+  const int rc2 = c->hip(hipStreamSynchronize(s), "sync");
+  if (rc || rc2) return rc ? rc : rc2;
+  if (st) std::memcpy(contactForce, st, vb);
   for (long long q = 0; q < 3ll * N; q++)
     if (!std::isfinite(contactForce[q]))
       return c->fail(PDG_E_NONFINITE, "NaN returned by contact force evaluation");
