@@ -1126,18 +1126,34 @@ int pdg_compute_damage(pdg_ctx* h, const double* y, const double* bdN, double* b
   if (!rc) rc = c->hip(hipMemsetAsync(c->d_near, 0, 8, s), "zero near");
   if (!rc) rc = c->hip(c->pass1(c->d_rec[c->cur], c->d_nbroken, true, nearCritical != nullptr), "pass1");
   unsigned long long near = 0;
+  // small meshes: damage and count come behind the bond bits' place in the
+  // staging buffer, under the one wait for those
+  const size_t at = (8 * (((size_t)c->B + 63) / 64) + 4 * (size_t)N + 63) & ~(size_t)63;
+  const size_t db = 8 * (size_t)N;
+  char* st = N > 0 && N <= kHostOrderMax && !rc ? c->stage(at + db + 8) : nullptr;
+  if (st) {
+    st += at;
+    hipLaunchKernelGGL(k_damage_out, blocks_of(N), dim3(256), 0, s, N, c->d_nbroken, c->d_row,
+                       c->d_perm, 0, c->d_y);
+    rc = c->hip(hipMemcpyAsync(st, c->d_y, db, hipMemcpyDeviceToHost, s), "d2h damage");
+  }
   if (!rc && nearCritical)
-    rc = c->hip(hipMemcpyAsync(&near, c->d_near, 8, hipMemcpyDeviceToHost, s), "d2h near");
+    rc = c->hip(hipMemcpyAsync(st ? st + db : (char*)&near, c->d_near, 8, hipMemcpyDeviceToHost, s), "d2h near");
   if (!rc) rc = c->download_mask(bdNP1);
   if (rc) {
     (void)hipStreamSynchronize(s);  // the copy of y reads the caller's array
     return rc;
   }
-  HostOut o(c, 8 * (size_t)N, true);
+  if (st) {
+    std::memcpy(damage, st, db);
+    if (nearCritical) std::memcpy(nearCritical, st + db, 8);
+    return PDG_OK;
+  }
+  HostOut o(c, db, true);
   if (N > 0)
     hipLaunchKernelGGL(k_damage_out, blocks_of(N), dim3(256), 0, s, N, c->d_nbroken, c->d_row,
                        c->d_perm, 0, o.next());
-  rc = o.add(damage, c->d_y, 8 * (size_t)N);
+  rc = o.add(damage, c->d_y, db);
   if (!rc) rc = o.finish();
   if (rc) return rc;
   if (nearCritical) *nearCritical = (long long)near;
