@@ -1393,6 +1393,7 @@ int pdg_verlet_run_persistent(pdg_ctx* h, int nsteps, double dt, double t0, int 
   if (tl != 4 && tl != 8 && tl != 16)
     return c->fail(PDG_E_UNSUPPORTED, "persistent run uses 4, 8 or 16 lanes per node");
   if (!initialEval && nsteps == 0) return PDG_OK;
+  const RunUnderWay under_way(c->device);
   (void)hipSetDevice(c->device);
   hipStream_t s = c->stream;
   VerletArgs va{};

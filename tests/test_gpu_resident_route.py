@@ -95,3 +95,27 @@ def test_runs_on_several_threads_are_launched():
         time.sleep(0.2)  # runs that met are remembered for a tenth of a second
         other.verlet_run(40, p["dt"])
         assert other.last_run_route() == "resident"
+
+
+def test_a_run_beside_a_persistent_one_is_launched():
+    """A persistent run's workgroups wait for each other without a limit, so no
+    resident run takes places from it."""
+    import threading
+    import time
+    (long, p), (other, _) = _context((50, 50, 4)), _context((50, 50, 4))
+    with long, other:
+        for c in (long, other):
+            c.upload_state()
+        other.verlet_run(40, p["dt"])
+        alone = other.download_state()
+        thread = threading.Thread(target=lambda: long.verlet_run_persistent(20000, p["dt"]))
+        thread.start()
+        time.sleep(0.05)
+        other.upload_state()
+        other.verlet_run(40, p["dt"])
+        route, under_way = other.last_run_route(), thread.is_alive()
+        together = other.download_state()
+        thread.join()
+        assert route == "launched" or not under_way
+        for k, v in alone.items():
+            assert np.array_equal(v, together[k]), k
