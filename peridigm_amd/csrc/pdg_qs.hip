@@ -802,7 +802,13 @@ __global__ __launch_bounds__(RB) void k_coarse_columns(CoarseGrid G, int nc, int
 
 // M = P^T K P, symmetrised, from the probes' rows of R: entry (target t,
 // source g) stands in the row of g's colour when t and g are within reach on
-// every axis, and is 0 otherwise
+// every axis, and is 0 otherwise. The diagonal is raised by kCoarseShift of
+// itself: on small meshes some functions depend on others (grid points with few
+// nodes), and the pivots of rounding noise that no cut separates from true ones
+// would make the inverse indefinite. On 1,087 random meshes of 8 to 700 nodes
+// PCG fails on 3 % without a shift and on none with 1e-10 to 1e-14; 1e-12 of the
+// diagonal changes the inverse no more than rounding does.
+constexpr double kCoarseShift = 1e-12;
 struct ProbeColours {
   int reach, stride, d[3];  // colours per axis
 };
@@ -820,8 +826,9 @@ __global__ __launch_bounds__(RB) void k_coarse_matrix(CoarseGrid G, ProbeColours
   auto row = [&](const int g[3], int k) {
     return (((g[2] % pc.stride) * pc.d[1] + g[1] % pc.stride) * pc.d[0] + g[0] % pc.stride) * 3 + k;
   };
-  M[e] = near ? 0.5 * (R[(size_t)row(a, i - 3 * pi) * nc + j] + R[(size_t)row(b, j - 3 * pj) * nc + i])
-              : 0.0;
+  const double m =
+      near ? 0.5 * (R[(size_t)row(a, i - 3 * pi) * nc + j] + R[(size_t)row(b, j - 3 * pj) * nc + i]) : 0.0;
+  M[e] = i == j ? m * (1.0 + kCoarseShift) : m;
 }
 
 __global__ __launch_bounds__(RB) void k_coarse_dmax(int nc, const double* __restrict__ M, double* dmax) {
@@ -836,84 +843,84 @@ __global__ __launch_bounds__(RB) void k_coarse_dmax(int nc, const double* __rest
   }
 }
 
-// One step of the block Gauss-Jordan inversion of a symmetric positive matrix
-// (no pivoting needed): rows and columns p0 .. p0 + kGj - 1 leave. With the
-// pivot block's inverse P, out = in - in(:, K) P in(K, :) outside the pivots'
-// rows and columns, P in(K, :) in the rows, -in(:, K) P in the columns and P
-// where they meet. Every block inverts the pivot block itself and takes a tile
-// of the matrix; steps alternate between two buffers. A pivot at or below
-// 1e-12 of the largest diagonal entry of the start (or a NaN) is dropped: its
-// row and column become 0. Latency of the pivots' serial chain bounds it: 30
-// steps of 13 us at 480 functions, where factorising on the host took 30 ms.
+// One step of the Gauss-Jordan inversion of a symmetric positive matrix (no
+// pivoting needed): the pivots p0 .. p0 + kGj - 1 leave one by one. Every block
+// takes a tile of the matrix with the pivots' rows and columns beside it, all in
+// registers: a thread has 3 x 3 entries of the tile, 3 of the rows, 3 of the
+// columns and one of the pivot block, and only the leaving row and column pass
+// through LDS (in turn through two buffers, so a pivot takes one barrier). Steps
+// alternate between two matrices. Taking the pivot block's inverse times rows
+// and columns instead, one product a step, loses digits with the block's
+// condition number and made inverses of small meshes indefinite. A pivot at or
+// below 1e-10 of the largest diagonal entry of the start (or a NaN) is dropped:
+// its row and column become 0. Latency of the pivots' serial chain bounds it:
+// 30 steps of 12.5 us at 480 functions, where factorising on the host took 30 ms.
 constexpr int kGj = 16;
-constexpr int kGjTile = 48;
+constexpr int kGjSide = 3;  // entries a thread along each side of the tile
+constexpr int kGjTile = kGj * kGjSide;
+static_assert(RB == kGj * kGj, "a thread per entry of the pivot block");
 __global__ __launch_bounds__(RB) void k_gj_step(int nc, int p0, const double* __restrict__ in,
                                                 const double* __restrict__ dmax,
                                                 double* __restrict__ out) {
-  __shared__ double P[kGj][kGj + 1];
-  __shared__ double rows[kGj][kGjTile + 1];   // in(K, tile columns), then P times it
-  __shared__ double cols[kGjTile][kGj + 1];   // in(tile rows, K)
+  __shared__ double lead[2][2][kGj + kGjTile];  // pivot row, column: of the block, of the tile
   const int b = min(kGj, nc - p0);
+  const int ty = threadIdx.x / kGj, tx = threadIdx.x % kGj;
   const int i0 = blockIdx.y * kGjTile, j0 = blockIdx.x * kGjTile;
-  const int pi = threadIdx.x / kGj, pj = threadIdx.x % kGj;
-  const double cut = 1e-12 * *dmax;
-  P[pi][pj] = pi < b && pj < b ? in[(size_t)(p0 + pi) * nc + p0 + pj] : 0.0;
-  for (int e = threadIdx.x; e < kGj * kGjTile; e += RB) {
-    const int k = e / kGjTile, j = e - kGjTile * k;
-    rows[k][j] = k < b && j0 + j < nc ? in[(size_t)(p0 + k) * nc + j0 + j] : 0.0;
-    const int r = e / kGj, q = e - kGj * r;
-    cols[r][q] = q < b && i0 + r < nc ? in[(size_t)(i0 + r) * nc + p0 + q] : 0.0;
+  const double cut = 1e-10 * *dmax;
+  auto entry = [&](int i, int j) { return i < nc && j < nc ? in[(size_t)i * nc + j] : 0.0; };
+  double v[kGjSide][kGjSide], row[kGjSide], col[kGjSide];
+  double pv = entry(p0 + ty, p0 + tx);
+#pragma unroll
+  for (int a = 0; a < kGjSide; a++) {
+    row[a] = entry(p0 + ty, j0 + tx + kGj * a);
+    col[a] = entry(i0 + ty + kGj * a, p0 + tx);
+#pragma unroll
+    for (int c = 0; c < kGjSide; c++) v[a][c] = entry(i0 + ty + kGj * a, j0 + tx + kGj * c);
   }
-  __syncthreads();
-  unsigned dropped = 0u;
   for (int p = 0; p < b; p++) {
-    const double d = P[p][p], rp = P[p][pj], cp = P[pi][p], v = P[pi][pj];
-    __syncthreads();
-    if (!(d > cut)) {
-      dropped |= 1u << p;
-      continue;
-    }
-    const double id = 1.0 / d;
-    P[pi][pj] = pi == p ? (pj == p ? id : rp * id) : (pj == p ? -cp * id : v - cp * (rp * id));
-    __syncthreads();
-  }
-  if (dropped >> pi & 1u || dropped >> pj & 1u) P[pi][pj] = 0.0;
-  for (int e = threadIdx.x; e < kGj * kGjTile; e += RB) {
-    const int k = e / kGjTile, r = e / kGj, q = e - kGj * r;
-    if (dropped >> k & 1u) rows[k][e - kGjTile * k] = 0.0;
-    if (dropped >> q & 1u) cols[r][q] = 0.0;
-  }
-  __syncthreads();
-  double t[kGj * kGjTile / RB];
+    double* R = lead[p & 1][0];
+    double* C = lead[p & 1][1];
+    if (ty == p) {
+      R[tx] = pv;
 #pragma unroll
-  for (int m = 0; m < kGj * kGjTile / RB; m++) {
-    const int e = threadIdx.x + m * RB, k = e / kGjTile, j = e - kGjTile * k;
-    const int jk = j0 + j - p0;  // pivot column
-    double v = 0.0;
-    for (int q = 0; q < kGj; q++) v += P[k][q] * rows[q][j];
-    t[m] = jk >= 0 && jk < b ? P[k][jk] : v;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int m = 0; m < kGj * kGjTile / RB; m++) {
-    const int e = threadIdx.x + m * RB, k = e / kGjTile;
-    rows[k][e - kGjTile * k] = t[m];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < kGjTile * kGjTile; e += RB) {
-    const int r = e / kGjTile, j = e - kGjTile * r;
-    if (i0 + r >= nc || j0 + j >= nc) continue;
-    const int ik = i0 + r - p0, jk = j0 + j - p0;
-    double v;
-    if (ik >= 0 && ik < b) {
-      v = rows[ik][j];
-    } else {
-      double s = 0.0;
-      for (int q = 0; q < kGj; q++) s += cols[r][q] * rows[q][j];
-      v = (jk >= 0 && jk < b ? 0.0 : in[(size_t)(i0 + r) * nc + j0 + j]) - s;
+      for (int c = 0; c < kGjSide; c++) R[kGj * (c + 1) + tx] = row[c];
     }
-    out[(size_t)(i0 + r) * nc + j0 + j] = v;
+    if (tx == p) {
+      C[ty] = pv;
+#pragma unroll
+      for (int a = 0; a < kGjSide; a++) C[kGj * (a + 1) + ty] = col[a];
+    }
+    __syncthreads();
+    const double d = R[p];
+    const bool kept = d > cut;
+    const double id = kept ? 1.0 / d : 0.0;
+    const double cp = kept ? C[ty] : 0.0, rp = kept ? R[tx] * id : 0.0;
+    pv = ty == p ? (tx == p ? id : rp) : (tx == p ? -cp * id : pv - cp * rp);
+    double rs[kGjSide];
+#pragma unroll
+    for (int c = 0; c < kGjSide; c++) {
+      rs[c] = kept ? R[kGj * (c + 1) + tx] * id : 0.0;
+      row[c] = ty == p ? rs[c] : row[c] - cp * rs[c];
+    }
+#pragma unroll
+    for (int a = 0; a < kGjSide; a++) {
+      const double cs = kept ? C[kGj * (a + 1) + ty] : 0.0;
+      col[a] = tx == p ? -cs * id : col[a] - cs * rp;
+#pragma unroll
+      for (int c = 0; c < kGjSide; c++) v[a][c] -= cs * rs[c];
+    }
   }
+  // p0 and the tile's corner are multiples of kGj: where a thread's entry of the
+  // tile lies in the pivots' rows or columns, it is the one the thread has of them
+#pragma unroll
+  for (int a = 0; a < kGjSide; a++)
+#pragma unroll
+    for (int c = 0; c < kGjSide; c++) {
+      const int i = i0 + ty + kGj * a, j = j0 + tx + kGj * c;
+      if (i >= nc || j >= nc) continue;
+      const bool ip = i0 + kGj * a == p0, jp = j0 + kGj * c == p0;
+      out[(size_t)i * nc + j] = ip ? (jp ? pv : row[c]) : (jp ? col[a] : v[a][c]);
+    }
 }
 
 // Probe vector of the coarse set-up: the sum of the coarse functions (g, k0),
